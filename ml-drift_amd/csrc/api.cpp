@@ -811,6 +811,9 @@ int mldhip_op_launch(mldhip_op* op, void* stream_ptr) {
       if (GetTuning().force_generic <= 0 && FcW8RingSupported(a)) {
         e = LaunchFcW8Ring(a, stream, &op->last_kernel);
       } else
+      if (GetTuning().force_generic <= 0 && FcW8RingOSupported(a)) {
+        e = LaunchFcW8RingO(a, stream, &op->last_kernel);
+      } else
       // packed groups: the matrix-core GEMM with one launch plane per matrix where it serves the shape
       if (GetTuning().force_generic <= 0 && FcW4MfmaPackedSupported(a)) {
         e = LaunchFcW4Mfma(a, stream, &op->last_kernel);

@@ -1,8 +1,9 @@
-// FullyConnected over ringed uint8 weights whose ring runs over the input channels
-// (ConvRuntimeCheckDesc::ring_i_offset_index over a kOSpatialIOGroupI4O4 buffer,
-// common/kernels/fully_connected.cc:424-441, 676-706), 1..4 tokens per row: the matmul of a decode
-// step with a cache as its weights (attention probabilities x value cache), where the cache is
-// long and the output narrow.
+// FullyConnected over ringed uint8 weights: the matmuls of a decode step with a cache as their weights.
+//
+// The ring over the output channels (query x key cache) is fc_w8_ring_o_kernel, at the end.  The ring over
+// the input channels (ConvRuntimeCheckDesc::ring_i_offset_index over a kOSpatialIOGroupI4O4 buffer,
+// common/kernels/fully_connected.cc:424-441, 676-706: attention probabilities x value cache) has a long
+// window and a narrow output.
 //
 // The reference's kernel walks the source slices and gathers, for source channel c, the word of
 // ring channel (c + offset) % ring_size: four 4-byte reads per slice and output slice.  Here the
@@ -13,6 +14,8 @@
 // source channels 4 w - offset % 4 + {0, 1, 2, 3}; those outside [0, channels multiplied) count as
 // zero.  That needs ring_size % 4 == 0.
 //
+// Two kernels walk it: fc_w8_ring_i_column_kernel (one launch; below) and, for the longest windows at up to 4
+// tokens, fc_w8_ring_i_kernel, described here.
 // Work-group = 256 threads = LS lanes along the output slices x 256 / LS rows in flight, four
 // rows per thread and pass; the window is split across blockIdx.x, the slices (in chunks of LS)
 // across blockIdx.y, the dst rows of a launch with batched weights across blockIdx.z.  Every
@@ -244,6 +247,361 @@ __global__ __launch_bounds__(256) void fc_w8_ring_finish_kernel(RingParams p) {
   }
 }
 
+// ------------------------------------------------------------------------------------------
+// The same walk in one launch: a work-group owns one output slice (4 channels) and MT tokens and walks
+// the whole window by itself, so there are no partial sums and no second kernel.
+//
+// What bounds it: the dependent launch (1.55 us), then how fast a CU takes pieces that lie in lines of their
+// own: a wave's load of 16-byte blocks a whole row (Ns x 16 bytes) apart touches 64 lines, its load of the
+// activations of two tokens 32.  So the slice below a row's own comes from the neighbouring lane instead
+// of memory and two tokens travel in one load (8 tokens x 8192 positions x 256 channels: 6.4 -> 5.8 us;
+// 74.7 us on the unspecialised kernel that served more than 4 tokens; one token 10.4 us with the window
+// split, 5.0 here).  Neighbouring slices share the lines of the weights, so runs of 8 slices are
+// dealt to one XCD, whose L2 fetches a line once.  A thread owns window rows tid, tid + THREADS, ...; the
+// loads of two rows are in flight per thread, at 1024 threads a cache of 8192 positions at once.
+// ------------------------------------------------------------------------------------------
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ half2_t AsHalf2(uint32_t v) { return __builtin_bit_cast(half2_t, v); }
+
+// Sum over the 64 lanes of four values (lane l ends with value 2 * (l / 32) + (l / 16) % 2) by register
+// exchanges that halve what a lane carries, then data-parallel moves over the 16 lanes that are left.
+__device__ __forceinline__ float AddRow16(float v) {
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+  const uint32_t up = __builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x104 /* row_shl:4 */, 0xf, 0x5, false);
+  const uint32_t both = __builtin_amdgcn_update_dpp(up, __float_as_uint(v), 0x114 /* row_shr:4 */, 0xf, 0xA, false);
+  v += __uint_as_float(both);
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x4E /* quad_perm:[2,3,0,1] */, 0xf, 0xf, false));
+  v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0xB1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, false));
+  return v;
+}
+__device__ __forceinline__ float SwapAdd32(float a, float b) {
+  const u32x2 e = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(e[0]) + __uint_as_float(e[1]);
+}
+__device__ __forceinline__ float SwapAdd16(float a, float b) {
+  const u32x2 e = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(e[0]) + __uint_as_float(e[1]);
+}
+
+// One slice of MT neighbouring tokens as it lies in memory: MT x 4 values in 32-bit words.
+typedef uint32_t u32x4_word __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_word __attribute__((ext_vector_type(2), aligned(4)));
+template <typename T> constexpr int kWordsPerToken = (int)sizeof(T);
+template <typename T, int MT>
+__device__ __forceinline__ void LoadTokens(const T* p, size_t i, uint32_t (&v)[MT * kWordsPerToken<T>]) {
+  if constexpr (MT * kWordsPerToken<T> == 2) {
+    const u32x2_word r = *reinterpret_cast<const u32x2_word*>(p + i);
+    v[0] = r[0];
+    v[1] = r[1];
+  } else {
+#pragma unroll
+    for (int q = 0; q < MT * kWordsPerToken<T> / 4; ++q) {
+      const u32x4_word r = reinterpret_cast<const u32x4_word*>(p + i)[q];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[q * 4 + j] = r[j];
+    }
+  }
+}
+
+// acc[c] += sum_i a_i (u_ic - 128) over one block (word i = ring channel i, byte c = output channel c) and
+// asum += sum_i a_i, where a_i is value 4 - sh + i of the eight values {lo, hi}.
+__device__ __forceinline__ void MultiplyRow(const float (&u)[4][4], const uint32_t* lo, const uint32_t* hi, int sh, float (&acc)[4],
+                                            float& asum) {
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = __uint_as_float(lo[i]);
+    v[4 + i] = __uint_as_float(hi[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = sh == 0 ? v[4 + i] : (sh == 1 ? v[3 + i] : (sh == 2 ? v[2 + i] : v[1 + i]));
+    asum += a;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = fmaf(a, u[i][c], acc[c]);
+  }
+}
+__device__ __forceinline__ void MultiplyRow(const half2_t (&u)[2][4], const uint32_t* lo, const uint32_t* hi, int sh, float (&acc)[4],
+                                            float& asum) {
+  // the words {y0, y1, y2} that hold halfs 4 - sh .. 7 - sh, shifted by one half where sh is odd
+  const uint32_t y0 = sh == 0 ? hi[0] : (sh <= 2 ? lo[1] : lo[0]);
+  const uint32_t y1 = sh == 0 ? hi[1] : (sh <= 2 ? hi[0] : lo[1]);
+  const uint32_t y2 = sh <= 2 ? hi[1] : hi[0];
+  const uint32_t by = (sh & 1) * 16;
+  const half2_t a01 = AsHalf2(__builtin_amdgcn_alignbit(y1, y0, by)), a23 = AsHalf2(__builtin_amdgcn_alignbit(y2, y1, by));
+  const half2_t one = {(_Float16)1.0f, (_Float16)1.0f};
+  asum = __builtin_amdgcn_fdot2(a23, one, __builtin_amdgcn_fdot2(a01, one, asum, false), false);
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    acc[c] = __builtin_amdgcn_fdot2(a23, u[1][c], __builtin_amdgcn_fdot2(a01, u[0][c], acc[c], false), false);
+}
+// u - 128 of one block, in the form the multiply takes (fp16 tensors: pairs of input channels; exact)
+__device__ __forceinline__ void Centre(const u32x4& blk, float (&u)[4][4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) u[i][c] = (float)((blk[i] >> (8 * c)) & 0xFFu) - 128.0f;
+}
+__device__ __forceinline__ void Centre(const u32x4& blk, half2_t (&u)[2][4]) {
+  const half2_t off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const uint32_t sel = 0x0c000c00u | (uint32_t)c | ((uint32_t)(4 + c) << 16);
+      u[j][c] = AsHalf2(__builtin_amdgcn_perm(blk[2 * j + 1], blk[2 * j], sel) | 0x64006400u) + off;
+    }
+}
+template <typename T> struct RingTypes;
+template <> struct RingTypes<float> { typedef float centred[4][4]; };
+template <> struct RingTypes<__half> { typedef half2_t centred[2][4]; };
+
+// scale * (sum - zp * sum(a)) of output channel n, in the destination type, plus the bias
+template <typename T>
+__device__ __forceinline__ void RingWrite(const RingParams& p, int wb, int n, size_t o, float sum, float asum) {
+  float s = p.scalar_scale, z = p.has_zero_point ? p.scalar_zero_point : 0.0f;
+  if (p.scale_kind == kScaleLinear) {
+    s = LoadF(static_cast<const T*>(p.scale), (size_t)wb * p.ns * 4 + n);
+    if (p.zero_point) z = LoadF(static_cast<const T*>(p.zero_point), (size_t)wb * p.ns * 4 + n);
+  }
+  const float r = s * fmaf(-z, asum, sum);
+  T* dst = static_cast<T*>(p.dst);
+  const T* bias = static_cast<const T*>(p.bias);
+  if constexpr (std::is_same<T, float>::value) {
+    dst[o] = bias ? r + bias[n] : r;
+  } else {
+    __half h = __float2half_rn(r);
+    if (bias) h = __hadd(h, bias[n]);
+    dst[o] = h;
+  }
+}
+
+// (MT <= p.m: the last work-group along the tokens starts at token m - MT, and only it writes what is left)
+template <typename T, int MT, int THREADS>
+__global__ __launch_bounds__(THREADS) void fc_w8_ring_i_column_kernel(RingParams p) {
+  constexpr int U = 2, WAVES = THREADS / 64, NW = kWordsPerToken<T>;
+  __shared__ float red[WAVES][MT][5];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // runs of 8 slices on one XCD (work-groups go round-robin to the 8 of them)
+  const int j = blockIdx.x >> 3;
+  const int ds = (j >> 3) * 64 + (blockIdx.x & 7) * 8 + (j & 7);
+  if (ds >= RingDstEndSlice(p)) return;  // (the whole work-group)
+  const int row = blockIdx.z, tok_first = blockIdx.y * MT, tok0 = min(tok_first, p.m - MT);
+  int wb = p.batch_ids ? p.batch_ids[row] : 0;
+  wb = min(max(wb, 0), p.weights_batch - 1);
+  const size_t act_stride = (size_t)p.src_rows * p.m;
+  const T* act = static_cast<const T*>(p.act) + ((size_t)min(row, p.src_rows - 1) * p.m + tok0) * 4;
+  const int off = ((p.params[p.ring_index] % p.ring_size) + p.ring_size) % p.ring_size;
+  const int sh = off & 3, row0 = off >> 2;
+  const int ks_end = RingSrcEndSlices(p);
+  const int nrows = ks_end > 0 ? (sh + ks_end * 4 + 3) >> 2 : 0;  // window rows touched (at most ring_rows + 1)
+  const u32x4* wcol = p.weights + (size_t)wb * p.ring_rows * p.ns + ds;
+
+  float acc[MT][4], asum[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    asum[t] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[t][c] = 0.0f;
+  }
+  for (int base = wave * 64; base < nrows; base += THREADS * U) {  // (the same for the whole wave: lanes exchange below)
+    u32x4 blk[U];
+    uint32_t first[U][MT * NW], hi[U][MT * NW];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int w_wave = base + u * THREADS, w = w_wave + lane;
+      int kb = row0 + min(w, nrows - 1);
+      if (kb >= p.ring_rows) kb -= p.ring_rows;
+      blk[u] = wcol[(size_t)kb * p.ns];
+      // slice w holds source channels 4 w .. 4 w + 3; the row needs 4 w - sh .. 4 w - sh + 3, the rest of which is
+      // the slice of the lane below (lane 0: a load of its own, one line for the wave)
+      LoadTokens<T, MT>(act, (size_t)min(w, ks_end - 1) * act_stride * 4, hi[u]);
+      LoadTokens<T, MT>(act, (size_t)max(min(w_wave, ks_end) - 1, 0) * act_stride * 4, first[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int w = base + u * THREADS + lane;
+      const bool lo_ok = w >= 1 && w - 1 < ks_end, hi_ok = w < ks_end;  // (a row past the window has neither)
+      typename RingTypes<T>::centred cu;
+      Centre(blk[u], cu);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        uint32_t lo[NW], hv[NW];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+          const uint32_t below = __builtin_amdgcn_update_dpp(first[u][t * NW + i], hi[u][t * NW + i], 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+          lo[i] = lo_ok ? below : 0u;
+          hv[i] = hi_ok ? hi[u][t * NW + i] : 0u;
+        }
+        MultiplyRow(cu, lo, hv, sh, acc[t], asum[t]);
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const float v = AddRow16(SwapAdd16(SwapAdd32(acc[t][0], acc[t][2]), SwapAdd32(acc[t][1], acc[t][3])));
+    const float s32 = SwapAdd32(asum[t], asum[t]);
+    const float a = AddRow16(SwapAdd16(s32, s32));
+    if ((lane & 15) == 0) red[wave][t][2 * (lane >> 5) + ((lane >> 4) & 1)] = v;
+    if (lane == 0) red[wave][t][4] = a;
+  }
+  __syncthreads();
+  if (tid >= MT * 4) return;
+  const int t = tid >> 2, c = tid & 3;
+  if (tok0 + t < tok_first) return;
+  float sum = 0.0f, as = 0.0f;
+#pragma unroll
+  for (int q = 0; q < WAVES; ++q) {
+    sum += red[q][t][c];
+    as += red[q][t][4];
+  }
+  RingWrite<T>(p, wb, ds * 4 + c, ((size_t)ds * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as);
+}
+
+// ------------------------------------------------------------------------------------------
+// Ring over the output channels of a kOSpatialIOGroupO4I4 buffer (GetRingedOAddresses,
+// fully_connected.cc:411-422, 680-697): query x key cache.  Word (ks, o) of the buffer holds input
+// channels 4 ks .. 4 ks + 3 of ring channel o, one per byte; dst channel c is ring channel
+// (c + offset) % ring_size.  A thread owns one dst slice, whose four words lie one after the other
+// (one 16-byte load from a 4-byte boundary), except in the slice that the end of the ring cuts.
+//
+// Work-group = 16 slices x 16 K lanes (K-slices k, k + 16, ...; 4 of them in a wave), MT tokens.  What bounds
+// it is latency: the ring's start has to be read before the first weight address is known.  So the
+// activations, which do not depend on it, go to LDS meanwhile (the 16 lanes of a K-slice read the same
+// 8 or 16 bytes per token), the weights of four K-slices per thread are then in flight at once, and the
+// sums meet by register exchanges inside a wave and through 4 KB of LDS across the waves.  8 tokens x 8192
+// positions x 256 channels, 2.1 MB: 4.0 us (5.3 with the activations from memory and the whole reduction
+// through LDS, 10.1 us on the unspecialised kernel that served it).
+// ------------------------------------------------------------------------------------------
+__device__ __forceinline__ void CentreO(const u32x4& w, float (&u)[4][4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) u[i][c] = (float)((w[c] >> (8 * i)) & 0xFFu) - 128.0f;
+}
+__device__ __forceinline__ void CentreO(const u32x4& w, half2_t (&u)[2][4]) {
+  const half2_t off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    u[0][c] = AsHalf2(__builtin_amdgcn_perm(0u, w[c], 0x0c010c00u) | 0x64006400u) + off;
+    u[1][c] = AsHalf2(__builtin_amdgcn_perm(0u, w[c], 0x0c030c02u) | 0x64006400u) + off;
+  }
+}
+
+template <typename T, int MT>
+__global__ __launch_bounds__(256) void fc_w8_ring_o_kernel(RingParams p) {
+  constexpr int KL = 16, U = 4, NW = kWordsPerToken<T>, CHUNK = 256;  // K-slices staged at a time
+  __shared__ uint32_t acts[CHUNK][MT * NW];
+  __shared__ float red[4][MT][64], reda[4][MT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sl = tid & 15, kl = tid >> 4;
+  const int row = blockIdx.z, tok_first = blockIdx.y * MT, tok0 = min(tok_first, p.m - MT);
+  const size_t act_stride = (size_t)p.src_rows * p.m;
+  const T* act = static_cast<const T*>(p.act) + ((size_t)min(row, p.src_rows - 1) * p.m + tok0) * 4;
+  const int ks_end = RingSrcEndSlices(p), ns_end = RingDstEndSlice(p);
+  if ((int)blockIdx.x * 16 >= ns_end) return;  // (the whole work-group)
+  const int ds = min((int)blockIdx.x * 16 + sl, p.ns - 1);
+  int wb = p.batch_ids ? p.batch_ids[row] : 0;
+  wb = min(max(wb, 0), p.weights_batch - 1);
+  const int off = ((p.params[p.ring_index] % p.ring_size) + p.ring_size) % p.ring_size;
+  const uint32_t* w32 = reinterpret_cast<const uint32_t*>(p.weights) + (size_t)wb * p.ks * p.ring_size;
+  const int o0 = (int)(((long)ds * 4 + off) % p.ring_size);
+  const bool whole = o0 + 4 <= p.ring_size;
+  float acc[MT][4], asum[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    asum[t] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[t][c] = 0.0f;
+  }
+  for (int chunk = 0; chunk < ks_end; chunk += CHUNK) {
+    const int count = min(ks_end - chunk, CHUNK);
+    if (chunk > 0) __syncthreads();  // (everybody is done with the chunk before)
+    for (int i = tid; i < count; i += 256) {
+      uint32_t v[MT * NW];
+      LoadTokens<T, MT>(act, (size_t)(chunk + i) * act_stride * 4, v);
+#pragma unroll
+      for (int q = 0; q < MT * NW; ++q) acts[i][q] = v[q];
+    }
+    bool staged = false;
+    for (int k0 = kl; k0 < count || !staged; k0 += KL * U) {
+      u32x4 w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t* base = w32 + (size_t)(chunk + min(k0 + u * KL, count - 1)) * p.ring_size;
+        if (whole) {
+          w[u] = *reinterpret_cast<const u32x4_word*>(base + o0);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) w[u][c] = base[o0 + c < p.ring_size ? o0 + c : o0 + c - p.ring_size];
+        }
+      }
+      if (!staged) __syncthreads();  // (once per chunk and thread: the first pass of every thread)
+      staged = true;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u * KL;
+        if (k < count) {
+          typename RingTypes<T>::centred cu;
+          CentreO(w[u], cu);
+          uint32_t v[MT * NW];
+#pragma unroll
+          for (int q = 0; q < MT * NW; ++q) v[q] = acts[k][q];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) MultiplyRow(cu, v + t * NW, v + t * NW, 0, acc[t], asum[t]);
+        }
+      }
+    }
+  }
+  // lane = slice + 16 x K lane of the wave; two exchanges leave it with channel 2 * (lane / 32) + (lane / 16) % 2
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    red[wave][t][lane] = SwapAdd16(SwapAdd32(acc[t][0], acc[t][2]), SwapAdd32(acc[t][1], acc[t][3]));
+    const float s32 = SwapAdd32(asum[t], asum[t]);
+    const float a = SwapAdd16(s32, s32);
+    if (lane == 0) reda[wave][t] = a;
+  }
+  __syncthreads();
+  if (tid >= MT * 64) return;
+  const int c = tid & 3, t = (tid >> 2) % MT, s = (tid >> 2) / MT;
+  const int slice = blockIdx.x * 16 + s;
+  if (slice >= ns_end || tok0 + t < tok_first) return;
+  float sum = 0.0f, as = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    sum += red[q][t][c * 16 + s];
+    as += reda[q][t];
+  }
+  RingWrite<T>(p, wb, slice * 4 + c, ((size_t)slice * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as);
+}
+
+template <typename T, int MT>
+hipError_t LaunchColumnT(const RingParams& p, bool small, hipStream_t stream) {
+  const dim3 grid(DivUp(p.ns, 64) * 64, DivUp(p.m, MT), p.rows);
+  if (small)
+    hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, 256>), grid, dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, 1024>), grid, dim3(1024), 0, stream, p);
+  return hipGetLastError();
+}
+template <typename T>
+hipError_t LaunchColumn(const RingParams& p, int slots, bool small, hipStream_t stream) {
+  if (slots == 4) return LaunchColumnT<T, 4>(p, small, stream);
+  if (slots == 2) return LaunchColumnT<T, 2>(p, small, stream);
+  return LaunchColumnT<T, 1>(p, small, stream);
+}
+template <typename T>
+hipError_t LaunchRingO(const RingParams& p, int slots, hipStream_t stream) {
+  const dim3 grid(DivUp(p.ns, 16), DivUp(p.m, slots), p.rows), block(256);
+  if (slots == 4)
+    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, 4>), grid, block, 0, stream, p);
+  else if (slots == 2)
+    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, 2>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, 1>), grid, block, 0, stream, p);
+  return hipGetLastError();
+}
+
 template <typename T, int LS>
 hipError_t LaunchRingT(const RingParams& p, bool dst_f16, hipStream_t stream) {
   const dim3 grid(p.parts, DivUp(p.ns, LS), p.rows);
@@ -270,24 +628,44 @@ size_t FcW8RingWorkspaceFloats(int max_tokens, int o) {
   return std::min((size_t)kRingMaxParts * rows_tokens * (n_pad + 4), (size_t)8 << 20);
 }
 
+bool RingShapeOk(const FcArgs& a) {
+  if (a.params == nullptr || a.weight_bits != 8 || a.ring_size < 4 || a.ring_size % 4 != 0) return false;
+  if (a.packed_params_offset >= 0 || a.scale_kind == kScaleBlock || a.act_f16 != a.dst_f16) return false;
+  return a.m >= 1 && a.rows >= 1 && a.rows <= 65535;
+}
+// Window rows up to which one work-group per slice walks the window by itself.  Its time grows with the rows
+// (3.6 us at 2048, 6.4 at 4096, 12.1 at 8192 for 256 channels and one token), that of the split window hardly
+// does (7.4, 7.8, 8.8 us), but the split window reads 32 activations per row and thread at 4 tokens (15.7,
+// 16.4, 17.4 us against 4.2, 7.0, 11.8) and serves no more than 4.
+int ColumnMaxRows(int tokens) { return tokens == 1 ? 4097 : 8193; }
+bool ColumnPreferred(const FcArgs& a) {
+  return a.m > 4 || std::min(DivUp(a.k, 4), a.ring_size / 4) + 1 <= ColumnMaxRows(a.m);
+}
+bool PartsSupported(const FcArgs& a) {
+  if (a.m > 4 || (long)a.rows * a.m > 16 || a.partial == nullptr) return false;
+  // at least one part must fit the workspace
+  return (size_t)a.rows * 4 * ((size_t)DivUp(a.n, 4) * 4 + 4) <= a.partial_floats;
+}
+
 bool FcW8RingSupported(const FcArgs& a) {
-  if (a.params == nullptr || a.ring_i_index < 0 || a.ring_o_index >= 0) return false;
-  if (a.weight_bits != 8 || a.ring_size < 4 || a.ring_size % 4 != 0) return false;
-  if (a.packed_params_offset >= 0 || a.scale_kind == kScaleBlock) return false;
-  if (a.act_f16 != a.dst_f16) return false;
-  if (a.m < 1 || a.m > 4 || a.rows < 1 || (long)a.rows * a.m > 16) return false;
+  if (!RingShapeOk(a) || a.ring_i_index < 0 || a.ring_o_index >= 0) return false;
   if (a.k > a.ring_size) return false;  // (the window stays within one turn of the ring)
   const int ns = DivUp(a.n, 4);
   if (EffectiveGroup(a.group, ns) != ns) return false;
   const int w_ks = DivUp(a.weights_k > 0 ? a.weights_k : a.k, 4);
   if (a.ring_size > 4 * w_ks || (a.weights_batch > 1 && a.ring_size != 4 * w_ks)) return false;
-  if (a.partial == nullptr) return false;
-  // at least one part must fit the workspace
-  return (size_t)a.rows * 4 * ((size_t)ns * 4 + 4) <= a.partial_floats;
+  return a.m <= 64;
 }
 
-hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kernel_name) {
-  if (!FcW8RingSupported(a)) return hipErrorInvalidValue;
+// Ring over the output channels.  Below 64 KB of weights a launch costs what a launch costs on either
+// kernel, and the unspecialised one keeps those.
+bool FcW8RingOSupported(const FcArgs& a) {
+  if (!RingShapeOk(a) || a.ring_o_index < 0 || a.ring_i_index >= 0) return false;
+  if (a.m > 64) return false;
+  return (size_t)DivUp(a.k, 4) * DivUp(a.n, 4) * 16 >= 65536;
+}
+
+static RingParams MakeRingParams(const FcArgs& a) {
   RingParams p;
   p.act = a.act;
   p.weights = reinterpret_cast<const u32x4*>(a.weights);
@@ -303,7 +681,7 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
   p.ns = DivUp(a.n, 4);
   p.ring_size = a.ring_size;
   p.ring_rows = a.ring_size / 4;
-  p.ring_index = a.ring_i_index;
+  p.ring_index = a.ring_i_index >= 0 ? a.ring_i_index : a.ring_o_index;
   p.src_end_ch_index = a.src_end_ch_index;
   p.dst_end_ch_index = a.dst_end_ch_index;
   p.k_channels = a.k;
@@ -314,19 +692,46 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
   p.has_zero_point = a.has_zero_point ? 1 : 0;
   p.scalar_scale = a.scalar_scale;
   p.scalar_zero_point = a.scalar_zero_point;
+  p.parts = 1;
+  return p;
+}
+
+hipError_t LaunchFcW8RingO(const FcArgs& a, hipStream_t stream, const char** kernel_name) {
+  if (!FcW8RingOSupported(a)) return hipErrorInvalidValue;
+  const RingParams p = MakeRingParams(a);
+  if (kernel_name) *kernel_name = "fc_w8_ring_o_kernel";
+  // token slots: as above (4 tokens x 8192 positions x 256 channels: 3.6 us with two, 3.9 with four; 8 tokens x 16384 x
+  // 128: 4.2 against 4.1)
+  int slots = (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 4) >= 512 ? 4 : 2;
+  while (slots > p.m) slots /= 2;
+  return a.act_f16 ? LaunchRingO<__half>(p, slots, stream) : LaunchRingO<float>(p, slots, stream);
+}
+
+hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kernel_name) {
+  if (!FcW8RingSupported(a)) return hipErrorInvalidValue;
+  RingParams p = MakeRingParams(a);
+  if (kernel_name) *kernel_name = "fc_w8_ring_i_kernel";
+  const int window = std::min(p.ks + 1, p.ring_rows + 1);
+  if (ColumnPreferred(a) || !PartsSupported(a)) {
+    // token slots of a work-group: two, so that the slices of a narrow cache (64 for a head of 256) occupy the chip
+    // (8 tokens x 8192 positions x 256 channels: 5.8 us, 8.6 with one slot, 6.2 with four); four where they do anyway
+    // (4096 positions x 512 channels: 5.25 against 5.8 us)
+    int slots = (long)p.ns * p.rows * DivUp(p.m, 4) >= 256 ? 4 : 2;
+    while (slots > p.m) slots /= 2;
+    const bool small = window <= 512;
+    return a.act_f16 ? LaunchColumn<__half>(p, slots, small, stream) : LaunchColumn<float>(p, slots, small, stream);
+  }
   // lanes along the output slices: a power of two up to 64; parts: about 32 KB of weights each, at
   // most what the workspace holds
   int ls = 16;
   while (ls < 64 && ls < p.ns) ls *= 2;
   const int rows_in_flight = kRingThreads / ls * RingUnroll(p.m == 1 ? 1 : (p.m == 2 ? 2 : 4));
-  const int window = std::min(p.ks + 1, p.ring_rows + 1);
   const size_t bytes = (size_t)window * p.ns * 16;
   int parts = (int)std::min<size_t>(kRingMaxParts, std::max<size_t>(1, bytes / 32768));
   parts = std::min(parts, std::max(1, DivUp(window, rows_in_flight)));
   const size_t per_part = (size_t)a.rows * 4 * ((size_t)p.ns * 4 + 4);
   parts = (int)std::min<size_t>(parts, a.partial_floats / per_part);
   p.parts = std::max(parts, 1);
-  if (kernel_name) *kernel_name = "fc_w8_ring_i_kernel";
   if (a.act_f16) {
     if (ls == 16) return LaunchRingT<__half, 16>(p, a.dst_f16, stream);
     if (ls == 32) return LaunchRingT<__half, 32>(p, a.dst_f16, stream);

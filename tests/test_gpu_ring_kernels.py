@@ -1,0 +1,113 @@
+"""GPU parity of the two kernels that serve ringed uint8 weights at decode sizes (fc_w8_ring_i_column_kernel:
+ring over the input channels, any window that one work-group walks; fc_w8_ring_o_kernel: ring over the output
+channels from 64 KB of weights on), against the float64 product over the rolled weights: more tokens than the
+partial-sum kernel takes, window lengths around a pass of the work-group, slices that the end of the ring cuts,
+widths that fill no group of 8 slices, batched weights, bounds, fp16 activations below the normal range."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+import mldhip as M
+import workloads as W
+from test_oracle_ring import make, rolled_product
+
+
+def run(axis, src_c, dst_c, ring, tokens, offsets, f16, batch=1, seed=1, src_end=None, dst_end=None, tiny=False):
+    import torch
+    td, mt = (np.float16, M.FLOAT16) if f16 else (np.float32, M.FLOAT32)
+    q, _, scale, zp, bias = make(seed, src_c, dst_c, ring, axis, batch)
+    rng = np.random.default_rng(seed)
+    act = rng.uniform(-1, 1, size=(batch * tokens, src_c))
+    if tiny:  # probabilities of a long softmax: most of them are fp16 subnormals
+        act = np.exp(rng.normal(-12.0, 3.0, size=act.shape))
+        bias = bias * 0.0
+    act, scale, bias = (v.astype(td).astype(np.float32) for v in (act, scale, bias))
+    w_o, w_i = q.shape[0], q.shape[3]
+    desc = M.make_desc(M.UINT8, M.LAYOUT_I4O4 if axis == "i" else M.LAYOUT_O4I4, (w_o + 3) // 4)
+    packed = M.rearrange_int8_as_uint8(q, desc)
+    ns = (dst_c + 3) // 4
+    pad = lambda v: np.tile(np.pad(v, (0, ns * 4 - dst_c)).astype(td), batch)
+    kw = {"ring_%s_offset_index" % axis: 1, "ring_size": ring, ("src" if axis == "i" else "dst") + "_channels": src_c if axis == "i" else dst_c}
+    if batch > 1:
+        kw["weights_batch"] = batch
+    if src_end is not None:
+        kw["src_end_ch_index"] = 2
+    if dst_end is not None:
+        kw["dst_end_ch_index"] = 3
+    op = M.fc_create(M.PRECISION_F32_F16 if f16 else M.PRECISION_F32, mt, mt, w_o, w_i, desc, has_bias=True, has_zero_point_tensor=True,
+                     scale_shape=(dst_c, 1), max_tokens=batch * tokens, **kw)
+    params = np.array([-1, 0, src_end or 0, dst_end or 0], np.int32)
+    d_params = torch.from_numpy(params).cuda()
+    cuda = lambda v: torch.from_numpy(np.ascontiguousarray(v)).cuda()
+    srcs = [cuda(W.to_slices(act).astype(td))]
+    if batch > 1:
+        srcs.append(torch.arange(batch, dtype=torch.int32, device="cuda"))
+    bias_t = np.pad(bias, (0, ns * 4 - dst_c)).astype(td)
+    srcs += [cuda(packed), cuda(pad(scale)), cuda(pad(zp)), cuda(bias_t), d_params]
+    out = torch.zeros((ns, batch * tokens, 4), dtype=torch.float16 if f16 else torch.float32, device="cuda")
+    op.bind(srcs, [out])
+    op.set_shape(1, batch, tokens) if batch > 1 else op.set_shape(1, 1, tokens)
+    for off in offsets:
+        params[1] = off
+        d_params.copy_(torch.from_numpy(params))
+        out.fill_(7.0)
+        print("ring kernel", axis, src_c, dst_c, ring, "tokens", tokens, "batch", batch, "offset", off, "f16", f16, src_end, dst_end, flush=True)
+        op.launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert op.kernel_name == "fc_w8_ring_%s_kernel" % axis, op.kernel_name
+        got = W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
+        n_written = dst_c if dst_end is None else min((dst_end + 31) // 32 * 32, ns * 4)
+        if n_written < dst_c:
+            assert np.all(got[:, n_written:] == 7.0)
+        active = None if src_end is None else (min(src_end, src_c) + 3) // 4 * 4
+        for b in range(batch):
+            for t in range(tokens):
+                a = act[b * tokens + t]
+                exact = rolled_product(q, a, scale, zp, bias, axis, ring, off, b, src_c, dst_c, active=active)[:n_written]
+                # fp32 sums of src_c products, in any order: (src_c + 8) roundings of the sum of magnitudes at worst; fp16
+                # results are rounded twice (result, bias)
+                mag = np.abs(a).sum() * 131.0 * scale[:n_written].astype(np.float64)
+                tol = 2.0 ** -24 * (src_c + 8) * mag + (2.0 ** -10 * (np.abs(exact) + np.abs(bias[:n_written])) + 2.0 ** -24 if f16 else
+                                                        2.0 ** -22 * np.abs(exact))
+                assert np.all(np.abs(got[b * tokens + t][:n_written] - exact) <= tol), (b, t, off)
+
+
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("tokens", [1, 2, 3, 5, 8, 16])
+def test_ring_i_token_counts(f16, tokens):
+    run("i", 300, 72, 1024, tokens, [0, 1, 722, 1023, -6], f16, seed=tokens)
+
+
+@pytest.mark.parametrize("src_c,ring", [(1021, 1024), (2044, 2052), (2048, 2048), (4096, 4104), (4097, 8192), (8190, 8192), (12, 16)])
+def test_ring_i_windows(src_c, ring):
+    """Windows around one and two rows per thread at both work-group sizes, full turns of the ring, a short one."""
+    run("i", src_c, 40, ring, 6, [0, 3, ring - 2], True, seed=src_c)
+
+
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("tokens", [1, 2, 4, 7, 9])
+def test_ring_o_token_counts(f16, tokens):
+    run("o", 68, 1000, 1024, tokens, [0, 1, 722, 1023, -6], f16, seed=tokens)
+
+
+@pytest.mark.parametrize("src_c,dst_c,ring", [(256, 2048, 2048), (64, 4093, 4096), (30, 8192, 8192), (260, 515, 1000)])
+def test_ring_o_shapes(src_c, dst_c, ring):
+    run("o", src_c, dst_c, ring, 8, [0, 5, ring - 1], True, seed=dst_c)
+
+
+def test_ring_batches_and_bounds():
+    run("i", 512, 320, 512, 5, [0, 258], True, batch=3, src_end=301, dst_end=70)
+    run("o", 128, 600, 1024, 6, [3, 900], True, batch=2, src_end=61, dst_end=200)
+    run("o", 128, 600, 1024, 3, [3, 900], False, batch=2)
+
+
+def test_ring_i_subnormal_probabilities():
+    run("i", 8192, 64, 8192, 8, [0, 4099], True, tiny=True)
+
+
+@pytest.mark.parametrize("src_c,tokens,f16", [(16384, 1, True), (16389, 1, True), (20000, 1, False), (32769, 3, True), (33000, 2, True),
+                                              (33000, 5, True)])
+def test_ring_i_windows_around_the_split(src_c, tokens, f16):
+    """Window lengths where the launcher passes from one work-group per slice to the split window (up to 4 tokens)."""
+    run("i", src_c, 24, (src_c + 7) // 4 * 4, tokens, [0, 2, src_c // 2 + 1], f16, seed=src_c)
