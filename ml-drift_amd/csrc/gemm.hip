@@ -88,8 +88,8 @@ struct GemmParams {
   int xcd_m;        // fp16 path: the 8 XCDs form an xcd_m x (8 / xcd_m) grid over (token tiles, channel tiles)
   int gate_activation;  // gated fp16 launch: MLDHIP_GATE_*
   int dual;             // fp16 path: a work-group owns two neighbouring channel tiles
-  // fp16 path, packed groups (ConvRuntimeCheckDesc::PackedGroups): blockIdx.z = weight matrix g of
-  // pg_groups; its tokens are min(pg_params[pg_offset + g], pg_max) many from token
+  // fp16 path, packed groups (ConvRuntimeCheckDesc::PackedGroups): the tokens of weight matrix g of
+  // pg_groups are min(pg_params[pg_offset + g], pg_max) many from token
   // pg_params[pg_offset + pg_groups + g] of the one source row.  pg_groups = 0: not set.
   const int32_t* pg_params;
   int pg_offset, pg_groups, pg_max;
@@ -531,9 +531,9 @@ __global__ __launch_bounds__(kI8Threads) void conv_int8_mfma_kernel(GemmParams p
 // differences are at the kernel).
 //
 // Work-group = WAVES waves on one output tile of 128 channels x (FM*32) tokens; the waves split
-// K WAVES ways and add their fp32 tiles through LDS at the end (fixed order).  Compiled shapes:
-// 32 and 64 tokens with 8 waves (two per SIMD), 128 tokens with 4 waves (one per SIMD, its 256
-// accumulators in the AGPR half of the register file).  Inside a wave every
+// K WAVES ways and add their fp32 tiles through LDS at the end (fixed order; a single wave stores its sums
+// itself).  Compiled shapes: 32 and 64 tokens with 8 waves (two per SIMD), 128 tokens with 4 waves (one
+// per SIMD, its 256 accumulators in the AGPR half of the register file); packed groups: 1, 2, 4 and 8 waves.  Inside a wave every
 // MFMA operand comes straight from global memory in the layout the instruction wants:
 //  - A (weights): the 32 "rows" of MFMA number t are the output channels 4*i + t, i = lane % 32,
 //    so a lane's two 8-byte blocks (K-slices 2q, 2q+1 of slice i; 8 input channels x 4 output
@@ -598,8 +598,19 @@ __device__ __forceinline__ W4Segment PickSegment(const GemmParams& p, int index)
   return sg;
 }
 
+// Sum over lanes 0 .. l of the wave.
+__device__ __forceinline__ int WaveInclusiveSum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111 /* row_shr:1 */, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112 /* row_shr:2 */, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114 /* row_shr:4 */, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118 /* row_shr:8 */, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142 /* row_bcast:15 */, 0xa, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143 /* row_bcast:31 */, 0xc, 0xf, false);
+  return v;
+}
+
 template <int WB, int FM, int U, int WAVES, bool ZP, bool PAIR, bool MULTI, int MODE = kModePlain>
-__global__ __launch_bounds__(WAVES * 64) void fc_w4_mfma_direct_kernel(GemmParams p) {
+__global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct_kernel(GemmParams p) {
   constexpr bool GATED = MODE == kModeGated, DUAL = MODE == kModeDual;
   static_assert(WB == 4 || WB == 8, "uint4 or uint8 weights");
   static_assert(!GATED || (!ZP && !MULTI), "the gated pair is symmetric and is the whole launch");
@@ -608,10 +619,10 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_mfma_direct_kernel(GemmParam
   typedef typename std::conditional<WB == 8, u32x4, u32x2>::type wblk_t;
   constexpr int BN = 128;
   constexpr int BM = FM * 32;
-  static_assert(WAVES == 4 || WAVES == 8, "the reduction's LDS buffers are sized for 4 or 8 waves");
-  // K reduction buffers: [phase parity][copy][register within the phase][lane], 128 KB
-  constexpr int RPH = WAVES == 4 ? 16 : 8;  // accumulator registers (x 4 MFMAs) per phase
-  __shared__ float4 red[2][WAVES][RPH][64];
+  static_assert(WAVES == 1 || WAVES == 2 || WAVES == 4 || WAVES == 8, "the reduction's LDS buffers are sized for up to 8 waves");
+  // K reduction buffers: [phase parity][copy][register within the phase][lane], up to 128 KB
+  constexpr int RPH = WAVES == 4 && FM == 4 ? 16 : 8;  // accumulator registers (x 4 MFMAs) per phase
+  __shared__ float4 red[WAVES == 1 ? 1 : 2][WAVES][WAVES == 1 ? 1 : RPH][64];
 
   // One batch of scalar loads for what the prologue reads.  (Left alone, the compiler fetches
   // every argument where it is first used: seven scalar round trips, one behind the other, in
@@ -636,24 +647,47 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_mfma_direct_kernel(GemmParam
   const int tiles_n = DUAL ? (tiles_n_all + 1) / 2 : tiles_n_all;        // channel tiles of the grid
   // Packed groups: this work-group's matrix and the run of tokens it multiplies (else: all tokens).
   int m_lo = 0, m_hi = p.m, pg_e = 0;
-  const int tiles_m = p.geo_tiles_m;  // (packed groups: the tiles of the largest group)
-  if (p.pg_groups > 0) {
-    pg_e = blockIdx.z;
-    const int size = min(p.pg_params[p.pg_offset + pg_e], p.pg_max);
-    const int off = p.pg_params[p.pg_offset + p.pg_groups + pg_e];
-    if (off < 0) return;
-    m_lo = off;
-    m_hi = min(off + size, p.m);
-  }
+  const int tiles_m = p.geo_tiles_m;  // (packed groups: the most token tiles that the groups can have together)
   const int xcd = blockIdx.x % 8, local = blockIdx.x / 8;
   const int xm = p.xcd_m;
   const int rect_m = p.geo_rect_m, rect_n = p.geo_rect_n;
   // local / rect_m by the host's reciprocal (exact: local and rect_m are below 2^16)
   const int local_n = rect_m == 1 ? local : (int)__umulhi((uint32_t)local, p.geo_rect_m_magic);
   const int local_m = local - local_n * rect_m;
-  const int tm = (xcd & (xm - 1)) * rect_m + local_m;
+  // (packed groups: neighbouring token tiles go to different XCDs, so that the numbers that turn out to have no
+  // tokens are spread over them)
+  int tm = p.pg_groups > 0 ? local_m * xm + (xcd & (xm - 1)) : (xcd & (xm - 1)) * rect_m + local_m;
   const int tn_grid = (xcd >> p.geo_xm_shift) * rect_n + local_n;
   if (tm >= tiles_m || tn_grid >= tiles_n) return;
+  if (p.pg_groups > 0) {
+    // Token tile tm of the launch -> a group and the tile inside it.  The group sizes are known on the device
+    // only and add up to at most p.m tokens, whatever the largest of them may be, so the launch has a
+    // tile for every BM tokens and one more per group, numbered group after group; a wave counts the
+    // tiles of 64 groups at a time.
+    int first = 0, found = -1;
+    for (int g0 = 0; g0 < p.pg_groups && found < 0; g0 += 64) {
+      const int g = g0 + lane;
+      int count = 0;
+      if (g < p.pg_groups) {  // (a group without a place in the tensor has no tiles, one past its end is cut)
+        const int offset = p.pg_params[p.pg_offset + p.pg_groups + g];
+        const int size = min(min(p.pg_params[p.pg_offset + g], p.pg_max), p.m - offset);
+        count = offset < 0 ? 0 : (max(size, 0) + BM - 1) / BM;
+      }
+      const int end = first + WaveInclusiveSum(count);
+      const uint64_t beyond = __ballot(end > tm);
+      if (beyond != 0) {
+        const int src = __builtin_ctzll(beyond);
+        found = g0 + src;
+        tm -= __builtin_amdgcn_readlane(end - count, src);
+      } else {
+        first = __builtin_amdgcn_readlane(end, 63);
+      }
+    }
+    if (found < 0) return;  // (the whole work-group: every wave counts the same)
+    pg_e = found;
+    m_lo = p.pg_params[p.pg_offset + p.pg_groups + pg_e];
+    m_hi = min(m_lo + min(p.pg_params[p.pg_offset + pg_e], p.pg_max), p.m);
+  }
   // channel tile of the launch -> matrix of the launch (return value) and tile inside it
   auto locate = [&](int& tile) {
     int seg_index = 0;
@@ -1026,6 +1060,19 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_mfma_direct_kernel(GemmParam
     *reinterpret_cast<u32x2*>(sgx.dst + ((size_t)slice * p.m + mi) * 4) = o;
   };
   static_assert(16 % RPH == 0 && RPH % WAVES == 0, "phases tile the 16 registers, waves tile a phase");
+  if constexpr (WAVES == 1) {  // the wave holds whole sums
+#pragma unroll
+    for (int fm = 0; fm < FM; ++fm) {
+      const int mi = token(fm);
+      if (mi >= m_hi) continue;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int slice = slice0 + 8 * (v >> 2) + 4 * g2 + (v & 3);
+        if (slice < sg.ns) store(sg, slice, mi, make_float4(acc[0][fm][v], acc[1][fm][v], acc[2][fm][v], acc[3][fm][v]));
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int fm = 0; fm < FM; ++fm) {
     const int mi = token(fm);
@@ -1126,6 +1173,48 @@ void LaunchDirect(int weight_bits, bool zp, dim3 grid, hipStream_t stream, const
     LaunchDirectW<8, FM, U, WAVES, PAIR, kModePlain>(zp, grid, stream, p);
   else
     LaunchDirectW<4, FM, U, WAVES, PAIR, kModePlain>(zp, grid, stream, p);
+}
+
+template <int FM, int WAVES>
+void LaunchPackedW(int weight_bits, bool zp, dim3 grid, hipStream_t stream, const GemmParams& p) {
+  const dim3 block(WAVES * 64);
+  if (weight_bits == 8 && zp)
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, true, false, false>), grid, block, 0, stream, p);
+  else if (weight_bits == 8)
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, false, false, false>), grid, block, 0, stream, p);
+  else if (zp)
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, true, false, false>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, false, false, false>), grid, block, 0, stream, p);
+}
+// Waves that share the K of a tile of packed groups.  One wave per tile needs no reduction through LDS (8
+// waves on 768 input channels: 80 us, one wave 41), more of them fill the chip when the tiles are few.
+// The estimate: rounds of the waves that are resident at a time (one per SIMD at 128-token tiles, two at
+// 64, three at 32), a round being a wave's share of the K-steps plus what a work-group costs around its
+// loop, in steps.  Over six layer shapes and 4 .. 1024 tokens per group the choice was within 10 % of the best.
+int PackedWaves(double tiles, int fm, int steps) {
+  const double slots = fm == 4 ? 1024.0 : (fm == 2 ? 2048.0 : 3072.0);
+  int best = 1;
+  double best_cost = 0.0;
+  for (int waves = 1; waves <= (fm == 4 ? 4 : 8); waves *= 2) {
+    const double around = waves == 1 ? 8.0 : (waves == 2 ? 12.0 : (waves == 4 ? 16.0 : 40.0));
+    const double x = tiles * waves / slots;
+    const double rounds = x <= 1.0 ? 1.0 : x + 0.35 * (std::ceil(x) - x);
+    const double cost = rounds * ((double)steps / waves + around);
+    if (waves == 1 || cost < best_cost) {
+      best = waves;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+template <int FM>
+void LaunchPacked(int weight_bits, bool zp, int waves, dim3 grid, hipStream_t stream, const GemmParams& p) {
+  if (waves == 1) LaunchPackedW<FM, 1>(weight_bits, zp, grid, stream, p);
+  if (waves == 2) LaunchPackedW<FM, 2>(weight_bits, zp, grid, stream, p);
+  if (waves == 4) LaunchPackedW<FM, 4>(weight_bits, zp, grid, stream, p);
+  if constexpr (FM != 4)
+    if (waves == 8) LaunchPackedW<FM, 8>(weight_bits, zp, grid, stream, p);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1581,7 +1670,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   const bool gated = gate_activation != 0;
   if (gated && count != 2) return hipErrorInvalidValue;
   const FcArgs& a = args[0];
-  // packed groups: one launch plane per weight matrix, token tiles sized for the largest group
+  // packed groups: the token tiles of all groups, found on the device from their sizes
   const bool packed = a.params != nullptr && a.packed_params_offset >= 0;
   if (packed && (count != 1 || gated || a.weights_batch < 1 || a.packed_max_group_size < 1)) return hipErrorInvalidValue;
   GemmParams p = {};
@@ -1643,14 +1732,14 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   const Tuning& tune = GetTuning();
   // the geometry the work-groups would otherwise divide out: waves = waves of the work-group that
   // share one tile's K (all of them, or half in the gated and two-tile modes)
-  auto set_geometry = [&p](int tiles_m, int tiles_n_grid, int fm, bool halves) {
+  auto set_geometry = [&p](int tiles_m, int tiles_n_grid, int waves, bool halves) {
     const int xn = 8 / p.xcd_m;
     p.geo_tiles_m = tiles_m;
     p.geo_rect_m = DivUp(tiles_m, p.xcd_m);
     p.geo_rect_n = DivUp(tiles_n_grid, xn);
     p.geo_xm_shift = p.xcd_m == 8 ? 3 : (p.xcd_m == 4 ? 2 : (p.xcd_m == 2 ? 1 : 0));
     p.geo_rect_m_magic = p.geo_rect_m > 1 ? (uint32_t)((((uint64_t)1 << 32) + p.geo_rect_m - 1) / p.geo_rect_m) : 0u;
-    const int waves = fm == 4 ? 4 : 8, kw = halves ? waves / 2 : waves, prefetch = 4;
+    const int kw = halves ? waves / 2 : waves, prefetch = 4;
     const int shares = kw * p.ksplit, steps_total = DivUp(p.k, 16);
     p.geo_per_wave = DivUp(DivUp(steps_total, shares), prefetch) * prefetch;
   };
@@ -1681,23 +1770,31 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     p.pg_groups = a.weights_batch;
     p.pg_max = std::min(a.packed_max_group_size, a.m);
     p.ksplit = 1;
-    // token tiles of 32, 64 or (groups of hundreds of tokens) 128 tokens; a group starts at any token,
-    // so the tiles are read token by token (no 16-byte token pairs)
-    int fm = p.pg_max <= 32 ? 1 : (p.pg_max >= 256 ? 4 : 2);
+    // Token tiles of 32, 64 or 128 tokens by the average group (the largest group is a bound that real
+    // groups stay far below: 512 tokens over 128 experts, 8 each, are 32 tokens per group on average and
+    // may be 512 in one).  128 experts of 2048 -> 768 at that average: 45.8 / 35.9 / 47.7 us with 32- / 64- /
+    // 128-token tiles; 8 experts of 4096 -> 14336 at an average of 512: 704 / 561 / 537 us; 4 tokens on
+    // average: 25.6 / 27.1 / 40.5 us.  A group starts at any token, so the tiles are read token by token
+    // (no 16-byte token pairs).
+    const double average = (double)a.m / a.weights_batch;
+    int fm = p.pg_max <= 32 || average <= 20.0 ? 1 : (average >= 512.0 ? 4 : 2);
     if (tune.gemm_fm == 1 || tune.gemm_fm == 2 || tune.gemm_fm == 4) fm = tune.gemm_fm;
-    const int tiles_m = DivUp(p.pg_max, fm * 32);
-    p.xcd_m = 1;  // few token tiles per matrix: the XCDs share the channel tiles
+    // (a group of s tokens has ceil(s / BM) <= s / BM + 1 tiles; a group without tokens has none)
+    const int tiles_m = (int)std::min<long>((long)a.m / (fm * 32) + std::min(a.weights_batch, a.m),
+                                            (long)a.weights_batch * DivUp(p.pg_max, fm * 32));
+    p.xcd_m = 8;  // an XCD owns whole token tiles: the channel tiles of a group share its activations
     if (tune.gemm_xcd_m == 1 || tune.gemm_xcd_m == 2 || tune.gemm_xcd_m == 4 || tune.gemm_xcd_m == 8) p.xcd_m = tune.gemm_xcd_m;
-    const dim3 grid(8 * DivUp(tiles_m, p.xcd_m) * DivUp(tiles_n, 8 / p.xcd_m), 1, a.weights_batch);
+    const dim3 grid(8 * DivUp(tiles_m, p.xcd_m) * DivUp(tiles_n, 8 / p.xcd_m));
     if (grid.x / 8 >= (1u << 16)) return hipErrorInvalidValue;  // (the reciprocal of rect_m is exact below 2^16)
-    set_geometry(tiles_m, tiles_n, fm, false);
+    const int waves = PackedWaves((average / (fm * 32) + 0.5) * a.weights_batch * tiles_n, fm, DivUp(a.k, 16));
+    set_geometry(tiles_m, tiles_n, waves, false);
     const bool zp = p.seg[0].zp != nullptr;
     if (fm == 4)
-      LaunchDirect<4, 4, 4, false, false>(a.weight_bits, zp, grid, stream, p);
+      LaunchPacked<4>(a.weight_bits, zp, waves, grid, stream, p);
     else if (fm == 2)
-      LaunchDirect<2, 4, 8, false, false>(a.weight_bits, zp, grid, stream, p);
+      LaunchPacked<2>(a.weight_bits, zp, waves, grid, stream, p);
     else
-      LaunchDirect<1, 4, 8, false, false>(a.weight_bits, zp, grid, stream, p);
+      LaunchPacked<1>(a.weight_bits, zp, waves, grid, stream, p);
     return hipGetLastError();
   }
   // token tile and K split follow the launch as a whole (all channels of all matrices)
@@ -1727,8 +1824,8 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   if (p.xcd_m != 1 && p.xcd_m != 2 && p.xcd_m != 4 && p.xcd_m != 8) p.xcd_m = 8;
   const dim3 grid(8 * DivUp(tiles_m, p.xcd_m) * DivUp(tiles_n, 8 / p.xcd_m), p.ksplit);
   if (grid.x / 8 >= (1u << 16)) return hipErrorInvalidValue;  // (the reciprocal of rect_m is exact below 2^16)
-  set_geometry(tiles_m, tiles_n, fm, gated || p.dual);
   const bool zp = p.seg[0].zp != nullptr;
+  set_geometry(tiles_m, tiles_n, fm == 4 ? 4 : 8, gated || p.dual);
   if (fm == 4)
     LaunchDirect<4, 4, 4, true, true>(a.weight_bits, zp, grid, stream, p);
   else if (fm == 2 && pair)

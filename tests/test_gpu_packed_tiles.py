@@ -1,0 +1,62 @@
+"""GPU parity of the packed-groups GEMM's tile numbering and wave counts: a launch has one token tile for every
+tile's worth of tokens plus one per group, found on the device from the group sizes, and 1, 2, 4 or 8 waves
+share the K of a tile.  More groups than a wave counts at a time, empty ones between, one group with nearly every
+token, sizes around the tile edges, and shapes that reach every (token tile, wave count) pair; against the
+per-matrix float64 product."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+import workloads as W
+from test_gpu_packed_groups import run_device
+from test_oracle_fc import batch_ids_float_weights, make_packed_groups_case
+
+
+def run(oracle, sizes, k, n, bits=4, groups=1, zp=False, max_group=None, group=None, seed=1, gap=0):
+    sizes = np.asarray(sizes, np.int32)
+    offsets = (np.cumsum(sizes) - sizes + gap * np.arange(len(sizes))).astype(np.int32)
+    tokens = int(sizes.sum()) + gap * len(sizes)
+    c = make_packed_groups_case(seed, tokens, 1, k, n, len(sizes), bits, groups, zp)
+    got = run_device(c, np.float16, sizes=sizes, offsets=offsets, max_group_size=max_group or tokens, fill=7.0, group=group)
+    wf = batch_ids_float_weights(oracle, c).astype(np.float64)
+    src = c["packed_src"].astype(np.float16).astype(np.float64)
+    limit = max_group or tokens
+    for g, (s, off) in enumerate(zip(sizes, offsets)):
+        live = slice(int(off), int(off) + min(int(s), limit))
+        ref = src[live] @ wf[:, g, :].T
+        # weights are rounded to fp16 (2^-11 relative, twice with a zero point), results once more; sums in fp32
+        tol = 2.0 ** -10 * (np.abs(src[live]) @ np.abs(wf[:, g, :]).T) / np.sqrt(k) * 4 + 2.0 ** -10 * np.abs(ref) + 1e-6
+        assert np.all(np.abs(got[live] - ref) <= tol), (g, s)
+        assert np.all(got[live.stop:int(off) + int(s)] == 7.0)
+    if gap:
+        for g in range(len(sizes)):
+            end = int(offsets[g] + sizes[g])
+            assert np.all(got[end:end + gap] == 7.0), g
+
+
+@pytest.mark.parametrize("sizes", [
+    [0] * 66 + [1, 0, 31, 32, 33, 0, 64, 65],                       # the first 64 groups are empty
+    [1] * 130,                                                      # three countings, every group one tile
+    [3, 700, 0, 2, 1],                                              # nearly everything in one group
+    list(range(40, 140)),                                           # one and two (128-token: one and two) tiles each
+    [600, 1, 520, 640],                                             # 128-token tiles
+])
+@pytest.mark.parametrize("gap", [0, 1])
+def test_tile_numbering(oracle, sizes, gap):
+    run(oracle, sizes, 64, 132, seed=len(sizes), gap=gap)
+
+
+# 64, 256, 1024 and 8192 input channels: 1, 2, 4 and 8 waves where tiles are few
+@pytest.mark.parametrize("sizes,k,n", [
+    ([18, 0, 20, 5], 64, 128), ([16] * 20, 256, 388), ([9, 12], 1024, 256), ([20, 3], 8192, 128),  # 32-token tiles
+    ([40] * 12, 64, 256), ([40] * 12, 256, 260), ([64, 65], 1024, 256), ([33, 90], 8192, 132),     # 64-token tiles
+    ([530, 600], 64, 640), ([515, 700], 256, 132), ([513, 600], 1024, 260),                         # 128-token tiles, up to 4 waves
+])
+@pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False)])
+def test_wave_counts(oracle, sizes, k, n, bits, zp):
+    run(oracle, sizes, k, n, bits=bits, groups=2 if bits == 4 else 1, zp=zp, seed=k + n)
+
+
+def test_largest_group_bound(oracle):
+    run(oracle, [70, 5, 90, 33], 128, 128, max_group=64)
