@@ -1579,6 +1579,251 @@ __global__ __launch_bounds__(256) void fc_w4_splitk_reduce_kernel(GemmParams p) 
   reinterpret_cast<u32x2*>(sg.dst)[idx] = o2;
 }
 
+// ------------------------------------------------------------------------------------------
+// int4 weights, a few tokens (up to FT * 16): small batches and speculated tokens.
+//
+// The layer's weights are the bytes that matter, so work-groups are cut along the output channels as
+// finely as it takes to give the CUs some: 4 T output slices (16 T channels) each, K (or a run of it)
+// dealt to the 8 waves step by step and added through LDS in wave order.  v_mfma_f32_16x16x32_f16: columns = tokens, row R of MFMA number t =
+// channel (R % (4 / T)) * T + t of slice R / (4 / T).  At T = 4 a lane unpacks every channel of
+// the two blocks that it loads; at T = 1 four lanes load the same blocks and unpack one channel each (a
+// lane-constant shift, mask and exponent), which costs L1 bandwidth, not HBM.  A lane holds one
+// token of whole 4-channel slices at the end: one 8-byte store.  Weights are dequantized as in the kernel
+// above (round_fp16((u - 8) * s)).  kSkinnySteps steps of 32 input channels are in flight per wave; the
+// activations' descriptor ends with the wave's share of K, so steps past it add zeros.
+// Bound: first-load latency and the launch for layers of 2048 channels, then the vector ALU's unpacking.
+// Against 32-token tiles of 128 channels (24 work-groups for the q/k/v projections of 2048 channels), in a step
+// of 18 layers (hidden 2048, MLP 16384, group 32): 988 -> 620 us at 8 tokens, 999 -> 632 at 16, 1008 -> 741
+// at 32; q/k/v 10.3 -> 6.1 us, o 10.4 -> 5.7, down 16.7 -> 7.4 (profiler figures, its second launch 4.1 either way).
+// ------------------------------------------------------------------------------------------
+constexpr int kSkinnyWaves = 8;
+constexpr int kSkinnySteps = 8;
+constexpr int kSkinnyMaxTokens = 32;
+constexpr int kSkinnySplitK = 8192;  // input channels from which K is cut between work-groups
+
+template <int T, int FT, bool ZP, bool MULTI>
+__global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(GemmParams p) {
+  typedef float float4v_t __attribute__((ext_vector_type(4)));
+  constexpr int Q = 4 / T;  // rows per slice; tiles per strip of 16 slices
+  constexpr int U = FT == 1 ? kSkinnySteps : kSkinnySteps / 2;  // (registers)
+  __shared__ float4 red[kSkinnyWaves][T * FT][64];
+
+  asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.group_shift), "s"(p.b_bytes), "s"(p.act), "s"(p.magic_lo), "s"(p.magic_hi),
+               "s"(p.mask_lo), "s"(p.mask_hi), "s"(p.segments), "s"(p.geo_per_wave), "s"(p.ksplit));
+  asm volatile("" : : "s"(p.seg[0].w4), "s"(p.seg[0].scale), "s"(p.seg[0].ns), "s"(p.seg[0].group), "s"(p.seg[0].tile_end),
+               "s"(p.seg[0].a_bytes), "s"(p.seg[0].s_bytes), "s"(p.seg[0].dst), "s"(p.seg[0].bias), "s"(p.seg[0].partial));
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  // The Q tiles of one strip of 16 slices (the 128-byte rows of the library's layout) run on one XCD, whose L2 then
+  // fetches each line once.  (Runs of neighbouring strips per XCD: 1 % slower.)
+  const int local = blockIdx.x / 8;
+  int tile = ((local / Q) * 8 + blockIdx.x % 8) * Q + local % Q;
+  if (tile >= p.seg[MULTI ? p.segments - 1 : 0].tile_end) return;
+  int si = 0;
+  if (MULTI && tile >= p.seg[0].tile_end) {
+    si = (p.segments > 2 && tile >= p.seg[1].tile_end) ? 2 : 1;
+    tile -= p.seg[si - 1].tile_end;
+  }
+  const W4Segment sg = PickSegment<MULTI>(p, si);
+  const int slice0 = tile * (4 * T);
+  const int nsi = slice0 + r / Q;  // the slice whose weights this lane unpacks
+  const int ch0 = (r % Q) * T;     // and its first channel
+
+  const int per_wave = p.geo_per_wave;
+  // Step i of wave w is step i * kSkinnyWaves + w of the work-group's run of K: the work-group walks the weights front
+  // to back, 8 KB of neighbouring rows at a time (with a run per wave, 64 KB apart at K = 16384, the waves of all
+  // work-groups hit the same few memory channels: 23 us for 2048 channels).
+  const int s_begin = (int)blockIdx.y * per_wave * kSkinnyWaves + wave;
+  const uint32_t row_w = (uint32_t)sg.group * 8u, row_x = (uint32_t)p.m * 8u;
+  const uint32_t x_end = (uint32_t)min((uint64_t)p.b_bytes, (uint64_t)(blockIdx.y + 1u) * (uint32_t)(per_wave * kSkinnyWaves) * 8u * row_x);
+  constexpr uint32_t kOob = 0x7FFFFFF0u;
+  const __amdgpu_buffer_rsrc_t rsrc_w =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sg.w4), 0, sg.a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(p.act), 0, x_end, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_s =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(sg.scale), 0, sg.s_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_z =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(ZP ? sg.zp : sg.scale), 0, sg.s_bytes, 0x00020000);
+
+  // Byte offsets of the next step to fetch.  (The launcher bounds every buffer, and what the prefetch runs past
+  // it, below 2^31: no offset wraps.)
+  const uint32_t nsi_group = sg.group_shift >= 0 ? (uint32_t)nsi >> sg.group_shift : (uint32_t)(nsi / sg.group);
+  const uint32_t col_w = (nsi_group * (uint32_t)p.ks * (uint32_t)sg.group + ((uint32_t)nsi - nsi_group * (uint32_t)sg.group)) * 8u;
+  const bool n_ok = nsi < sg.ns;
+  const uint32_t k0 = (uint32_t)s_begin * 8u + 2u * (uint32_t)g;  // the first of this lane's two K-slices
+  uint32_t vw = n_ok ? k0 * row_w + col_w : kOob;
+  const uint32_t vs = n_ok ? (uint32_t)nsi * 8u + (uint32_t)(ch0 * 2) : kOob;
+  const uint32_t group_bytes = (uint32_t)sg.ns * 8u;
+  uint32_t vx[FT];
+#pragma unroll
+  for (int ft = 0; ft < FT; ++ft) vx[ft] = ft * 16 + r < p.m ? k0 * row_x + (uint32_t)(ft * 16 + r) * 8u : kOob;
+
+  u32x2 rw[U][2], rx[U][FT][2], rsc[U], rzp[U];
+  auto load_channels = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t at) {  // T halfs
+    u32x2 v = {0u, 0u};
+    if constexpr (T == 1) v[0] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc, at, 0, 0);
+    if constexpr (T == 2) v[0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, 0);
+    if constexpr (T == 4) v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, 0);
+    return v;
+  };
+  auto load_step = [&](int s, int u) {
+    const uint32_t at = vs + (uint32_t)(s >> (p.group_shift - 1)) * group_bytes;
+    rsc[u] = load_channels(rsrc_s, at);
+    if (ZP) rzp[u] = load_channels(rsrc_z, at);
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) {
+      rx[u][ft][0] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_x, vx[ft], 0, 0);
+      rx[u][ft][1] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_x, vx[ft] + row_x, 0, 0);
+      vx[ft] += kSkinnyWaves * 8u * row_x;
+    }
+    rw[u][0] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_w, vw, 0, 0);
+    rw[u][1] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_w, vw + row_w, 0, 0);
+    vw += kSkinnyWaves * 8u * row_w;
+  };
+
+  float4v_t acc[T][FT];
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft) acc[t][ft] = float4v_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+  // Nibble pattern of a channel: even channels are read in bits 0..3 (1024 + u), odd ones in bits 4..7
+  // (64 + u), channels 2 and 3 after a shift by 8.  Constants of the instruction where the channel is one
+  // (T = 2, 4), of the lane at T = 1.
+  uint32_t magic_lo = p.magic_lo, magic_hi = p.magic_hi;
+  asm volatile("" : "+v"(magic_lo), "+v"(magic_hi));
+  const uint32_t lane_shift = T == 4 ? 0u : (uint32_t)(ch0 >> 1) * 8u;
+  const bool lane_odd = T == 1 && (ch0 & 1);
+  const uint32_t lane_mask = lane_odd ? p.mask_hi : p.mask_lo, lane_magic = lane_odd ? magic_hi : magic_lo;
+  const half2_t off_lo = {(_Float16)-1032.0f, (_Float16)-1032.0f}, off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
+  const half2_t lane_off = lane_odd ? off_hi : off_lo;
+
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {  // (in the order of their use: waiting for one step leaves the younger ones in flight)
+    load_step(s_begin + u * kSkinnyWaves, u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  auto multiply_step = [&](int u) {
+    u32x4 blk = {rw[u][0][0], rw[u][0][1], rw[u][1][0], rw[u][1][1]}, blk8 = blk;
+    if constexpr (T == 4) blk8 = u32x4{blk[0] >> 8, blk[1] >> 8, blk[2] >> 8, blk[3] >> 8};
+    else blk = u32x4{blk[0] >> lane_shift, blk[1] >> lane_shift, blk[2] >> lane_shift, blk[3] >> lane_shift};
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const half2_t sp = AsHalf2(rsc[u][t >> 1]);
+      const half2_t s2 = (t & 1) ? __builtin_shufflevector(sp, sp, 1, 1) : __builtin_shufflevector(sp, sp, 0, 0);
+      half2_t mzs = {(_Float16)0.0f, (_Float16)0.0f};
+      if (ZP) {
+        const half2_t zq = AsHalf2(rzp[u][t >> 1]);
+        mzs = -(((t & 1) ? __builtin_shufflevector(zq, zq, 1, 1) : __builtin_shufflevector(zq, zq, 0, 0)) * s2);
+      }
+      const half2_t off = T == 1 ? lane_off : ((t & 1) ? off_hi : off_lo);
+      u32x4 aop;
+#pragma unroll
+      for (int wd = 0; wd < 4; ++wd) {
+        const uint32_t x = T == 4 && (t & 2) ? blk8[wd] : blk[wd];
+        const uint32_t bits = T == 1 ? ((x & lane_mask) | lane_magic)
+                                     : ((t & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo));
+        const half2_t centred = AsHalf2(bits) + off;  // exact: u - 8
+        aop[wd] = AsU32(ZP ? __builtin_elementwise_fma(centred, s2, mzs) : centred * s2);
+      }
+#pragma unroll
+      for (int ft = 0; ft < FT; ++ft) {
+        const u32x4 bop = {rx[u][ft][0][0], rx[u][ft][0][1], rx[u][ft][1][0], rx[u][ft][1][1]};
+        acc[t][ft] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, aop), __builtin_bit_cast(half8_t, bop),
+                                                            acc[t][ft], 0, 0, 0);
+      }
+    }
+  };
+  // All steps but the last U are refilled; the last U have loops of their own, so that no wait has to allow for a
+  // refill that may not be there.
+  int s0 = 0;
+  for (; s0 + U < per_wave; s0 += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      multiply_step(u);
+      __builtin_amdgcn_sched_barrier(0);
+      load_step(s_begin + (s0 + U + u) * kSkinnyWaves, u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    multiply_step(u);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // Register v of lane (r, g) is row 4 g + v: slice g T + q of the tile holds its channel c in
+  // acc[c % T], register q Q + c / T.
+#pragma unroll
+  for (int q = 0; q < T; ++q)
+#pragma unroll
+    for (int ft = 0; ft < FT; ++ft)
+      red[wave][q * FT + ft][lane] = make_float4(acc[0][ft][q * Q], acc[1 % T][ft][q * Q + 1 / T], acc[2 % T][ft][q * Q + 2 / T],
+                                                 acc[3 % T][ft][q * Q + 3 / T]);
+  __syncthreads();
+  for (int part = wave; part < T * FT; part += kSkinnyWaves) {
+    const int slice = slice0 + g * T + part / FT, token = (part % FT) * 16 + r;
+    if (slice >= sg.ns || token >= p.m) continue;
+    float4 sum = red[0][part][lane];
+#pragma unroll
+    for (int w = 1; w < kSkinnyWaves; ++w) {
+      const float4 o = red[w][part][lane];
+      sum.x += o.x;
+      sum.y += o.y;
+      sum.z += o.z;
+      sum.w += o.w;
+    }
+    if (p.ksplit > 1) {
+      reinterpret_cast<float4*>(sg.partial)[((size_t)blockIdx.y * sg.ns + slice) * p.m + token] = sum;
+      continue;
+    }
+    __half h[4] = {__float2half_rn(sum.x), __float2half_rn(sum.y), __float2half_rn(sum.z), __float2half_rn(sum.w)};
+    if (sg.bias) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) h[c] = __hadd(h[c], sg.bias[slice * 4 + c]);
+    }
+    u32x2 o2;
+    o2[0] = (uint32_t)__half_as_ushort(h[0]) | ((uint32_t)__half_as_ushort(h[1]) << 16);
+    o2[1] = (uint32_t)__half_as_ushort(h[2]) | ((uint32_t)__half_as_ushort(h[3]) << 16);
+    *reinterpret_cast<u32x2*>(sg.dst + ((size_t)slice * p.m + token) * 4) = o2;
+  }
+}
+
+// Channel tile (slices / 4) and K split of the kernel for a few tokens.  Strips of 16 slices where
+// they give most CUs a work-group, or where K is long enough to be cut between work-groups (a second
+// launch adds the shares); else narrower tiles, which cost every CU the L1 bandwidth of a whole strip.
+// (16384 -> 2048 channels at 8 tokens: 23 us in 128 tiles of 16 channels without a split, 7.4 + 4.1 us in
+// 32 strips x 8.  2048 channels of K end inside one batch of loads: no split.)
+int SkinnyTile(int k, int n) {
+  const int strips = DivUp(n, 64);
+  if (strips >= 200 || k >= kSkinnySplitK) return 4;
+  return strips * 2 >= 200 ? 2 : 1;
+}
+int SkinnyKSplit(int k, int n) {
+  if (k < kSkinnySplitK) return 1;
+  int s = 1;  // (every wave keeps at least 8 steps)
+  while (s < 8 && DivUp(n, 64) * s * 2 <= 256 && k / 32 / (kSkinnyWaves * s * 2) >= kSkinnySteps) s *= 2;
+  return s;
+}
+
+template <int T, int FT>
+void LaunchSkinny(bool zp, const GemmParams& p, hipStream_t stream) {
+  const int tiles = p.seg[p.segments - 1].tile_end, unit = 8 * (4 / T);
+  const dim3 grid((unsigned)(DivUp(tiles, unit) * unit), p.ksplit), block(kSkinnyWaves * 64);
+  const bool multi = p.segments > 1;
+  if (zp && multi)
+    hipLaunchKernelGGL((fc_w4_mfma_skinny_kernel<T, FT, true, true>), grid, block, 0, stream, p);
+  else if (zp)
+    hipLaunchKernelGGL((fc_w4_mfma_skinny_kernel<T, FT, true, false>), grid, block, 0, stream, p);
+  else if (multi)
+    hipLaunchKernelGGL((fc_w4_mfma_skinny_kernel<T, FT, false, true>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((fc_w4_mfma_skinny_kernel<T, FT, false, false>), grid, block, 0, stream, p);
+}
+
 // Token tile of the int4 GEMM in blocks of 32 tokens.  64 tokens when that still yields a
 // work-group for half the CUs, else 32 (more work-groups beat a K split across them).  128 tokens (one wave per SIMD, every
 // dequantized weight feeds four MFMAs) when the launch fills the chip anyway and the rounds of
@@ -1797,6 +2042,32 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
       LaunchPacked<1>(a.weight_bits, zp, waves, grid, stream, p);
     return hipGetLastError();
   }
+  auto launch_reduce = [&] {  // (a K split across work-groups)
+    if (p.ksplit <= 1) return;
+    size_t items = 0;
+    for (int i = 0; i < count; ++i) items += (size_t)p.seg[i].ns * a.m;
+    hipLaunchKernelGGL(fc_w4_splitk_reduce_kernel, dim3((unsigned)DivUp((long)items, 256L)), dim3(256), 0, stream, p);
+  };
+  // A few tokens: fc_w4_mfma_skinny_kernel.  Up to 32: at 48 and 64 tokens its four blocks of 16 and the 64-token tiles of
+  // the direct kernel take the same time (1050 / 1068 us per 18-layer step); below 5 the token forms of the GEMVs are
+  // faster (628 us at 4 tokens against 870 before the loop was pipelined) and callers come here only where those do not serve.
+  // (gemm_fm and gemm_ksplit ask for the direct kernel's shapes.)
+  if (!gated && a.weight_bits == 4 && a.m <= kSkinnyMaxTokens && tune.gemm_fm <= 0 && tune.gemm_ksplit <= 0) {
+    const int t = SkinnyTile(p.k, n_total);
+    p.ksplit = SkinnyKSplit(p.k, n_total);
+    for (int i = 0; i < count; ++i)
+      while (p.ksplit > 1 && (size_t)p.ksplit * p.seg[i].ns * 4 * a.m > args[i].partial_floats) p.ksplit /= 2;
+    int tiles = 0;
+    for (int i = 0; i < count; ++i) p.seg[i].tile_end = tiles += DivUp(p.seg[i].ns, 4 * t);
+    p.geo_per_wave = DivUp(DivUp(p.ks, 8), kSkinnyWaves * p.ksplit);
+    const bool zp = p.seg[0].zp != nullptr;
+    if (a.m <= 16)
+      (t == 4 ? LaunchSkinny<4, 1> : t == 2 ? LaunchSkinny<2, 1> : LaunchSkinny<1, 1>)(zp, p, stream);
+    else
+      (t == 4 ? LaunchSkinny<4, 2> : t == 2 ? LaunchSkinny<2, 2> : LaunchSkinny<1, 2>)(zp, p, stream);
+    launch_reduce();
+    return hipGetLastError();
+  }
   // token tile and K split follow the launch as a whole (all channels of all matrices)
   int fm = W4TokenBlocks(a.m, n_total);
   if (tune.gemm_fm > 0) fm = tune.gemm_fm == 1 ? 1 : (tune.gemm_fm == 4 && a.m % 2 == 0 ? 4 : 2);
@@ -1834,11 +2105,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     LaunchDirect<2, 4, 8, false, false>(a.weight_bits, zp, grid, stream, p);
   else
     LaunchDirect<1, 4, 8, false, false>(a.weight_bits, zp, grid, stream, p);
-  if (p.ksplit > 1) {
-    size_t items = 0;
-    for (int i = 0; i < count; ++i) items += (size_t)p.seg[i].ns * a.m;
-    hipLaunchKernelGGL(fc_w4_splitk_reduce_kernel, dim3((unsigned)DivUp((long)items, 256L)), dim3(256), 0, stream, p);
-  }
+  launch_reduce();
   return hipGetLastError();
 }
 
@@ -1884,7 +2151,7 @@ hipError_t LaunchFcW4MfmaGated(const FcArgs& gate, const FcArgs& up, int activat
 size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n) {
   size_t need = 0;
   for (int m = kGemvMaxTokens + 1; m <= max_tokens; ++m) {
-    const int s = W4KSplit(m, k, n);
+    const int s = std::max(W4KSplit(m, k, n), m <= kSkinnyMaxTokens ? SkinnyKSplit(k, n) : 1);
     if (s > 1) need = std::max(need, (size_t)s * DivUp(n, 4) * 4 * m);
   }
   return need;

@@ -1,0 +1,57 @@
+"""The matrix-core kernel for 5..32 tokens over uint4 weights: channel tiles of 4, 8 and 16 slices, one and two blocks
+of 16 tokens, K cut between work-groups, K tails, ragged channels, zero points, several matrices per launch;
+against the float64 product of the dequantized weights."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+import mldhip as M
+import workloads as W
+from test_gpu_fc import textbook
+from test_gpu_gemm import run_w4
+
+
+def check(got, case):
+    # as dequantized, a weight is rounded to fp16 (2^-11 relative, and the zero point's product with the scale once more),
+    # the result once; random signs: the errors of a sum grow with the root of the sum of squares
+    ref = textbook(case)
+    act = case["act"].astype(np.float64)
+    assert got.shape == ref.shape
+    rms = np.sqrt(np.mean(ref ** 2)) + 1e-9
+    assert np.all(np.isfinite(got)) and act.shape[0] == ref.shape[0]
+    err = np.abs(got - ref)
+    assert np.all(err <= 2.0 ** -10 * np.abs(ref) + 6 * 2.0 ** -10 * rms), float(err.max() / rms)
+
+
+# channel tiles: 12800 channels = 200 strips (16 slices), 6400 and 6396 (8), fewer (4); K >= 8192: cut in 2, 4 and 8
+@pytest.mark.parametrize("m", [5, 16, 17, 32])
+@pytest.mark.parametrize("k,n,groups", [(64, 12800, 2), (96, 6400, 1), (250, 6396, 1), (2048, 264, 64), (1000, 4, 1),
+                                        (8192, 2052, 64), (9001, 64, 1), (16384, 2048, 128), (2112, 128, 33)])
+def test_shapes(m, k, n, groups):
+    zp = (k + n) % 3 == 0
+    case = W.make_fc_case(seed=m + k, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=groups, with_bias=m % 2 == 1,
+                          with_zero_point=zp)
+    print("skinny", m, k, n, groups, zp, flush=True)
+    check(run_w4(case), case)
+
+
+@pytest.mark.parametrize("m", [7, 20])
+@pytest.mark.parametrize("k,shapes", [(512, (260, 36, 1024)), (8192, (128, 2048)), (64, (12000, 800, 4))])
+def test_several_matrices(m, k, shapes):
+    """One launch of several matrices gives what single launches give within rounding, tile ends inside a strip among
+    them."""
+    cases = [W.make_fc_case(seed=i + m, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=k // 32) for i, n in enumerate(shapes)]
+    for c in cases[1:]:
+        c["act"] = cases[0]["act"]
+    devs = [W.FcDevice(c) for c in cases]
+    for d in devs[1:]:
+        d.act = devs[0].act
+        srcs = [d.act, d.weights, d.scale]
+        d.op.bind(srcs, [d.out])
+    import torch
+    M.fc_launch_fused([d.op for d in devs], torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for d, c in zip(devs, cases):
+        assert d.op.kernel_name == "fc_w4_mfma_gemm_kernel"
+        check(d.result(), c)
