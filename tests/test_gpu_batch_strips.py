@@ -13,6 +13,6 @@ from test_oracle_fc import make_batch_ids_case
                                                      (31, 1, 96, 64, 7)])
 def test_batched_strips(oracle, rows, src_rows, k, n, batch):
     c = make_batch_ids_case(rows + k, rows, 1, src_rows, k, n, batch, 4, k // 32, False)
-    got, name = run_device(c, np.float16)
+    got, name = run_device(c, np.float16, group=16)
     assert name == ("fc_w4_strip_kernel" if n // 64 * rows >= 32 else "fc_w4_stream_kernel"), name
     check_batch(c, np.float16, got, oracle)
