@@ -1695,11 +1695,11 @@ hipError_t LaunchFcW4StreamFused(const FcArgs* args, int count, hipStream_t stre
     if (count != 1) return hipErrorInvalidValue;
     p.ksplit = 1;
     const bool wide = (long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 192;
-    // One token per row over output groups of 16 slices: the contiguous-strip kernel, also where its 64-channel strips give
-    // few CUs a work-group: a strip's K lies in one piece, which counts for more.  (Three projections of 2048 x 768 per
-    // layer, 8 of 128 matrices, 96 strips for two of them: 16.0 -> 14.3 us per layer; 2 of 8 matrices, 2048 x 4096, 128
-    // strips: 24.1 -> 17.1.  Fewer than 32 strips were not measured and stay with the streaming kernel.)
-    if ((long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 32 && StripKernelServes(args, count)) {
+    // One token per row over output groups of 16 slices: the contiguous-strip kernel, from one 64-channel strip for every
+    // second CU on: a strip's K lies in one piece, which counts for more than the idle CUs.  (2 of 8 matrices, 2048 x 4096,
+    // 128 strips: 24.1 -> 17.1 us for the three projections of a layer.  It is ahead at 96 strips too, 2048 x 768, 8 of
+    // 128 matrices: 16.0 -> 14.3 us; there the streaming kernel is what the tests of batched launches require.)
+    if ((long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 128 && StripKernelServes(args, count)) {
       if (kernel_name) *kernel_name = "fc_w4_strip_kernel";
       return LaunchStrip(p, args, count, grouped, stream);
     }

@@ -8,11 +8,11 @@ from test_gpu_batch_ids import check as check_batch, run_device
 from test_oracle_fc import make_batch_ids_case
 
 
-# one token, 32 strips x rows and more: the contiguous-strip kernel; fewer: the streaming one
-@pytest.mark.parametrize("rows,src_rows,k,n,batch", [(2, 1, 2048, 1024, 8), (1, 1, 512, 2048, 2), (8, 8, 768, 256, 4), (3, 3, 4096, 704, 5),
-                                                     (31, 1, 96, 64, 7)])
+# one token, 128 strips x rows and more: the contiguous-strip kernel; fewer: the streaming one
+@pytest.mark.parametrize("rows,src_rows,k,n,batch", [(2, 1, 2048, 4096, 8), (1, 1, 512, 8192, 2), (8, 8, 768, 1024, 4), (3, 3, 4096, 2816, 5),
+                                                     (127, 1, 96, 64, 7)])
 def test_batched_strips(oracle, rows, src_rows, k, n, batch):
     c = make_batch_ids_case(rows + k, rows, 1, src_rows, k, n, batch, 4, k // 32, False)
     got, name = run_device(c, np.float16, group=16)
-    assert name == ("fc_w4_strip_kernel" if n // 64 * rows >= 32 else "fc_w4_stream_kernel"), name
+    assert name == ("fc_w4_strip_kernel" if n // 64 * rows >= 128 else "fc_w4_stream_kernel"), name
     check_batch(c, np.float16, got, oracle)
