@@ -1580,7 +1580,7 @@ __global__ __launch_bounds__(256) void fc_w4_splitk_reduce_kernel(GemmParams p) 
 }
 
 // ------------------------------------------------------------------------------------------
-// int4 weights, a few tokens (up to FT * 16): small batches and speculated tokens.
+// int4 weights, a few tokens (token tiles of FT * 16 along grid.z): small batches, speculated tokens, short prompts.
 //
 // The layer's weights are the bytes that matter, so work-groups are cut along the output channels as
 // finely as it takes to give the CUs some: 4 T output slices (16 T channels) each, K (or a run of it)
@@ -1595,10 +1595,12 @@ __global__ __launch_bounds__(256) void fc_w4_splitk_reduce_kernel(GemmParams p) 
 // Against 32-token tiles of 128 channels (24 work-groups for the q/k/v projections of 2048 channels), in a step
 // of 18 layers (hidden 2048, MLP 16384, group 32): 988 -> 620 us at 8 tokens, 999 -> 632 at 16, 1008 -> 741
 // at 32; q/k/v 10.3 -> 6.1 us, o 10.4 -> 5.7, down 16.7 -> 7.4 (profiler figures, its second launch 4.1 either way).
+// Several token tiles read one strip's weights on one XCD (grid.x is a multiple of 8): 2048 -> 2048 at 128 tokens 8.4 -> 5.7 us.
 // ------------------------------------------------------------------------------------------
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnySteps = 8;
-constexpr int kSkinnyMaxTokens = 32;
+constexpr int kSkinnyMaxTokens = 32;        // one token tile
+constexpr int kSkinnyMaxTiledTokens = 384;  // token tiles of 32 along grid.z
 constexpr int kSkinnySplitK = 8192;  // input channels from which K is cut between work-groups
 
 template <int T, int FT, bool ZP, bool MULTI>
@@ -1630,6 +1632,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
   const int slice0 = tile * (4 * T);
   const int nsi = slice0 + r / Q;  // the slice whose weights this lane unpacks
   const int ch0 = (r % Q) * T;     // and its first channel
+  const int token0 = (int)blockIdx.z * (FT * 16);
 
   const int per_wave = p.geo_per_wave;
   // Step i of wave w is step i * kSkinnyWaves + w of the work-group's run of K: the work-group walks the weights front
@@ -1658,7 +1661,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
   const uint32_t group_bytes = (uint32_t)sg.ns * 8u;
   uint32_t vx[FT];
 #pragma unroll
-  for (int ft = 0; ft < FT; ++ft) vx[ft] = ft * 16 + r < p.m ? k0 * row_x + (uint32_t)(ft * 16 + r) * 8u : kOob;
+  for (int ft = 0; ft < FT; ++ft) vx[ft] = token0 + ft * 16 + r < p.m ? k0 * row_x + (uint32_t)(token0 + ft * 16 + r) * 8u : kOob;
 
   u32x2 rw[U][2], rx[U][FT][2], rsc[U], rzp[U];
   auto load_channels = [&](__amdgpu_buffer_rsrc_t rsrc, uint32_t at) {  // T halfs
@@ -1765,7 +1768,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
                                                  acc[3 % T][ft][q * Q + 3 / T]);
   __syncthreads();
   for (int part = wave; part < T * FT; part += kSkinnyWaves) {
-    const int slice = slice0 + g * T + part / FT, token = (part % FT) * 16 + r;
+    const int slice = slice0 + g * T + part / FT, token = token0 + (part % FT) * 16 + r;
     if (slice >= sg.ns || token >= p.m) continue;
     float4 sum = red[0][part][lane];
 #pragma unroll
@@ -1792,27 +1795,44 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
   }
 }
 
-// Channel tile (slices / 4) and K split of the kernel for a few tokens.  Strips of 16 slices where
-// they give most CUs a work-group, or where K is long enough to be cut between work-groups (a second
-// launch adds the shares); else narrower tiles, which cost every CU the L1 bandwidth of a whole strip.
-// (16384 -> 2048 channels at 8 tokens: 23 us in 128 tiles of 16 channels without a split, 7.4 + 4.1 us in
-// 32 strips x 8.  2048 channels of K end inside one batch of loads: no split.)
-int SkinnyTile(int k, int n) {
-  const int strips = DivUp(n, 64);
-  if (strips >= 200 || k >= kSkinnySplitK) return 4;
-  return strips * 2 >= 200 ? 2 : 1;
-}
-int SkinnyKSplit(int k, int n) {
+// K split of the kernel for a few tokens.  (16384 -> 2048 channels at 8 tokens: 23 us in 128 tiles of 16 channels
+// without a split, 7.4 + 4.1 us in 32 strips x 8.  2048 channels of K end inside one batch of loads: no split.)
+int SkinnyKSplit(int k, int n, int token_tiles) {
   if (k < kSkinnySplitK) return 1;
   int s = 1;  // (every wave keeps at least 8 steps)
-  while (s < 8 && DivUp(n, 64) * s * 2 <= 256 && k / 32 / (kSkinnyWaves * s * 2) >= kSkinnySteps) s *= 2;
+  while (s < 8 && DivUp(n, 64) * token_tiles * s * 2 <= 256 && k / 32 / (kSkinnyWaves * s * 2) >= kSkinnySteps) s *= 2;
   return s;
+}
+struct SkinnyPlan {
+  int tile, ksplit;  // tile 0: not served
+};
+// The kernel is taken where a work-group per CU holds the whole launch, on the narrowest tiles for which it does: its tiles
+// are smaller than the direct kernel's 128 channels, which leave most CUs idle there, but every token tile unpacks the
+// weights again, and a second round costs more than idle CUs.  A strip's tiles run on one XCD of 32 CUs, so the count is
+// per XCD (18 strips x 6 token tiles in halves, 216 work-groups but 36 on two XCDs: 8.3 us against 7.3 of the direct
+// kernel; 16 strips, 32 on each: 4.1 against 6.4).  Us, direct / here: 2048 -> 2048 channels at 64 tokens 8.4 / 5.4, 128
+// 8.4 / 5.7, 256 8.7 / 6.9, 384 9.2 / 10.3 in 384 work-groups; 2048 -> 2560 in three matrices at 128 9.3 / 7.4; 2048 ->
+// 5632 at 64 10.6 / 7.9, 100 10.7 / 11.1 in 352; 5632 -> 2048 at 128 19.2 / 13.4.  Up to 32 tokens, over 280 random launches
+// of more than 256 strips, the direct kernel was 5 to 20 % ahead, except where up to 16 tokens meet a K that fills the one
+// batch of loads (1536..2048 channels: 4 % behind).  Long K, above 32 tokens, only where it is cut at least 4 ways: 16384 -> 2048 at 64
+// tokens 19.8 / 16.0, at 100, cut in 2, 20.4 / 23.3.  More than 384 tokens were not measured.
+SkinnyPlan PlanSkinny(int m, int k, int n) {
+  const int token_tiles = DivUp(m, 32), strips_xcd = DivUp(DivUp(n, 64), 8);
+  if (m > kSkinnyMaxTiledTokens) return {0, 1};
+  if (k >= kSkinnySplitK) {
+    const int s = SkinnyKSplit(k, n, token_tiles);
+    return m <= kSkinnyMaxTokens || (s >= 4 && strips_xcd * token_tiles * s <= 32) ? SkinnyPlan{4, s} : SkinnyPlan{0, 1};
+  }
+  for (int t = 1; t <= 4; t *= 2)
+    if ((long)strips_xcd * (4 / t) * token_tiles <= 32) return {t, 1};
+  constexpr int kBatch = kSkinnyWaves * kSkinnySteps * 32;  // input channels of one batch of loads
+  return m <= 16 && k <= kBatch && k >= kBatch * 3 / 4 ? SkinnyPlan{4, 1} : SkinnyPlan{0, 1};
 }
 
 template <int T, int FT>
 void LaunchSkinny(bool zp, const GemmParams& p, hipStream_t stream) {
   const int tiles = p.seg[p.segments - 1].tile_end, unit = 8 * (4 / T);
-  const dim3 grid((unsigned)(DivUp(tiles, unit) * unit), p.ksplit), block(kSkinnyWaves * 64);
+  const dim3 grid((unsigned)(DivUp(tiles, unit) * unit), p.ksplit, DivUp(p.m, FT * 16)), block(kSkinnyWaves * 64);
   const bool multi = p.segments > 1;
   if (zp && multi)
     hipLaunchKernelGGL((fc_w4_mfma_skinny_kernel<T, FT, true, true>), grid, block, 0, stream, p);
@@ -2048,13 +2068,15 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     for (int i = 0; i < count; ++i) items += (size_t)p.seg[i].ns * a.m;
     hipLaunchKernelGGL(fc_w4_splitk_reduce_kernel, dim3((unsigned)DivUp((long)items, 256L)), dim3(256), 0, stream, p);
   };
-  // A few tokens: fc_w4_mfma_skinny_kernel.  Up to 32: at 48 and 64 tokens its four blocks of 16 and the 64-token tiles of
-  // the direct kernel take the same time (1050 / 1068 us per 18-layer step); below 5 the token forms of the GEMVs are
+  // Few tokens, or few tiles: fc_w4_mfma_skinny_kernel.  Below 5 tokens the token forms of the GEMVs are
   // faster (628 us at 4 tokens against 870 before the loop was pipelined) and callers come here only where those do not serve.
-  // (gemm_fm and gemm_ksplit ask for the direct kernel's shapes.)
-  if (!gated && a.weight_bits == 4 && a.m <= kSkinnyMaxTokens && tune.gemm_fm <= 0 && tune.gemm_ksplit <= 0) {
-    const int t = SkinnyTile(p.k, n_total);
-    p.ksplit = SkinnyKSplit(p.k, n_total);
+  // (gemm_fm, gemm_ksplit and the others ask for the direct kernel's shapes.)
+  const SkinnyPlan skinny = PlanSkinny(a.m, p.k, n_total);
+  const bool direct_asked = tune.gemm_fm > 0 || tune.gemm_ksplit > 0 ||
+                            (a.m > kSkinnyMaxTokens && (tune.gemm_no_pair > 0 || tune.gemm_dual >= 0 || tune.gemm_xcd_m > 0));
+  if (!gated && a.weight_bits == 4 && skinny.tile > 0 && !direct_asked) {
+    const int t = skinny.tile;
+    p.ksplit = skinny.ksplit;
     for (int i = 0; i < count; ++i)
       while (p.ksplit > 1 && (size_t)p.ksplit * p.seg[i].ns * 4 * a.m > args[i].partial_floats) p.ksplit /= 2;
     int tiles = 0;
@@ -2151,7 +2173,7 @@ hipError_t LaunchFcW4MfmaGated(const FcArgs& gate, const FcArgs& up, int activat
 size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n) {
   size_t need = 0;
   for (int m = kGemvMaxTokens + 1; m <= max_tokens; ++m) {
-    const int s = std::max(W4KSplit(m, k, n), m <= kSkinnyMaxTokens ? SkinnyKSplit(k, n) : 1);
+    const int s = std::max(W4KSplit(m, k, n), PlanSkinny(m, k, n).ksplit);
     if (s > 1) need = std::max(need, (size_t)s * DivUp(n, 4) * 4 * m);
   }
   return need;

@@ -1,5 +1,5 @@
-"""The matrix-core kernel for 5..32 tokens over uint4 weights: channel tiles of 4, 8 and 16 slices, one and two blocks
-of 16 tokens, K cut between work-groups, K tails, ragged channels, zero points, several matrices per launch;
+"""The matrix-core kernel for few tokens over uint4 weights: channel tiles of 4, 8 and 16 slices, one and two blocks
+of 16 tokens, several token tiles, K cut between work-groups, K tails, ragged channels, zero points, several matrices per launch;
 against the float64 product of the dequantized weights."""
 import numpy as np
 import pytest
@@ -36,7 +36,7 @@ def test_shapes(m, k, n, groups):
     check(run_w4(case), case)
 
 
-@pytest.mark.parametrize("m", [7, 20])
+@pytest.mark.parametrize("m", [7, 20, 75])
 @pytest.mark.parametrize("k,shapes", [(512, (260, 36, 1024)), (8192, (128, 2048)), (64, (12000, 800, 4))])
 def test_several_matrices(m, k, shapes):
     """One launch of several matrices gives what single launches give within rounding, tile ends inside a strip among
@@ -55,3 +55,16 @@ def test_several_matrices(m, k, shapes):
     for d, c in zip(devs, cases):
         assert d.op.kernel_name == "fc_w4_mfma_gemm_kernel"
         check(d.result(), c)
+
+
+# several token tiles: 16, 32 and 64 channels where they make at most 256 work-groups, one more channel than that, the last
+# token count, K cut in 4 and not cut far enough, ragged tokens, channels and K
+@pytest.mark.parametrize("m,k,n,groups", [(33, 64, 2048, 2), (64, 96, 2052, 1), (97, 250, 1028, 1), (128, 512, 2048, 16), (256, 96, 2048, 3),
+                                          (257, 64, 1792, 1), (384, 2112, 1300, 33), (384, 64, 4, 1), (385, 64, 260, 2), (300, 1000, 12, 1),
+                                          (64, 8192, 2048, 64), (63, 8192, 2052, 64), (70, 9001, 100, 1)])
+def test_token_tiles(m, k, n, groups):
+    zp = n % 8 != 0
+    case = W.make_fc_case(seed=m + k, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=groups, with_bias=m % 2 == 1,
+                          with_zero_point=zp)
+    print("token tiles", m, k, n, groups, zp, flush=True)
+    check(run_w4(case), case)
