@@ -631,6 +631,9 @@ size_t FcW8RingWorkspaceFloats(int max_tokens, int o) {
 bool RingShapeOk(const FcArgs& a) {
   if (a.params == nullptr || a.weight_bits != 8 || a.ring_size < 4 || a.ring_size % 4 != 0) return false;
   if (a.packed_params_offset >= 0 || a.scale_kind == kScaleBlock || a.act_f16 != a.dst_f16) return false;
+  // one output group (more dst channels than a ring over the output channels holds: refused by the unspecialised kernel)
+  const int ns = DivUp(a.n, 4);
+  if (EffectiveGroup(a.group, ns) != ns) return false;
   return a.m >= 1 && a.rows >= 1 && a.rows <= 65535;
 }
 // Window rows up to which one work-group per slice walks the window by itself.  Its time grows with the rows
@@ -650,8 +653,6 @@ bool PartsSupported(const FcArgs& a) {
 bool FcW8RingSupported(const FcArgs& a) {
   if (!RingShapeOk(a) || a.ring_i_index < 0 || a.ring_o_index >= 0) return false;
   if (a.k > a.ring_size) return false;  // (the window stays within one turn of the ring)
-  const int ns = DivUp(a.n, 4);
-  if (EffectiveGroup(a.group, ns) != ns) return false;
   const int w_ks = DivUp(a.weights_k > 0 ? a.weights_k : a.k, 4);
   if (a.ring_size > 4 * w_ks || (a.weights_batch > 1 && a.ring_size != 4 * w_ks)) return false;
   return a.m <= 64;

@@ -111,3 +111,21 @@ def test_ring_i_subnormal_probabilities():
 def test_ring_i_windows_around_the_split(src_c, tokens, f16):
     """Window lengths where the launcher passes from one work-group per slice to the split window (up to 4 tokens)."""
     run("i", src_c, 24, (src_c + 7) // 4 * 4, tokens, [0, 2, src_c // 2 + 1], f16, seed=src_c)
+
+
+@pytest.mark.parametrize("src_c,dst_c,ring", [(16, 40, 32), (256, 2052, 1024), (64, 8192, 8188)])
+def test_ring_o_refuses_more_channels_than_the_ring(src_c, dst_c, ring):
+    """dst channels that would wrap the ring: an error at any size, and nothing is launched."""
+    import torch
+    desc = M.make_desc(M.UINT8, M.LAYOUT_O4I4, ring // 4)
+    op = M.fc_create(M.PRECISION_F32_F16, M.FLOAT16, M.FLOAT16, ring, src_c, desc, scale_shape=(dst_c, 1), max_tokens=2,
+                     ring_o_offset_index=0, ring_size=ring, dst_channels=dst_c)
+    half = lambda *shape: torch.zeros(shape, dtype=torch.float16, device="cuda")
+    out = torch.full((dst_c // 4, 2, 4), 7.0, dtype=torch.float16, device="cuda")
+    op.bind([half(src_c // 4, 2, 4), torch.zeros(ring * src_c, dtype=torch.uint8, device="cuda"), half(dst_c),
+             torch.zeros(1, dtype=torch.int32, device="cuda")], [out])
+    op.set_shape(1, 1, 2)
+    with pytest.raises(M.MldhipError):
+        op.launch(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.all(out == 7.0)
