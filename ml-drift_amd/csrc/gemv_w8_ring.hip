@@ -84,6 +84,38 @@ __device__ __forceinline__ int RingDstEndSlice(const RingParams& p) {
   return min(max(DstEndSlice(p.params[p.dst_end_ch_index], p.ns), 0), p.ns);
 }
 
+// sum_i a_i (u_i - 128 - z) for dst channel n of token `token` in row `row`, one product after the other.  The kernels sum
+// a_i (u_i - 128) and a_i apart and subtract z times the latter, which turns infinite activations into NaN (without a
+// zero point too: -0 * inf); the rare sum of that kind is done over here, as the unspecialised kernel does all of them.
+// The arguments are read again from where the kernel got them: kept for this, they would hold 20 scalar registers
+// through the whole kernel (and a quarter of the column kernel's speed: one work-group less per CU).
+__device__ __forceinline__ bool RingSumInfinite(float asum) { return __builtin_expect(!(fabsf(asum) <= 3.4028235e38f), 0); }
+template <typename T, bool RING_O>
+__device__ __forceinline__ float RingSumByProducts(int row, int token, int n, float z) {
+  typedef const __attribute__((address_space(4))) RingParams* args_t;
+  args_t p = (args_t)__builtin_amdgcn_kernarg_segment_ptr();  // (RingParams is each kernel's first argument)
+  asm volatile("" : "+s"(p) : : "memory");
+  const int ring = p->ring_size, ring_start = ((p->params[p->ring_index] % ring) + ring) % ring;
+  int slices = p->ks;
+  if (p->src_end_ch_index >= 0) slices = SrcEndSlices(p->params[p->src_end_ch_index], p->k_channels, slices);
+  int wb = p->batch_ids ? p->batch_ids[row] : 0;
+  wb = min(max(wb, 0), p->weights_batch - 1);
+  const T* act = static_cast<const T*>(p->act) + ((size_t)min(row, p->src_rows - 1) * p->m + token) * 4;
+  const uint32_t* w32 = reinterpret_cast<const uint32_t*>(p->weights) +
+                        (RING_O ? (size_t)wb * p->ks * ring : ((size_t)wb * p->ring_rows * p->ns + (n >> 2)) * 4);
+  uint32_t at = ((uint32_t)ring_start + (RING_O ? (uint32_t)n : 0u)) % (uint32_t)ring;  // ring channel
+  float sum = 0.0f;
+  for (int ks = 0; ks < slices; ++ks) {
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t word = RING_O ? w32[(size_t)ks * ring + at] : w32[(size_t)(at >> 2) * p->ns * 4 + (at & 3)];
+      const float u = (float)((word >> (8 * (RING_O ? i : n & 3))) & 0xFFu);
+      sum = fmaf(LoadF(act, (size_t)ks * p->src_rows * p->m * 4 + i), u - (128.0f + z), sum);
+      if (!RING_O) at = at + 1 == (uint32_t)ring ? 0u : at + 1;
+    }
+  }
+  return sum;
+}
+
 template <typename T, int LS, int MT>
 __global__ __launch_bounds__(kRingThreads) void fc_w8_ring_i_kernel(RingParams p) {
   constexpr int RW = kRingThreads / LS;  // window rows in flight per pass
@@ -234,7 +266,8 @@ __global__ __launch_bounds__(256) void fc_w8_ring_finish_kernel(RingParams p) {
     s = LoadF(static_cast<const T*>(p.scale), (size_t)wb * n_all + n);
     if (p.zero_point) z = LoadF(static_cast<const T*>(p.zero_point), (size_t)wb * n_all + n);
   }
-  const float r = s * fmaf(-z, asum, sum);
+  float r = s * fmaf(-z, asum, sum);
+  if (RingSumInfinite(asum)) r = s * RingSumByProducts<T, false>(row, t, n, z);
   const size_t o = ((size_t)(n >> 2) * p.rows * p.m + (size_t)row * p.m + t) * 4 + (n & 3);
   DstT* dst = static_cast<DstT*>(p.dst);
   const DstT* bias = static_cast<const DstT*>(p.bias);
@@ -358,14 +391,15 @@ template <> struct RingTypes<float> { typedef float centred[4][4]; };
 template <> struct RingTypes<__half> { typedef half2_t centred[2][4]; };
 
 // scale * (sum - zp * sum(a)) of output channel n, in the destination type, plus the bias
-template <typename T>
-__device__ __forceinline__ void RingWrite(const RingParams& p, int wb, int n, size_t o, float sum, float asum) {
+template <typename T, bool RING_O>
+__device__ __forceinline__ void RingWrite(const RingParams& p, int wb, int n, size_t o, float sum, float asum, int row, int token) {
   float s = p.scalar_scale, z = p.has_zero_point ? p.scalar_zero_point : 0.0f;
   if (p.scale_kind == kScaleLinear) {
     s = LoadF(static_cast<const T*>(p.scale), (size_t)wb * p.ns * 4 + n);
     if (p.zero_point) z = LoadF(static_cast<const T*>(p.zero_point), (size_t)wb * p.ns * 4 + n);
   }
-  const float r = s * fmaf(-z, asum, sum);
+  float r = s * fmaf(-z, asum, sum);
+  if (RingSumInfinite(asum)) r = s * RingSumByProducts<T, RING_O>(row, token, n, z);
   T* dst = static_cast<T*>(p.dst);
   const T* bias = static_cast<const T*>(p.bias);
   if constexpr (std::is_same<T, float>::value) {
@@ -456,7 +490,7 @@ __global__ __launch_bounds__(THREADS) void fc_w8_ring_i_column_kernel(RingParams
     sum += red[q][t][c];
     as += red[q][t][4];
   }
-  RingWrite<T>(p, wb, ds * 4 + c, ((size_t)ds * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as);
+  RingWrite<T, false>(p, wb, ds * 4 + c, ((size_t)ds * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as, row, tok0 + t);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -572,7 +606,7 @@ __global__ __launch_bounds__(256) void fc_w8_ring_o_kernel(RingParams p) {
     sum += red[q][t][c * 16 + s];
     as += reda[q][t];
   }
-  RingWrite<T>(p, wb, slice * 4 + c, ((size_t)slice * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as);
+  RingWrite<T, true>(p, wb, slice * 4 + c, ((size_t)slice * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as, row, tok0 + t);
 }
 
 template <typename T, int MT>

@@ -129,3 +129,44 @@ def test_ring_o_refuses_more_channels_than_the_ring(src_c, dst_c, ring):
         op.launch(torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     assert torch.all(out == 7.0)
+
+
+# column walk, split window (one token over more than 16384 positions), ring over the output channels
+@pytest.mark.parametrize("axis,src_c,dst_c,ring,tokens", [("i", 300, 72, 1024, 5), ("i", 20000, 24, 20004, 1), ("o", 68, 1000, 1024, 3)])
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("zero_point", [True, False])
+def test_ring_infinite_activations(axis, src_c, dst_c, ring, tokens, f16, zero_point):
+    """An infinite activation gives the infinities and NaNs of the unspecialised kernel, which multiplies every product by
+    itself: infinite where no weight of the channel is exactly its zero point, with the product's sign."""
+    import torch
+    td, mt = (torch.float16, M.FLOAT16) if f16 else (torch.float32, M.FLOAT32)
+    rng = np.random.default_rng(src_c)
+    o, i = (dst_c, ring) if axis == "i" else (ring, src_c)
+    desc = M.make_desc(M.UINT8, M.LAYOUT_I4O4 if axis == "i" else M.LAYOUT_O4I4, (o + 3) // 4)
+    packed = M.rearrange_int8_as_uint8(rng.integers(-2, 3, size=(o, 1, 1, i), dtype=np.int8), desc)
+    act = rng.uniform(-1, 1, size=(tokens, src_c))
+    act[0, src_c // 2] = np.inf
+    if tokens > 1:
+        act[1, 3], act[1, src_c - 1] = -np.inf, -np.inf
+    ns = (dst_c + 3) // 4
+    kw = {"ring_%s_offset_index" % axis: 0, "ring_size": ring, ("src" if axis == "i" else "dst") + "_channels": src_c if axis == "i" else dst_c}
+    op = M.fc_create(M.PRECISION_F32_F16 if f16 else M.PRECISION_F32, mt, mt, o, i, desc, scale_shape=(dst_c, 1), max_tokens=tokens,
+                     has_zero_point_tensor=zero_point, **kw)
+    srcs = [torch.from_numpy(W.to_slices(act)).to(td).cuda(), torch.from_numpy(packed).cuda(), torch.full((ns * 4,), 0.01, dtype=td, device="cuda")]
+    if zero_point:
+        srcs.append(torch.from_numpy(rng.integers(-2, 3, size=ns * 4)).to(td).cuda())
+    srcs.append(torch.tensor([ring // 3], dtype=torch.int32, device="cuda"))
+    results = []
+    for generic in (0, 1):
+        out = torch.full((ns, tokens, 4), 7.0, dtype=td, device="cuda")
+        op.bind(srcs, [out])
+        op.set_shape(1, 1, tokens)
+        with M.tuning(force_generic=generic):
+            op.launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert op.kernel_name == ("fc_generic_kernel" if generic else "fc_w8_ring_%s_kernel" % axis)
+        results.append(W.from_slices(out.cpu().numpy().astype(np.float64), dst_c))
+    got, ref = results
+    assert np.isinf(ref[0]).any() and np.isnan(ref[0]).any()
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
+    assert np.array_equal(got[np.isinf(got)], ref[np.isinf(ref)])
