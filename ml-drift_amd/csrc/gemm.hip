@@ -656,7 +656,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   const int local_m = local - local_n * rect_m;
   // (packed groups: neighbouring token tiles go to different XCDs, so that the numbers that turn out to have no
   // tokens are spread over them)
-  int tm = p.pg_groups > 0 ? local_m * xm + (xcd & (xm - 1)) : (xcd & (xm - 1)) * rect_m + local_m;
+  int tm = p.pg_groups > 0 ? ((int)blockIdx.z * rect_m + local_m) * xm + (xcd & (xm - 1)) : (xcd & (xm - 1)) * rect_m + local_m;
   const int tn_grid = (xcd >> p.geo_xm_shift) * rect_n + local_n;
   if (tm >= tiles_m || tn_grid >= tiles_n) return;
   if (p.pg_groups > 0) {
@@ -2049,10 +2049,18 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
                                             (long)a.weights_batch * DivUp(p.pg_max, fm * 32));
     p.xcd_m = 8;  // an XCD owns whole token tiles: the channel tiles of a group share its activations
     if (tune.gemm_xcd_m == 1 || tune.gemm_xcd_m == 2 || tune.gemm_xcd_m == 4 || tune.gemm_xcd_m == 8) p.xcd_m = tune.gemm_xcd_m;
-    const dim3 grid(8 * DivUp(tiles_m, p.xcd_m) * DivUp(tiles_n, 8 / p.xcd_m));
-    if (grid.x / 8 >= (1u << 16)) return hipErrorInvalidValue;  // (the reciprocal of rect_m is exact below 2^16)
+    // The launch has at most 2^16 - 1 tiles per XCD and plane (the reciprocal of rect_m is exact below 2^16); more token
+    // tiles go to further planes along grid.z, and more channel tiles than that to more XCDs.
+    constexpr int kPlaneTiles = (1 << 16) - 1;
+    while (p.xcd_m > 1 && DivUp(tiles_n, 8 / p.xcd_m) > kPlaneTiles) p.xcd_m /= 2;
+    const int rect_n = DivUp(tiles_n, 8 / p.xcd_m);
+    if (rect_n > kPlaneTiles) return hipErrorInvalidValue;
+    const int rect_m = std::min(DivUp(tiles_m, p.xcd_m), kPlaneTiles / rect_n), planes = DivUp(DivUp(tiles_m, p.xcd_m), rect_m);
+    if (planes > 65535) return hipErrorInvalidValue;
+    const dim3 grid(8 * rect_m * rect_n, 1, planes);
     const int waves = PackedWaves((average / (fm * 32) + 0.5) * a.weights_batch * tiles_n, fm, DivUp(a.k, 16));
-    set_geometry(tiles_m, tiles_n, waves, false);
+    set_geometry(std::min(tiles_m, rect_m * p.xcd_m), tiles_n, waves, false);
+    p.geo_tiles_m = tiles_m;
     const bool zp = p.seg[0].zp != nullptr;
     if (fm == 4)
       LaunchPacked<4>(a.weight_bits, zp, waves, grid, stream, p);

@@ -8,6 +8,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
+import mldhip as M
 import workloads as W
 from test_gpu_packed_groups import run_device
 from test_oracle_fc import batch_ids_float_weights, make_packed_groups_case
@@ -60,3 +61,32 @@ def test_wave_counts(oracle, sizes, k, n, bits, zp):
 
 def test_largest_group_bound(oracle):
     run(oracle, [70, 5, 90, 33], 128, 128, max_group=64)
+
+
+@pytest.mark.parametrize("groups,n,k", [(16384, 4100, 16), (2048, 64, 32)])
+def test_many_small_groups(groups, n, k):
+    """Every token a group of its own: 16384 token tiles x 33 channel tiles are more than 2^16 per XCD.  Matrix g holds one
+    code in every place and each channel a scale of its own, small enough that every result is exact."""
+    import torch
+    g = torch.arange(groups, device="cuda")
+    ns = W.div_up(n, 4)
+    desc = M.fc_int4_weights_desc(n, k, reference=True)
+    assert M.packed_bytes(desc, n, groups, 1, k) == groups * W.div_up(k, 4) * ns * 8
+    code = (g % 16).to(torch.uint8)
+    weights = (code * 17).repeat_interleave(W.div_up(k, 4) * ns * 8)  # (one matrix after the other)
+    channel_scale = (1 + torch.arange(ns * 4, device="cuda") % 7).half() / 64
+    scale = channel_scale.repeat(groups)
+    act = torch.randint(-2, 3, (groups, k), device="cuda").half()
+    src = act.view(groups, k // 4, 4).transpose(0, 1).contiguous()
+    params = torch.cat([torch.ones_like(g), g]).to(torch.int32)
+    out = torch.full((ns, groups, 4), 7.0, dtype=torch.float16, device="cuda")
+    op = M.fc_create(M.PRECISION_F32_F16, M.FLOAT16, M.FLOAT16, n, k, desc, scale_shape=(n, 1), max_tokens=groups, packed_groups=(0, groups, 1))
+    op.bind([src, weights, scale, params], [out])
+    op.set_shape(1, 1, groups)
+    print("packed groups", groups, n, k, flush=True)
+    op.launch(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert op.kernel_name == "fc_w4_mfma_gemm_kernel"
+    got = out.transpose(0, 1).reshape(groups, ns * 4)[:, :n].float()
+    sums = act.float().sum(dim=1) * (code.float() - 8)
+    assert torch.equal(got, sums[:, None] * channel_scale.float()[None, :n])
