@@ -495,6 +495,10 @@ int mldhip_fc_int4_decode_noalloc(const void* src, const void* weights, const vo
  * at the current shape (GPUOperation::flops_/read_size_/write_size_,
  * common/task/gpu_operation.h:190-195). */
 const char* mldhip_op_kernel_name(const mldhip_op* op);
+/* The form of that kernel the last launch of a FullyConnected took, where several run under one name (for tests; the texts may
+ * change): "direct" / "skinny 64x32 k4" (channels x tokens of a work-group, parts of K) / "packed 64x8" (tokens of a tile, waves
+ * that share its K) under fc_w4_mfma_gemm_kernel, "column" / "split" under fc_w8_ring_i_kernel; else empty. */
+const char* mldhip_op_kernel_variant(const mldhip_op* op);
 int mldhip_op_cost(const mldhip_op* op, uint64_t* bytes, uint64_t* flops);
 
 void mldhip_op_destroy(mldhip_op* op);

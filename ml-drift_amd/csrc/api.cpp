@@ -106,6 +106,7 @@ struct mldhip_op {
   float* partial = nullptr;
   size_t partial_floats = 0;
   const char* last_kernel = "";
+  const char* last_variant = "";  // the form of that kernel
   // bytes every object needs at the current shape (kept up to date by create and set_shape, so that
   // a launch checks its bindings without touching the heap)
   std::vector<size_t> need_src, need_dst;
@@ -742,6 +743,8 @@ static int BuildFcArgs(mldhip_op* op, FcArgs* out) {
   a.scalar_zero_point = d.has_scalar_zero_point ? d.scalar_zero_point : 0.0f;
   a.partial = op->partial;
   a.partial_floats = op->partial_floats;
+  op->last_variant = "";
+  a.variant = &op->last_variant;
   if (op->idx_params >= 0) {
     a.params = static_cast<const int32_t*>(op->src_ptr[op->idx_params]);
     a.src_end_ch_index = d.src_end_ch_index;
@@ -986,6 +989,7 @@ int mldhip_fc_int4_decode_noalloc(const void* src, const void* weights, const vo
 }
 
 const char* mldhip_op_kernel_name(const mldhip_op* op) { return op ? op->last_kernel : ""; }
+const char* mldhip_op_kernel_variant(const mldhip_op* op) { return op ? op->last_variant : ""; }
 
 int mldhip_op_cost(const mldhip_op* op, uint64_t* bytes, uint64_t* flops) {
   if (!op) return Fail(MLDHIP_INVALID_ARGUMENT, "null op");

@@ -1908,6 +1908,8 @@ hipError_t LaunchConvInt8Tile(const GemmParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+int Log2(int power_of_two) { return __builtin_ctz((unsigned)power_of_two); }
+
 // What the matrix-core kernel can run at all (any token count).
 bool DirectGemmShapeOk(const FcArgs& a) {
   if ((a.weight_bits != 4 && a.weight_bits != 8) || !a.act_f16 || !a.dst_f16) return false;
@@ -1994,6 +1996,9 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   if (kernel_name)
     *kernel_name = gated ? (a.weight_bits == 8 ? "fc_w8_gated_mfma_gemm_kernel" : "fc_w4_gated_mfma_gemm_kernel")
                          : (a.weight_bits == 8 ? "fc_w8_mfma_gemm_kernel" : "fc_w4_mfma_gemm_kernel");
+  auto set_variant = [&](const char* name) {
+    for (int i = 0; i < count; ++i) SetVariant(args[i].variant, name);
+  };
   const Tuning& tune = GetTuning();
   // the geometry the work-groups would otherwise divide out: waves = waves of the work-group that
   // share one tile's K (all of them, or half in the gated and two-tile modes)
@@ -2062,6 +2067,10 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     set_geometry(std::min(tiles_m, rect_m * p.xcd_m), tiles_n, waves, false);
     p.geo_tiles_m = tiles_m;
     const bool zp = p.seg[0].zp != nullptr;
+    static const char* const kForms[3][4] = {{"packed 32x1", "packed 32x2", "packed 32x4", "packed 32x8"},
+                                             {"packed 64x1", "packed 64x2", "packed 64x4", "packed 64x8"},
+                                             {"packed 128x1", "packed 128x2", "packed 128x4", ""}};
+    set_variant(kForms[Log2(fm)][Log2(waves)]);
     if (fm == 4)
       LaunchPacked<4>(a.weight_bits, zp, waves, grid, stream, p);
     else if (fm == 2)
@@ -2091,6 +2100,12 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     for (int i = 0; i < count; ++i) p.seg[i].tile_end = tiles += DivUp(p.seg[i].ns, 4 * t);
     p.geo_per_wave = DivUp(DivUp(p.ks, 8), kSkinnyWaves * p.ksplit);
     const bool zp = p.seg[0].zp != nullptr;
+#define MLD_SKINNY_FORMS(shape) {"skinny " shape " k1", "skinny " shape " k2", "skinny " shape " k4", "skinny " shape " k8"}
+    static const char* const kForms[3][2][4] = {{MLD_SKINNY_FORMS("16x16"), MLD_SKINNY_FORMS("16x32")},
+                                                {MLD_SKINNY_FORMS("32x16"), MLD_SKINNY_FORMS("32x32")},
+                                                {MLD_SKINNY_FORMS("64x16"), MLD_SKINNY_FORMS("64x32")}};
+#undef MLD_SKINNY_FORMS
+    set_variant(kForms[Log2(t)][a.m > 16][Log2(p.ksplit)]);
     if (a.m <= 16)
       (t == 4 ? LaunchSkinny<4, 1> : t == 2 ? LaunchSkinny<2, 1> : LaunchSkinny<1, 1>)(zp, p, stream);
     else
@@ -2098,6 +2113,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     launch_reduce();
     return hipGetLastError();
   }
+  set_variant("direct");
   // token tile and K split follow the launch as a whole (all channels of all matrices)
   int fm = W4TokenBlocks(a.m, n_total);
   if (tune.gemm_fm > 0) fm = tune.gemm_fm == 1 ? 1 : (tune.gemm_fm == 4 && a.m % 2 == 0 ? 4 : 2);

@@ -754,8 +754,10 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
     int slots = (long)p.ns * p.rows * DivUp(p.m, 4) >= 256 ? 4 : 2;
     while (slots > p.m) slots /= 2;
     const bool small = window <= 512;
+    SetVariant(a.variant, "column");
     return a.act_f16 ? LaunchColumn<__half>(p, slots, small, stream) : LaunchColumn<float>(p, slots, small, stream);
   }
+  SetVariant(a.variant, "split");
   // lanes along the output slices: a power of two up to 64; parts: about 32 KB of weights each, at
   // most what the workspace holds
   int ls = 16;

@@ -54,6 +54,10 @@ __host__ __device__ inline int DstEndSlice(int end_ch, int ns) {
   return s < 0 ? 0 : (s > ns ? ns : s);
 }
 
+inline void SetVariant(const char** variant, const char* name) {
+  if (variant) *variant = name;
+}
+
 // One FullyConnected launch.  Tensors are slice-major: act [Ks][m][4], dst [Ns][m][4].
 struct FcArgs {
   const void* act = nullptr;
@@ -97,6 +101,7 @@ struct FcArgs {
   // ring_size output channels.
   int ring_o_index = -1, ring_i_index = -1, ring_size = 0;
   int weights_k = 0;  // input channels of the weights buffer (ring_i); 0 = k
+  const char** variant = nullptr;  // out: the form of the kernel that was launched (mldhip_op_kernel_variant)
 };
 
 // Split-K workspace sizing for the streaming GEMV.
