@@ -579,7 +579,7 @@ __device__ __forceinline__ void SwapRegisters(u32x4& a, u32x4& b) {
 // channel tiles (2j, 2j + 1 of the launch), one per half.  The two halves read the same
 // activations, so every activation tile is fetched from L2 once for 256 channels, and there are
 // half as many work-groups and reduction rounds; for launches with many tiles.
-enum { kModePlain = 0, kModeGated = 1, kModeDual = 2 };
+enum { kModePlain = 0, kModeGated = 1, kModeDual = 2, kModePacked = 3 };
 // Entry `index` of the launch's matrix list, by value.  Every field of every entry sits at a fixed
 // offset of the kernel arguments, so all of them are fetched by one batch of scalar loads and
 // chosen with scalar selects; indexing the list with a run-time number makes the entry's loads
@@ -611,7 +611,8 @@ __device__ __forceinline__ int WaveInclusiveSum(int v) {
 
 template <int WB, int FM, int U, int WAVES, bool ZP, bool PAIR, bool MULTI, int MODE = kModePlain>
 __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct_kernel(GemmParams p) {
-  constexpr bool GATED = MODE == kModeGated, DUAL = MODE == kModeDual;
+  constexpr bool GATED = MODE == kModeGated, DUAL = MODE == kModeDual, HALVES = GATED || DUAL, PACKED = MODE == kModePacked;
+  static_assert(!PACKED || (!PAIR && !MULTI), "packed groups: one matrix per group, tokens read one by one");
   static_assert(WB == 4 || WB == 8, "uint4 or uint8 weights");
   static_assert(!GATED || (!ZP && !MULTI), "the gated pair is symmetric and is the whole launch");
   static_assert(!PAIR || FM % 2 == 0, "pairs of token blocks");
@@ -624,15 +625,15 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   constexpr int RPH = WAVES == 4 && FM == 4 ? 16 : 8;  // accumulator registers (x 4 MFMAs) per phase
   __shared__ float4 red[WAVES == 1 ? 1 : 2][WAVES][WAVES == 1 ? 1 : RPH][64];
 
-  // One batch of scalar loads for what the prologue reads.  (Left alone, the compiler fetches
+  // One batch of scalar loads (in one statement: of two, the compiler may wait for the first) for what the prologue reads.  (Left alone, it fetches
   // every argument where it is first used: seven scalar round trips, one behind the other, in
   // front of the first operand load.  Input-only operands keep the pointers' address spaces.)
-  asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.ksplit), "s"(p.xcd_m), "s"(p.pg_groups), "s"(p.group_shift),
+  asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.ksplit), "s"(p.xcd_m), "s"(p.group_shift),
                "s"(p.b_bytes), "s"(p.act), "s"(p.magic_lo), "s"(p.magic_hi), "s"(p.mask_lo), "s"(p.mask_hi), "s"(p.segments),
                "s"(p.geo_tiles_m), "s"(p.geo_rect_m), "s"(p.geo_rect_n), "s"(p.geo_xm_shift), "s"(p.geo_rect_m_magic),
-               "s"(p.geo_per_wave));
-  asm volatile("" : : "s"(p.seg[0].w4), "s"(p.seg[0].scale), "s"(p.seg[0].ns), "s"(p.seg[0].group), "s"(p.seg[0].tile_end),
-               "s"(p.seg[0].a_bytes), "s"(p.seg[0].s_bytes), "s"(p.seg[0].dst), "s"(p.seg[0].bias), "s"(p.seg[0].partial));
+               "s"(p.geo_per_wave), "s"(p.seg[0].w4), "s"(p.seg[0].scale), "s"(ZP ? p.seg[0].zp : p.seg[0].scale), "s"(p.seg[0].ns),
+               "s"(p.seg[0].group), "s"(p.seg[0].tile_end), "s"(p.seg[0].a_bytes), "s"(p.seg[0].s_bytes), "s"(p.seg[0].dst),
+               "s"(p.seg[0].bias), "s"(p.seg[0].partial));
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -656,10 +657,11 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   const int local_m = local - local_n * rect_m;
   // (packed groups: neighbouring token tiles go to different XCDs, so that the numbers that turn out to have no
   // tokens are spread over them)
-  int tm = p.pg_groups > 0 ? ((int)blockIdx.z * rect_m + local_m) * xm + (xcd & (xm - 1)) : (xcd & (xm - 1)) * rect_m + local_m;
+  int tm = PACKED ? ((int)blockIdx.z * rect_m + local_m) * xm + (xcd & (xm - 1)) : (xcd & (xm - 1)) * rect_m + local_m;
   const int tn_grid = (xcd >> p.geo_xm_shift) * rect_n + local_n;
   if (tm >= tiles_m || tn_grid >= tiles_n) return;
-  if (p.pg_groups > 0) {
+  const int matrices = PACKED ? p.pg_groups : 1;
+  if constexpr (PACKED) {
     // Token tile tm of the launch -> a group and the tile inside it.  The group sizes are known on the device
     // only and add up to at most p.m tokens, whatever the largest of them may be, so the launch has a
     // tile for every BM tokens and one more per group, numbered group after group; a wave counts the
@@ -697,8 +699,8 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
     }
     return seg_index;
   };
-  constexpr int KW = MODE != kModePlain ? WAVES / 2 : WAVES;  // waves that share one tile's K
-  const int half = MODE != kModePlain ? __builtin_amdgcn_readfirstlane(wave / KW) : 0;
+  constexpr int KW = HALVES ? WAVES / 2 : WAVES;  // waves that share one tile's K
+  const int half = HALVES ? __builtin_amdgcn_readfirstlane(wave / KW) : 0;
   int tn = DUAL ? 2 * tn_grid + half : tn_grid;
   const bool tile_ok = !DUAL || tn < tiles_n_all;  // the last pair of an odd count has one tile
   if (!tile_ok) tn = 0;
@@ -728,7 +730,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   const uint32_t k_slices_end = (uint32_t)(t_begin + per_wave) * 4u;
   // (packed groups over output groups: the buffer of all matrices, see w_base)
   const uint32_t w_end = one_group ? (uint32_t)min((uint64_t)sg.a_bytes, (uint64_t)k_slices_end * row_w)
-                                   : sg.a_bytes * (uint32_t)max(p.pg_groups, 1);
+                                   : sg.a_bytes * (uint32_t)matrices;
   const uint32_t x_end = min((uint64_t)p.b_bytes, (uint64_t)k_slices_end * row_x);
 
   constexpr uint32_t kOob = 0x7FFFFFF0u;
@@ -766,7 +768,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   const uint32_t nsi_group = sg.group_shift >= 0 ? (uint32_t)nsi >> sg.group_shift : (uint32_t)(nsi / sg.group);
   const uint32_t nsi_in_group = (uint32_t)nsi - nsi_group * (uint32_t)sg.group;
   const uint32_t col_w = one_group ? (uint32_t)nsi * kBlk
-                                   : ((nsi_group * (uint32_t)max(p.pg_groups, 1) + (uint32_t)pg_e) * (uint32_t)p.ks * (uint32_t)sg.group +
+                                   : ((nsi_group * (uint32_t)matrices + (uint32_t)pg_e) * (uint32_t)p.ks * (uint32_t)sg.group +
                                       nsi_in_group) * kBlk;
   uint32_t vw0 = n_ok ? ((uint32_t)t_begin * 4u + (uint32_t)g2 * 2u) * row_w + col_w : kOob;
   const uint32_t vs = n_ok ? (uint32_t)nsi * 8u : kOob;
@@ -779,7 +781,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
     const int mi = token(PAIR ? 2 * i : i);
     vx[i] = mi < m_hi ? ((uint32_t)t_begin * 4u + (uint32_t)g2 * 2u) * row_x + (uint32_t)mi * 8u : kOob;
   }
-  const uint32_t group_bytes = (uint32_t)sg.ns * 8u * (uint32_t)max(p.pg_groups, 1);  // one scale group: [matrices][Ns][4] halfs
+  const uint32_t group_bytes = (uint32_t)sg.ns * 8u * (uint32_t)matrices;  // one scale group: [matrices][Ns][4] halfs
 
   wblk_t rw[U][2];
   u32x2 rsc[U], rzp[U], rx[U][NX][2];
@@ -1099,7 +1101,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
         }
         const int v = ph * RPH + j;
         const int slice_l = 8 * (v >> 2) + 4 * g2 + (v & 3);  // slice inside the tile
-        if constexpr (MODE != kModePlain) {
+        if constexpr (HALVES) {
           float4 sum_b = red[buf][KW][j][lane];
 #pragma unroll
           for (int c = KW + 1; c < WAVES; ++c) {
@@ -1179,13 +1181,13 @@ template <int FM, int WAVES>
 void LaunchPackedW(int weight_bits, bool zp, dim3 grid, hipStream_t stream, const GemmParams& p) {
   const dim3 block(WAVES * 64);
   if (weight_bits == 8 && zp)
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, true, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, true, false, false, kModePacked>), grid, block, 0, stream, p);
   else if (weight_bits == 8)
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, false, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, false, false, false, kModePacked>), grid, block, 0, stream, p);
   else if (zp)
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, true, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, true, false, false, kModePacked>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, false, false, false>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, false, false, false, kModePacked>), grid, block, 0, stream, p);
 }
 // Waves that share the K of a tile of packed groups.  One wave per tile needs no reduction through LDS (8
 // waves on 768 input channels: 80 us, one wave 41), more of them fill the chip when the tiles are few.
