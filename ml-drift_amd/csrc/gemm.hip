@@ -669,26 +669,26 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
     int first = 0, found = -1;
     for (int g0 = 0; g0 < p.pg_groups && found < 0; g0 += 64) {
       const int g = g0 + lane;
-      int count = 0;
+      int offset = 0, size = 0;
       if (g < p.pg_groups) {  // (a group without a place in the tensor has no tiles, one past its end is cut)
-        const int offset = p.pg_params[p.pg_offset + p.pg_groups + g];
-        const int size = min(min(p.pg_params[p.pg_offset + g], p.pg_max), p.m - offset);
-        count = offset < 0 ? 0 : (max(size, 0) + BM - 1) / BM;
+        offset = p.pg_params[p.pg_offset + p.pg_groups + g];
+        size = offset < 0 ? 0 : max(min(min(p.pg_params[p.pg_offset + g], p.pg_max), p.m - offset), 0);
       }
+      const int count = (size + BM - 1) / BM;
       const int end = first + WaveInclusiveSum(count);
       const uint64_t beyond = __ballot(end > tm);
       if (beyond != 0) {
         const int src = __builtin_ctzll(beyond);
         found = g0 + src;
         tm -= __builtin_amdgcn_readlane(end - count, src);
+        m_lo = __builtin_amdgcn_readlane(offset, src);
+        m_hi = m_lo + __builtin_amdgcn_readlane(size, src);
       } else {
         first = __builtin_amdgcn_readlane(end, 63);
       }
     }
     if (found < 0) return;  // (the whole work-group: every wave counts the same)
     pg_e = found;
-    m_lo = p.pg_params[p.pg_offset + p.pg_groups + pg_e];
-    m_hi = min(m_lo + min(p.pg_params[p.pg_offset + pg_e], p.pg_max), p.m);
   }
   // channel tile of the launch -> matrix of the launch (return value) and tile inside it
   auto locate = [&](int& tile) {
@@ -1191,9 +1191,10 @@ void LaunchPackedW(int weight_bits, bool zp, dim3 grid, hipStream_t stream, cons
 }
 // Waves that share the K of a tile of packed groups.  One wave per tile needs no reduction through LDS (8
 // waves on 768 input channels: 80 us, one wave 41), more of them fill the chip when the tiles are few.
-// The estimate: rounds of the waves that are resident at a time (one per SIMD at 128-token tiles, two at
-// 64, three at 32), a round being a wave's share of the K-steps plus what a work-group costs around its
-// loop, in steps.  Over six layer shapes and 4 .. 1024 tokens per group the choice was within 10 % of the best.
+// The estimate: rounds of `slots` waves, a round being a wave's share of the K-steps plus what a work-group
+// costs around its loop, in steps.  The constants are fitted, not counted (what registers and LDS let a CU hold is
+// 16, 10, 8 and 8 waves of 32-token tiles in work-groups of 1, 2, 4 and 8, 8 of 64-token ones, 4 of 128-token ones; slots
+// counted that way chose no better).  Over six layer shapes and 4 .. 1024 tokens per group the choice was within 10 % of the best.
 int PackedWaves(double tiles, int fm, int steps) {
   const double slots = fm == 4 ? 1024.0 : (fm == 2 ? 2048.0 : 3072.0);
   int best = 1;
@@ -1209,6 +1210,27 @@ int PackedWaves(double tiles, int fm, int steps) {
     }
   }
   return best;
+}
+// XCD grid of a launch of packed groups: xcd_m XCDs share the token tiles, 8 / xcd_m the channel tiles.  An XCD that owns whole
+// token tiles (8) has the channel tiles of a group share its activations in one L2, but where token tiles are few some XCDs
+// get one more of them than others, or none: 16 groups over 9 tokens (K 3776, 2244 channels) 30 us, 17 with the channel tiles
+// spread.  So: the widest xcd_m within 5 % of the fewest tiles on an XCD, by the tiles that groups of the average size and of up to
+// 1.67 times that have (every group with tokens one tile, or average / tile + 1/2 of them).  Over 5557 random launches (2 .. 256
+// groups, up to 1024 tokens per group, K 64 .. 14336, 128 .. 4096 channels) none got slower than at 8 by more than 8 %, and 1.8 % are won on average.
+int PackedXcdGrid(int m, int groups, int largest, int tile, int tiles_n) {
+  const double average = std::min((double)m / groups, (double)largest);
+  const bool one_each = 1.67 * average <= tile || largest <= tile;
+  double tiles = one_each ? groups * (1.0 - std::exp(-average)) : groups * (average / tile + 0.5);
+  tiles = std::min({tiles, (double)m / tile + std::min(groups, m), (double)groups * DivUp(largest, tile)});
+  auto busiest = [&](int xm) {
+    double t = tiles / xm + 0.5 * (1.0 - 1.0 / xm);
+    if (one_each) t = std::min(t, (double)DivUp(std::min(groups, m), xm));
+    return t * DivUp(tiles_n, 8 / xm);
+  };
+  const double fewest = std::min({busiest(1), busiest(2), busiest(4), busiest(8)});
+  int xm = 8;
+  while (xm > 1 && busiest(xm) > 1.05 * fewest) xm /= 2;
+  return xm;
 }
 template <int FM>
 void LaunchPacked(int weight_bits, bool zp, int waves, dim3 grid, hipStream_t stream, const GemmParams& p) {
@@ -2054,7 +2076,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     // (a group of s tokens has ceil(s / BM) <= s / BM + 1 tiles; a group without tokens has none)
     const int tiles_m = (int)std::min<long>((long)a.m / (fm * 32) + std::min(a.weights_batch, a.m),
                                             (long)a.weights_batch * DivUp(p.pg_max, fm * 32));
-    p.xcd_m = 8;  // an XCD owns whole token tiles: the channel tiles of a group share its activations
+    p.xcd_m = PackedXcdGrid(a.m, a.weights_batch, p.pg_max, fm * 32, tiles_n);
     if (tune.gemm_xcd_m == 1 || tune.gemm_xcd_m == 2 || tune.gemm_xcd_m == 4 || tune.gemm_xcd_m == 8) p.xcd_m = tune.gemm_xcd_m;
     // The launch has at most 2^16 - 1 tiles per XCD and plane (the reciprocal of rect_m is exact below 2^16); more token
     // tiles go to further planes along grid.z, and more channel tiles than that to more XCDs.

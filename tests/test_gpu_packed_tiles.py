@@ -90,3 +90,23 @@ def test_many_small_groups(groups, n, k):
     got = out.transpose(0, 1).reshape(groups, ns * 4)[:, :n].float()
     sums = act.float().sum(dim=1) * (code.float() - 8)
     assert torch.equal(got, sums[:, None] * channel_scale.float()[None, :n])
+
+
+# every form of the launch (tokens of a tile x waves that share its K)
+@pytest.mark.parametrize("sizes,k,n,form", [
+    ([3] * 20, 64, 516, "32x1"), ([3] * 20, 256, 260, "32x2"), ([12, 20, 4] * 4, 512, 388, "32x4"), ([9, 0, 3], 4096, 128, "32x8"),
+    ([30, 0, 31, 33, 64, 20, 32, 40, 30, 20], 64, 516, "64x1"), ([40] * 12, 256, 260, "64x2"), ([40, 100, 3], 1024, 132, "64x4"),
+    ([40, 100, 3], 4096, 132, "64x8"), ([530, 600], 64, 640, "128x1"), ([515, 700], 256, 132, "128x2"), ([513, 600], 1024, 260, "128x4")])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_forms(oracle, monkeypatch, sizes, k, n, form, bits):
+    ops, create = [], M.fc_create
+    monkeypatch.setattr(M, "fc_create", lambda *a, **kw: ops.append(create(*a, **kw)) or ops[-1])
+    run(oracle, sizes, k, n, bits=bits, seed=k + n)
+    assert ops[-1].kernel_variant == "packed " + form
+
+
+# token tiles on the XCDs: as many as XCDs and one more, fewer, all in one group, more groups than tokens; channel tiles 1, 2, 9, 18
+@pytest.mark.parametrize("sizes", [[1] * 9, [1] * 8, [0, 2, 0], [0] * 30 + [3] + [0] * 30, [40, 33, 0, 64, 1, 65, 70, 40, 2], [300]])
+@pytest.mark.parametrize("n", [100, 256, 1152, 2244])
+def test_tiles_over_the_xcds(oracle, sizes, n):
+    run(oracle, sizes, 64, n, seed=n + len(sizes))
