@@ -1838,17 +1838,29 @@ struct SkinnyPlan {
 // 8.4 / 5.7, 256 8.7 / 6.9, 384 9.2 / 10.3 in 384 work-groups; 2048 -> 2560 in three matrices at 128 9.3 / 7.4; 2048 ->
 // 5632 at 64 10.6 / 7.9, 100 10.7 / 11.1 in 352; 5632 -> 2048 at 128 19.2 / 13.4.  Up to 32 tokens, over 280 random launches
 // of more than 256 strips, the direct kernel was 5 to 20 % ahead, except where up to 16 tokens meet a K that fills the one
-// batch of loads (1536..2048 channels: 4 % behind).  Long K, above 32 tokens, only where it is cut at least 4 ways: 16384 -> 2048 at 64
-// tokens 19.8 / 16.0, at 100, cut in 2, 20.4 / 23.3.  More than 384 tokens were not measured.
+// batch of loads (1536..2048 channels), where it was 4 % behind.  More than 384 tokens were not measured.
+// Long K (3471 random launches; direct time / time here, median): up to 32 tokens this kernel is ahead where it is cut at least
+// as often as the direct one (4 and 4 ways 1.20..1.34, 2 and 2 1.23..1.30), else behind (2 against 4 ways 0.91..0.98, whole
+// against 2 ways 0.95 at 17..32 tokens), but for 16 tokens and fewer in whole strips (1.07); two rounds 0.79..0.94 (14336 ->
+// 28672 at 24 tokens 0.8).  Above 32 tokens only where it is cut at least 4 ways: 16384 -> 2048 at 64 tokens 19.8 / 16.0, at 100,
+// cut in 2, 20.4 / 23.3; whole K of 6144 and more in 64-channel tiles against a direct kernel cut in 2: 0.92..1.01.  64-channel
+// tiles up to 16 tokens from more than 512 input channels on: 0.97 below.
+int W4KSplit(int m, int k, int n);
 SkinnyPlan PlanSkinny(int m, int k, int n) {
   const int token_tiles = DivUp(m, 32), strips_xcd = DivUp(DivUp(n, 64), 8);
   if (m > kSkinnyMaxTiledTokens) return {0, 1};
+  const int direct_split = W4KSplit(m, k, n);
   if (k >= kSkinnySplitK) {
     const int s = SkinnyKSplit(k, n, token_tiles);
-    return m <= kSkinnyMaxTokens || (s >= 4 && strips_xcd * token_tiles * s <= 32) ? SkinnyPlan{4, s} : SkinnyPlan{0, 1};
+    if ((long)strips_xcd * token_tiles * s > 32) return {0, 1};
+    const bool taken = m > kSkinnyMaxTokens ? s >= 4 : s >= direct_split || (m <= 16 && s == 1);
+    return taken ? SkinnyPlan{4, s} : SkinnyPlan{0, 1};
   }
   for (int t = 1; t <= 4; t *= 2)
-    if ((long)strips_xcd * (4 / t) * token_tiles <= 32) return {t, 1};
+    if ((long)strips_xcd * (4 / t) * token_tiles <= 32) {
+      if (t == 4 && (m > kSkinnyMaxTokens ? direct_split > 1 : m <= 16 && k <= 512)) return {0, 1};
+      return {t, 1};
+    }
   constexpr int kBatch = kSkinnyWaves * kSkinnySteps * 32;  // input channels of one batch of loads
   return m <= 16 && k <= kBatch && k >= kBatch * 3 / 4 ? SkinnyPlan{4, 1} : SkinnyPlan{0, 1};
 }

@@ -68,3 +68,44 @@ def test_token_tiles(m, k, n, groups):
                           with_zero_point=zp)
     print("token tiles", m, k, n, groups, zp, flush=True)
     check(run_w4(case), case)
+
+
+# which kernel a launch takes, and both results: K cut in 1, 2, 4 and 8 and every tile of the kernel; against it two rounds of
+# work-groups, a direct kernel cut more often, whole K of 6144 and more above 32 tokens, one batch of short K in whole strips
+@pytest.mark.parametrize("m,k,n,zp,form", [
+    (16, 64, 2048, True, "skinny 16x16 k1"), (33, 512, 1024, True, "skinny 16x32 k1"), (9, 64, 8192, False, "skinny 32x16 k1"),
+    (17, 96, 8100, True, "skinny 32x32 k1"), (12, 544, 16384, False, "skinny 64x16 k1"), (20, 64, 12804, True, "skinny 64x32 k1"),
+    (16, 2048, 17000, False, "skinny 64x16 k1"), (7, 8192, 9000, True, "skinny 64x16 k1"), (5, 8192, 5000, False, "skinny 64x16 k2"),
+    (32, 8200, 4100, True, "skinny 64x32 k2"), (16, 8192, 4096, False, "skinny 64x16 k4"), (24, 8192, 2052, True, "skinny 64x32 k4"),
+    (64, 8192, 2048, False, "skinny 64x32 k4"), (16, 16384, 1024, True, "skinny 64x16 k8"), (30, 16384, 2000, False, "skinny 64x32 k8"),
+    (16, 512, 16384, True, "direct"), (20, 64, 16640, False, "direct"), (16, 1504, 17000, False, "direct"), (16, 8192, 17000, False, "direct"),
+    (17, 8192, 9000, False, "direct"), (8, 12288, 5000, False, "direct"), (33, 8192, 4096, False, "direct"), (64, 6144, 5000, False, "direct"),
+    (385, 64, 260, True, "direct")])
+def test_kernel_choice(m, k, n, zp, form):
+    case = W.make_fc_case(seed=m + k, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=k // 32 if k % 32 == 0 else 1,
+                          with_bias=m % 2 == 1, with_zero_point=zp)
+    print("kernel choice", m, k, n, zp, form, flush=True)
+    dev = W.FcDevice(case)
+    dev.run()
+    got = dev.result()
+    assert (dev.op.kernel_name, dev.op.kernel_variant) == ("fc_w4_mfma_gemm_kernel", form)
+    check(got, case)
+
+
+@pytest.mark.parametrize("m,k,shapes,form", [(7, 512, (260, 36, 1024), "skinny 16x16 k1"), (20, 8192, (128, 2048), "skinny 64x32 k4"),
+                                             (75, 96, (1500, 800, 4), "skinny 32x32 k1"), (24, 8192, (9000, 4000), "direct")])
+def test_several_matrices_with_zero_points(m, k, shapes, form):
+    cases = [W.make_fc_case(seed=i + m, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=k // 32, with_zero_point=True)
+             for i, n in enumerate(shapes)]
+    for c in cases[1:]:
+        c["act"] = cases[0]["act"]
+    devs = [W.FcDevice(c) for c in cases]
+    for d in devs[1:]:
+        d.act = devs[0].act
+        d.op.bind([d.act, d.weights, d.scale, d.zero_point], [d.out])
+    import torch
+    M.fc_launch_fused([d.op for d in devs], torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    for d, c in zip(devs, cases):
+        assert d.op.kernel_variant == form
+        check(d.result(), c)
