@@ -1675,7 +1675,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
       __builtin_amdgcn_make_buffer_rsrc(const_cast<__half*>(ZP ? sg.zp : sg.scale), 0, sg.s_bytes, 0x00020000);
 
   // Byte offsets of the next step to fetch.  (The launcher bounds every buffer, and what the prefetch runs past
-  // it, below 2^31: no offset wraps.)
+  // it, below 2^31, SkinnyOffsetsFit: no offset wraps, those that start at kOob neither.)
   const uint32_t nsi_group = sg.group_shift >= 0 ? (uint32_t)nsi >> sg.group_shift : (uint32_t)(nsi / sg.group);
   const uint32_t col_w = (nsi_group * (uint32_t)p.ks * (uint32_t)sg.group + ((uint32_t)nsi - nsi_group * (uint32_t)sg.group)) * 8u;
   const bool n_ok = nsi < sg.ns;
@@ -1863,6 +1863,17 @@ SkinnyPlan PlanSkinny(int m, int k, int n) {
     }
   constexpr int kBatch = kSkinnyWaves * kSkinnySteps * 32;  // input channels of one batch of loads
   return m <= 16 && k <= kBatch && k >= kBatch * 3 / 4 ? SkinnyPlan{4, 1} : SkinnyPlan{0, 1};
+}
+
+// The prefetch ends with whole batches of steps in every wave: K-slices up to which offsets are formed.
+bool SkinnyOffsetsFit(const GemmParams& p) {
+  const int unroll = p.m <= 16 ? kSkinnySteps : kSkinnySteps / 2;
+  const uint64_t per_slice = (uint64_t)kSkinnyWaves * 8;
+  const uint64_t end = ((uint64_t)(p.ksplit - 1) * p.geo_per_wave + (uint64_t)DivUp(p.geo_per_wave, unroll) * unroll) * per_slice;
+  const uint64_t past = end > (uint64_t)p.ks ? end - p.ks : 0;
+  uint64_t most = p.b_bytes + past * p.m * 8;
+  for (int i = 0; i < p.segments; ++i) most = std::max<uint64_t>(most, p.seg[i].a_bytes + past * p.seg[i].group * 8);
+  return most < 0x7FFFFFF0u;
 }
 
 template <int T, int FT>
@@ -2129,25 +2140,29 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
                             (a.m > kSkinnyMaxTokens && (tune.gemm_no_pair > 0 || tune.gemm_dual >= 0 || tune.gemm_xcd_m > 0));
   if (!gated && a.weight_bits == 4 && skinny.tile > 0 && !direct_asked) {
     const int t = skinny.tile;
-    p.ksplit = skinny.ksplit;
+    GemmParams q = p;
+    q.ksplit = skinny.ksplit;
     for (int i = 0; i < count; ++i)
-      while (p.ksplit > 1 && (size_t)p.ksplit * p.seg[i].ns * 4 * a.m > args[i].partial_floats) p.ksplit /= 2;
+      while (q.ksplit > 1 && (size_t)q.ksplit * q.seg[i].ns * 4 * a.m > args[i].partial_floats) q.ksplit /= 2;
     int tiles = 0;
-    for (int i = 0; i < count; ++i) p.seg[i].tile_end = tiles += DivUp(p.seg[i].ns, 4 * t);
-    p.geo_per_wave = DivUp(DivUp(p.ks, 8), kSkinnyWaves * p.ksplit);
-    const bool zp = p.seg[0].zp != nullptr;
+    for (int i = 0; i < count; ++i) q.seg[i].tile_end = tiles += DivUp(q.seg[i].ns, 4 * t);
+    q.geo_per_wave = DivUp(DivUp(q.ks, 8), kSkinnyWaves * q.ksplit);
+    if (SkinnyOffsetsFit(q)) {
+      p = q;
+      const bool zp = p.seg[0].zp != nullptr;
 #define MLD_SKINNY_FORMS(shape) {"skinny " shape " k1", "skinny " shape " k2", "skinny " shape " k4", "skinny " shape " k8"}
-    static const char* const kForms[3][2][4] = {{MLD_SKINNY_FORMS("16x16"), MLD_SKINNY_FORMS("16x32")},
-                                                {MLD_SKINNY_FORMS("32x16"), MLD_SKINNY_FORMS("32x32")},
-                                                {MLD_SKINNY_FORMS("64x16"), MLD_SKINNY_FORMS("64x32")}};
+      static const char* const kForms[3][2][4] = {{MLD_SKINNY_FORMS("16x16"), MLD_SKINNY_FORMS("16x32")},
+                                                  {MLD_SKINNY_FORMS("32x16"), MLD_SKINNY_FORMS("32x32")},
+                                                  {MLD_SKINNY_FORMS("64x16"), MLD_SKINNY_FORMS("64x32")}};
 #undef MLD_SKINNY_FORMS
-    set_variant(kForms[Log2(t)][a.m > 16][Log2(p.ksplit)]);
-    if (a.m <= 16)
-      (t == 4 ? LaunchSkinny<4, 1> : t == 2 ? LaunchSkinny<2, 1> : LaunchSkinny<1, 1>)(zp, p, stream);
-    else
-      (t == 4 ? LaunchSkinny<4, 2> : t == 2 ? LaunchSkinny<2, 2> : LaunchSkinny<1, 2>)(zp, p, stream);
-    launch_reduce();
-    return hipGetLastError();
+      set_variant(kForms[Log2(t)][a.m > 16][Log2(p.ksplit)]);
+      if (a.m <= 16)
+        (t == 4 ? LaunchSkinny<4, 1> : t == 2 ? LaunchSkinny<2, 1> : LaunchSkinny<1, 1>)(zp, p, stream);
+      else
+        (t == 4 ? LaunchSkinny<4, 2> : t == 2 ? LaunchSkinny<2, 2> : LaunchSkinny<1, 2>)(zp, p, stream);
+      launch_reduce();
+      return hipGetLastError();
+    }
   }
   set_variant("direct");
   // token tile and K split follow the launch as a whole (all channels of all matrices)

@@ -109,3 +109,32 @@ def test_several_matrices_with_zero_points(m, k, shapes, form):
     for d, c in zip(devs, cases):
         assert d.op.kernel_variant == form
         check(d.result(), c)
+
+
+@pytest.mark.parametrize("k,n,form", [(1600, 2600000, "direct"), (2048, 1000000, "skinny 64x16 k1")])
+def test_offsets_below_two_gib(k, n, form):
+    """A batch of loads that would reach past 2 GiB of one matrix's offsets (1600 input channels of 2048 in a batch, 2.08 GB of
+    weights) goes to the direct kernel; channels at both ends and between against float64."""
+    import torch
+    m, ks, ns = 8, k // 4, n // 4
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    desc = M.fc_int4_weights_desc(n, k, reference=True)
+    weights = torch.randint(-2 ** 31, 2 ** 31, (ks * ns * 2,), dtype=torch.int32, device="cuda", generator=gen)
+    act = torch.randn((ks, m, 4), device="cuda", generator=gen).half()
+    scale = (torch.rand((k // 32, ns * 4), device="cuda", generator=gen) * 0.01).half()  # (groups of 32: few-token per-channel layers have a kernel of their own)
+    out = torch.zeros((ns, m, 4), dtype=torch.float16, device="cuda")
+    op = M.fc_create(M.PRECISION_F32_F16, M.FLOAT16, M.FLOAT16, n, k, desc, scale_shape=(n, k // 32), max_tokens=m)
+    op.bind([act, weights, scale], [out])
+    op.set_shape(1, 1, m)
+    print("offsets", k, n, flush=True)
+    op.launch(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert op.kernel_variant == form
+    words = weights.view(ks, ns, 2)
+    for s in (0, 1, ns // 3, ns - 1):
+        w = words[:, s].cpu().numpy().view(np.uint32)  # [ks][2]: bits 16 (i % 2) + 4 c of word i / 2
+        u = np.stack([[(w[:, i // 2] >> (16 * (i % 2) + 4 * c)) & 15 for c in range(4)] for i in range(4)])  # [i][c][ks]
+        wf = (u.transpose(2, 0, 1).reshape(k, 4).astype(np.float64) - 8) * scale[:, 4 * s:4 * s + 4].double().cpu().numpy().repeat(32, axis=0)
+        ref = act.double().cpu().numpy().transpose(1, 0, 2).reshape(m, k) @ wf
+        err = np.abs(out[s].double().cpu().numpy() - ref)
+        assert np.all(err <= 2.0 ** -10 * np.abs(ref) + 6 * 2.0 ** -10 * np.sqrt(np.mean(ref ** 2)))
