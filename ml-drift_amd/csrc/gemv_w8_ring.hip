@@ -59,6 +59,7 @@ struct RingParams {
   int scale_kind, has_zero_point;
   float scalar_scale, scalar_zero_point;
   int parts;
+  int xcd_mask, xcd_runs;  // column kernel
 };
 
 __device__ __forceinline__ float LoadF(const float* p, size_t i) { return p[i]; }
@@ -390,16 +391,9 @@ template <typename T> struct RingTypes;
 template <> struct RingTypes<float> { typedef float centred[4][4]; };
 template <> struct RingTypes<__half> { typedef half2_t centred[2][4]; };
 
-// scale * (sum - zp * sum(a)) of output channel n, in the destination type, plus the bias
-template <typename T, bool RING_O>
-__device__ __forceinline__ void RingWrite(const RingParams& p, int wb, int n, size_t o, float sum, float asum, int row, int token) {
-  float s = p.scalar_scale, z = p.has_zero_point ? p.scalar_zero_point : 0.0f;
-  if (p.scale_kind == kScaleLinear) {
-    s = LoadF(static_cast<const T*>(p.scale), (size_t)wb * p.ns * 4 + n);
-    if (p.zero_point) z = LoadF(static_cast<const T*>(p.zero_point), (size_t)wb * p.ns * 4 + n);
-  }
-  float r = s * fmaf(-z, asum, sum);
-  if (RingSumInfinite(asum)) r = s * RingSumByProducts<T, RING_O>(row, token, n, z);
+// One result in the destination type, plus the bias
+template <typename T>
+__device__ __forceinline__ void RingStore(const RingParams& p, int n, size_t o, float r) {
   T* dst = static_cast<T*>(p.dst);
   const T* bias = static_cast<const T*>(p.bias);
   if constexpr (std::is_same<T, float>::value) {
@@ -410,6 +404,17 @@ __device__ __forceinline__ void RingWrite(const RingParams& p, int wb, int n, si
     dst[o] = h;
   }
 }
+// scale * (sum - zp * sum(a)) of output channel n (the rare second store comes last, out of the way of the first)
+template <typename T, bool RING_O>
+__device__ __forceinline__ void RingWrite(const RingParams& p, int wb, int n, size_t o, float sum, float asum, int row, int token) {
+  float s = p.scalar_scale, z = p.has_zero_point ? p.scalar_zero_point : 0.0f;
+  if (p.scale_kind == kScaleLinear) {
+    s = LoadF(static_cast<const T*>(p.scale), (size_t)wb * p.ns * 4 + n);
+    if (p.zero_point) z = LoadF(static_cast<const T*>(p.zero_point), (size_t)wb * p.ns * 4 + n);
+  }
+  RingStore<T>(p, n, o, s * fmaf(-z, asum, sum));
+  if (RingSumInfinite(asum)) RingStore<T>(p, n, o, s * RingSumByProducts<T, RING_O>(row, token, n, z));
+}
 
 // (MT <= p.m: the last work-group along the tokens starts at token m - MT, and only it writes what is left)
 template <typename T, int MT, int THREADS>
@@ -417,9 +422,13 @@ __global__ __launch_bounds__(THREADS) void fc_w8_ring_i_column_kernel(RingParams
   constexpr int U = 2, WAVES = THREADS / 64, NW = kWordsPerToken<T>;
   __shared__ float red[WAVES][MT][5];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // runs of 8 slices on one XCD (work-groups go round-robin to the 8 of them)
-  const int j = blockIdx.x >> 3;
-  const int ds = (j >> 3) * 64 + (blockIdx.x & 7) * 8 + (j & 7);
+  // runs of 8 slices on one XCD (work-groups go round-robin to the 8 of them); fewer than 8 runs: what one
+  // of them does not hold at a time goes to others (20 channels, 16 rows of 49 tokens: all on XCD 0 else); not less, since
+  // the tokens of a row share its weights, and the rows the lines of the activations
+  constexpr int kSpreadShift = THREADS == 1024 ? 3 : 5;  // (8 slices x 8 or 32 token tiles fill 32 CUs)
+  const int plane = blockIdx.z * ((p.m + MT - 1) / MT) + blockIdx.y;
+  const int j = blockIdx.x >> 3, run = (blockIdx.x - ((plane >> kSpreadShift) & p.xcd_mask) * p.xcd_runs) & 7;
+  const int ds = (j >> 3) * 64 + run * 8 + (j & 7);
   if (ds >= RingDstEndSlice(p)) return;  // (the whole work-group)
   const int row = blockIdx.z, tok_first = blockIdx.y * MT, tok0 = min(tok_first, p.m - MT);
   int wb = p.batch_ids ? p.batch_ids[row] : 0;
@@ -728,6 +737,7 @@ static RingParams MakeRingParams(const FcArgs& a) {
   p.scalar_scale = a.scalar_scale;
   p.scalar_zero_point = a.scalar_zero_point;
   p.parts = 1;
+  p.xcd_mask = p.xcd_runs = 0;
   return p;
 }
 
@@ -754,6 +764,8 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
     int slots = (long)p.ns * p.rows * DivUp(p.m, 4) >= 256 ? 4 : 2;
     while (slots > p.m) slots /= 2;
     const bool small = window <= 512;
+    p.xcd_runs = std::min(8, DivUp(p.ns, 8));
+    p.xcd_mask = p.xcd_runs == 1 ? 7 : (p.xcd_runs == 2 ? 3 : (p.xcd_runs <= 4 ? 1 : 0));
     SetVariant(a.variant, "column");
     return a.act_f16 ? LaunchColumn<__half>(p, slots, small, stream) : LaunchColumn<float>(p, slots, small, stream);
   }
