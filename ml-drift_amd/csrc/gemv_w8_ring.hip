@@ -679,26 +679,95 @@ bool RingShapeOk(const FcArgs& a) {
   if (EffectiveGroup(a.group, ns) != ns) return false;
   return a.m >= 1 && a.rows >= 1 && a.rows <= 65535;
 }
-// Window rows up to which one work-group per slice walks the window by itself.  Its time grows with the rows
-// (3.6 us at 2048, 6.4 at 4096, 12.1 at 8192 for 256 channels and one token), that of the split window hardly
-// does (7.4, 7.8, 8.8 us), but the split window reads 32 activations per row and thread at 4 tokens (15.7,
-// 16.4, 17.4 us against 4.2, 7.0, 11.8) and serves no more than 4.
-int ColumnMaxRows(int tokens) { return tokens == 1 ? 4097 : 8193; }
-bool ColumnPreferred(const FcArgs& a) {
-  return a.m > 4 || std::min(DivUp(a.k, 4), a.ring_size / 4) + 1 <= ColumnMaxRows(a.m);
-}
 bool PartsSupported(const FcArgs& a) {
   if (a.m > 4 || (long)a.rows * a.m > 16 || a.partial == nullptr) return false;
   // at least one part must fit the workspace
   return (size_t)a.rows * 4 * ((size_t)DivUp(a.n, 4) * 4 + 4) <= a.partial_floats;
 }
 
+int RingWindow(const FcArgs& a) { return std::min(DivUp(a.k, 4), a.ring_size / 4) + 1; }
+
+// Token slots of a column work-group: two, so that the slices of a narrow cache (64 for a head of 256) occupy the chip
+// (8 tokens x 8192 positions x 256 channels: 5.8 us, 8.6 with one slot, 6.2 with four); four where they do anyway
+// (4096 positions x 512 channels: 5.25 against 5.8 us).
+int ColumnSlots(const FcArgs& a) {
+  int slots = (long)DivUp(a.n, 4) * a.rows * DivUp(a.m, 4) >= 256 ? 4 : 2;
+  while (slots > a.m) slots /= 2;
+  return slots;
+}
+
+// The split window: lanes along the output slices (a power of two up to 64) and parts of about 32 KB of weights each, at most
+// what the workspace holds.
+struct RingSplit {
+  int lanes, parts, rows_in_flight;
+};
+RingSplit SplitWindow(const FcArgs& a) {
+  const int ns = DivUp(a.n, 4), window = RingWindow(a);
+  RingSplit r;
+  r.lanes = 16;
+  while (r.lanes < 64 && r.lanes < ns) r.lanes *= 2;
+  r.rows_in_flight = kRingThreads / r.lanes * RingUnroll(a.m == 1 ? 1 : (a.m == 2 ? 2 : 4));
+  const size_t bytes = (size_t)window * ns * 16;
+  int parts = (int)std::min<size_t>(kRingMaxParts, std::max<size_t>(1, bytes / 32768));
+  parts = std::min(parts, std::max(1, DivUp(window, r.rows_in_flight)));
+  const size_t per_part = (size_t)a.rows * 4 * ((size_t)ns * 4 + 4);
+  r.parts = std::max(1, (int)std::min<size_t>(parts, a.partial_floats / per_part));
+  return r;
+}
+
+// Which kernel takes the ring over the input channels.  A column work-group reads 16 bytes of a line of its own per window row, so
+// its time grows with window x slices x token tiles over the CUs (2000 positions x 2500 channels x 39 tokens 2150 us, the
+// unspecialised kernel 560); the split window reads whole lines but is two launches with 32 activations per row and thread (8192
+// positions x 256 channels, one token: 10.4 us, 5.0 in columns; 3088 x 2352, 16 rows of one token: 24 against 73).  Times in us, each
+// the root of the sum of squares of a work-group's chain and of the busiest share of the work, plus the weights' bytes; fitted to
+// 9319 random launches (windows of 128 .. 65536 positions, 4 .. 8192 channels, 1 .. 64 tokens x 1 .. 16 rows, fp16 and fp32) to
+// within 17 % in nine of ten.  Their choice is slower than what served these launches without the column kernel by more than 10 %
+// in 49 of them (in 1625 if it takes them all).
+double RingMegabytes(const FcArgs& a) { return 16e-6 * a.rows * DivUp(a.n, 4) * RingWindow(a); }
+double ColumnUs(const FcArgs& a) {
+  struct Cost {
+    double pass, row, act, group;  // per pass of 1024 threads; per 1000 rows: weights, activations; per work-group of 1024 threads
+  };
+  static const Cost kCost[2][3] = {{{1.5, 1.4, 0.82, 0.18}, {1.8, 1.2, 0.83, 0.46}, {4.3, 1.5, 0.68, 1.1}},   // fp16: 1, 2, 4 slots
+                                   {{1.7, 1.2, 0.65, 0.49}, {2.6, 1.2, 0.72, 1.2}, {8.5, 2.0, 0.49, 2.9}}};  // fp32
+  const int ns = DivUp(a.n, 4), window = RingWindow(a), slots = ColumnSlots(a);
+  const bool small = window <= 512;
+  const Cost& c = kCost[a.act_f16 ? 0 : 1][slots == 1 ? 0 : (slots == 2 ? 1 : 2)];
+  // work-groups of the busiest XCD, as the kernel deals them
+  const int runs = std::min(8, DivUp(ns, 8)), copies = runs == 1 ? 8 : (runs == 2 ? 4 : (runs <= 4 ? 2 : 1));
+  const long planes = (long)DivUp(a.m, slots) * a.rows, together = small ? 32 : 8;
+  const long shared = planes <= together ? planes : std::max(together, (planes + copies - 1) / copies);
+  const double cus = (ns / 64 * 8 + std::min(8, ns % 64)) * (double)shared / 32.0;  // work-groups per CU
+  const double lines = std::min(1.0, a.src_rows * (double)a.m * (a.act_f16 ? 8 : 16) / 128.0);  // lines that a row's activations touch
+  const double chain = small ? 0.0 : std::max(1.0, std::ceil(cus / 2.0)) * DivUp(window, 2048) * c.pass;
+  const double work = cus * (window * (c.row + c.act * lines) / 1000.0 + c.group * (small ? 0.31 : 1.0));
+  return 3.0 + std::hypot(chain, work) + 0.16 * RingMegabytes(a);
+}
+double SplitUs(const FcArgs& a) {
+  struct Cost {
+    double fixed, pass, group, sum;
+  };
+  static const Cost kCost[3] = {{4.1, 2.7, 0.66, 1.5}, {5.0, 2.4, 0.88, 1.0}, {4.4, 4.7, 2.2, 1.7}};  // 1, 2, 3..4 tokens
+  const RingSplit r = SplitWindow(a);
+  const Cost& c = kCost[a.m == 1 ? 0 : (a.m == 2 ? 1 : 2)];
+  const double groups = (double)r.parts * DivUp(DivUp(a.n, 4), r.lanes) * a.rows;
+  const int passes = DivUp(DivUp(RingWindow(a), r.parts), r.rows_in_flight);
+  return c.fixed + std::hypot(std::max(1.0, std::ceil(groups / 512)) * passes * c.pass, groups / 256 * c.group) +
+         DivUp(r.parts, 128) * c.sum + 0.16 * DivUp(a.n, 4) * 4 * a.m * a.rows / 4096 + 0.055 * RingMegabytes(a);
+}
+double UnspecialisedUs(const FcArgs& a) {
+  const double groups = (double)DivUp(DivUp(a.n, 4), 16) * DivUp(a.m, 4) * a.rows, steps = DivUp(a.k, 64);
+  return 5.9 + std::hypot(0.74 * steps, groups / 256 * (0.47 * steps + 1.1)) + 0.24 * RingMegabytes(a);
+}
+// (longer windows were not measured in columns, but at 8192 rows x 256 channels and one token: 12.1 us, 8.8 split)
+bool ColumnMeasured(const FcArgs& a) { return RingWindow(a) <= (a.m == 1 ? 4097 : 8193); }
+
 bool FcW8RingSupported(const FcArgs& a) {
   if (!RingShapeOk(a) || a.ring_i_index < 0 || a.ring_o_index >= 0) return false;
   if (a.k > a.ring_size) return false;  // (the window stays within one turn of the ring)
   const int w_ks = DivUp(a.weights_k > 0 ? a.weights_k : a.k, 4);
   if (a.ring_size > 4 * w_ks || (a.weights_batch > 1 && a.ring_size != 4 * w_ks)) return false;
-  return a.m <= 64;
+  return a.m <= 64 && (PartsSupported(a) || ColumnUs(a) <= UnspecialisedUs(a));
 }
 
 // Ring over the output channels.  Below 64 KB of weights a launch costs what a launch costs on either
@@ -745,7 +814,7 @@ hipError_t LaunchFcW8RingO(const FcArgs& a, hipStream_t stream, const char** ker
   if (!FcW8RingOSupported(a)) return hipErrorInvalidValue;
   const RingParams p = MakeRingParams(a);
   if (kernel_name) *kernel_name = "fc_w8_ring_o_kernel";
-  // token slots: as above (4 tokens x 8192 positions x 256 channels: 3.6 us with two, 3.9 with four; 8 tokens x 16384 x
+  // token slots: as ColumnSlots (4 tokens x 8192 positions x 256 channels: 3.6 us with two, 3.9 with four; 8 tokens x 16384 x
   // 128: 4.2 against 4.1)
   int slots = (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 4) >= 512 ? 4 : 2;
   while (slots > p.m) slots /= 2;
@@ -756,31 +825,18 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
   if (!FcW8RingSupported(a)) return hipErrorInvalidValue;
   RingParams p = MakeRingParams(a);
   if (kernel_name) *kernel_name = "fc_w8_ring_i_kernel";
-  const int window = std::min(p.ks + 1, p.ring_rows + 1);
-  if (ColumnPreferred(a) || !PartsSupported(a)) {
-    // token slots of a work-group: two, so that the slices of a narrow cache (64 for a head of 256) occupy the chip
-    // (8 tokens x 8192 positions x 256 channels: 5.8 us, 8.6 with one slot, 6.2 with four); four where they do anyway
-    // (4096 positions x 512 channels: 5.25 against 5.8 us)
-    int slots = (long)p.ns * p.rows * DivUp(p.m, 4) >= 256 ? 4 : 2;
-    while (slots > p.m) slots /= 2;
-    const bool small = window <= 512;
+  if (!PartsSupported(a) || (ColumnMeasured(a) && ColumnUs(a) <= SplitUs(a))) {
+    const int slots = ColumnSlots(a);
+    const bool small = RingWindow(a) <= 512;
     p.xcd_runs = std::min(8, DivUp(p.ns, 8));
     p.xcd_mask = p.xcd_runs == 1 ? 7 : (p.xcd_runs == 2 ? 3 : (p.xcd_runs <= 4 ? 1 : 0));
     SetVariant(a.variant, "column");
     return a.act_f16 ? LaunchColumn<__half>(p, slots, small, stream) : LaunchColumn<float>(p, slots, small, stream);
   }
   SetVariant(a.variant, "split");
-  // lanes along the output slices: a power of two up to 64; parts: about 32 KB of weights each, at
-  // most what the workspace holds
-  int ls = 16;
-  while (ls < 64 && ls < p.ns) ls *= 2;
-  const int rows_in_flight = kRingThreads / ls * RingUnroll(p.m == 1 ? 1 : (p.m == 2 ? 2 : 4));
-  const size_t bytes = (size_t)window * p.ns * 16;
-  int parts = (int)std::min<size_t>(kRingMaxParts, std::max<size_t>(1, bytes / 32768));
-  parts = std::min(parts, std::max(1, DivUp(window, rows_in_flight)));
-  const size_t per_part = (size_t)a.rows * 4 * ((size_t)p.ns * 4 + 4);
-  parts = (int)std::min<size_t>(parts, a.partial_floats / per_part);
-  p.parts = std::max(parts, 1);
+  const RingSplit split = SplitWindow(a);
+  const int ls = split.lanes;
+  p.parts = split.parts;
   if (a.act_f16) {
     if (ls == 16) return LaunchRingT<__half, 16>(p, a.dst_f16, stream);
     if (ls == 32) return LaunchRingT<__half, 32>(p, a.dst_f16, stream);

@@ -13,7 +13,7 @@ import workloads as W
 from test_oracle_ring import make, rolled_product
 
 
-def run(axis, src_c, dst_c, ring, tokens, offsets, f16, batch=1, seed=1, src_end=None, dst_end=None, tiny=False):
+def run(axis, src_c, dst_c, ring, tokens, offsets, f16, batch=1, seed=1, src_end=None, dst_end=None, tiny=False, kernel=None, form=None):
     import torch
     td, mt = (np.float16, M.FLOAT16) if f16 else (np.float32, M.FLOAT32)
     q, _, scale, zp, bias = make(seed, src_c, dst_c, ring, axis, batch)
@@ -55,7 +55,8 @@ def run(axis, src_c, dst_c, ring, tokens, offsets, f16, batch=1, seed=1, src_end
         print("ring kernel", axis, src_c, dst_c, ring, "tokens", tokens, "batch", batch, "offset", off, "f16", f16, src_end, dst_end, flush=True)
         op.launch(torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        assert op.kernel_name == "fc_w8_ring_%s_kernel" % axis, op.kernel_name
+        assert op.kernel_name == (kernel or "fc_w8_ring_%s_kernel" % axis), op.kernel_name
+        assert form is None or op.kernel_variant == form, op.kernel_variant
         got = W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
         n_written = dst_c if dst_end is None else min((dst_end + 31) // 32 * 32, ns * 4)
         if n_written < dst_c:
@@ -170,3 +171,15 @@ def test_ring_infinite_activations(axis, src_c, dst_c, ring, tokens, f16, zero_p
     assert np.isinf(ref[0]).any() and np.isnan(ref[0]).any()
     assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isinf(got), np.isinf(ref))
     assert np.array_equal(got[np.isinf(got)], ref[np.isinf(ref)])
+
+
+# the kernel by window, width, tokens and rows: column walk, split window (up to 4 tokens per row and 16 in all), unspecialised
+@pytest.mark.parametrize("src_c,dst_c,tokens,batch,f16,form", [
+    (1024, 64, 1, 1, True, "column"), (2100, 256, 4, 1, True, "column"), (16380, 24, 1, 1, True, "column"), (16388, 24, 1, 1, True, "split"),
+    (32760, 16, 3, 1, False, "column"), (32772, 16, 3, 1, False, "split"), (2048, 1200, 1, 4, True, "split"), (2560, 4096, 2, 1, False, "split"),
+    (640, 72, 5, 4, True, "column"), (4096, 20, 17, 1, True, "column"), (300, 40, 4, 5, False, "column"), (2100, 520, 9, 4, False, "unspecialised"),
+    (2100, 1400, 33, 1, True, "unspecialised"), (64, 12, 64, 1, True, "column")])
+def test_ring_i_kernel_choice(src_c, dst_c, tokens, batch, f16, form):
+    ring = (src_c + 3) // 4 * 4
+    run("i", src_c, dst_c, ring, tokens, [0, src_c // 2 + 1], f16, batch=batch, seed=src_c,
+        **(dict(kernel="fc_generic_kernel", form="") if form == "unspecialised" else dict(form=form)))
