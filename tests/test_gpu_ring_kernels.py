@@ -66,11 +66,14 @@ def run(axis, src_c, dst_c, ring, tokens, offsets, f16, batch=1, seed=1, src_end
             for t in range(tokens):
                 a = act[b * tokens + t]
                 exact = rolled_product(q, a, scale, zp, bias, axis, ring, off, b, src_c, dst_c, active=active)[:n_written]
-                # fp32 sums of src_c products, in any order: (src_c + 8) roundings of the sum of magnitudes at worst; fp16
-                # results are rounded twice (result, bias)
-                mag = np.abs(a).sum() * 131.0 * scale[:n_written].astype(np.float64)
-                tol = 2.0 ** -24 * (src_c + 8) * mag + (2.0 ** -10 * (np.abs(exact) + np.abs(bias[:n_written])) + 2.0 ** -24 if f16 else
-                                                        2.0 ** -22 * np.abs(exact))
+                # fp32 sums: the products of a thread one after the other (some 100 at most), then a tree; every partial sum is of
+                # the size of the root of the sum of squares (weights of random sign) or, in the zero point's half, of the
+                # sum of magnitudes; a lost slice of 4 channels is sqrt(4 / src_c) of the former, over 0.01 at 33000 channels.
+                # fp16 results are rounded twice (result, bias)
+                s_abs = scale[:n_written].astype(np.float64)
+                size = np.sqrt((a.astype(np.float64) ** 2).sum()) * 74.0  # (rms of a weight: 127 / sqrt(3))
+                tol = 2.0 ** -24 * s_abs * (128 * size + 64 * np.abs(a).sum()) + (
+                    2.0 ** -10 * (np.abs(exact) + np.abs(bias[:n_written])) + 2.0 ** -24 if f16 else 2.0 ** -22 * (np.abs(exact) + np.abs(bias[:n_written])))
                 assert np.all(np.abs(got[b * tokens + t][:n_written] - exact) <= tol), (b, t, off)
 
 
@@ -183,3 +186,46 @@ def test_ring_i_kernel_choice(src_c, dst_c, tokens, batch, f16, form):
     ring = (src_c + 3) // 4 * 4
     run("i", src_c, dst_c, ring, tokens, [0, src_c // 2 + 1], f16, batch=batch, seed=src_c,
         **(dict(kernel="fc_generic_kernel", form="") if form == "unspecialised" else dict(form=form)))
+
+
+# A single activation of 1, scales of 1, no zero point: the result is that input channel's weights, exactly.  The first and last
+# channel, both sides of the seams of a slice, a wave, a pass of 256 and of 1024 threads, and where the window meets the ring's end
+@pytest.mark.parametrize("axis,src_c,dst_c,ring,tokens,form", [
+    ("i", 1021, 40, 1024, 8, "column"), ("i", 8190, 12, 8192, 6, "column"), ("i", 16384, 24, 16384, 1, "column"), ("i", 32757, 8, 32760, 4, "column"),
+    ("i", 16390, 20, 16392, 1, "split"), ("i", 33000, 24, 33004, 3, "split"), ("i", 2560, 6400, 2560, 2, "split"),
+    ("o", 68, 1000, 1024, 7, ""), ("o", 260, 515, 1000, 4, ""), ("o", 1030, 64, 64, 2, "")])
+@pytest.mark.parametrize("f16", [True, False])
+def test_ring_one_channel(axis, src_c, dst_c, ring, tokens, form, f16):
+    import torch
+    td, mt = (torch.float16, M.FLOAT16) if f16 else (torch.float32, M.FLOAT32)
+    rng = np.random.default_rng(src_c + dst_c)
+    o, i = (dst_c, ring) if axis == "i" else (ring, src_c)
+    q = rng.integers(-127, 128, size=(o, 1, 1, i), dtype=np.int8)
+    desc = M.make_desc(M.UINT8, M.LAYOUT_I4O4 if axis == "i" else M.LAYOUT_O4I4, (o + 3) // 4)
+    packed = torch.from_numpy(M.rearrange_int8_as_uint8(q, desc)).cuda()
+    ns, ks = (dst_c + 3) // 4, (src_c + 3) // 4
+    kw = {"ring_%s_offset_index" % axis: 0, "ring_size": ring, ("src" if axis == "i" else "dst") + "_channels": src_c if axis == "i" else dst_c}
+    op = M.fc_create(M.PRECISION_F32_F16 if f16 else M.PRECISION_F32, mt, mt, o, i, desc, scale_shape=(dst_c, 1), max_tokens=tokens, **kw)
+    act = torch.zeros((ks, tokens, 4), dtype=td, device="cuda")
+    out = torch.zeros((ns, tokens, 4), dtype=td, device="cuda")
+    params = torch.zeros(1, dtype=torch.int32, device="cuda")
+    op.bind([act, packed, torch.ones(ns * 4, dtype=td, device="cuda"), params], [out])
+    op.set_shape(1, 1, tokens)
+    for off in (0, 1, 2, 3, ring - 1, ring - 6):
+        seams = [0, 3, 4, 255, 256, 1023, 1024, 2047, 2048, 4095, 4096, 8191, 8192, ring - off - 1, ring - off, src_c - 5, src_c - 4, src_c - 1]
+        places = sorted({c for c in seams if 0 <= c < src_c})
+        params.fill_(off)
+        for first in range(0, len(places), tokens):
+            some = [places[min(first + t, len(places) - 1)] for t in range(tokens)]
+            act.zero_()
+            for t, c in enumerate(some):
+                act[c // 4, t, c % 4] = 1.0
+            out.fill_(7.0)
+            print("one channel", axis, src_c, dst_c, ring, off, some, f16, flush=True)
+            op.launch(torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            assert (op.kernel_name, op.kernel_variant) == ("fc_w8_ring_%s_kernel" % axis, form)
+            got = W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
+            for t, c in enumerate(some):
+                want = q[:, 0, 0, (c + off) % ring] if axis == "i" else q[(np.arange(dst_c) + off) % ring, 0, 0, c]
+                assert np.array_equal(got[t], want.astype(np.float64)), (off, c)
