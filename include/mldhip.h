@@ -330,7 +330,8 @@ typedef struct {
    * mldhip_fc_batch_ids_create (the two ops of a layer read the same buffers).  The source is one row of tokens sorted by matrix; matrix g multiplies
    * the params[packed_params_offset + g] tokens that start at token
    * params[packed_params_offset + packed_num_groups + g] (fully_connected_util.cc:263-277), at most
-   * packed_max_group_size of them; dst tokens that belong to no group are not written.  "params" is
+   * packed_max_group_size of them; dst tokens that belong to no group are not written, and no token
+   * belongs to two groups.  "params" is
    * the last src object; mldhip_op_set_shape(op, 1, 1, tokens). */
   int32_t packed_params_offset, packed_num_groups, packed_max_group_size;
   /* Channels of the src / dst tensors where they differ from the weights' i / o: ringed weights

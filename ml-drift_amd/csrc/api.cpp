@@ -804,20 +804,21 @@ int mldhip_op_launch(mldhip_op* op, void* stream_ptr) {
       FcArgs a;
       if (int rc = BuildFcArgs(op, &a)) return rc;
       // Runtime channel bounds at 1..4 tokens run on the streaming GEMVs (which stop their K loop at the
-      // bound and skip the dst strips beyond it); ringed weights, packed groups off the matrix cores and
-      // bounds at more tokens on the unspecialised kernel.
+      // bound and skip the dst strips beyond it); packed groups off the matrix cores, bounds at more tokens and ringed
+      // weights that the kernels of their own do not take on the unspecialised kernel.
       const bool bounded = a.params != nullptr;
       const bool bounded_stream = bounded && a.packed_params_offset < 0 && a.ring_i_index < 0 && a.ring_o_index < 0 &&
                                   (FcW4StreamSupported(a) || FcW8StreamSupported(a));
       const bool force_generic = GetTuning().force_generic > 0 || (bounded && !bounded_stream);
-      // ringed weights over the input channels at a few tokens: the kernel that walks the ring's rows
+      // ringed weights: over the input channels the kernels that walk the ring's rows, where they are faster; over the output
+      // channels the kernel for 64 KB of weights and more
       if (GetTuning().force_generic <= 0 && FcW8RingSupported(a)) {
         e = LaunchFcW8Ring(a, stream, &op->last_kernel);
       } else
       if (GetTuning().force_generic <= 0 && FcW8RingOSupported(a)) {
         e = LaunchFcW8RingO(a, stream, &op->last_kernel);
       } else
-      // packed groups: the matrix-core GEMM with one launch plane per matrix where it serves the shape
+      // packed groups: the matrix-core GEMM over the token tiles of all groups where it serves the shape
       if (GetTuning().force_generic <= 0 && FcW4MfmaPackedSupported(a)) {
         e = LaunchFcW4Mfma(a, stream, &op->last_kernel);
       } else

@@ -1845,11 +1845,10 @@ struct SkinnyPlan {
 // 28672 at 24 tokens 0.8).  Above 32 tokens only where it is cut at least 4 ways: 16384 -> 2048 at 64 tokens 19.8 / 16.0, at 100,
 // cut in 2, 20.4 / 23.3; whole K of 6144 and more in 64-channel tiles against a direct kernel cut in 2: 0.92..1.01.  64-channel
 // tiles up to 16 tokens from more than 512 input channels on: 0.97 below.
-int W4KSplit(int m, int k, int n);
-SkinnyPlan PlanSkinny(int m, int k, int n) {
+// (direct_split: W4KSplit(m, k, n))
+SkinnyPlan PlanSkinny(int m, int k, int n, int direct_split) {
   const int token_tiles = DivUp(m, 32), strips_xcd = DivUp(DivUp(n, 64), 8);
   if (m > kSkinnyMaxTiledTokens) return {0, 1};
-  const int direct_split = W4KSplit(m, k, n);
   if (k >= kSkinnySplitK) {
     const int s = SkinnyKSplit(k, n, token_tiles);
     if ((long)strips_xcd * token_tiles * s > 32) return {0, 1};
@@ -1906,8 +1905,9 @@ int W4TokenBlocks(int m, int n) {
 // keeps at least 24 steps of 16 channels (below that the partial sums and the second kernel
 // cost more than the idle CUs: 2048 x 2048 at 128 tokens 10.9 -> 8.5 us without a split).
 int W4KSplit(int m, int k, int n) {
-  if (W4TokenBlocks(m, n) == 4) return 1;
-  const long tiles = (long)DivUp(n, 128) * DivUp(m, W4TokenBlocks(m, n) * 32);
+  const int fm = W4TokenBlocks(m, n);
+  if (fm == 4) return 1;
+  const long tiles = (long)DivUp(n, 128) * DivUp(m, fm * 32);
   const int steps = DivUp(k, 16);
   int s = 1;
   while (s < 8 && tiles * s * 2 <= 256 && steps / (8 * s * 2) >= 24) s *= 2;
@@ -2135,7 +2135,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   // Few tokens, or few tiles: fc_w4_mfma_skinny_kernel.  Below 5 tokens the token forms of the GEMVs are
   // faster (628 us at 4 tokens against 870 before the loop was pipelined) and callers come here only where those do not serve.
   // (gemm_fm, gemm_ksplit and the others ask for the direct kernel's shapes.)
-  const SkinnyPlan skinny = PlanSkinny(a.m, p.k, n_total);
+  const SkinnyPlan skinny = PlanSkinny(a.m, p.k, n_total, W4KSplit(a.m, p.k, n_total));
   const bool direct_asked = tune.gemm_fm > 0 || tune.gemm_ksplit > 0 ||
                             (a.m > kSkinnyMaxTokens && (tune.gemm_no_pair > 0 || tune.gemm_dual >= 0 || tune.gemm_xcd_m > 0));
   if (!gated && a.weight_bits == 4 && skinny.tile > 0 && !direct_asked) {
@@ -2248,7 +2248,7 @@ hipError_t LaunchFcW4MfmaGated(const FcArgs& gate, const FcArgs& up, int activat
 size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n) {
   size_t need = 0;
   for (int m = kGemvMaxTokens + 1; m <= max_tokens; ++m) {
-    const int s = std::max(W4KSplit(m, k, n), PlanSkinny(m, k, n).ksplit);
+    const int direct = W4KSplit(m, k, n), s = std::max(direct, PlanSkinny(m, k, n, direct).ksplit);
     if (s > 1) need = std::max(need, (size_t)s * DivUp(n, 4) * 4 * m);
   }
   return need;

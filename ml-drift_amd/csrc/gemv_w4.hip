@@ -1697,8 +1697,9 @@ hipError_t LaunchFcW4StreamFused(const FcArgs* args, int count, hipStream_t stre
     const bool wide = (long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 192;
     // One token per row over output groups of 16 slices: the contiguous-strip kernel, from one 64-channel strip for every
     // second CU on: a strip's K lies in one piece, which counts for more than the idle CUs.  (2 of 8 matrices, 2048 x 4096,
-    // 128 strips: 24.1 -> 17.1 us for the three projections of a layer.  It is ahead at 96 strips too, 2048 x 768, 8 of
-    // 128 matrices: 16.0 -> 14.3 us; there the streaming kernel is what the tests of batched launches require.)
+    // 128 strips: 24.1 -> 17.1 us for the three projections of a layer; of 2041 random launches of 96 .. 260 strips, K 256 ..
+    // 8192, one got 5 % slower by the line's move from 192 to 128.  Below 128 two shapes were timed, 96 strips of 2048 x 768 among
+    // them: 16.0 against 14.3 us, the strip kernel ahead there too; that is no line, and those launches stay on the streaming kernel.)
     if ((long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 128 && StripKernelServes(args, count)) {
       if (kernel_name) *kernel_name = "fc_w4_strip_kernel";
       return LaunchStrip(p, args, count, grouped, stream);

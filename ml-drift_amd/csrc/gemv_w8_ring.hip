@@ -14,8 +14,8 @@
 // source channels 4 w - offset % 4 + {0, 1, 2, 3}; those outside [0, channels multiplied) count as
 // zero.  That needs ring_size % 4 == 0.
 //
-// Two kernels walk it: fc_w8_ring_i_column_kernel (one launch; below) and, for the longest windows at up to 4
-// tokens, fc_w8_ring_i_kernel, described here.
+// Two kernels walk it: fc_w8_ring_i_column_kernel (one launch; below) and, for the longest windows and wide caches
+// at up to 4 tokens, fc_w8_ring_i_kernel, described here.
 // Work-group = 256 threads = LS lanes along the output slices x 256 / LS rows in flight, four
 // rows per thread and pass; the window is split across blockIdx.x, the slices (in chunks of LS)
 // across blockIdx.y, the dst rows of a launch with batched weights across blockIdx.z.  Every

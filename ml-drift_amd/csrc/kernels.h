@@ -95,8 +95,7 @@ struct FcArgs {
   // tokens of the one source row are sorted by weight matrix; params[offset + g] tokens starting at
   // token params[offset + weights_batch + g] are multiplied with matrix g.  offset < 0 = not set.
   int packed_params_offset = -1, packed_max_group_size = 0;
-  // Ringed weights (fully_connected.cc:411-441, 676-706; uint8, one output group, the unspecialised
-  // kernel): the offset is params[ring_*_index] modulo ring_size.  ring_i: k = src channels, the
+  // Ringed weights (fully_connected.cc:411-441, 676-706; uint8, one output group): the offset is params[ring_*_index] modulo ring_size.  ring_i: k = src channels, the
   // I4O4 buffer holds weights_k input channels; ring_o: n = dst channels, the O4I4 buffer holds
   // ring_size output channels.
   int ring_o_index = -1, ring_i_index = -1, ring_size = 0;
@@ -109,8 +108,8 @@ constexpr int kGemvMaxTokens = 4;
 constexpr int kGemvMaxKSplit = 32;
 
 hipError_t LaunchFcGeneric(const FcArgs& a, hipStream_t stream, const char** kernel_name);
-// Ringed uint8 weights with the ring over the input channels, up to 64 tokens per row: walks the ring's own
-// K-slice rows (aligned 16-byte blocks) and shifts the activations.
+// Ringed uint8 weights with the ring over the input channels, up to 64 tokens per row where that is faster than the
+// unspecialised kernel: walks the ring's own K-slice rows (aligned 16-byte blocks) and shifts the activations.
 bool FcW8RingSupported(const FcArgs& a);
 hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kernel_name);
 // The same with the ring over the output channels (query x key cache).
