@@ -625,9 +625,10 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   constexpr int RPH = WAVES == 4 && FM == 4 ? 16 : 8;  // accumulator registers (x 4 MFMAs) per phase
   __shared__ float4 red[WAVES == 1 ? 1 : 2][WAVES][WAVES == 1 ? 1 : RPH][64];
 
-  // One batch of scalar loads (in one statement: of two, the compiler may wait for the first) for what the prologue reads.  (Left alone, it fetches
-  // every argument where it is first used: seven scalar round trips, one behind the other, in
-  // front of the first operand load.  Input-only operands keep the pointers' address spaces.)
+  // One batch of scalar loads for what the prologue reads, in one statement (of two, the compiler may
+  // wait for the first).  (Left alone, it fetches every argument where it is first used: seven scalar
+  // round trips, one behind the other, in front of the first operand load.  Input-only operands keep
+  // the pointers' address spaces.)
   asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.ksplit), "s"(p.xcd_m), "s"(p.group_shift),
                "s"(p.b_bytes), "s"(p.act), "s"(p.magic_lo), "s"(p.magic_hi), "s"(p.mask_lo), "s"(p.mask_hi), "s"(p.segments),
                "s"(p.geo_tiles_m), "s"(p.geo_rect_m), "s"(p.geo_rect_n), "s"(p.geo_xm_shift), "s"(p.geo_rect_m_magic),
