@@ -562,8 +562,12 @@ __device__ __forceinline__ void SwapRegisters(u32x4& a, u32x4& b) {
 
 // ZP: the weights have a zero-point tensor (same shape as the scales): w = (u - shift) * s - zp * s,
 // one fused multiply-add per pair of weights (zp * s is formed once per channel and scale group).
-// PAIR (FM even, token count even): a lane's tokens for the MFMA pair (fm, fm+1) are neighbours
-// (2j, 2j+1 instead of j, j+32), so one 16-byte load brings both activation operands.
+// PAIR (FM even): a lane's tokens for the MFMA pair (fm, fm+1) are neighbours (2j, 2j+1 instead of j, j+32), so
+// one 16-byte load brings both activation operands.  With an odd token count every other row starts 8 bytes off a 16-byte
+// boundary, which these loads (4-byte alignment) take; the last token's partner is then the next row's first token, or, past
+// the buffer's end, zero (the range check is per 32-bit word), in a column of the MFMA that is never stored.  Tokens read one
+// by one there, without the 128-token and two-tile forms: 8191 tokens x 4096 x 14336 1216 us, 856 like this; 2047 x 2048 x 4096
+// 55.5 / 38.9; 333 x 1656 x 2900 with uint8 weights 16.1 / 15.1.
 // MULTI: the launch covers more than one matrix (the single-matrix instantiation reads its
 // arguments at fixed offsets instead of through a dependent scalar load).
 // WB: weight bits.  8: the packed buffer holds 16-byte blocks, word i = input channel i of the
@@ -1899,7 +1903,7 @@ void LaunchSkinny(bool zp, const GemmParams& p, hipStream_t stream) {
 int W4TokenBlocks(int m, int n) {
   const long tiles_n = DivUp(n, 128);
   const long tiles64 = tiles_n * DivUp(m, 64), tiles128 = tiles_n * DivUp(m, 128);
-  if (m % 2 == 0 && tiles128 >= 256 && 1.85 * DivUp(tiles128, 256L) < (double)DivUp(tiles64, 256L)) return 4;
+  if (tiles128 >= 256 && 1.85 * DivUp(tiles128, 256L) < (double)DivUp(tiles64, 256L)) return 4;
   return (m > 32 && tiles64 >= 128) ? 2 : 1;
 }
 // K split across work-groups: doubled while the grid stays within the CU count and every wave
@@ -2168,7 +2172,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   set_variant("direct");
   // token tile and K split follow the launch as a whole (all channels of all matrices)
   int fm = W4TokenBlocks(a.m, n_total);
-  if (tune.gemm_fm > 0) fm = tune.gemm_fm == 1 ? 1 : (tune.gemm_fm == 4 && a.m % 2 == 0 ? 4 : 2);
+  if (tune.gemm_fm > 0) fm = tune.gemm_fm == 1 ? 1 : (tune.gemm_fm == 4 ? 4 : 2);
   p.ksplit = 1;
   if (fm == W4TokenBlocks(a.m, n_total)) p.ksplit = W4KSplit(a.m, a.k, n_total);
   if (tune.gemm_ksplit > 0) p.ksplit = tune.gemm_ksplit;
@@ -2176,7 +2180,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   for (int i = 0; i < count; ++i)
     while (p.ksplit > 1 && (size_t)p.ksplit * p.seg[i].ns * 4 * a.m > args[i].partial_floats) p.ksplit /= 2;
   const int tiles_m = DivUp(a.m, fm * 32);
-  const bool pair = a.m % 2 == 0 && tune.gemm_no_pair <= 0;
+  const bool pair = tune.gemm_no_pair <= 0;
   // Two channel tiles per work-group when the rounds of 256 work-groups come out cheaper: a
   // two-tile work-group takes 1.87 x the time of a one-tile one, and a last round filled to the
   // fraction f costs 0.45 + 0.55 f of a full one (fitted to same-box timings of 14 shapes).

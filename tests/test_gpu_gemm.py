@@ -216,6 +216,27 @@ def test_gemm_two_tiles_per_work_group(oracle, bits, m, k, n, groups, zp):
         check_restatement(oracle, got[:small], sub, "kernel restatement")
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("fm,dual", [(2, 0), (2, 1), (4, 0), (4, 1)])
+@pytest.mark.parametrize("m,k,n,groups,zp", [(33, 64, 132, 2, False), (65, 136, 128, 1, True), (127, 96, 260, 3, False), (129, 1000, 388, 1, False)])
+def test_gemm_odd_token_counts(bits, fm, dual, m, k, n, groups, zp):
+    """An odd token count: the last token travels in a pair with the next row's first token (or with what lies past the tensor).
+    Each token's sums are formed in the same order as with one token more, so the results are the same bit for bit; the first
+    token is infinite, which may show in its own results only."""
+    case = W.make_fc_case(seed=m + k, m=m + 1, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups,
+                          with_bias=True, with_zero_point=zp)
+    with M.tuning(gemm_fm=fm, gemm_dual=dual, gemm_ksplit=1):
+        even = run_w4(case, reference_layout=True)
+        check_fp(even, textbook(case), case, "one token more")
+        odd = dict(case, m=m, act=np.array(case["act"][:m]))
+        odd["act"][0] = np.inf
+        dev = W.FcDevice(odd, reference_layout=True)
+        dev.run()
+        got = dev.result()
+    assert np.array_equal(got[1:], even[1:m])
+    assert not np.isfinite(got[0]).any()
+
+
 def test_gemm_modes_random_sweep():
     """Seeded sweep over shapes with the two-tile mode forced on and off and every token tile
     forced in turn: all against the textbook reference at the fp16 bar."""
