@@ -186,7 +186,7 @@ int mldhip_set_tuning(const char* name, int value) {
       {"gemv_one_chunk", &t.gemv_one_chunk},
       {"gemv_lpr", &t.gemv_lpr}, {"gemv_waves", &t.gemv_waves}, {"gemv_ksplit", &t.gemv_ksplit},
       {"gemv_narrow_max_mb", &t.gemv_narrow_max_mb}, {"gemm_fm", &t.gemm_fm}, {"gemm_ksplit", &t.gemm_ksplit},
-      {"gemm_no_pair", &t.gemm_no_pair}, {"gemm_dual", &t.gemm_dual}, {"gemm_xcd_m", &t.gemm_xcd_m},
+      {"gemm_no_pair", &t.gemm_no_pair}, {"gemm_waves", &t.gemm_waves}, {"gemm_dual", &t.gemm_dual}, {"gemm_xcd_m", &t.gemm_xcd_m},
       {"gemm_i8_fm", &t.gemm_i8_fm}, {"gemm_tiled", &t.gemm_tiled}};
   for (const auto& k : knobs)
     if (std::strcmp(name, k.name) == 0) {
@@ -367,7 +367,8 @@ static int AllocWorkspace(mldhip_op* op, int n, bool ring_i = false) {
   }
   const int n_pad = DivUp(n, 4) * 4;
   op->partial_floats = std::max((size_t)kGemvMaxKSplit * kGemvMaxTokens * n_pad,
-                                FcW4MfmaWorkspaceFloats(op->fc.max_tokens, op->fc.i, op->fc.o));
+                                FcW4MfmaWorkspaceFloats(op->fc.max_tokens, op->fc.i, op->fc.o, std::max(op->fc.scale_i, 1),
+                                                        op->fc.weights.type == MLDHIP_UINT8 ? 8 : 4));
   // (the ring over the input channels: partial sums of the parts of its window)
   if (ring_i) op->partial_floats = FcW8RingWorkspaceFloats(op->fc.max_tokens, op->fc.o);
   hipError_t e = hipMalloc(reinterpret_cast<void**>(&op->partial), op->partial_floats * sizeof(float));

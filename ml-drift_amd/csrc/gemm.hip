@@ -31,6 +31,7 @@ namespace {
 
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4_word __attribute__((ext_vector_type(4), aligned(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 typedef int int16v_t __attribute__((ext_vector_type(16)));
 typedef int int4v_t __attribute__((ext_vector_type(4)));
@@ -87,7 +88,6 @@ struct GemmParams {
   int group_shift;  // log2(group_size / 16) when that is a power of two, else -1 (not supported by the direct kernel)
   int xcd_m;        // fp16 path: the 8 XCDs form an xcd_m x (8 / xcd_m) grid over (token tiles, channel tiles)
   int gate_activation;  // gated fp16 launch: MLDHIP_GATE_*
-  int dual;             // fp16 path: a work-group owns two neighbouring channel tiles
   // fp16 path, packed groups (ConvRuntimeCheckDesc::PackedGroups): the tokens of weight matrix g of
   // pg_groups are min(pg_params[pg_offset + g], pg_max) many from token
   // pg_params[pg_offset + pg_groups + g] of the one source row.  pg_groups = 0: not set.
@@ -579,11 +579,7 @@ __device__ __forceinline__ void SwapRegisters(u32x4& a, u32x4& b) {
 // second half on up, each half splitting K among its waves; the main loop is the same.  In the
 // reduction the wave that adds the copies of a register adds the two halves separately and so
 // holds the gate and the up value of the same slice and token.
-// DUAL: the same split of the waves for an ordinary launch: the work-group owns two neighbouring
-// channel tiles (2j, 2j + 1 of the launch), one per half.  The two halves read the same
-// activations, so every activation tile is fetched from L2 once for 256 channels, and there are
-// half as many work-groups and reduction rounds; for launches with many tiles.
-enum { kModePlain = 0, kModeGated = 1, kModeDual = 2, kModePacked = 3 };
+enum { kModePlain = 0, kModeGated = 1, kModePacked = 2 };
 // Entry `index` of the launch's matrix list, by value.  Every field of every entry sits at a fixed
 // offset of the kernel arguments, so all of them are fetched by one batch of scalar loads and
 // chosen with scalar selects; indexing the list with a run-time number makes the entry's loads
@@ -615,7 +611,7 @@ __device__ __forceinline__ int WaveInclusiveSum(int v) {
 
 template <int WB, int FM, int U, int WAVES, bool ZP, bool PAIR, bool MULTI, int MODE = kModePlain>
 __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct_kernel(GemmParams p) {
-  constexpr bool GATED = MODE == kModeGated, DUAL = MODE == kModeDual, HALVES = GATED || DUAL, PACKED = MODE == kModePacked;
+  constexpr bool GATED = MODE == kModeGated, PACKED = MODE == kModePacked;
   static_assert(!PACKED || (!PAIR && !MULTI), "packed groups: one matrix per group, tokens read one by one");
   static_assert(WB == 4 || WB == 8, "uint4 or uint8 weights");
   static_assert(!GATED || (!ZP && !MULTI), "the gated pair is symmetric and is the whole launch");
@@ -649,8 +645,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   // tiles and the weight tiles of that rectangle, and the L2 fetches each of them once.  Inside
   // the rectangle the token tile runs fastest, so that the tiles in flight at any time reuse the
   // same few activation tiles while the weights stream through.
-  const int tiles_n_all = p.seg[MULTI ? p.segments - 1 : 0].tile_end;  // channel tiles of all matrices of the launch
-  const int tiles_n = DUAL ? (tiles_n_all + 1) / 2 : tiles_n_all;        // channel tiles of the grid
+  const int tiles_n = p.seg[MULTI ? p.segments - 1 : 0].tile_end;  // channel tiles of all matrices of the launch
   // Packed groups: this work-group's matrix and the run of tokens it multiplies (else: all tokens).
   int m_lo = 0, m_hi = p.m, pg_e = 0;
   const int tiles_m = p.geo_tiles_m;  // (packed groups: the most token tiles that the groups can have together)
@@ -663,8 +658,8 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   // (packed groups: neighbouring token tiles go to different XCDs, so that the numbers that turn out to have no
   // tokens are spread over them)
   int tm = PACKED ? ((int)blockIdx.z * rect_m + local_m) * xm + (xcd & (xm - 1)) : (xcd & (xm - 1)) * rect_m + local_m;
-  const int tn_grid = (xcd >> p.geo_xm_shift) * rect_n + local_n;
-  if (tm >= tiles_m || tn_grid >= tiles_n) return;
+  int tn = (xcd >> p.geo_xm_shift) * rect_n + local_n;
+  if (tm >= tiles_m || tn >= tiles_n) return;
   const int matrices = PACKED ? p.pg_groups : 1;
   if constexpr (PACKED) {
     // Token tile tm of the launch -> a group and the tile inside it.  The group sizes are known on the device
@@ -695,27 +690,20 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
     if (found < 0) return;  // (the whole work-group: every wave counts the same)
     pg_e = found;
   }
-  // channel tile of the launch -> matrix of the launch (return value) and tile inside it
-  auto locate = [&](int& tile) {
-    int seg_index = 0;
-    if (MULTI && p.segments > 1 && tile >= p.seg[0].tile_end) {
-      seg_index = (p.segments > 2 && tile >= p.seg[1].tile_end) ? 2 : 1;
-      tile -= p.seg[seg_index - 1].tile_end;
-    }
-    return seg_index;
-  };
-  constexpr int KW = HALVES ? WAVES / 2 : WAVES;  // waves that share one tile's K
-  const int half = HALVES ? __builtin_amdgcn_readfirstlane(wave / KW) : 0;
-  int tn = DUAL ? 2 * tn_grid + half : tn_grid;
-  const bool tile_ok = !DUAL || tn < tiles_n_all;  // the last pair of an odd count has one tile
-  if (!tile_ok) tn = 0;
-  const int si = locate(tn);
+  // channel tile of the launch -> matrix of the launch and tile inside it
+  int si = 0;
+  if (MULTI && tn >= p.seg[0].tile_end) {
+    si = (p.segments > 2 && tn >= p.seg[1].tile_end) ? 2 : 1;
+    tn -= p.seg[si - 1].tile_end;
+  }
+  constexpr int KW = GATED ? WAVES / 2 : WAVES;  // waves that share one tile's K
+  const int half = GATED ? __builtin_amdgcn_readfirstlane(wave / KW) : 0;
   const W4Segment sg = PickSegment<GATED || MULTI>(p, GATED ? half : (MULTI ? si : 0));
   const int slice0 = tn * (BN / 4);  // first output slice of the tile
   const int m0 = m_lo + tm * BM;
   if (m0 >= m_hi) return;  // (packed groups: a tile beyond the group's size; the whole work-group leaves)
   const int nsi = slice0 + i32;
-  const bool n_ok = tile_ok && nsi < sg.ns;
+  const bool n_ok = nsi < sg.ns;
 
   // This wave's range of 16-channel steps.  The buffer descriptors of the weights and the
   // activations end where the wave's share of K ends, so the prefetches that run past it (and
@@ -1039,23 +1027,10 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   // 8*(v/4) + 4*g2 + v%4 and token i32, and the four MFMAs hold the slice's four channels: one
   // 8-byte store.
   // GATED: copies 0 .. KW-1 are gate's, the others up's; the two sums are rounded to fp16 (+ bias)
-  // as the two FullyConnected nodes would store them, then combined in fp32.  DUAL: the two sums
-  // belong to the two tiles of the work-group.
-  int tile_b = 2 * tn_grid + 1;  // DUAL: the second tile
-  const bool tile_b_ok = DUAL && tile_b < tiles_n_all;
-  if (!tile_b_ok) tile_b = 0;
-  int tile_a = DUAL ? 2 * tn_grid : tn;
-  const int seg_a = DUAL ? locate(tile_a) : si, seg_b = DUAL ? locate(tile_b) : 0;
-  const W4Segment sga = PickSegment<!GATED && MULTI>(p, GATED ? 0 : (MULTI ? seg_a : 0));
-  const W4Segment sgb = PickSegment<GATED || MULTI>(p, GATED ? 1 : (MULTI ? seg_b : 0));
-  const int slice0_a = DUAL ? tile_a * (BN / 4) : slice0, slice0_b = tile_b * (BN / 4);
-  // one slice of four channels of one token: the K-split partial sums, or the fp16 result
-  auto store = [&](const W4Segment& sgx, int slice, int mi, const float4& sum) {
-    if (p.ksplit > 1) {
-      // this work-group's share of K: fp32 sums for the second pass
-      *reinterpret_cast<float4*>(sgx.partial + (((size_t)blockIdx.y * sgx.ns + slice) * p.m + mi) * 4) = sum;
-      return;
-    }
+  // as the two FullyConnected nodes would store them, then combined in fp32.
+  const W4Segment sga = PickSegment<false>(p, 0), sgb = p.seg[1];  // GATED: gate's and up's
+  // one slice of four channels: the K-split partial sums, or the fp16 result, of token mi and, where `both`, token mi + 1 behind it
+  auto round4 = [](const W4Segment& sgx, int slice, const float4& sum) {
     __half h[4] = {__float2half_rn(sum.x), __float2half_rn(sum.y), __float2half_rn(sum.z), __float2half_rn(sum.w)};
     if (sgx.bias) {
 #pragma unroll
@@ -1064,79 +1039,99 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
     u32x2 o;
     o[0] = (uint32_t)__half_as_ushort(h[0]) | ((uint32_t)__half_as_ushort(h[1]) << 16);
     o[1] = (uint32_t)__half_as_ushort(h[2]) | ((uint32_t)__half_as_ushort(h[3]) << 16);
-    *reinterpret_cast<u32x2*>(sgx.dst + ((size_t)slice * p.m + mi) * 4) = o;
+    return o;
   };
-  static_assert(16 % RPH == 0 && RPH % WAVES == 0, "phases tile the 16 registers, waves tile a phase");
+  auto write16 = [&](const W4Segment& sgx, int slice, int mi, bool both, u32x2 o0, u32x2 o1) {
+    __half* at = sgx.dst + ((size_t)slice * p.m + mi) * 4;
+    if (both)
+      *reinterpret_cast<u32x4_word*>(at) = u32x4_word{o0[0], o0[1], o1[0], o1[1]};
+    else
+      *reinterpret_cast<u32x2*>(at) = o0;
+  };
+  auto store = [&](const W4Segment& sgx, int slice, int mi, bool both, const float4& s0, const float4& s1) {
+    if (p.ksplit > 1) {
+      // this work-group's share of K: fp32 sums for the second pass
+      float4* at = reinterpret_cast<float4*>(sgx.partial + (((size_t)blockIdx.y * sgx.ns + slice) * p.m + mi) * 4);
+      at[0] = s0;
+      if (both) at[1] = s1;
+      return;
+    }
+    write16(sgx, slice, mi, both, round4(sgx, slice, s0), both ? round4(sgx, slice, s1) : u32x2{0u, 0u});
+  };
+  // Tokens that a lane finishes together: a pair that it holds is one 16-byte store.
+  constexpr int E = PAIR && (WAVES == 1 || (RPH / 2) % WAVES == 0) ? 2 : 1;
   if constexpr (WAVES == 1) {  // the wave holds whole sums
 #pragma unroll
-    for (int fm = 0; fm < FM; ++fm) {
+    for (int fm = 0; fm < FM; fm += E) {
       const int mi = token(fm);
       if (mi >= m_hi) continue;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int slice = slice0 + 8 * (v >> 2) + 4 * g2 + (v & 3);
-        if (slice < sg.ns) store(sg, slice, mi, make_float4(acc[0][fm][v], acc[1][fm][v], acc[2][fm][v], acc[3][fm][v]));
+        if (slice < sg.ns)
+          store(sg, slice, mi, E == 2 && mi + 1 < m_hi, make_float4(acc[0][fm][v], acc[1][fm][v], acc[2][fm][v], acc[3][fm][v]),
+                make_float4(acc[0][fm + E - 1][v], acc[1][fm + E - 1][v], acc[2][fm + E - 1][v], acc[3][fm + E - 1][v]));
       }
     }
-    return;
-  }
+  } else {
+    constexpr int RPT = RPH / E, PHASES = 16 / RPT;  // registers of a token within a phase; phases of a token
+    static_assert(16 % RPT == 0 && RPT % WAVES == 0, "phases tile the 16 registers, waves tile a phase");
+    auto put = [&](int phase) {  // this wave's copy of a phase
+      const int fm = phase / PHASES * E, ph = phase % PHASES;
 #pragma unroll
-  for (int fm = 0; fm < FM; ++fm) {
-    const int mi = token(fm);
+      for (int j = 0; j < RPT; ++j)
 #pragma unroll
-    for (int ph = 0; ph < 16 / RPH; ++ph) {
-      const int buf = (fm * (16 / RPH) + ph) & 1;
-#pragma unroll
-      for (int j = 0; j < RPH; ++j) {
-        const int v = ph * RPH + j;
-        red[buf][wave][j][lane] = make_float4(acc[0][fm][v], acc[1][fm][v], acc[2][fm][v], acc[3][fm][v]);
-      }
-      LdsBarrier();
-#pragma unroll
-      for (int q = 0; q < RPH / WAVES; ++q) {
-        const int j = q * WAVES + wave;
-        float4 sum = red[buf][0][j][lane];
-#pragma unroll
-        for (int c = 1; c < KW; ++c) {
-          const float4 o = red[buf][c][j][lane];
-          sum.x += o.x;
-          sum.y += o.y;
-          sum.z += o.z;
-          sum.w += o.w;
+        for (int e = 0; e < E; ++e) {
+          const int v = ph * RPT + j;
+          red[phase & 1][wave][j * E + e][lane] = make_float4(acc[0][fm + e][v], acc[1][fm + e][v], acc[2][fm + e][v], acc[3][fm + e][v]);
         }
-        const int v = ph * RPH + j;
-        const int slice_l = 8 * (v >> 2) + 4 * g2 + (v & 3);  // slice inside the tile
-        if constexpr (HALVES) {
-          float4 sum_b = red[buf][KW][j][lane];
+    };
+    put(0);
 #pragma unroll
-          for (int c = KW + 1; c < WAVES; ++c) {
-            const float4 o = red[buf][c][j][lane];
-            sum_b.x += o.x;
-            sum_b.y += o.y;
-            sum_b.z += o.z;
-            sum_b.w += o.w;
+    for (int phase = 0; phase < FM / E * PHASES; ++phase) {
+      const int fm = phase / PHASES * E, ph = phase % PHASES;
+      const int mi = token(fm);
+      const bool both = E == 2 && mi + 1 < m_hi;
+      LdsBarrier();
+      if (phase + 1 < FM / E * PHASES) put(phase + 1);
+#pragma unroll
+      for (int q = 0; q < RPT / WAVES; ++q) {
+        const int j = q * WAVES + wave;
+        auto add = [&](int first, int e) {  // KW copies from `first` on, in order
+          float4 sum = red[phase & 1][first][j * E + e][lane];
+#pragma unroll
+          for (int c = 1; c < KW; ++c) {
+            const float4 o = red[phase & 1][first + c][j * E + e][lane];
+            sum.x += o.x;
+            sum.y += o.y;
+            sum.z += o.z;
+            sum.w += o.w;
           }
-          if (DUAL) {
-            if (mi < m_hi && slice0_a + slice_l < sga.ns) store(sga, slice0_a + slice_l, mi, sum);
-            if (mi < m_hi && tile_b_ok && slice0_b + slice_l < sgb.ns) store(sgb, slice0_b + slice_l, mi, sum_b);
-          } else if (mi < m_hi && slice0 + slice_l < sga.ns) {
+          return sum;
+        };
+        const float4 s0 = add(0, 0), s1 = E == 2 ? add(0, E - 1) : s0;
+        const int v = ph * RPT + j;
+        const int slice_l = 8 * (v >> 2) + 4 * g2 + (v & 3);  // slice inside the tile
+        if constexpr (GATED) {
+          const float4 b0 = add(KW, 0), b1 = E == 2 ? add(KW, E - 1) : b0;
+          if (mi < m_hi && slice0 + slice_l < sga.ns) {
             const int slice = slice0 + slice_l;
-            const float g[4] = {sum.x, sum.y, sum.z, sum.w}, up[4] = {sum_b.x, sum_b.y, sum_b.z, sum_b.w};
-            __half h[4];
+            auto combine = [&](const float4& gate, const float4& up) {
+              const u32x2 hg = round4(sga, slice, gate), hu = round4(sgb, slice, up);
+              u32x2 o;
 #pragma unroll
-            for (int t4 = 0; t4 < 4; ++t4) {
-              __half hg = __float2half_rn(g[t4]), hu = __float2half_rn(up[t4]);
-              if (sga.bias) hg = __hadd(hg, sga.bias[slice * 4 + t4]);
-              if (sgb.bias) hu = __hadd(hu, sgb.bias[slice * 4 + t4]);
-              h[t4] = __float2half_rn(GatedActivation(p.gate_activation, __half2float(hg), __half2float(hu)));
-            }
-            u32x2 o;
-            o[0] = (uint32_t)__half_as_ushort(h[0]) | ((uint32_t)__half_as_ushort(h[1]) << 16);
-            o[1] = (uint32_t)__half_as_ushort(h[2]) | ((uint32_t)__half_as_ushort(h[3]) << 16);
-            *reinterpret_cast<u32x2*>(sga.dst + ((size_t)slice * p.m + mi) * 4) = o;
+              for (int i = 0; i < 2; ++i) {
+                const half2_t g = AsHalf2(hg[i]), u = AsHalf2(hu[i]);
+                const __half lo = __float2half_rn(GatedActivation(p.gate_activation, (float)g[0], (float)u[0]));
+                const __half hi = __float2half_rn(GatedActivation(p.gate_activation, (float)g[1], (float)u[1]));
+                o[i] = (uint32_t)__half_as_ushort(lo) | ((uint32_t)__half_as_ushort(hi) << 16);
+              }
+              return o;
+            };
+            write16(sga, slice, mi, both, combine(s0, b0), both ? combine(s1, b1) : u32x2{0u, 0u});
           }
         } else if (mi < m_hi && slice0 + slice_l < sg.ns) {
-          store(sg, slice0 + slice_l, mi, sum);
+          store(sg, slice0 + slice_l, mi, both, s0, s1);
         }
       }
     }
@@ -1155,31 +1150,20 @@ void LaunchDirectW(bool zp, dim3 grid, hipStream_t stream, const GemmParams& p) 
   else
     hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<WB, FM, U, WAVES, false, PAIR, false, MODE>), grid, block, 0, stream, p);
 }
-// DUAL_OK: the two-tile mode is compiled for this shape.
-template <int FM, int U, int WAVES, bool PAIR, bool DUAL_OK>
+template <int FM, int WAVES>
 void LaunchDirect(int weight_bits, bool zp, dim3 grid, hipStream_t stream, const GemmParams& p) {
-  if (p.gate_activation != 0) {  // gated pair: symmetric weights
-    if (weight_bits == 8)
-      hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, U, WAVES, false, PAIR, false, kModeGated>), grid,
-                         dim3(WAVES * 64), 0, stream, p);
-    else
-      hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, U, WAVES, false, PAIR, false, kModeGated>), grid,
-                         dim3(WAVES * 64), 0, stream, p);
-    return;
-  }
-  if constexpr (DUAL_OK) {
-    if (p.dual) {
-      if (weight_bits == 8)
-        LaunchDirectW<8, FM, U, WAVES, PAIR, kModeDual>(zp, grid, stream, p);
-      else
-        LaunchDirectW<4, FM, U, WAVES, PAIR, kModeDual>(zp, grid, stream, p);
-      return;
-    }
-  }
   if (weight_bits == 8)
-    LaunchDirectW<8, FM, U, WAVES, PAIR, kModePlain>(zp, grid, stream, p);
+    LaunchDirectW<8, FM, 4, WAVES, FM != 1, kModePlain>(zp, grid, stream, p);
   else
-    LaunchDirectW<4, FM, U, WAVES, PAIR, kModePlain>(zp, grid, stream, p);
+    LaunchDirectW<4, FM, 4, WAVES, FM != 1, kModePlain>(zp, grid, stream, p);
+}
+// (symmetric weights; half of the waves per matrix)
+template <int FM, int WAVES>
+void LaunchGated(int weight_bits, dim3 grid, hipStream_t stream, const GemmParams& p) {
+  if (weight_bits == 8)
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, false, FM != 1, false, kModeGated>), grid, dim3(WAVES * 64), 0, stream, p);
+  else
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, false, FM != 1, false, kModeGated>), grid, dim3(WAVES * 64), 0, stream, p);
 }
 
 template <int FM, int WAVES>
@@ -1850,7 +1834,7 @@ struct SkinnyPlan {
 // 28672 at 24 tokens 0.8).  Above 32 tokens only where it is cut at least 4 ways: 16384 -> 2048 at 64 tokens 19.8 / 16.0, at 100,
 // cut in 2, 20.4 / 23.3; whole K of 6144 and more in 64-channel tiles against a direct kernel cut in 2: 0.92..1.01.  64-channel
 // tiles up to 16 tokens from more than 512 input channels on: 0.97 below.
-// (direct_split: W4KSplit(m, k, n))
+// (direct_split: CoarseKSplit(m, k, n))
 SkinnyPlan PlanSkinny(int m, int k, int n, int direct_split) {
   const int token_tiles = DivUp(m, 32), strips_xcd = DivUp(DivUp(n, 64), 8);
   if (m > kSkinnyMaxTiledTokens) return {0, 1};
@@ -1895,8 +1879,8 @@ void LaunchSkinny(bool zp, const GemmParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((fc_w4_mfma_skinny_kernel<T, FT, false, false>), grid, block, 0, stream, p);
 }
 
-// Token tile of the int4 GEMM in blocks of 32 tokens.  64 tokens when that still yields a
-// work-group for half the CUs, else 32 (more work-groups beat a K split across them).  128 tokens (one wave per SIMD, every
+// Gated pairs: token tile in blocks of 32 tokens.  64 tokens when that still yields a
+// work-group for half the CUs, else 32.  128 tokens (one wave per SIMD, every
 // dequantized weight feeds four MFMAs) when the launch fills the chip anyway and the rounds of
 // 256 work-groups come out cheaper: a 128-token tile takes about 1.85 x the time of a 64-token
 // one.
@@ -1906,10 +1890,9 @@ int W4TokenBlocks(int m, int n) {
   if (tiles128 >= 256 && 1.85 * DivUp(tiles128, 256L) < (double)DivUp(tiles64, 256L)) return 4;
   return (m > 32 && tiles64 >= 128) ? 2 : 1;
 }
-// K split across work-groups: doubled while the grid stays within the CU count and every wave
-// keeps at least 24 steps of 16 channels (below that the partial sums and the second kernel
-// cost more than the idle CUs: 2048 x 2048 at 128 tokens 10.9 -> 8.5 us without a split).
-int W4KSplit(int m, int k, int n) {
+// Shares that K can be cut into with a work-group of 8 waves and 24 steps of 16 channels per wave on every second CU: the
+// measure that the kernel for a few tokens holds its own cut against.
+int CoarseKSplit(int m, int k, int n) {
   const int fm = W4TokenBlocks(m, n);
   if (fm == 4) return 1;
   const long tiles = (long)DivUp(n, 128) * DivUp(m, fm * 32);
@@ -1960,6 +1943,65 @@ hipError_t LaunchConvInt8Tile(const GemmParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// How a plain launch of the direct kernel is cut: token tiles of 32 fm tokens, waves that share a tile's K inside a
+// work-group, parts of K for work-groups of their own (added by the second kernel).
+struct DirectPlan {
+  int fm, waves, ksplit;
+};
+// Times in us: `around` is what a work-group does outside its loop, `step` a K-step of 16 channels with nobody else on its
+// SIMDs (latency), `busy` and `busy_around` the same per wave and work-group when a CU is full (issue slots, LDS); for uint8
+// weights the steps take step8 and busy8 times that.
+struct DirectForm {
+  int fm, waves, per_cu;  // per_cu: work-groups that share a CU
+  double step, around, busy, busy_around, step8, busy8;
+};
+// The forms and their times, fitted to 5200 random launches (5 .. 8192 tokens, K 128 .. 16384, 128 .. 32768 channels, uint4
+// and uint8, per-channel scales and groups of 32 .. 128, 20 % with zero points), each in every form, to within 7 .. 11 % in
+// nine of ten.  Many tiles: one wave per tile needs no reduction through LDS and its store overlaps the other tiles of
+// the CU; fewer tiles: more waves share a tile's K.  32-token tiles of 4 waves: four work-groups fit a CU, the best form of short
+// prompts.  Left out since the rest comes within 0.1 % without them: 8 waves on 64 tokens, 2 waves on 32 and 64, and work-groups of
+// two channel tiles.  One rule of rounds of 256 work-groups (8 waves per tile, 4 at 128 tokens) stood here before: over the
+// 3219 launches where every form was timed this one is 1.29 times as fast in the geometric mean (0.9 % behind the best form), 19
+// are slower by more than 4 %.  us, before / now: 8192 x 512 x 14336 210 / 156, 4096 x 1024 x 4096 46.6 / 39, 1000 x 2000 x
+// 5000 34.9 / 30, 700 x 700 x 2777 15.8 / 10.8, 512 x 2048 x 32768 73.7 / 66, 8192 x 4096 x 14336 832 / 791.
+const DirectForm kDirectForms[] = {
+    {1, 1, 16, 0.14, 1.1, 0.0431, 0.45, 1.12, 1.13}, {1, 4, 2, 0.11, 1.1, 0.0394, 0.96, 1.19, 1.13}, {1, 8, 1, 0.22, 1.4, 0.0292, 1.9, 1.12, 1.19},
+    {2, 1, 8, 0.15, 2.6, 0.0563, 0.61, 1.26, 1.15},  {2, 4, 2, 0.10, 2.3, 0.0577, 1.2, 1.43, 1.12},  {4, 1, 4, 0.24, 5.7, 0.0798, 1.6, 1.16, 1.07},
+    {4, 2, 2, 0.23, 5.2, 0.0811, 2.1, 1.18, 1.06},   {4, 4, 1, 0.15, 4.6, 0.0907, 3.0, 1.20, 1.08}};
+constexpr int kDirectMaxKSplit = 8;
+constexpr long kDirectMaxSplitTiles = 640;  // work-groups up to which K is cut
+// (depends on m through DivUp(m, 32) only; max_split: parts of K that the workspace holds)
+DirectPlan PlanDirect(int m, int k, int n, int tiles_n, int groups, int bits, int max_split) {
+  const int m32 = DivUp(m, 32) * 32, steps = DivUp(k, 16);
+  DirectPlan best = {4, 1, 1};
+  double best_us = 0.0, fm_work = 0.0;
+  int fm = 0, tiles_m = 0;
+  for (const DirectForm& f : kDirectForms) {
+    if (f.fm > 1 && m32 <= 16 * f.fm) continue;  // (a tile half of which would be empty)
+    if (f.fm != fm) {
+      fm = f.fm;
+      tiles_m = DivUp(m, 32 * fm);
+      const int xm = W4XcdGrid(tiles_m, tiles_n, 32 * fm, k, groups);
+      fm_work = (double)DivUp(tiles_m, xm) * DivUp(tiles_n, 8 / xm) / 32.0;  // tiles per CU of the busiest XCD
+    }
+    const long tiles = (long)tiles_m * tiles_n;
+    if ((fm == 1 && tiles > 2048) || (f.waves < 4 && tiles * f.waves < 96)) continue;  // (never the best there)
+    for (int s = 1; s <= max_split; s *= 2) {
+      if (s > 1 && (f.waves < 2 || tiles * s > kDirectMaxSplitTiles || steps < 4 * s * f.waves)) break;
+      const double work = fm_work * s, whole = std::ceil(work - 1e-9);
+      const int share = DivUp(DivUp(steps, f.waves * s), 4) * 4;
+      const double chain = std::ceil(whole / f.per_cu) * (share * f.step * (bits == 8 ? f.step8 : 1.0) + f.around);
+      const double busy = 0.5 * (whole + work) * (f.waves * share * f.busy * (bits == 8 ? f.busy8 : 1.0) + f.busy_around);
+      double us = std::sqrt(chain * chain + busy * busy);
+      if (s > 1) us += 2.6 + (fm == 4 ? 0.84e-6 : 1.2e-6) * s * m32 * (double)n;  // the second kernel
+      if (best_us == 0.0 || us < best_us) {
+        best = {fm, f.waves, s};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
 int Log2(int power_of_two) { return __builtin_ctz((unsigned)power_of_two); }
 
 // What the matrix-core kernel can run at all (any token count).
@@ -2140,8 +2182,8 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   // Few tokens, or few tiles: fc_w4_mfma_skinny_kernel.  Below 5 tokens the token forms of the GEMVs are
   // faster (628 us at 4 tokens against 870 before the loop was pipelined) and callers come here only where those do not serve.
   // (gemm_fm, gemm_ksplit and the others ask for the direct kernel's shapes.)
-  const SkinnyPlan skinny = PlanSkinny(a.m, p.k, n_total, W4KSplit(a.m, p.k, n_total));
-  const bool direct_asked = tune.gemm_fm > 0 || tune.gemm_ksplit > 0 ||
+  const SkinnyPlan skinny = PlanSkinny(a.m, p.k, n_total, CoarseKSplit(a.m, p.k, n_total));
+  const bool direct_asked = tune.gemm_fm > 0 || tune.gemm_waves > 0 || tune.gemm_ksplit > 0 ||
                             (a.m > kSkinnyMaxTokens && (tune.gemm_no_pair > 0 || tune.gemm_dual >= 0 || tune.gemm_xcd_m > 0));
   if (!gated && a.weight_bits == 4 && skinny.tile > 0 && !direct_asked) {
     const int t = skinny.tile;
@@ -2170,43 +2212,44 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     }
   }
   set_variant("direct");
-  // token tile and K split follow the launch as a whole (all channels of all matrices)
-  int fm = W4TokenBlocks(a.m, n_total);
-  if (tune.gemm_fm > 0) fm = tune.gemm_fm == 1 ? 1 : (tune.gemm_fm == 4 ? 4 : 2);
-  p.ksplit = 1;
-  if (fm == W4TokenBlocks(a.m, n_total)) p.ksplit = W4KSplit(a.m, a.k, n_total);
-  if (tune.gemm_ksplit > 0) p.ksplit = tune.gemm_ksplit;
-  if (gated) p.ksplit = 1;  // the epilogue needs whole sums
-  for (int i = 0; i < count; ++i)
-    while (p.ksplit > 1 && (size_t)p.ksplit * p.seg[i].ns * 4 * a.m > args[i].partial_floats) p.ksplit /= 2;
-  const int tiles_m = DivUp(a.m, fm * 32);
-  const bool pair = tune.gemm_no_pair <= 0;
-  // Two channel tiles per work-group when the rounds of 256 work-groups come out cheaper: a
-  // two-tile work-group takes 1.87 x the time of a one-tile one, and a last round filled to the
-  // fraction f costs 0.45 + 0.55 f of a full one (fitted to same-box timings of 14 shapes).
-  const bool dual_ok = !gated && pair && fm >= 2 && p.ksplit == 1;
-  auto rounds = [](long work_groups) {
-    const double r = work_groups / 256.0, whole = std::floor(r), f = r - whole;
-    return whole + (f > 0.0 ? 0.45 + 0.55 * f : 0.0);
+  // token tile, waves and K split follow the launch as a whole (all channels of all matrices)
+  DirectPlan plan = {W4TokenBlocks(a.m, n_total), 0, 1};  // gated: the epilogue needs whole sums
+  auto fits = [&](int split) {
+    bool ok = true;
+    for (int i = 0; i < count; ++i) ok = ok && (size_t)split * p.seg[i].ns * 4 * a.m <= args[i].partial_floats;
+    return ok;
   };
-  p.dual = dual_ok && 1.87 * rounds((long)DivUp(tiles_n, 2) * tiles_m) < 0.97 * rounds((long)tiles_n * tiles_m);
-  if (tune.gemm_dual >= 0) p.dual = dual_ok && tune.gemm_dual != 0;
-  if (p.dual) tiles_n = DivUp(tiles_n, 2);
+  int max_split = kDirectMaxKSplit;
+  while (max_split > 1 && !fits(max_split)) max_split /= 2;
+  if (!gated) plan = PlanDirect(a.m, a.k, n_total, tiles_n, p.groups, a.weight_bits, max_split);
+  if (tune.gemm_fm > 0) {
+    const int fm_asked = tune.gemm_fm == 1 || tune.gemm_fm == 4 ? tune.gemm_fm : 2;
+    if (fm_asked != plan.fm) plan = {fm_asked, fm_asked == 1 ? 8 : 4, 1};
+  }
+  if (tune.gemm_waves > 0) plan.waves = tune.gemm_waves;
+  if (tune.gemm_ksplit > 0 && !gated) plan.ksplit = tune.gemm_ksplit;
+  const int fm = plan.fm;
+  // (the forms that are compiled)
+  const int waves = gated ? (fm == 4 ? 4 : 8) : fm == 4 ? std::min(plan.waves, 4) : plan.waves == 1 ? 1 : (fm == 1 && plan.waves > 4 ? 8 : 4);
+  p.ksplit = plan.ksplit;
+  while (p.ksplit > 1 && !fits(p.ksplit)) p.ksplit /= 2;
+  const int tiles_m = DivUp(a.m, fm * 32);
   p.xcd_m = W4XcdGrid(tiles_m, tiles_n, fm * 32, a.k, p.groups);
   if (tune.gemm_xcd_m > 0) p.xcd_m = tune.gemm_xcd_m;
   if (p.xcd_m != 1 && p.xcd_m != 2 && p.xcd_m != 4 && p.xcd_m != 8) p.xcd_m = 8;
   const dim3 grid(8 * DivUp(tiles_m, p.xcd_m) * DivUp(tiles_n, 8 / p.xcd_m), p.ksplit);
   if (grid.x / 8 >= (1u << 16)) return hipErrorInvalidValue;  // (the reciprocal of rect_m is exact below 2^16)
   const bool zp = p.seg[0].zp != nullptr;
-  set_geometry(tiles_m, tiles_n, fm == 4 ? 4 : 8, gated || p.dual);
-  if (fm == 4)
-    LaunchDirect<4, 4, 4, true, true>(a.weight_bits, zp, grid, stream, p);
-  else if (fm == 2 && pair)
-    LaunchDirect<2, 4, 8, true, true>(a.weight_bits, zp, grid, stream, p);
-  else if (fm == 2)
-    LaunchDirect<2, 4, 8, false, false>(a.weight_bits, zp, grid, stream, p);
-  else
-    LaunchDirect<1, 4, 8, false, false>(a.weight_bits, zp, grid, stream, p);
+  set_geometry(tiles_m, tiles_n, waves, gated);
+  if (gated) {
+    (fm == 4 ? LaunchGated<4, 4> : fm == 2 ? LaunchGated<2, 8> : LaunchGated<1, 8>)(a.weight_bits, grid, stream, p);
+    return hipGetLastError();
+  }
+  typedef void (*launch_t)(int, bool, dim3, hipStream_t, const GemmParams&);
+  static const launch_t kLaunch[3][4] = {{LaunchDirect<1, 1>, nullptr, LaunchDirect<1, 4>, LaunchDirect<1, 8>},
+                                         {LaunchDirect<2, 1>, nullptr, LaunchDirect<2, 4>, nullptr},
+                                         {LaunchDirect<4, 1>, LaunchDirect<4, 2>, LaunchDirect<4, 4>, nullptr}};
+  kLaunch[Log2(fm)][Log2(waves)](a.weight_bits, zp, grid, stream, p);
   launch_reduce();
   return hipGetLastError();
 }
@@ -2250,11 +2293,21 @@ hipError_t LaunchFcW4MfmaGated(const FcArgs& gate, const FcArgs& up, int activat
   return LaunchDirectGemm(both, 2, activation, dst, stream, kernel_name);
 }
 
-size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n) {
+size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n, int groups, int bits) {
   size_t need = 0;
-  for (int m = kGemvMaxTokens + 1; m <= max_tokens; ++m) {
-    const int direct = W4KSplit(m, k, n), s = std::max(direct, PlanSkinny(m, k, n, direct).ksplit);
-    if (s > 1) need = std::max(need, (size_t)s * DivUp(n, 4) * 4 * m);
+  // (the direct kernel's plan depends on whole blocks of 32 tokens; no K split above kDirectMaxSplitTiles tiles of 128 tokens)
+  const int tiles_n = DivUp(n, 128);
+  for (long m = 32; m < (long)max_tokens + 32; m += 32) {
+    const int mc = (int)std::min<long>(m, max_tokens);
+    if (mc > kSkinnyMaxTiledTokens && (long)DivUp(mc, 128) * tiles_n * 2 > kDirectMaxSplitTiles) break;
+    int s = 1;
+    bool direct = mc > kSkinnyMaxTiledTokens || bits != 4;  // (is there a token count of the block that the direct kernel takes)
+    for (int t = std::max(mc - 31, kGemvMaxTokens + 1); bits == 4 && t <= mc && t <= kSkinnyMaxTiledTokens; ++t) {
+      const SkinnyPlan skinny = PlanSkinny(t, k, n, CoarseKSplit(t, k, n));
+      if (skinny.tile > 0) s = std::max(s, skinny.ksplit); else direct = true;
+    }
+    if (direct && mc > kGemvMaxTokens) s = std::max(s, PlanDirect(mc, k, n, tiles_n, groups, bits, kDirectMaxKSplit).ksplit);
+    if (s > 1) need = std::max(need, (size_t)s * DivUp(n, 4) * 4 * mc);
   }
   return need;
 }

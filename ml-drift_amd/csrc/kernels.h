@@ -179,7 +179,8 @@ struct Tuning {
   int gemv_lpr = -1, gemv_waves = -1, gemv_ksplit = -1, gemv_narrow_max_mb = -1;
   int gemv_rows_rpt = -1;       // rows per thread the row-interleaved GEMV sizes its work-groups for
   int gemv_one_chunk = -1;      // 0: never take the one-chunk form of the contiguous-strip GEMV
-  int gemm_fm = -1, gemm_ksplit = -1, gemm_no_pair = -1, gemm_dual = -1, gemm_xcd_m = -1;
+  int gemm_fm = -1, gemm_waves = -1, gemm_ksplit = -1, gemm_xcd_m = -1;
+  int gemm_no_pair = -1, gemm_dual = -1;  // (set: the direct kernel above 32 tokens; the forms that they chose between are gone)
   int gemm_i8_fm = -1;
   int gemm_tiled = -1;          // 1 / 0: always / never take the LDS-tiled int4 GEMM where it can run
 };
@@ -221,7 +222,7 @@ hipError_t LaunchFcW4Mfma(const FcArgs& a, hipStream_t stream, const char** kern
 hipError_t LaunchFcW4MfmaFused(const FcArgs* args, int count, hipStream_t stream, const char** kernel_name);
 // fp32 workspace the MFMA path wants for token counts up to max_tokens (K split across
 // work-groups); 0 when it never splits.
-size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n);
+size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n, int groups, int bits);
 // dst = activation(gate(x)) * up(x) on the matrix-core kernel (symmetric weights; uint4 at any token
 // count, uint8 above the GEMV token counts).
 bool FcW4MfmaGatedSupported(const FcArgs& gate, const FcArgs& up);

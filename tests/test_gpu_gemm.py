@@ -237,6 +237,24 @@ def test_gemm_odd_token_counts(bits, fm, dual, m, k, n, groups, zp):
     assert not np.isfinite(got[0]).any()
 
 
+@pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False)])
+@pytest.mark.parametrize("fm,waves", [(1, 1), (1, 4), (1, 8), (2, 1), (2, 4), (4, 1), (4, 2), (4, 4)])
+@pytest.mark.parametrize("m,k,n,groups,ksplit", [(5, 64, 4, 2, 1), (65, 136, 132, 1, 1), (128, 1056, 260, 33, 1), (131, 1024, 388, 1, 2), (257, 2048, 128, 4, 4)])
+def test_gemm_waves_per_tile(fm, waves, bits, zp, m, k, n, groups, ksplit):
+    """Every token tile with every number of waves that share a tile's K (one: whole sums in registers, tokens stored in pairs),
+    ragged tokens and channels, K that does not divide into the shares, K cut between work-groups too.  Weights are rounded to
+    fp16 (2^-11 relative, twice with a zero point), results once more; sums in fp32."""
+    case = W.make_fc_case(seed=m + n + bits, m=m, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups,
+                          with_bias=True, with_zero_point=zp)
+    with M.tuning(gemm_fm=fm, gemm_waves=waves, gemm_ksplit=ksplit):
+        got = run_w4(case)
+    ref = textbook(case)
+    check_fp(got, ref, case, "textbook")
+    w = case["w"].astype(np.float64) - (np.repeat(case["zero_point"], k // groups, axis=1) if zp else 0.0)
+    size = np.abs(case["act"].astype(np.float64)) @ np.abs(w * np.repeat(case["scale"], k // groups, axis=1)).T
+    assert np.all(np.abs(got - ref) <= 2.0 ** -10 * size / np.sqrt(k) * 4 + 2.0 ** -9 * (np.abs(ref) + 1.0))
+
+
 def test_gemm_modes_random_sweep():
     """Seeded sweep over shapes with the two-tile mode forced on and off and every token tile
     forced in turn: all against the textbook reference at the fp16 bar."""
