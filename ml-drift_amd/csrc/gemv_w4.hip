@@ -93,6 +93,8 @@ struct StreamParams {
   // slices beyond the bound are not written.
   const int32_t* rt_params;
   int src_end_idx, dst_end_idx, k_channels;
+  // batched launches in half strips: pairs of them per row, ceil(2^32 / pairs)
+  uint32_t pairs, pairs_magic;
 };
 
 __device__ __forceinline__ void StoreHalf(__half* dst, size_t i, float r, const __half* bias, size_t bi) {
@@ -123,6 +125,66 @@ __device__ __forceinline__ void LoadChunk(const StreamParams& p, const u32x4* wc
       a[j][m] = u32x2{ks < ks_live ? v[0] : 0u, ks < ks_live ? v[1] : 0u};
     }
   }
+}
+
+typedef uint32_t u32x2s __attribute__((ext_vector_type(2)));
+
+// Rows of 16 lanes: this lane ends with channels (lane % 16) * 8 + 4 * (lane / 32) + 2 * ((lane / 16) % 2) and the next.
+__device__ __forceinline__ float2 WaveStripSum16(const float acc[8]) {
+  float s4[4], s2[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x2s r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + 4]), false, false);
+    s4[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const u32x2s r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s4[i]), __float_as_uint(s4[i + 2]), false, false);
+    s2[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+  return make_float2(s2[0], s2[1]);
+}
+// LPR lanes (16 bytes each) cover a row; a wave holds 64 / LPR rows.  Sum over the rows of a wave
+// of the 8 channel sums of every lane; the result of channel (lane % LPR) * 8 + (lane / 8) % 8 is
+// returned in this lane (lanes that differ only in the bits between LPR and 8 hold the same
+// sums).  All 64 lanes must be active.
+// v + the value of the lane that differs in one bit of the lane number, as data-parallel moves
+// inside the rows of 16 lanes (no trip through the LDS crossbar): bits 0 and 1 are quad
+// permutations, bit 2 a shift by 4 lanes in either direction, each for the banks it is valid in.
+__device__ __forceinline__ float AddLaneXor1(float v) {
+  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0xB1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float AddLaneXor2(float v) {
+  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x4E /* quad_perm:[2,3,0,1] */, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float AddLaneXor4(float v) {
+  const uint32_t up = __builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x104 /* row_shl:4 */, 0xf, 0x5, false);
+  const uint32_t both = __builtin_amdgcn_update_dpp(up, __float_as_uint(v), 0x114 /* row_shr:4 */, 0xf, 0xA, false);
+  return v + __uint_as_float(both);
+}
+
+template <int LPR>
+__device__ __forceinline__ float WaveStripSum(const float acc[8], int lane) {
+  float s4[4], s2[2];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x2s r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + 4]), false, false);
+    s4[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const u32x2s r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s4[i]), __float_as_uint(s4[i + 2]), false, false);
+    s2[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    s2[i] += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(s2[i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+  float v = (lane & 8) ? s2[1] : s2[0];
+  // narrower rows: the lanes 4 (and 2) apart hold further rows of the same channels
+  if (LPR <= 4) v = AddLaneXor4(v);
+  if (LPR <= 2) v = AddLaneXor2(v);
+  if (LPR <= 1) v = AddLaneXor1(v);
+  return v;
 }
 
 // t[m][o] += sum over the chunk of a * (c_o + u), c_o = 1024 for even o, 64 for odd o;
@@ -176,8 +238,7 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
   constexpr int ROWS = THREADS / LPR;  // chunks the work-group covers per step
   constexpr int RPW = 64 / LPR;        // rows per wave
   constexpr int STRIP = LPR * 8;       // output channels per work-group
-  __shared__ float red[ROWS][M][STRIP];
-  __shared__ float red2[(THREADS / STRIP > 0 ? THREADS / STRIP : 1)][M][STRIP];
+  __shared__ float red[WAVES][M][STRIP];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -194,7 +255,16 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
   const int row_u4 = sg.row_u4;
   // BATCHED: this row's matrix (an id outside the batch is clamped into it), its source row
   // (one shared row is broadcast) and the token strides of the two tensors
-  const int brow = BATCHED ? (int)blockIdx.z : 0;
+  // Half strips (LPR = 4) of one 128-byte row segment run on one XCD, whose L2 then fetches its lines once: work-groups L and
+  // L + 8 (of 16 in a row) are the two halves of a strip.  (8 of 128 matrices 2048 x 768 and 768 x 2048, one token: the
+  // three launches of a layer 15.1 -> 13.4 us; dealt one after the other, each line came from HBM to two L2.)
+  int brow = BATCHED ? (int)blockIdx.z : 0;
+  if (BATCHED && LPR == 4) {
+    const uint32_t pair = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
+    brow = (int)(p.pairs == 1 ? pair : __umulhi(pair, p.pairs_magic));
+    strip = 2 * (int)(pair - (uint32_t)brow * p.pairs) + (int)((blockIdx.x >> 3) & 1u);
+    if (brow >= p.rows || strip >= p.seg[0].strip_end) return;
+  }
   int wb = BATCHED ? p.batch_ids[brow] : 0;
   if (BATCHED) wb = __builtin_amdgcn_readfirstlane(min(max(wb, 0), p.weights_batch - 1));
   const u32x4* weights = sg.weights;
@@ -227,36 +297,33 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
 #pragma unroll
     for (int o = 0; o < 8; ++o) acc[m][o] = 0.0f;
 
-  // The per-channel scale and the bias of the output this thread writes at the end (output
-  // tid % STRIP of the strip, for every token it handles): fetched now, so that their latency
-  // does not follow the reduction.
-  // (Unconditional loads of the raw halfs at a clamped index: a branch, or a conversion, here
-  // would make the kernel wait for them before it issues the weight loads.)
+  int c = c_begin + row;
+  u32x4 zv = {0u, 0u, 0u, 0u};  // zero points of this thread's 8 channels (halfs)
+  if (ZP && !GROUPED) zv = *reinterpret_cast<const u32x4*>(zp_base + (size_t)2 * pcol * 4);
+  // The per-channel scale and the bias of the output this thread writes at the end (output tid % STRIP of the strip, for
+  // every token it handles): fetched now, so that their latency does not follow the reduction (behind the weights: 3 % slower
+  // over the one-token launches of a mixture of experts).  (Unconditional loads of the raw halfs at a clamped index: a
+  // branch, or a conversion, here would make the kernel wait for them before it issues the weight loads.)
   const int n_out = min(strip * STRIP + tid % STRIP, sg.n_pad - 1);
   const unsigned short* bias_src = reinterpret_cast<const unsigned short*>(sg.bias ? sg.bias : sg.scale);
   const unsigned short out_scale_raw = reinterpret_cast<const unsigned short*>(scale_base)[n_out];
   const unsigned short out_bias_raw = bias_src[n_out];
-
-  int c = c_begin + row;
-  u32x4 zv = {0u, 0u, 0u, 0u};  // zero points of this thread's 8 channels (halfs)
-  if (ZP && !GROUPED) zv = *reinterpret_cast<const u32x4*>(zp_base + (size_t)2 * pcol * 4);
-  if (c < c_end) {
-    u32x4 w[8];
-    u32x2 a[8][M];
-    LoadChunk<M>(p, wcol, rstride, c, w, a, ks_live, act_stride, act_tok0);
+  u32x4 w[8];
+  u32x2 a[8][M];
+  const bool first = c < c_end;
+  if (first) LoadChunk<M>(p, wcol, rstride, c, w, a, ks_live, act_stride, act_tok0);
+  if (first) {
     while (true) {
       const int cn = c + ROWS;
       const bool more = cn < c_end;
-      u32x4 wn[8];
+      u32x4 sv, wn[8];
       u32x2 an[8][M];
-      if (more) LoadChunk<M>(p, wcol, rstride, cn, wn, an, ks_live, act_stride, act_tok0);
-      u32x4 sv;
-      if (GROUPED) {
-        int g = c / p.group_chunks;
-        if (g >= p.groups) g = p.groups - 1;
+      if (GROUPED) {  // (in front of the next chunk's weights: loads return in order)
+        const int g = min(c / p.group_chunks, p.groups - 1);
         sv = *reinterpret_cast<const u32x4*>(scale_base + (size_t)g * group_stride + (size_t)2 * pcol * 4);
         if (ZP) zv = *reinterpret_cast<const u32x4*>(zp_base + (size_t)g * group_stride + (size_t)2 * pcol * 4);
       }
+      if (more) LoadChunk<M>(p, wcol, rstride, cn, wn, an, ks_live, act_stride, act_tok0);
       float t[M][8], asum[M];
 #pragma unroll
       for (int m = 0; m < M; ++m) {
@@ -290,27 +357,14 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
     }
   }
 
-  // K reduction inside the work-group, through LDS only: every thread stores its 8*M sums,
-  // PARTS threads per output add ROWS/PARTS rows each, then one thread per output adds the
-  // PARTS results.
-  constexpr int PARTS = THREADS / STRIP >= 1 ? (THREADS / STRIP > ROWS ? ROWS : THREADS / STRIP) : 1;
-  constexpr int RPP = ROWS / PARTS;  // rows per part
+  // K reduction inside the work-group: the rows of a wave by register exchanges, the waves through LDS, in wave order.
 #pragma unroll
   for (int m = 0; m < M; ++m) {
-    float4* dst4 = reinterpret_cast<float4*>(&red[row][m][col * 8]);
-    dst4[0] = make_float4(acc[m][0], acc[m][1], acc[m][2], acc[m][3]);
-    dst4[1] = make_float4(acc[m][4], acc[m][5], acc[m][6], acc[m][7]);
-  }
-  __syncthreads();
-  const int nl = tid % STRIP;
-  const int part = tid / STRIP;
-  if (part < PARTS) {
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float v = 0.0f;
-#pragma unroll
-      for (int r = 0; r < RPP; ++r) v += red[part * RPP + r][m][nl];
-      red2[part][m][nl] = v;
+    if constexpr (LPR == 16) {
+      const float2 v = WaveStripSum16(acc[m]);
+      *reinterpret_cast<float2*>(&red[wave][m][col * 8 + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1)]) = v;
+    } else {
+      red[wave][m][col * 8 + ((lane >> 3) & 7)] = WaveStripSum<LPR>(acc[m], lane);
     }
   }
   __syncthreads();
@@ -321,7 +375,7 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
     if (n >= ns_live * 4) continue;
     float v = 0.0f;
 #pragma unroll
-    for (int q = 0; q < PARTS; ++q) v += red2[q][m][ol];
+    for (int q = 0; q < WAVES; ++q) v += red[q][m][ol];
     if (p.ksplit == 1) {
       if (!GROUPED) v *= __half2float(__ushort_as_half(out_scale_raw));
       __half h = __float2half_rn(v);
@@ -359,157 +413,6 @@ __global__ __launch_bounds__(256) void fc_w4_reduce_kernel(StreamParams p, int n
   }
   v *= scale;
   StoreHalf(sg.dst, ((size_t)(n >> 2) * p.m + m) * 4 + (n & 3), v, sg.bias, (size_t)n);
-}
-
-// ------------------------------------------------------------------------------------------
-// Gated pair: dst = activation(gate(x)) * up(x), the MLP step that follows the gate and up
-// projections in the decoder layers of the LLM sample (samples/llm/gemma3_model_builder.cc:
-// 1054-1090 CreateGeluTanhMulOp, samples/llm/qwen3_model_builder.cc:850-883 CreateSiluMulOp).
-// The two projections run as in the kernel above, in one work-group per strip (seg[0] = gate,
-// seg[1] = up, same shape); their sums are rounded to fp16 (+ bias) exactly as the two separate
-// FullyConnected nodes would store them, then combined in fp32 in the operation order of the
-// sample's elementwise kernel.  Only seg[0].dst is written.
-// ------------------------------------------------------------------------------------------
-template <int LPR, int WAVES, int M, bool GROUPED>
-__global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamParams p, int activation) {
-  constexpr int THREADS = WAVES * 64;
-  constexpr int ROWS = THREADS / LPR;
-  constexpr int RPW = 64 / LPR;
-  constexpr int STRIP = LPR * 8;
-  constexpr int PARTS = THREADS / STRIP > ROWS ? ROWS : THREADS / STRIP;
-  constexpr int RPP = ROWS / PARTS;
-  __shared__ float red[ROWS][2 * M][STRIP];
-  __shared__ float red2[PARTS][2 * M][STRIP];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int col = lane % LPR;
-  const int row = wave * RPW + lane / LPR;
-  const int strip = blockIdx.x;
-  const int row_u4 = p.seg[0].row_u4;
-  const int pcol_raw = strip * LPR + col;
-  const int pcol = pcol_raw < row_u4 ? pcol_raw : row_u4 - 1;  // clamp: loads stay in range, result unused
-  const int rstride = p.seg[0].gu4;
-  const size_t wcol_off = (size_t)(pcol / rstride) * p.ks * rstride + pcol % rstride;
-
-  // scales / biases of the output this thread finishes, fetched ahead (raw halfs, clamped index)
-  const int n_out = min(strip * STRIP + tid % STRIP, p.seg[0].n_pad - 1);
-  unsigned short scale_raw[2], bias_raw[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const unsigned short* bias_src = reinterpret_cast<const unsigned short*>(p.seg[q].bias ? p.seg[q].bias : p.seg[q].scale);
-    scale_raw[q] = reinterpret_cast<const unsigned short*>(p.seg[q].scale)[n_out];
-    bias_raw[q] = bias_src[n_out];
-  }
-
-  float acc[2][M][8];
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-#pragma unroll
-    for (int m = 0; m < M; ++m)
-#pragma unroll
-      for (int o = 0; o < 8; ++o) acc[q][m][o] = 0.0f;
-
-  for (int c = row; c < p.chunks; c += ROWS) {
-    u32x4 w[2][8];
-    u32x2 a[8][M];
-    LoadChunk<M>(p, p.seg[0].weights + wcol_off, rstride, c, w[0], a, p.ks);
-    {
-      const int ks0 = c * 8;
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        w[1][j] = __builtin_nontemporal_load(p.seg[1].weights + wcol_off + (size_t)min(ks0 + j, p.ks - 1) * rstride);
-    }
-    u32x4 sv[2];
-    if (GROUPED) {
-      int g = c / p.group_chunks;
-      if (g >= p.groups) g = p.groups - 1;
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        sv[q] = *reinterpret_cast<const u32x4*>(p.seg[q].scale + ((size_t)g * p.seg[q].ns + 2 * pcol) * 4);
-    }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      float t[M][8], asum[M];
-#pragma unroll
-      for (int m = 0; m < M; ++m) {
-        asum[m] = 0.0f;
-#pragma unroll
-        for (int o = 0; o < 8; ++o) t[m][o] = 0.0f;
-      }
-      ComputeChunk<M>(p, w[q], a, t, asum);
-#pragma unroll
-      for (int m = 0; m < M; ++m)
-#pragma unroll
-        for (int o = 0; o < 8; ++o) {
-          const float centered = fmaf((o & 1) ? -72.0f : -1032.0f, asum[m], t[m][o]);
-          if (GROUPED) {
-            const half2_t sp = AsHalf2(sv[q][o >> 1]);
-            acc[q][m][o] = fmaf((float)sp[o & 1], centered, acc[q][m][o]);
-          } else {
-            acc[q][m][o] += centered;
-          }
-        }
-    }
-  }
-
-#pragma unroll
-  for (int q = 0; q < 2; ++q)
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      float4* dst4 = reinterpret_cast<float4*>(&red[row][q * M + m][col * 8]);
-      dst4[0] = make_float4(acc[q][m][0], acc[q][m][1], acc[q][m][2], acc[q][m][3]);
-      dst4[1] = make_float4(acc[q][m][4], acc[q][m][5], acc[q][m][6], acc[q][m][7]);
-    }
-  __syncthreads();
-  const int nl = tid % STRIP;
-  const int part = tid / STRIP;
-  if (part < PARTS) {
-#pragma unroll
-    for (int qm = 0; qm < 2 * M; ++qm) {
-      float v = 0.0f;
-#pragma unroll
-      for (int r = 0; r < RPP; ++r) v += red[part * RPP + r][qm][nl];
-      red2[part][qm][nl] = v;
-    }
-  }
-  __syncthreads();
-  const int n0 = strip * STRIP;
-  for (int idx = tid; idx < M * STRIP; idx += THREADS) {
-    const int m = idx / STRIP, ol = idx % STRIP;
-    const int n = n0 + ol;
-    if (n >= p.seg[0].n_pad) continue;
-    float gu[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      float v = 0.0f;
-#pragma unroll
-      for (int k = 0; k < PARTS; ++k) v += red2[k][q * M + m][ol];
-      if (!GROUPED) v *= __half2float(__ushort_as_half(scale_raw[q]));
-      __half h = __float2half_rn(v);
-      if (p.seg[q].bias) h = __hadd(h, __ushort_as_half(bias_raw[q]));
-      gu[q] = __half2float(h);
-    }
-    p.seg[0].dst[((size_t)(n >> 2) * M + m) * 4 + (n & 3)] = __float2half_rn(GatedActivation(activation, gu[0], gu[1]));
-  }
-}
-
-template <int LPR, int WAVES>
-hipError_t LaunchGatedM(const StreamParams& p, bool grouped, int activation, dim3 grid, hipStream_t stream) {
-  const dim3 block(WAVES * 64);
-#define MLD_GATED(MM)                                                                                             \
-  if (grouped)                                                                                                    \
-    hipLaunchKernelGGL((fc_w4_gated_stream_kernel<LPR, WAVES, MM, true>), grid, block, 0, stream, p, activation); \
-  else                                                                                                            \
-    hipLaunchKernelGGL((fc_w4_gated_stream_kernel<LPR, WAVES, MM, false>), grid, block, 0, stream, p, activation);
-  switch (p.m) {
-    case 1: MLD_GATED(1) break;
-    case 2: MLD_GATED(2) break;
-    default: return hipErrorInvalidValue;
-  }
-#undef MLD_GATED
-  return hipGetLastError();
 }
 
 template <int LPR, int WAVES, int M, bool GROUPED, bool ZP>
@@ -591,49 +494,103 @@ hipError_t LaunchBatchedM(const StreamParams& p, bool grouped, dim3 grid, hipStr
 // of a row with a DPP rotate), after which lane l holds channel (l % 8) * 8 + l / 8 of the
 // strip; across waves through 4 KB of LDS, fixed order.
 // ------------------------------------------------------------------------------------------
-typedef uint32_t u32x2s __attribute__((ext_vector_type(2)));
+// ------------------------------------------------------------------------------------------
+// Gated pair: dst = activation(gate(x)) * up(x), the MLP step that follows the gate and up
+// projections in the decoder layers of the LLM sample (samples/llm/gemma3_model_builder.cc:
+// 1054-1090 CreateGeluTanhMulOp, samples/llm/qwen3_model_builder.cc:850-883 CreateSiluMulOp).
+// The two projections run as in the streaming kernel above, in one work-group per strip of 64 channels (seg[0] = gate,
+// seg[1] = up, same shape); their sums are rounded to fp16 (+ bias) exactly as the two separate
+// FullyConnected nodes would store them, then combined in fp32 in the operation order of the
+// sample's elementwise kernel.  Only seg[0].dst is written.
+// Bound: HBM, with at most one strip per CU (14336 channels: 224).  A thread has one chunk of both matrices in flight, 16 loads;
+// 16 waves hold all of K = 4096 at once: gate, up and down of 4096 x 14336, 20.8 -> 20.1 us a layer (two chunks per thread
+// of 8 waves, the same bytes in flight: 21.6; the waves' sums through LDS instead of register exchanges: the same).
+// ------------------------------------------------------------------------------------------
+template <int WAVES, int M, bool GROUPED>
+__global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamParams p, int activation) {
+  constexpr int LPR = 8, ROWS = WAVES * 64 / LPR, STRIP = LPR * 8;
+  __shared__ float red[WAVES][2 * M][STRIP];
 
-// LPR lanes (16 bytes each) cover a row; a wave holds 64 / LPR rows.  Sum over the rows of a wave
-// of the 8 channel sums of every lane; the result of channel (lane % LPR) * 8 + (lane / 8) % 8 is
-// returned in this lane (lanes that differ only in the bits between LPR and 8 hold the same
-// sums).  All 64 lanes must be active.
-// v + the value of the lane that differs in one bit of the lane number, as data-parallel moves
-// inside the rows of 16 lanes (no trip through the LDS crossbar): bits 0 and 1 are quad
-// permutations, bit 2 a shift by 4 lanes in either direction, each for the banks it is valid in.
-__device__ __forceinline__ float AddLaneXor1(float v) {
-  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0xB1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float AddLaneXor2(float v) {
-  return v + __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x4E /* quad_perm:[2,3,0,1] */, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float AddLaneXor4(float v) {
-  const uint32_t up = __builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x104 /* row_shl:4 */, 0xf, 0x5, false);
-  const uint32_t both = __builtin_amdgcn_update_dpp(up, __float_as_uint(v), 0x114 /* row_shr:4 */, 0xf, 0xA, false);
-  return v + __uint_as_float(both);
-}
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int col = lane % LPR;
+  const int row = tid / LPR;
+  const int strip = blockIdx.x;
+  const int row_u4 = p.seg[0].row_u4;
+  const int pcol_raw = strip * LPR + col;
+  const int pcol = pcol_raw < row_u4 ? pcol_raw : row_u4 - 1;  // clamp: loads stay in range, result unused
+  const int rstride = p.seg[0].gu4;
+  const size_t wcol_off = (size_t)(pcol / rstride) * p.ks * rstride + pcol % rstride;
 
-template <int LPR>
-__device__ __forceinline__ float WaveStripSum(const float acc[8], int lane) {
-  float s4[4], s2[2];
+  float acc[2][M][8];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const u32x2s r = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[i]), __float_as_uint(acc[i + 4]), false, false);
-    s4[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int m = 0; m < M; ++m)
+#pragma unroll
+      for (int o = 0; o < 8; ++o) acc[q][m][o] = 0.0f;
+
+  for (int c = row; c < p.chunks; c += ROWS) {
+    u32x4 w[2][8], sv[2];
+    u32x2 a[8][M];
+    LoadChunk<M>(p, p.seg[0].weights + wcol_off, rstride, c, w[0], a, p.ks);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      w[1][j] = __builtin_nontemporal_load(p.seg[1].weights + wcol_off + (size_t)min(c * 8 + j, p.ks - 1) * rstride);
+    if (GROUPED) {
+      const int g = min(c / p.group_chunks, p.groups - 1);
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        sv[q] = *reinterpret_cast<const u32x4*>(p.seg[q].scale + ((size_t)g * p.seg[q].ns + 2 * pcol) * 4);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      float t[M][8], asum[M];
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        asum[m] = 0.0f;
+#pragma unroll
+        for (int o = 0; o < 8; ++o) t[m][o] = 0.0f;
+      }
+      ComputeChunk<M>(p, w[q], a, t, asum);
+#pragma unroll
+      for (int m = 0; m < M; ++m)
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+          const float centered = fmaf((o & 1) ? -72.0f : -1032.0f, asum[m], t[m][o]);
+          if (GROUPED) {
+            const half2_t sp = AsHalf2(sv[q][o >> 1]);
+            acc[q][m][o] = fmaf((float)sp[o & 1], centered, acc[q][m][o]);
+          } else {
+            acc[q][m][o] += centered;
+          }
+        }
+    }
   }
+
+  // the rows of a wave by register exchanges, the waves through LDS, in wave order
+  const int ch_wave = col * 8 + ((lane >> 3) & 7);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const u32x2s r = __builtin_amdgcn_permlane16_swap(__float_as_uint(s4[i]), __float_as_uint(s4[i + 2]), false, false);
-    s2[i] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int m = 0; m < M; ++m) red[wave][q * M + m][ch_wave] = WaveStripSum<LPR>(acc[q][m], lane);
+  __syncthreads();
+  const int m = tid / STRIP, ol = tid % STRIP;
+  const int n = strip * STRIP + ol;
+  if (m >= M || n >= p.seg[0].n_pad) return;
+  float gu[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < WAVES; ++k) v += red[k][q * M + m][ol];
+    if (!GROUPED) v *= __half2float(p.seg[q].scale[n]);
+    __half h = __float2half_rn(v);
+    if (p.seg[q].bias) h = __hadd(h, p.seg[q].bias[n]);
+    gu[q] = __half2float(h);
   }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    s2[i] += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(s2[i]), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
-  float v = (lane & 8) ? s2[1] : s2[0];
-  // narrower rows: the lanes 4 (and 2) apart hold further rows of the same channels
-  if (LPR <= 4) v = AddLaneXor4(v);
-  if (LPR <= 2) v = AddLaneXor2(v);
-  if (LPR <= 1) v = AddLaneXor1(v);
-  return v;
+  p.seg[0].dst[((size_t)(n >> 2) * M + m) * 4 + (n & 3)] = __float2half_rn(GatedActivation(activation, gu[0], gu[1]));
 }
 
 // Launch parameters of the strip kernel: what a single-matrix launch reads sits in the first
@@ -1708,7 +1665,9 @@ hipError_t LaunchFcW4StreamFused(const FcArgs* args, int count, hipStream_t stre
     const int lpr_b = wide ? 8 : 4, rows_b = wide ? 64 : 64;
     p.chunks_per_split = DivUp(p.chunks, rows_b) * rows_b;
     p.seg[0].strip_end = DivUp(p.seg[0].row_u4, lpr_b);
-    const dim3 grid_b(p.seg[0].strip_end, 1, a.rows);
+    p.pairs = (uint32_t)DivUp(p.seg[0].strip_end, 2);
+    p.pairs_magic = (uint32_t)((((uint64_t)1 << 32) + p.pairs - 1) / p.pairs);
+    const dim3 grid_b = wide ? dim3(p.seg[0].strip_end, 1, a.rows) : dim3(DivUp((int)p.pairs * a.rows, 8) * 16);
     return wide ? LaunchBatchedM<8, 8>(p, grouped, grid_b, stream) : LaunchBatchedM<4, 4>(p, grouped, grid_b, stream);
   }
 
@@ -1848,10 +1807,19 @@ hipError_t LaunchFcW4Gated(const FcArgs& gate, const FcArgs& up, int activation,
   p.src_end_idx = p.dst_end_idx = -1;
   p.k_channels = gate.k;
   if (kernel_name) *kernel_name = "fc_w4_gated_stream_kernel";
-  // 128-byte row segments, 8 waves: 64 rows of chunks per pass (one pass covers K = 2048); the
-  // 16-wave shape would spill with the two sets of accumulators
+  // 128-byte row segments, 8 waves: 64 rows of chunks (K = 2048); 16 for longer K where the registers suffice (two tokens, or
+  // group-wise scales next to both matrices' weights, would spill)
   const dim3 grid(DivUp(p.seg[0].row_u4, 8));
-  return LaunchGatedM<8, 8>(p, grouped, activation, grid, stream);
+#define MLD_GATED(W, M, G) hipLaunchKernelGGL((fc_w4_gated_stream_kernel<W, M, G>), grid, dim3(W * 64), 0, stream, p, activation)
+  if (p.m == 1 && p.chunks > 64 && !grouped)
+    MLD_GATED(16, 1, false);
+  else if (p.m == 1) {
+    if (grouped) MLD_GATED(8, 1, true); else MLD_GATED(8, 1, false);
+  } else {
+    if (grouped) MLD_GATED(8, 2, true); else MLD_GATED(8, 2, false);
+  }
+#undef MLD_GATED
+  return hipGetLastError();
 }
 
 hipError_t LaunchFcW4Stream(const FcArgs& a, hipStream_t stream, const char** kernel_name) {
