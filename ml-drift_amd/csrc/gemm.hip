@@ -1544,10 +1544,12 @@ __global__ __launch_bounds__(kTlThreads) void fc_w4_mfma_tiled_kernel(GemmParams
 
 // Second pass of a K split across work-groups: adds the parts in a fixed order, converts, adds
 // the bias.  One thread per (slice, token).
-__global__ __launch_bounds__(256) void fc_w4_splitk_reduce_kernel(GemmParams p) {
+// Bound by latency: the parts come from other XCDs' writes.  Up to eight of them in flight, in work-groups of one wave, so that small
+// launches use more CUs (the step of 18 layers at 8 tokens, one such launch each: 620 -> 611 us; four at a time in 4 waves before).
+__global__ __launch_bounds__(64) void fc_w4_splitk_reduce_kernel(GemmParams p) {
   // items of all matrices of the launch, matrix after matrix (the list entries by value: fixed
   // argument offsets, one batch of scalar loads)
-  uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+  uint32_t idx = blockIdx.x * 64u + threadIdx.x;
   const uint32_t m = (uint32_t)p.m;
   const uint32_t items0 = (uint32_t)p.seg[0].ns * m, items1 = (uint32_t)p.seg[1].ns * m;
   int si = 0;
@@ -1563,15 +1565,15 @@ __global__ __launch_bounds__(256) void fc_w4_splitk_reduce_kernel(GemmParams p) 
   const uint32_t items = (uint32_t)sg.ns * m;
   if (idx >= items) return;
   const float4* part = reinterpret_cast<const float4*>(sg.partial) + idx;
-  // the shares are added in their order, four loads in flight at a time
-  float4 sum = part[0];
+  // the shares are added in their order, up to eight loads in flight at a time
+  float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const int ksplit = p.ksplit;
-  for (int s0 = 1; s0 < ksplit; s0 += 4) {
-    float4 o[4];
+  for (int s0 = 0; s0 < ksplit; s0 += 8) {
+    float4 o[8];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = part[(size_t)min(s0 + j, ksplit - 1) * items];
+    for (int j = 0; j < 8; ++j) o[j] = part[(size_t)min(s0 + j, ksplit - 1) * items];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < 8; ++j) {
       if (s0 + j < ksplit) {
         sum.x += o[j].x;
         sum.y += o[j].y;
@@ -2177,7 +2179,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     if (p.ksplit <= 1) return;
     size_t items = 0;
     for (int i = 0; i < count; ++i) items += (size_t)p.seg[i].ns * a.m;
-    hipLaunchKernelGGL(fc_w4_splitk_reduce_kernel, dim3((unsigned)DivUp((long)items, 256L)), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL(fc_w4_splitk_reduce_kernel, dim3((unsigned)DivUp((long)items, 64L)), dim3(64), 0, stream, p);
   };
   // Few tokens, or few tiles: fc_w4_mfma_skinny_kernel.  Below 5 tokens the token forms of the GEMVs are
   // faster (628 us at 4 tokens against 870 before the loop was pipelined) and callers come here only where those do not serve.
