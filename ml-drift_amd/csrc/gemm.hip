@@ -612,7 +612,7 @@ __device__ __forceinline__ int WaveInclusiveSum(int v) {
 template <int WB, int FM, int U, int WAVES, bool ZP, bool PAIR, bool MULTI, int MODE = kModePlain>
 __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct_kernel(GemmParams p) {
   constexpr bool GATED = MODE == kModeGated, PACKED = MODE == kModePacked;
-  static_assert(!PACKED || (!PAIR && !MULTI), "packed groups: one matrix per group, tokens read one by one");
+  static_assert(!PACKED || !MULTI, "packed groups: one matrix per group");
   static_assert(WB == 4 || WB == 8, "uint4 or uint8 weights");
   static_assert(!GATED || (!ZP && !MULTI), "the gated pair is symmetric and is the whole launch");
   static_assert(!PAIR || FM % 2 == 0, "pairs of token blocks");
@@ -1170,13 +1170,13 @@ template <int FM, int WAVES>
 void LaunchPackedW(int weight_bits, bool zp, dim3 grid, hipStream_t stream, const GemmParams& p) {
   const dim3 block(WAVES * 64);
   if (weight_bits == 8 && zp)
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, true, false, false, kModePacked>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, true, FM != 1, false, kModePacked>), grid, block, 0, stream, p);
   else if (weight_bits == 8)
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, false, false, false, kModePacked>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<8, FM, 4, WAVES, false, FM != 1, false, kModePacked>), grid, block, 0, stream, p);
   else if (zp)
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, true, false, false, kModePacked>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, true, FM != 1, false, kModePacked>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, false, false, false, kModePacked>), grid, block, 0, stream, p);
+    hipLaunchKernelGGL((fc_w4_mfma_direct_kernel<4, FM, 4, WAVES, false, FM != 1, false, kModePacked>), grid, block, 0, stream, p);
 }
 // Waves that share the K of a tile of packed groups.  One wave per tile needs no reduction through LDS (8
 // waves on 768 input channels: 80 us, one wave 41), more of them fill the chip when the tiles are few.
@@ -2140,8 +2140,9 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
     // groups stay far below: 512 tokens over 128 experts, 8 each, are 32 tokens per group on average and
     // may be 512 in one).  128 experts of 2048 -> 768 at that average: 45.8 / 35.9 / 47.7 us with 32- / 64- /
     // 128-token tiles; 8 experts of 4096 -> 14336 at an average of 512: 704 / 561 / 537 us; 4 tokens on
-    // average: 25.6 / 27.1 / 40.5 us.  A group starts at any token, so the tiles are read token by token
-    // (no 16-byte token pairs).
+    // average: 25.6 / 27.1 / 40.5 us.  A group starts at any token and its last token may be paired with the next group's
+    // first, whose column is not stored; read token by token instead, 4096 tokens of 128 experts took 143 us for the three
+    // projections of a layer, 133 in pairs.
     const double average = (double)a.m / a.weights_batch;
     int fm = p.pg_max <= 32 || average <= 20.0 ? 1 : (average >= 512.0 ? 4 : 2);
     if (tune.gemm_fm == 1 || tune.gemm_fm == 2 || tune.gemm_fm == 4) fm = tune.gemm_fm;
