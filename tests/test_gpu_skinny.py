@@ -138,3 +138,30 @@ def test_offsets_below_two_gib(k, n, form):
         ref = act.double().cpu().numpy().transpose(1, 0, 2).reshape(m, k) @ wf
         err = np.abs(out[s].double().cpu().numpy() - ref)
         assert np.all(err <= 2.0 ** -10 * np.abs(ref) + 6 * 2.0 ** -10 * np.sqrt(np.mean(ref ** 2)))
+
+
+# 64-channel tiles up to 16 tokens, whose codes are multiplied before they are scaled: K tails, the last slices of a matrix, K cut in
+# 8, activations with a mean (codes and what they carry beside u - 8 cancel), one token with an infinite value
+@pytest.mark.parametrize("m,k,n,groups", [(5, 544, 12804, 17), (16, 2048, 16384, 64), (8, 1056, 12800, 33), (11, 8192, 2052, 64), (16, 9001, 100, 1)])
+def test_codes_before_scales(m, k, n, groups):
+    case = W.make_fc_case(seed=m + k, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=groups, with_bias=True)
+    case["act"] = (case["act"].astype(np.float32) + 2.0).astype(np.float16)
+    print("codes before scales", m, k, n, groups, flush=True)
+    dev = W.FcDevice(case)
+    dev.run()
+    got = dev.result()
+    assert dev.op.kernel_variant.startswith("skinny 64x16 k"), dev.op.kernel_variant
+    # per step of 32 channels: sums of up to 1039 |a|, 2^-23 of them lost per addition at most; then as `check`
+    ref = textbook(case)
+    act, scale = np.abs(case["act"].astype(np.float64)), np.abs(case["scale"].astype(np.float64))
+    steps = act.sum(axis=1, keepdims=True) * 1039 * 2.0 ** -23 * 32 @ scale.max(axis=1, keepdims=True).T
+    err = np.abs(got - ref)
+    assert np.all(err <= 2.0 ** -10 * (np.abs(ref) + np.abs(ref).mean()) + steps), float((err / (np.abs(ref) + 1)).max())
+    inf = dict(case, act=np.array(case["act"]))
+    inf["act"][m - 1, k - 1] = np.inf
+    dev = W.FcDevice(inf)
+    dev.run()
+    got_inf = dev.result()
+    assert np.array_equal(got_inf[:m - 1], got[:m - 1])
+    sign = np.sign(case["w"][:, k - 1].astype(np.float64) * case["scale"][:, -1].astype(np.float16).astype(np.float64))
+    assert np.array_equal(got_inf[m - 1], np.where(sign == 0, np.nan, np.copysign(np.inf, sign)), equal_nan=True)
