@@ -147,7 +147,12 @@ __global__ __launch_bounds__(1024) void quantize_kernel(QuantParams p) {
   const int lr = threadIdx.x / TT;
   const int wave = threadIdx.x / 64;
   const int waves = blockDim.x / 64;
-  const int tok_raw = blockIdx.x * TT + lt;
+  // A slice of 8 fp16 tokens is half a 128-byte line: work-groups L and L + 8, which run on one XCD, take the two halves, so
+  // that one L2 fetches the line (2048 tokens x 2048 channels with the int8 product behind it 43.0 -> 42.0 us, 41.1 -> 40.0 on another
+  // card).  The last work-groups, fewer than 16, keep their own places.
+  int tile = blockIdx.x;
+  if (TT * sizeof(RawT) < 128 && tile < (int)(gridDim.x & ~15u)) tile = (tile & ~15) + 2 * (tile & 7) + ((tile >> 3) & 1);
+  const int tok_raw = tile * TT + lt;
   const bool tok_ok = tok_raw < p.tokens;
   const int tok = tok_ok ? tok_raw : p.tokens - 1;
   const int s16_count = (p.slices + 3) / 4;

@@ -93,6 +93,20 @@ def test_config4_activation_quantization(oracle):
         assert np.all(np.abs(deq - x.astype(np.float32)) <= 0.51 * params[:, 0:1] + 1e-6)
 
 
+# token tiles of 8: 15 (none swapped), 16, 17, 32 and 33 of them, the last one full or not
+@pytest.mark.parametrize("tokens", [120, 121, 128, 129, 256, 263])
+@pytest.mark.parametrize("dtype", [np.float16, np.float32])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_tiles_of_eight_tokens(oracle, tokens, dtype, symmetric):
+    rng = np.random.default_rng(tokens)
+    src = W.to_slices(edge_tensor(rng, tokens, 180)).astype(dtype)
+    codes, params = run_quant(src, tokens, 180, M.PACKED_INT8C16, symmetric, True)
+    osrc = oracle.f32_to_f16_bits(src.astype(np.float32)) if dtype == np.float16 else src
+    rcodes, rparams = oracle.quantize(osrc, tokens, 180, M.PACKED_INT8C16, symmetric, True)
+    assert np.array_equal(params.view(np.uint32), rparams.view(np.uint32))
+    assert np.array_equal(codes, rcodes)
+
+
 def test_batched_seed_element(oracle):
     # tokens = (y*W+x)*B+b: the asymmetric search of token t starts from element (b = t % B, 0, 0, 0)
     rng = np.random.default_rng(3)
