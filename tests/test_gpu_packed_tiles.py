@@ -105,6 +105,17 @@ def test_forms(oracle, monkeypatch, sizes, k, n, form, bits):
     assert ops[-1].kernel_variant == "packed " + form
 
 
+# a 32-token tile for every CU and more
+@pytest.mark.parametrize("sizes,k,n,form", [
+    ([8] * 40, 256, 1000, "32x4"), ([5] * 90, 512, 388, "32x4"), ([6, 0] * 70, 128, 772, "32x1"), ([9, 1, 20] * 30, 64, 900, "32x1")])
+@pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False)])
+def test_forms_of_many_small_groups(oracle, monkeypatch, sizes, k, n, form, bits, zp):
+    ops, create = [], M.fc_create
+    monkeypatch.setattr(M, "fc_create", lambda *a, **kw: ops.append(create(*a, **kw)) or ops[-1])
+    run(oracle, sizes, k, n, bits=bits, groups=2 if bits == 4 else 1, zp=zp, seed=k + n)
+    assert ops[-1].kernel_variant == "packed " + form
+
+
 # token tiles on the XCDs: as many as XCDs and one more, fewer, all in one group, more groups than tokens; channel tiles 1, 2, 9, 18
 @pytest.mark.parametrize("sizes", [[1] * 9, [1] * 8, [0, 2, 0], [0] * 30 + [3] + [0] * 30, [40, 33, 0, 64, 1, 65, 70, 40, 2], [300]])
 @pytest.mark.parametrize("n", [100, 256, 1152, 2244])
