@@ -566,7 +566,7 @@ __device__ __forceinline__ void SwapRegisters(u32x4& a, u32x4& b) {
 // one 16-byte load brings both activation operands.  With an odd token count every other row starts 8 bytes off a 16-byte
 // boundary, which these loads (4-byte alignment) take; the last token's partner is then the next row's first token, or, past
 // the buffer's end, zero (the range check is per 32-bit word), in a column of the MFMA that is never stored.  Tokens read one
-// by one there, without the 128-token and two-tile forms: 8191 tokens x 4096 x 14336 1216 us, 856 like this; 2047 x 2048 x 4096
+// by one there, in 64-token tiles at most: 8191 tokens x 4096 x 14336 1216 us, 856 like this; 2047 x 2048 x 4096
 // 55.5 / 38.9; 333 x 1656 x 2900 with uint8 weights 16.1 / 15.1.
 // MULTI: the launch covers more than one matrix (the single-matrix instantiation reads its
 // arguments at fixed offsets instead of through a dependent scalar load).
@@ -2245,7 +2245,7 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   };
   const Tuning& tune = GetTuning();
   // the geometry the work-groups would otherwise divide out: waves = waves of the work-group that
-  // share one tile's K (all of them, or half in the gated and two-tile modes)
+  // share one tile's K (all of them, or half in the gated mode)
   auto set_geometry = [&p](int tiles_m, int tiles_n_grid, int waves, bool halves) {
     const int xn = 8 / p.xcd_m;
     p.geo_tiles_m = tiles_m;
