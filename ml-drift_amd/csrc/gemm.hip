@@ -1641,18 +1641,13 @@ __global__ __launch_bounds__(64) void fc_w4_splitk_reduce_kernel(GemmParams p) {
 // the two blocks that it loads; at T = 1 four lanes load the same blocks and unpack one channel each (a
 // lane-constant shift, mask and exponent), which costs L1 bandwidth, not HBM.  A lane holds one
 // token of whole 4-channel slices at the end: one 8-byte store.  Weights are dequantized as in the kernel
-// above (round_fp16((u - 8) * s)).  kSkinnySteps steps of 32 input channels are in flight per wave; the
+// above (round_fp16((u - 8) * s)): the matrix cores never see the 1024 + u of the unpacking, whose product with a large activation
+// would leave its rounding in channels where the weight is zero.  kSkinnySteps steps of 32 input channels are in flight per wave; the
 // activations' descriptor ends with the wave's share of K, so steps past it add zeros.
 // Bound: first-load latency and the launch for layers of 2048 channels, then the vector ALU's unpacking.
 // Against 32-token tiles of 128 channels (24 work-groups for the q/k/v projections of 2048 channels), in a step
 // of 18 layers (hidden 2048, MLP 16384, group 32): 988 -> 620 us at 8 tokens, 999 -> 632 at 16, 1008 -> 741
 // at 32; q/k/v 10.3 -> 6.1 us, o 10.4 -> 5.7, down 16.7 -> 7.4 (profiler figures, its second launch 4.1 either way).
-// RAW (64-channel tiles, up to 16 tokens, no zero points): a step's codes go to the matrix cores as they are unpacked (1024 + u,
-// 64 + u), a constant matrix starts the sums with -(1024 + 8) and
-// -(64 + 8) times the activations, and the step's sums are scaled as they are added: 36 vector instructions per step instead of
-// 52, and no rounding of the weights.  The scales of a row of the result, which is a slice, come from LDS.  Four steps in
-// flight leave registers for two work-groups per CU (eight: 606 us).  A step of 18 layers at 8 tokens 611 -> 565 us; 2048 ->
-// 32768 at 8 tokens 12.0 -> 11.0.  In narrower tiles the loads are what counts: no faster there.
 // Several token tiles read one strip's weights on one XCD (grid.x is a multiple of 8): 2048 -> 2048 at 128 tokens 8.4 -> 5.7 us.
 // ------------------------------------------------------------------------------------------
 constexpr int kSkinnyWaves = 8;
@@ -1661,18 +1656,12 @@ constexpr int kSkinnyMaxTokens = 32;        // one token tile
 constexpr int kSkinnyMaxTiledTokens = 384;  // token tiles of 32 along grid.z
 constexpr int kSkinnySplitK = 8192;  // input channels from which K is cut between work-groups
 
-// K-steps in flight per wave (what the registers of two work-groups per CU allow)
-__host__ __device__ constexpr int SkinnyUnroll(int t, int ft, bool zp) { return ft != 1 || (t == 4 && !zp) ? kSkinnySteps / 2 : kSkinnySteps; }
-
 template <int T, int FT, bool ZP, bool MULTI>
 __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(GemmParams p) {
   typedef float float4v_t __attribute__((ext_vector_type(4)));
   constexpr int Q = 4 / T;  // rows per slice; tiles per strip of 16 slices
-  constexpr bool RAW = T == 4 && FT == 1 && !ZP;
-  constexpr int U = SkinnyUnroll(T, FT, ZP);
+  constexpr int U = FT == 1 ? kSkinnySteps : kSkinnySteps / 2;  // (registers)
   __shared__ float4 red[kSkinnyWaves][T * FT][64];
-  // RAW: the scales of a batch of U steps, wave by wave: [step][slice][4] halfs
-  __shared__ __align__(16) __half scales[RAW ? kSkinnyWaves : 1][RAW ? U : 1][RAW ? 16 * T : 1];
 
   asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.group_shift), "s"(p.b_bytes), "s"(p.act), "s"(p.magic_lo), "s"(p.magic_hi),
                "s"(p.mask_lo), "s"(p.mask_hi), "s"(p.segments), "s"(p.geo_per_wave), "s"(p.ksplit));
@@ -1724,8 +1713,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
   const uint32_t col_w = (nsi_group * (uint32_t)p.ks * (uint32_t)sg.group + ((uint32_t)nsi - nsi_group * (uint32_t)sg.group)) * 8u;
   const bool n_ok = nsi < sg.ns;
   const uint32_t k0 = (uint32_t)s_begin * 8u + 2u * (uint32_t)g;  // the first of this lane's two K-slices
-  const uint32_t vw_first = n_ok ? k0 * row_w + col_w : kOob;
-  uint32_t vw = vw_first;
+  uint32_t vw = n_ok ? k0 * row_w + col_w : kOob;
   const uint32_t vs = n_ok ? (uint32_t)nsi * 8u + (uint32_t)(ch0 * 2) : kOob;
   const uint32_t group_bytes = (uint32_t)sg.ns * 8u;
   uint32_t vx[FT];
@@ -1740,33 +1728,9 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
     if constexpr (T == 4) v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, at, 0, 0);
     return v;
   };
-  // RAW: a lane's share of the scales of U steps from step s on: 64 / U lanes per step
-  constexpr int kShare = U * T / 2;  // bytes
-  u32x4 batch_scales = {0u, 0u, 0u, 0u};
-  auto load_scales = [&](int s) {
-    const uint32_t at = (uint32_t)((s + (lane / (64 / U)) * kSkinnyWaves) >> (p.group_shift - 1)) * group_bytes + (uint32_t)slice0 * 8u +
-                        (uint32_t)(lane % (64 / U)) * kShare;
-    if constexpr (kShare == 2) batch_scales[0] = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsrc_s, at, 0, 0);
-    if constexpr (kShare == 4) batch_scales[0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_s, at, 0, 0);
-    if constexpr (kShare == 8) {
-      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc_s, at, 0, 0);
-      batch_scales[0] = v[0];
-      batch_scales[1] = v[1];
-    }
-    if constexpr (kShare == 16) batch_scales = __builtin_amdgcn_raw_buffer_load_b128(rsrc_s, at, 0, 0);
-  };
-  auto put_scales = [&] {
-    uint8_t* to = reinterpret_cast<uint8_t*>(&scales[RAW ? wave : 0][0][0]) + lane * kShare;
-    __builtin_amdgcn_wave_barrier();
-    if constexpr (kShare == 2) *reinterpret_cast<uint16_t*>(to) = (uint16_t)batch_scales[0];
-    if constexpr (kShare == 4) *reinterpret_cast<uint32_t*>(to) = batch_scales[0];
-    if constexpr (kShare == 8) *reinterpret_cast<u32x2*>(to) = u32x2{batch_scales[0], batch_scales[1]};
-    if constexpr (kShare == 16) *reinterpret_cast<u32x4*>(to) = batch_scales;
-    __builtin_amdgcn_wave_barrier();  // (the wave's own items: its LDS accesses are in order)
-  };
-  auto load_step = [&](int s, int u, bool with_scale) {
+  auto load_step = [&](int s, int u) {
     const uint32_t at = vs + (uint32_t)(s >> (p.group_shift - 1)) * group_bytes;
-    if (with_scale) rsc[u] = load_channels(rsrc_s, at);
+    rsc[u] = load_channels(rsrc_s, at);
     if (ZP) rzp[u] = load_channels(rsrc_z, at);
 #pragma unroll
     for (int ft = 0; ft < FT; ++ft) {
@@ -1796,50 +1760,13 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
   const half2_t off_lo = {(_Float16)-1032.0f, (_Float16)-1032.0f}, off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
   const half2_t lane_off = lane_odd ? off_hi : off_lo;
 
-  // RAW: what the codes carry beside u - 8 (1024 + 8, 64 + 8), as a constant matrix whose product with the activations starts
-  // the sums of a step; a matrix of odd and even channels has both.
-  const uint32_t off_word[2] = {T == 1 ? (lane_odd ? 0xD480D480u : 0xE408E408u) : 0xE408E408u, 0xD480D480u};  // -1032, -72
   __builtin_amdgcn_sched_barrier(0);
-  if (RAW) load_scales(s_begin);
 #pragma unroll
   for (int u = 0; u < U; ++u) {  // (in the order of their use: waiting for one step leaves the younger ones in flight)
-    load_step(s_begin + u * kSkinnyWaves, u, !RAW);
+    load_step(s_begin + u * kSkinnyWaves, u);
     __builtin_amdgcn_sched_barrier(0);
   }
-  float activations = 0.0f;
-  auto multiply_raw = [&](int u) {
-    u32x4 blk = {rw[u][0][0], rw[u][0][1], rw[u][1][0], rw[u][1][1]}, blk8 = blk;
-    if constexpr (T == 4) blk8 = u32x4{blk[0] >> 8, blk[1] >> 8, blk[2] >> 8, blk[3] >> 8};
-    else blk = u32x4{blk[0] >> lane_shift, blk[1] >> lane_shift, blk[2] >> lane_shift, blk[3] >> lane_shift};
-    const half8_t bop = __builtin_bit_cast(half8_t, u32x4{rx[u][0][0][0], rx[u][0][0][1], rx[u][0][1][0], rx[u][0][1][1]});
-    float4v_t start[2];
-#pragma unroll
-    for (int i = 0; i < (T == 1 ? 1 : 2); ++i)
-      start[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, u32x4{off_word[i], off_word[i], off_word[i], off_word[i]}), bop,
-                                                        float4v_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-    activations += start[0][0];
-    // rows 4 g .. 4 g + 3: channel v T + t of the T slices from g T on
-    uint32_t sc[2 * T];
-    const uint32_t* from = reinterpret_cast<const uint32_t*>(&scales[RAW ? wave : 0][RAW ? u : 0][RAW ? g * 4 * T : 0]);
-#pragma unroll
-    for (int i = 0; i < 2 * T; ++i) sc[i] = from[i];
-    float4v_t d[T];
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      u32x4 aop;
-#pragma unroll
-      for (int wd = 0; wd < 4; ++wd) {
-        const uint32_t x = T == 4 && (t & 2) ? blk8[wd] : blk[wd];
-        aop[wd] = T == 1 ? ((x & lane_mask) | lane_magic) : ((t & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo));
-      }
-      d[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, aop), bop, start[T == 1 ? 0 : t & 1], 0, 0, 0);
-    }
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[t][0][v] = fmaf((float)AsHalf2(sc[(v * T + t) >> 1])[(v * T + t) & 1], d[t][v], acc[t][0][v]);
-  };
-  auto multiply_dequantized = [&](int u) {
+  auto multiply_step = [&](int u) {
     u32x4 blk = {rw[u][0][0], rw[u][0][1], rw[u][1][0], rw[u][1][1]}, blk8 = blk;
     if constexpr (T == 4) blk8 = u32x4{blk[0] >> 8, blk[1] >> 8, blk[2] >> 8, blk[3] >> 8};
     else blk = u32x4{blk[0] >> lane_shift, blk[1] >> lane_shift, blk[2] >> lane_shift, blk[3] >> lane_shift};
@@ -1870,55 +1797,22 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
       }
     }
   };
-  auto multiply_step = [&](int u) {
-    if constexpr (RAW) multiply_raw(u); else multiply_dequantized(u);
-  };
   // All steps but the last U are refilled; the last U have loops of their own, so that no wait has to allow for a
   // refill that may not be there.
   int s0 = 0;
   for (; s0 + U < per_wave; s0 += U) {
-    if (RAW) {
-      put_scales();
-      load_scales(s_begin + (s0 + U) * kSkinnyWaves);
-      __builtin_amdgcn_sched_barrier(0);
-    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       multiply_step(u);
       __builtin_amdgcn_sched_barrier(0);
-      load_step(s_begin + (s0 + U + u) * kSkinnyWaves, u, !RAW);
+      load_step(s_begin + (s0 + U + u) * kSkinnyWaves, u);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (RAW) put_scales();
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     multiply_step(u);
     __builtin_amdgcn_sched_barrier(0);
-  }
-
-  if constexpr (RAW) {
-    // An infinite activation meets its codes and what they carry with opposite signs there: NaN, where (u - 8) * s * a may
-    // be infinite.  The rare token with one has its sums done over from dequantized weights.
-    const bool infinite = !(fabsf(activations) <= 3.4028235e38f);
-    if (__builtin_expect(__any(infinite), 0)) {
-      float4v_t raw[T];
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        raw[t] = acc[t][0];
-        acc[t][0] = float4v_t{0.0f, 0.0f, 0.0f, 0.0f};
-      }
-      vw = vw_first;
-      vx[0] = token0 + r < p.m ? k0 * row_x + (uint32_t)(token0 + r) * 8u : kOob;
-      for (int i = 0; i < per_wave; ++i) {
-        load_step(s_begin + i * kSkinnyWaves, 0, true);
-        multiply_dequantized(0);
-      }
-#pragma unroll
-      for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) acc[t][0][v] = infinite ? acc[t][0][v] : raw[t][v];
-    }
   }
 
   // Register v of lane (r, g) is row 4 g + v: slice g T + q of the tile holds its channel c in
@@ -2005,7 +1899,7 @@ SkinnyPlan PlanSkinny(int m, int k, int n, int direct_split) {
 
 // The prefetch ends with whole batches of steps in every wave: K-slices up to which offsets are formed.
 bool SkinnyOffsetsFit(const GemmParams& p) {
-  const int unroll = kSkinnySteps;
+  const int unroll = p.m <= 16 ? kSkinnySteps : kSkinnySteps / 2;
   const uint64_t per_slice = (uint64_t)kSkinnyWaves * 8;
   const uint64_t end = ((uint64_t)(p.ksplit - 1) * p.geo_per_wave + (uint64_t)DivUp(p.geo_per_wave, unroll) * unroll) * per_slice;
   const uint64_t past = end > (uint64_t)p.ks ? end - p.ks : 0;
