@@ -503,13 +503,15 @@ hipError_t LaunchBatchedM(const StreamParams& p, bool grouped, dim3 grid, hipStr
 // FullyConnected nodes would store them, then combined in fp32 in the operation order of the
 // sample's elementwise kernel.  Only seg[0].dst is written.
 // Bound: HBM, with at most one strip per CU (14336 channels: 224).  A thread has one chunk of both matrices in flight, 16 loads;
-// 16 waves hold all of K = 4096 at once: gate, up and down of 4096 x 14336, 20.8 -> 20.1 us a layer (two chunks per thread
-// of 8 waves, the same bytes in flight: 21.6; the waves' sums through LDS instead of register exchanges: the same).
+// 16 waves hold all of K = 4096 at once: gate and up of 4096 x 14336 12.9 -> 12.2 us.  Chunks 64 apart are added first and
+// rows in the order of 8 waves, so that a result does not depend on the number of waves or tokens.
 // ------------------------------------------------------------------------------------------
 template <int WAVES, int M, bool GROUPED>
 __global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamParams p, int activation) {
-  constexpr int LPR = 8, ROWS = WAVES * 64 / LPR, STRIP = LPR * 8;
-  __shared__ float red[WAVES][2 * M][STRIP];
+  constexpr int LPR = 8, ROWS = WAVES * 64 / LPR, STRIP = LPR * 8, PARTS = 8;
+  static_assert(WAVES == PARTS || WAVES == 2 * PARTS, "8 parts of 8 rows, or of 8 pairs of rows");
+  __shared__ float red[ROWS][2 * M][STRIP];
+  __shared__ float red2[PARTS][2 * M][STRIP];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -522,6 +524,16 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamPa
   const int pcol = pcol_raw < row_u4 ? pcol_raw : row_u4 - 1;  // clamp: loads stay in range, result unused
   const int rstride = p.seg[0].gu4;
   const size_t wcol_off = (size_t)(pcol / rstride) * p.ks * rstride + pcol % rstride;
+
+  // scales / biases of the output this thread finishes, fetched ahead (raw halfs, clamped index)
+  const int n_out = min(strip * STRIP + lane, p.seg[0].n_pad - 1);
+  unsigned short scale_raw[2], bias_raw[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const unsigned short* bias_src = reinterpret_cast<const unsigned short*>(p.seg[q].bias ? p.seg[q].bias : p.seg[q].scale);
+    scale_raw[q] = reinterpret_cast<const unsigned short*>(p.seg[q].scale)[n_out];
+    bias_raw[q] = bias_src[n_out];
+  }
 
   float acc[2][M][8];
 #pragma unroll
@@ -569,12 +581,27 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamPa
     }
   }
 
-  // the rows of a wave by register exchanges, the waves through LDS, in wave order
-  const int ch_wave = col * 8 + ((lane >> 3) & 7);
 #pragma unroll
   for (int q = 0; q < 2; ++q)
 #pragma unroll
-    for (int m = 0; m < M; ++m) red[wave][q * M + m][ch_wave] = WaveStripSum<LPR>(acc[q][m], lane);
+    for (int m = 0; m < M; ++m) {
+      float4* dst4 = reinterpret_cast<float4*>(&red[row][q * M + m][col * 8]);
+      dst4[0] = make_float4(acc[q][m][0], acc[q][m][1], acc[q][m][2], acc[q][m][3]);
+      dst4[1] = make_float4(acc[q][m][4], acc[q][m][5], acc[q][m][6], acc[q][m][7]);
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PARTS * 2 * M / WAVES; ++i) {
+    const int part = wave % PARTS, qm = i * (WAVES / PARTS) + wave / PARTS;
+    float v = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      float x = red[part * 8 + r][qm][lane];
+      if (WAVES > PARTS) x += red[part * 8 + r + ROWS / 2][qm][lane];
+      v += x;
+    }
+    red2[part][qm][lane] = v;
+  }
   __syncthreads();
   const int m = tid / STRIP, ol = tid % STRIP;
   const int n = strip * STRIP + ol;
@@ -584,10 +611,10 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamPa
   for (int q = 0; q < 2; ++q) {
     float v = 0.0f;
 #pragma unroll
-    for (int k = 0; k < WAVES; ++k) v += red[k][q * M + m][ol];
-    if (!GROUPED) v *= __half2float(p.seg[q].scale[n]);
+    for (int k = 0; k < PARTS; ++k) v += red2[k][q * M + m][ol];
+    if (!GROUPED) v *= __half2float(__ushort_as_half(scale_raw[q]));
     __half h = __float2half_rn(v);
-    if (p.seg[q].bias) h = __hadd(h, p.seg[q].bias[n]);
+    if (p.seg[q].bias) h = __hadd(h, __ushort_as_half(bias_raw[q]));
     gu[q] = __half2float(h);
   }
   p.seg[0].dst[((size_t)(n >> 2) * M + m) * 4 + (n & 3)] = __float2half_rn(GatedActivation(activation, gu[0], gu[1]));
@@ -1807,11 +1834,12 @@ hipError_t LaunchFcW4Gated(const FcArgs& gate, const FcArgs& up, int activation,
   p.src_end_idx = p.dst_end_idx = -1;
   p.k_channels = gate.k;
   if (kernel_name) *kernel_name = "fc_w4_gated_stream_kernel";
-  // 128-byte row segments, 8 waves: 64 rows of chunks (K = 2048); 16 for longer K where the registers suffice (two tokens, or
-  // group-wise scales next to both matrices' weights, would spill)
+  // 128-byte row segments, 8 waves: 64 rows of chunks (K = 2048); 16 where they hold all of K and 8 do not (us with 8 / 16:
+  // 4096 x 14336 12.9 / 12.2, 2560 x 16384 10.1 / 10.0; longer K: 5120 x 16384 15.4 / 15.8, 8192 x 16384 23.7 / 24.0) and the
+  // registers suffice (two tokens, or group-wise scales next to both matrices' weights, would spill)
   const dim3 grid(DivUp(p.seg[0].row_u4, 8));
 #define MLD_GATED(W, M, G) hipLaunchKernelGGL((fc_w4_gated_stream_kernel<W, M, G>), grid, dim3(W * 64), 0, stream, p, activation)
-  if (p.m == 1 && p.chunks > 64 && !grouped)
+  if (p.m == 1 && p.chunks > 64 && p.chunks <= 128 && !grouped)
     MLD_GATED(16, 1, false);
   else if (p.m == 1) {
     if (grouped) MLD_GATED(8, 1, true); else MLD_GATED(8, 1, false);

@@ -395,6 +395,31 @@ def run_gated_pair(oracle, m, k, n, groups, bias, kind, expect_kernel, ulp_check
     assert np.array_equal(gate.out.cpu().numpy(), g16) and np.array_equal(up.out.cpu().numpy(), u16)
 
 
+@pytest.mark.parametrize("k,n,groups", [(2048, 8192, 1), (2052, 8192, 1), (2592, 8192, 1), (4000, 8200, 1), (4096, 14336, 1), (4100, 4096, 1),
+                                        (5120, 8192, 1), (4096, 8192, 128)])
+def test_gated_pair_same_sums_for_one_and_two_tokens(k, n, groups):
+    """A token's sums are formed in one order, alone (16 waves where K is 2049..4096, else 8) or beside another token (8 waves):
+    the results are the same bit for bit."""
+    torch = torch_cuda()
+    cases = [W.make_fc_case(seed=k + i, m=2, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=groups, with_bias=True) for i in range(2)]
+    cases[1]["act"] = cases[0]["act"]
+    print("gated", k, n, groups, flush=True)
+
+    def gated(tokens):
+        gate, up = (W.FcDevice(dict(c, m=len(tokens), act=np.array(c["act"][tokens]))) for c in cases)
+        up.op.set_src(0, gate.act)
+        dst = torch.zeros_like(gate.out)
+        M.fc_launch_gated(gate.op, up.op, M.GATE_SILU, dst, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert gate.op.kernel_name == "fc_w4_gated_stream_kernel", gate.op.kernel_name
+        return W.from_slices(dst.cpu().numpy(), n)
+
+    both = gated([0, 1])
+    assert np.any(both != 0)
+    for t in range(2):
+        assert np.array_equal(gated([t])[0], both[t]), t
+
+
 @pytest.mark.parametrize("m,k,n,groups,bias", [(3, 512, 72, 16, False), (16, 2048, 2048, 1, True),
                                                (64, 1024, 1032, 32, True), (77, 352, 200, 11, False),
                                                (128, 2048, 16384, 64, False), (130, 96, 260, 1, True),
