@@ -107,6 +107,7 @@ struct mldhip_op {
   size_t partial_floats = 0;
   const char* last_kernel = "";
   const char* last_variant = "";  // the form of that kernel
+  int last_tiles[3] = {0, 0, 0};  // and how its work was cut
   // bytes every object needs at the current shape (kept up to date by create and set_shape, so that
   // a launch checks its bindings without touching the heap)
   std::vector<size_t> need_src, need_dst;
@@ -746,6 +747,8 @@ static int BuildFcArgs(mldhip_op* op, FcArgs* out) {
   a.partial_floats = op->partial_floats;
   op->last_variant = "";
   a.variant = &op->last_variant;
+  std::fill_n(op->last_tiles, 3, 0);
+  a.tiles = op->last_tiles;
   if (op->idx_params >= 0) {
     a.params = static_cast<const int32_t*>(op->src_ptr[op->idx_params]);
     a.src_end_ch_index = d.src_end_ch_index;
@@ -992,6 +995,13 @@ int mldhip_fc_int4_decode_noalloc(const void* src, const void* weights, const vo
 
 const char* mldhip_op_kernel_name(const mldhip_op* op) { return op ? op->last_kernel : ""; }
 const char* mldhip_op_kernel_variant(const mldhip_op* op) { return op ? op->last_variant : ""; }
+int mldhip_op_kernel_tiles(const mldhip_op* op, int* tokens, int* waves, int* k_parts) {
+  if (!op || !tokens || !waves || !k_parts) return Fail(MLDHIP_INVALID_ARGUMENT, "null argument");
+  *tokens = op->last_tiles[0];
+  *waves = op->last_tiles[1];
+  *k_parts = op->last_tiles[2];
+  return MLDHIP_OK;
+}
 
 int mldhip_op_cost(const mldhip_op* op, uint64_t* bytes, uint64_t* flops) {
   if (!op) return Fail(MLDHIP_INVALID_ARGUMENT, "null op");

@@ -2280,6 +2280,12 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   const int waves = gated ? (fm == 4 ? 4 : 8) : fm == 4 ? std::min(plan.waves, 4) : plan.waves == 1 ? 1 : (fm == 1 && plan.waves > 4 ? 8 : 4);
   p.ksplit = plan.ksplit;
   while (p.ksplit > 1 && !fits(p.ksplit)) p.ksplit /= 2;
+  for (int i = 0; i < count; ++i)
+    if (args[i].tiles) {
+      args[i].tiles[0] = fm * 32;
+      args[i].tiles[1] = waves;
+      args[i].tiles[2] = p.ksplit;
+    }
   const int tiles_m = DivUp(a.m, fm * 32);
   p.xcd_m = W4XcdGrid(tiles_m, tiles_n, fm * 32, a.k, p.groups);
   if (tune.gemm_xcd_m > 0) p.xcd_m = tune.gemm_xcd_m;

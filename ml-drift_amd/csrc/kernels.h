@@ -101,6 +101,7 @@ struct FcArgs {
   int ring_o_index = -1, ring_i_index = -1, ring_size = 0;
   int weights_k = 0;  // input channels of the weights buffer (ring_i); 0 = k
   const char** variant = nullptr;  // out: the form of the kernel that was launched (mldhip_op_kernel_variant)
+  int* tiles = nullptr;            // out: tokens of a tile, waves, parts of K (mldhip_op_kernel_tiles)
 };
 
 // Split-K workspace sizing for the streaming GEMV.

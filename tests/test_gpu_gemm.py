@@ -194,21 +194,33 @@ def test_w4_gemm_tiled_kernel_full_size(oracle):
         check_restatement(oracle, got[rows], sub, "kernel restatement (%s 32 tokens)" % name)
 
 
-@pytest.mark.parametrize("bits,m,k,n,groups,zp", [(4, 64, 512, 384, 4, False),    # 3 channel tiles: the last pair holds one
-                                                  (4, 130, 352, 1000, 11, True),   # ragged channels and tokens, 64-token tile
-                                                  (4, 256, 96, 260, 1, False),
-                                                  (8, 128, 1024, 640, 8, True),
-                                                  (4, 4096, 64, 2048, 2, True),    # 128-token tile
-                                                  (8, 2050, 96, 1100, 1, False)])
-def test_gemm_two_tiles_per_work_group(oracle, bits, m, k, n, groups, zp):
-    """The two-tile mode (half of a work-group's waves per channel tile), forced on shapes of test
-    size: odd tile counts, ragged edges, zero points, both weight types, both token tiles; and
-    the same bytes as the one-tile mode where the K shares coincide is not required - the bar is
-    the FullyConnected one."""
+def run_form(case, form, reference_layout=False, max_tokens=None):
+    """The case in one form of the direct kernel (tokens of a tile, waves, parts of K), which the launch has to have taken; twice, with
+    the same bits.  `max_tokens` beyond the case's own sizes the workspace for more parts of K than its own plan has."""
+    print("form", {k: case[k] for k in ("m", "k", "n", "groups", "weight_bits")}, form, flush=True)
+    with M.tuning(gemm_fm=form[0] // 32, gemm_waves=form[1], gemm_ksplit=form[2]):
+        dev = W.FcDevice(case, reference_layout=reference_layout, max_tokens=max_tokens)
+        dev.run()
+        got = dev.result()
+        assert (dev.op.kernel_variant, dev.op.kernel_tiles) == ("direct", form)
+        dev.out.zero_()
+        dev.run()
+        assert np.array_equal(got, dev.result(), equal_nan=True)
+    return got
+
+
+FORMS = [(32, 1), (32, 4), (32, 8), (64, 1), (64, 4), (128, 1), (128, 2), (128, 4)]
+
+
+@pytest.mark.parametrize("bits,m,k,n,groups,zp", [(4, 64, 512, 384, 4, False), (4, 130, 352, 1000, 11, True), (4, 256, 96, 260, 1, False),
+                                                  (8, 128, 1024, 640, 8, True), (4, 4096, 64, 2048, 2, True), (8, 2050, 96, 1100, 1, False)])
+@pytest.mark.parametrize("form", [(64, 4, 1), (128, 1, 1)])
+def test_gemm_forms_against_the_restatement(oracle, form, bits, m, k, n, groups, zp):
+    """64- and 128-token tiles, four waves and one, odd channel tile counts, ragged edges, zero points, both weight types: the
+    FullyConnected bar and, where it is affordable, the restatement of the reference's kernel."""
     case = W.make_fc_case(seed=m + n + bits, m=m, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups,
                           with_bias=True, with_zero_point=zp)
-    with M.tuning(gemm_dual=1):
-        got = run_w4(case)
+    got = run_form(case, form)
     check_fp(got, textbook(case), case, "textbook")
     small = m if restatement_affordable(case) else min(m, 64)
     sub = dict(case, m=small, act=case["act"][:small])
@@ -217,47 +229,77 @@ def test_gemm_two_tiles_per_work_group(oracle, bits, m, k, n, groups, zp):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("fm,dual", [(2, 0), (2, 1), (4, 0), (4, 1)])
+@pytest.mark.parametrize("form", [(64, 4, 1), (64, 1, 1), (128, 1, 1), (128, 4, 1)])
 @pytest.mark.parametrize("m,k,n,groups,zp", [(33, 64, 132, 2, False), (65, 136, 128, 1, True), (127, 96, 260, 3, False), (129, 1000, 388, 1, False)])
-def test_gemm_odd_token_counts(bits, fm, dual, m, k, n, groups, zp):
+def test_gemm_odd_token_counts(bits, form, m, k, n, groups, zp):
     """An odd token count: the last token travels in a pair with the next row's first token (or with what lies past the tensor).
     Each token's sums are formed in the same order as with one token more, so the results are the same bit for bit; the first
     token is infinite, which may show in its own results only."""
     case = W.make_fc_case(seed=m + k, m=m + 1, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups,
                           with_bias=True, with_zero_point=zp)
-    with M.tuning(gemm_fm=fm, gemm_dual=dual, gemm_ksplit=1):
-        even = run_w4(case, reference_layout=True)
-        check_fp(even, textbook(case), case, "one token more")
-        odd = dict(case, m=m, act=np.array(case["act"][:m]))
-        odd["act"][0] = np.inf
-        dev = W.FcDevice(odd, reference_layout=True)
-        dev.run()
-        got = dev.result()
+    even = run_form(case, form, reference_layout=True)
+    check_fp(even, textbook(case), case, "one token more")
+    odd = dict(case, m=m, act=np.array(case["act"][:m]))
+    odd["act"][0] = np.inf
+    got = run_form(odd, form, reference_layout=True)
     assert np.array_equal(got[1:], even[1:m])
     assert not np.isfinite(got[0]).any()
 
 
+def check_sums(got, case, label):
+    """Weights are rounded to fp16 (2^-11 relative, twice with a zero point), results once more; sums in fp32."""
+    k, groups = case["k"], case["groups"]
+    ref = textbook(case)
+    check_fp(got, ref, case, label)
+    w = case["w"].astype(np.float64) - (np.repeat(case["zero_point"], k // groups, axis=1) if case["zero_point"] is not None else 0.0)
+    size = np.abs(case["act"].astype(np.float64)) @ np.abs(w * np.repeat(case["scale"], k // groups, axis=1)).T
+    assert np.all(np.abs(got - ref) <= 2.0 ** -10 * size / np.sqrt(k) * 4 + 2.0 ** -9 * (np.abs(ref) + 1.0)), label
+
+
 @pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False)])
-@pytest.mark.parametrize("fm,waves", [(1, 1), (1, 4), (1, 8), (2, 1), (2, 4), (4, 1), (4, 2), (4, 4)])
-@pytest.mark.parametrize("m,k,n,groups,ksplit", [(5, 64, 4, 2, 1), (65, 136, 132, 1, 1), (128, 1056, 260, 33, 1), (131, 1024, 388, 1, 2), (257, 2048, 128, 4, 4)])
+@pytest.mark.parametrize("fm,waves", FORMS)
+@pytest.mark.parametrize("m,k,n,groups,ksplit", [(5, 64, 4, 2, 1), (65, 136, 132, 1, 1), (128, 1056, 260, 33, 1), (131, 4072, 388, 1, 2), (257, 4096, 128, 4, 4),
+                                                 (70, 4096, 260, 128, 8)])
 def test_gemm_waves_per_tile(fm, waves, bits, zp, m, k, n, groups, ksplit):
     """Every token tile with every number of waves that share a tile's K (one: whole sums in registers, tokens stored in pairs),
-    ragged tokens and channels, K that does not divide into the shares, K cut between work-groups too.  Weights are rounded to
-    fp16 (2^-11 relative, twice with a zero point), results once more; sums in fp32."""
+    ragged tokens and channels, K that does not divide into the shares, K cut between work-groups too."""
     case = W.make_fc_case(seed=m + n + bits, m=m, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups,
                           with_bias=True, with_zero_point=zp)
-    with M.tuning(gemm_fm=fm, gemm_waves=waves, gemm_ksplit=ksplit):
-        got = run_w4(case)
-    ref = textbook(case)
-    check_fp(got, ref, case, "textbook")
-    w = case["w"].astype(np.float64) - (np.repeat(case["zero_point"], k // groups, axis=1) if zp else 0.0)
-    size = np.abs(case["act"].astype(np.float64)) @ np.abs(w * np.repeat(case["scale"], k // groups, axis=1)).T
-    assert np.all(np.abs(got - ref) <= 2.0 ** -10 * size / np.sqrt(k) * 4 + 2.0 ** -9 * (np.abs(ref) + 1.0))
+    got = run_form(case, (fm, waves, ksplit), max_tokens=520)  # (520 tokens of these matrices: parts of K for 2 x 257)
+    check_sums(got, case, "textbook")
+
+
+@pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False), (8, True)])
+@pytest.mark.parametrize("fm,waves", FORMS)
+@pytest.mark.parametrize("m,ksplit", [(33, 1), (129, 4), (258, 2)])
+def test_gemm_forms_of_several_matrices(fm, waves, bits, zp, m, ksplit):
+    """Three matrices in one launch (4 + 1 + 3 channel tiles, ragged) in every form, odd token counts and K cut between
+    work-groups among them; the same bits as three launches of that form where K is whole."""
+    import torch
+    k = 4096 if ksplit > 1 else 200
+    cases = [W.make_fc_case(seed=60 + i + m, m=m, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=2 if ksplit > 1 else 1, with_bias=True,
+                            with_zero_point=zp) for i, n in enumerate((388, 100, 260))]
+    for c in cases[1:]:
+        c["act"] = cases[0]["act"]
+    print("several matrices", fm, waves, bits, zp, m, ksplit, flush=True)
+    with M.tuning(gemm_fm=fm // 32, gemm_waves=waves, gemm_ksplit=ksplit):
+        devs = [W.FcDevice(c, max_tokens=1025) for c in cases]
+        for d in devs[1:]:
+            d.op.set_src(0, devs[0].act)
+        M.fc_launch_fused([d.op for d in devs], torch.cuda.current_stream().cuda_stream)
+        results = [d.result() for d in devs]
+        for d, c, got in zip(devs, cases, results):
+            assert (d.op.kernel_variant, d.op.kernel_tiles) == ("direct", (fm, waves, ksplit))
+            check_sums(got, c, "n=%d" % c["n"])
+            d.out.zero_()
+            d.run()
+            assert d.op.kernel_tiles == (fm, waves, ksplit)
+            assert np.array_equal(got, d.result())
 
 
 def test_gemm_modes_random_sweep():
-    """Seeded sweep over shapes with the two-tile mode forced on and off and every token tile
-    forced in turn: all against the textbook reference at the fp16 bar."""
+    """Seeded sweep over shapes with every token tile forced in turn, in the waves and K parts of the form or of
+    the plan: all against the textbook reference at the fp16 bar."""
     rng = np.random.default_rng(31)
     for it in range(24):
         bits = int(rng.choice([4, 8]))
@@ -271,42 +313,14 @@ def test_gemm_modes_random_sweep():
         zp = bool(rng.random() < 0.4)
         case = W.make_fc_case(seed=900 + it, m=m, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups,
                               with_bias=bool(it % 2), with_zero_point=zp)
-        with M.tuning(gemm_dual=it % 2, gemm_fm=[1, 2, 4][it % 3]):
+        with M.tuning(gemm_waves=-1 if it % 2 else 1, gemm_fm=[1, 2, 4][it % 3]):
             got = run_w4(case, reference_layout=bool((it // 6) % 2))
         check_fp(got, textbook(case), case, "sweep %d" % it)
 
 
-def test_gemm_two_tiles_fused_launch():
-    """Three matrices in one two-tile launch: pairs of tiles that straddle two matrices (3 + 1 + 2
-    channel tiles) against the single one-tile launches."""
-    import torch
-    m, k = 128, 512
-    cases = [W.make_fc_case(seed=60 + i, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=4, with_bias=True)
-             for i, n in enumerate((384, 100, 256))]
-    for c in cases[1:]:
-        c["act"] = cases[0]["act"]
-    devs = [W.FcDevice(c) for c in cases]
-    for d in devs[1:]:
-        d.op.set_src(0, devs[0].act)
-    single = []
-    with M.tuning(gemm_dual=0):
-        for d in devs:
-            d.run()
-            single.append(d.result())
-            d.out.zero_()
-    with M.tuning(gemm_dual=1):
-        M.fc_launch_fused([d.op for d in devs], torch.cuda.current_stream().cuda_stream)
-    for d, c, ref in zip(devs, cases, single):
-        got = d.result()
-        check_fp(got, textbook(c), c, "two-tile fused")
-        rms = np.sqrt(np.mean(textbook(c) ** 2))
-        assert np.abs(got - ref).max() <= 2e-3 * rms  # another K split among the waves: fp32 summation order
-
-
 def test_fused_prefill_2048_tokens_default_modes():
     """q / k / v of the decoder stack (2048 -> 2048, 256, 256, group 32) at 2048 tokens in one launch with
-    the dispatcher's own choices (128-token tiles, two channel tiles per work-group, pairs that
-    straddle matrices): every output against the textbook reference."""
+    the dispatcher's own choices: every output against the textbook reference."""
     import torch
     m, k = 2048, 2048
     cases = [W.make_fc_case(seed=70 + i, m=m, k=k, n=n, weight_bits=4, tensor_dtype=np.float16, groups=64)
@@ -321,10 +335,16 @@ def test_fused_prefill_2048_tokens_default_modes():
         check_fp(d.result(), textbook(c), c, "fused prefill n=%d" % c["n"])
 
 
-def test_gemm_two_tiles_chosen_for_large_launches():
-    """4096 x 4096 x 4096 (1024 tiles) runs in the two-tile mode by default and meets the bar."""
-    case = W.make_fc_case(seed=5, m=4096, k=4096, n=4096, weight_bits=4, tensor_dtype=np.float16, groups=1)
-    got = run_w4(case)
+# many tiles: one wave each; one tile per CU and fewer: waves share its K; K is cut between work-groups where
+# even those leave CUs idle
+@pytest.mark.parametrize("m,k,n,bits,groups,form", [(4096, 4096, 4096, 4, 1, (128, 1, 1)), (512, 4096, 4096, 4, 128, (64, 4, 1)), (333, 1656, 2900, 8, 1, (64, 4, 1)),
+                                                    (128, 8192, 2048, 8, 1, (64, 4, 8))])
+def test_gemm_forms_chosen(m, k, n, bits, groups, form):
+    case = W.make_fc_case(seed=5, m=m, k=k, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=groups)
+    dev = W.FcDevice(case)
+    dev.run()
+    got = dev.result()
+    assert (dev.op.kernel_variant, dev.op.kernel_tiles) == ("direct", form)
     check_fp(got, textbook(case), case, "textbook")
 
 
