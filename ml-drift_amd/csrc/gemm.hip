@@ -2029,7 +2029,9 @@ DirectPlan PlanDirect(int m, int k, int n, int tiles_n, int groups, int bits, in
       fm_work = (double)DivUp(tiles_m, xm) * DivUp(tiles_n, 8 / xm) / 32.0;  // tiles per CU of the busiest XCD
     }
     const long tiles = (long)tiles_m * tiles_n;
-    if ((fm == 1 && tiles > 2048) || (f.waves < 4 && tiles * f.waves < 96)) continue;  // (never the best there)
+    // (never the best there: 2560 -> 262208 at 48 tokens 152 us, 111 in 64-token tiles.  Up to 32 tokens no other tile is left: 16
+    // tokens of the same layer take 102 us, 154 in a 128-token tile of one wave)
+    if ((fm == 1 && m32 > 32 && tiles > 2048) || (f.waves < 4 && tiles * f.waves < 96)) continue;
     for (int s = 1; s <= max_split; s *= 2) {
       if (s > 1 && (f.waves < 2 || tiles * s > kDirectMaxSplitTiles || steps < 4 * s * f.waves)) break;
       const double work = fm_work * s, whole = std::ceil(work - 1e-9);

@@ -335,6 +335,19 @@ def test_fused_prefill_2048_tokens_default_modes():
         check_fp(d.result(), textbook(c), c, "fused prefill n=%d" % c["n"])
 
 
+# up to 32 tokens over more channels than 2048 tiles of 128 (a vocabulary projection): 32-token tiles as below that line
+@pytest.mark.parametrize("m,bits", [(5, 8), (16, 4), (32, 4), (32, 8)])
+@pytest.mark.parametrize("n", [262144, 262208, 300004])
+def test_gemm_few_tokens_of_many_channels(m, n, bits):
+    case = W.make_fc_case(seed=m, m=m, k=64, n=n, weight_bits=bits, tensor_dtype=np.float16, groups=2, with_bias=True)
+    print("many channels", m, n, bits, flush=True)
+    dev = W.FcDevice(case)
+    dev.run()
+    got = dev.result()
+    assert dev.op.kernel_variant == "direct" and dev.op.kernel_tiles[0] == 32, dev.op.kernel_tiles
+    check_sums(got, case, "textbook")
+
+
 # many tiles: one wave each; one tile per CU and fewer: waves share its K; K is cut between work-groups where
 # even those leave CUs idle
 @pytest.mark.parametrize("m,k,n,bits,groups,form", [(4096, 4096, 4096, 4, 1, (128, 1, 1)), (512, 4096, 4096, 4, 128, (64, 4, 1)), (333, 1656, 2900, 8, 1, (64, 4, 1)),
