@@ -652,7 +652,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   const int xcd = blockIdx.x % 8, local = blockIdx.x / 8;
   const int xm = p.xcd_m;
   const int rect_m = p.geo_rect_m, rect_n = p.geo_rect_n;
-  // local / rect_m by the host's reciprocal (exact: local and rect_m are below 2^16)
+  // local / rect_m by the host's reciprocal (exact for every number that the host launches)
   const int local_n = rect_m == 1 ? local : (int)__umulhi((uint32_t)local, p.geo_rect_m_magic);
   const int local_m = local - local_n * rect_m;
   // (packed groups: neighbouring token tiles go to different XCDs, so that the numbers that turn out to have no
@@ -2014,20 +2014,24 @@ const DirectForm kDirectForms[] = {
     {4, 2, 2, 0.23, 5.2, 0.0811, 2.1, 1.18, 1.06},   {4, 4, 1, 0.15, 4.6, 0.0907, 3.0, 1.20, 1.08}};
 constexpr int kDirectMaxKSplit = 8;
 constexpr long kDirectMaxSplitTiles = 640;  // work-groups up to which K is cut
+constexpr long kDirectMaxRectTiles = 1L << 17;  // tiles of an XCD's rectangle in one launch
 // (depends on m through DivUp(m, 32) only; max_split: parts of K that the workspace holds)
 DirectPlan PlanDirect(int m, int k, int n, int tiles_n, int groups, int bits, int max_split) {
   const int m32 = DivUp(m, 32) * 32, steps = DivUp(k, 16);
   DirectPlan best = {4, 1, 1};
   double best_us = 0.0, fm_work = 0.0;
   int fm = 0, tiles_m = 0;
+  long rect_tiles = 0;
   for (const DirectForm& f : kDirectForms) {
     if (f.fm > 1 && m32 <= 16 * f.fm) continue;  // (a tile half of which would be empty)
     if (f.fm != fm) {
       fm = f.fm;
       tiles_m = DivUp(m, 32 * fm);
       const int xm = W4XcdGrid(tiles_m, tiles_n, 32 * fm, k, groups);
-      fm_work = (double)DivUp(tiles_m, xm) * DivUp(tiles_n, 8 / xm) / 32.0;  // tiles per CU of the busiest XCD
+      rect_tiles = (long)DivUp(tiles_m, xm) * DivUp(tiles_n, 8 / xm);
+      fm_work = rect_tiles / 32.0;  // tiles per CU of the busiest XCD
     }
+    if (rect_tiles >= kDirectMaxRectTiles) continue;  // (larger tiles may fit; none: the launch is refused)
     const long tiles = (long)tiles_m * tiles_n;
     // (never the best there: 2560 -> 262208 at 48 tokens 152 us, 111 in 64-token tiles.  Up to 32 tokens no other tile is left: 16
     // tokens of the same layer take 102 us, 154 in a 128-token tile of one wave)
@@ -2292,10 +2296,13 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   p.xcd_m = W4XcdGrid(tiles_m, tiles_n, fm * 32, a.k, p.groups);
   if (tune.gemm_xcd_m > 0) p.xcd_m = tune.gemm_xcd_m;
   if (p.xcd_m != 1 && p.xcd_m != 2 && p.xcd_m != 4 && p.xcd_m != 8) p.xcd_m = 8;
-  const dim3 grid(8 * DivUp(tiles_m, p.xcd_m) * DivUp(tiles_n, 8 / p.xcd_m), p.ksplit);
-  if (grid.x / 8 >= (1u << 16)) return hipErrorInvalidValue;  // (the reciprocal of rect_m is exact below 2^16)
-  const bool zp = p.seg[0].zp != nullptr;
   set_geometry(tiles_m, tiles_n, waves, gated);
+  // (the reciprocal of rect_m is exact for numbers whose product with its excess is below 2^32: all below 2^16)
+  const long rect_tiles = (long)p.geo_rect_m * p.geo_rect_n;
+  const uint64_t excess = (uint64_t)p.geo_rect_m_magic * p.geo_rect_m & 0xFFFFFFFFu;
+  if (rect_tiles >= kDirectMaxRectTiles || (rect_tiles - 1) * excess >> 32) return hipErrorInvalidValue;
+  const dim3 grid(8 * (unsigned)rect_tiles, p.ksplit);
+  const bool zp = p.seg[0].zp != nullptr;
   if (gated) {
     (fm == 4 ? LaunchGated<4, 4> : fm == 2 ? LaunchGated<2, 8> : LaunchGated<1, 8>)(a.weight_bits, grid, stream, p);
     return hipGetLastError();

@@ -348,6 +348,36 @@ def test_gemm_few_tokens_of_many_channels(m, n, bits):
     check_sums(got, case, "textbook")
 
 
+@pytest.mark.parametrize("m,n,tokens", [(16384, 262144, 64), (8192, 1100000, 128), (8191, 1100000, 128)])
+def test_gemm_more_tiles_than_16_bits(m, n, tokens):
+    """65536 and more tiles per XCD: 64-token tiles as planned, 128-token ones where those are more than 2^17.  Channels at both ends
+    and between against float64, every output written."""
+    import torch
+    k, ks, ns = 32, 8, n // 4
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    desc = M.fc_int4_weights_desc(n, k, reference=True)
+    weights = torch.randint(-2 ** 31, 2 ** 31, (ks * ns * 2,), dtype=torch.int32, device="cuda", generator=gen)
+    act = torch.randn((ks, m, 4), device="cuda", generator=gen).half()
+    scale = (torch.rand((1, ns * 4), device="cuda", generator=gen) * 0.01).half()
+    out = torch.full((ns, m, 4), float("nan"), dtype=torch.float16, device="cuda")
+    op = M.fc_create(M.PRECISION_F32_F16, M.FLOAT16, M.FLOAT16, n, k, desc, scale_shape=(n, 1), max_tokens=m)
+    op.bind([act, weights, scale], [out])
+    op.set_shape(1, 1, m)
+    print("many tiles", m, n, flush=True)
+    op.launch(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert op.kernel_variant == "direct" and op.kernel_tiles[0] == tokens, op.kernel_tiles
+    assert all(bool(torch.isfinite(out[i:i + 4096]).all()) for i in range(0, ns, 4096))
+    words = weights.view(ks, ns, 2)
+    x = act.double().cpu().numpy().transpose(1, 0, 2).reshape(m, k)
+    for s in [0, 1, ns - 1] + [ns // 7 * i + i for i in range(1, 7)]:
+        w = words[:, s].cpu().numpy().view(np.uint32)  # [ks][2]: bits 16 (i % 2) + 4 c of word i / 2
+        u = np.stack([[(w[:, i // 2] >> (16 * (i % 2) + 4 * c)) & 15 for c in range(4)] for i in range(4)])  # [i][c][ks]
+        ref = x @ ((u.transpose(2, 0, 1).reshape(k, 4).astype(np.float64) - 8) * scale[:, 4 * s:4 * s + 4].double().cpu().numpy())
+        err = np.abs(out[s].double().cpu().numpy() - ref)
+        assert np.all(err <= 2.0 ** -10 * np.abs(ref) + 6 * 2.0 ** -10 * np.sqrt(np.mean(ref ** 2))), s
+
+
 # many tiles: one wave each; one tile per CU and fewer: waves share its K; K is cut between work-groups where
 # even those leave CUs idle
 @pytest.mark.parametrize("m,k,n,bits,groups,form", [(4096, 4096, 4096, 4, 1, (128, 1, 1)), (512, 4096, 4096, 4, 128, (64, 4, 1)), (333, 1656, 2900, 8, 1, (64, 4, 1)),
