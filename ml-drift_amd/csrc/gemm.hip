@@ -2283,7 +2283,10 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   if (tune.gemm_ksplit > 0 && !gated) plan.ksplit = tune.gemm_ksplit;
   const int fm = plan.fm;
   // (the forms that are compiled)
-  const int waves = gated ? (fm == 4 ? 4 : 8) : fm == 4 ? std::min(plan.waves, 4) : plan.waves == 1 ? 1 : (fm == 1 && plan.waves > 4 ? 8 : 4);
+  const int waves = gated ? (fm == 4 ? 4 : 8)
+                    : plan.waves == 1 ? 1
+                    : fm == 4         ? (plan.waves < 4 ? 2 : 4)
+                                      : (fm == 1 && plan.waves > 4 ? 8 : 4);
   p.ksplit = plan.ksplit;
   while (p.ksplit > 1 && !fits(p.ksplit)) p.ksplit /= 2;
   for (int i = 0; i < count; ++i)

@@ -269,6 +269,19 @@ def test_gemm_waves_per_tile(fm, waves, bits, zp, m, k, n, groups, ksplit):
     check_sums(got, case, "textbook")
 
 
+@pytest.mark.parametrize("fm,asked,waves", [(32, 2, 4), (32, 3, 4), (32, 5, 8), (32, 100, 8), (64, 2, 4), (64, 8, 4), (128, 3, 2), (128, 8, 4)])
+def test_gemm_waves_without_a_form(fm, asked, waves):
+    """A number of waves that has no form takes the next one that has, with its own geometry: all of K is summed."""
+    case = W.make_fc_case(seed=asked, m=65, k=1056, n=132, weight_bits=4, tensor_dtype=np.float16, groups=33)
+    with M.tuning(gemm_fm=fm // 32, gemm_waves=asked, gemm_ksplit=1):
+        dev = W.FcDevice(case)
+        dev.run()
+        got = dev.result()
+        assert dev.op.kernel_tiles == (fm, waves, 1)
+    assert np.array_equal(got, run_form(case, (fm, waves, 1)))
+    check_sums(got, case, "textbook")
+
+
 @pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False), (8, True)])
 @pytest.mark.parametrize("fm,waves", FORMS)
 @pytest.mark.parametrize("m,ksplit", [(33, 1), (129, 4), (258, 2)])
