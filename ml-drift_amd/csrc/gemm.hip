@@ -2014,6 +2014,10 @@ const DirectForm kDirectForms[] = {
     {4, 2, 2, 0.23, 5.2, 0.0811, 2.1, 1.18, 1.06},   {4, 4, 1, 0.15, 4.6, 0.0907, 3.0, 1.20, 1.08}};
 constexpr int kDirectMaxKSplit = 8;
 constexpr long kDirectMaxSplitTiles = 640;  // work-groups up to which K is cut
+// fp32 partial sums that an op's own workspace has room for (8.4 MB; every op has one, and a model hundreds of ops).  With room for
+// any cut, 14336 -> 4096 would hold 42 MB; by the times below 0.2 % of 129 .. 8192 tokens of up to 16384 x 16384 in the geometric
+// mean, 2 % of those launches 4 .. 20 %.
+constexpr size_t kDirectMaxSplitFloats = (size_t)1 << 21;
 constexpr long kDirectMaxRectTiles = 1L << 17;  // tiles of an XCD's rectangle in one launch
 // (depends on m through DivUp(m, 32) only; max_split: parts of K that the workspace holds)
 DirectPlan PlanDirect(int m, int k, int n, int tiles_n, int groups, int bits, int max_split) {
@@ -2371,8 +2375,11 @@ size_t FcW4MfmaWorkspaceFloats(int max_tokens, int k, int n, int groups, int bit
       const SkinnyPlan skinny = PlanSkinny(t, k, n, CoarseKSplit(t, k, n));
       if (skinny.tile > 0) s = std::max(s, skinny.ksplit); else direct = true;
     }
-    if (direct && mc > kGemvMaxTokens) s = std::max(s, PlanDirect(mc, k, n, tiles_n, groups, bits, kDirectMaxKSplit).ksplit);
-    if (s > 1) need = std::max(need, (size_t)s * DivUp(n, 4) * 4 * mc);
+    const size_t floats = (size_t)DivUp(n, 4) * 4 * mc;  // of one part
+    int max_split = kDirectMaxKSplit;
+    while (max_split > 1 && max_split * floats > kDirectMaxSplitFloats) max_split /= 2;
+    if (direct && mc > kGemvMaxTokens) s = std::max(s, PlanDirect(mc, k, n, tiles_n, groups, bits, max_split).ksplit);
+    if (s > 1) need = std::max(need, s * floats);
   }
   return need;
 }

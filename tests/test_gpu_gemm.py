@@ -282,6 +282,17 @@ def test_gemm_waves_without_a_form(fm, asked, waves):
     check_sums(got, case, "textbook")
 
 
+@pytest.mark.parametrize("bits,k,n,max_tokens", [(4, 14336, 4096, 8192), (4, 16384, 2048, 8192), (8, 14336, 4096, 1280), (4, 16384, 3072, 384)])
+def test_gemm_workspace_of_an_op(bits, k, n, max_tokens):
+    """The partial sums of K parts that an op has room for: at most 2^21 floats (every op of a model holds its own); 2 MiB of
+    granularity per allocation."""
+    import torch
+    desc = M.fc_int8_weights_desc(n, k) if bits == 8 else M.fc_int4_weights_desc(n, k)
+    free = torch.cuda.mem_get_info()[0]
+    ops = [M.fc_create(M.PRECISION_F32_F16, M.FLOAT16, M.FLOAT16, n, k, desc, scale_shape=(n, k // 32), max_tokens=max_tokens) for _ in range(4)]
+    assert free - torch.cuda.mem_get_info()[0] <= len(ops) * (4 * 2 ** 21 + 2 ** 21)
+
+
 @pytest.mark.parametrize("bits,zp", [(4, False), (4, True), (8, False), (8, True)])
 @pytest.mark.parametrize("fm,waves", FORMS)
 @pytest.mark.parametrize("m,ksplit", [(33, 1), (129, 4), (258, 2)])
