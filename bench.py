@@ -52,7 +52,7 @@ def parse():
                         "c5-decode: the weights as mldhip_fc_int4_weights_desc_decode asks for them (the default) or, "
                         "with 'library', in the layout mldhip_fc_int4_weights_desc asks for; c5-prefill with 'decode': "
                         "the prefill step over the decode ops' layout (one copy of the weights for both graphs)")
-    p.add_argument("--tune", default="", help="tuning knobs for the run, e.g. gemv_ksplit=1,gemm_dual=0 (mldhip_set_tuning)")
+    p.add_argument("--tune", default="", help="tuning knobs for the run, e.g. gemv_ksplit=1,gemm_fm=2 (mldhip_set_tuning)")
     p.add_argument("--no-cpu-baseline", action="store_true")
     p.add_argument("--no-graph", action="store_true", help="time an eager launch loop instead of a graph replay")
     p.add_argument("--cpu-seconds", type=float, default=12.0)

@@ -1996,14 +1996,15 @@ struct DirectPlan {
 // SIMDs (latency), `busy` and `busy_around` the same per wave and work-group when a CU is full (issue slots, LDS); for uint8
 // weights the steps take step8 and busy8 times that.
 struct DirectForm {
-  int fm, waves, per_cu;  // per_cu: work-groups that share a CU
+  int fm, waves, per_cu;  // per_cu: work-groups that share a CU (LDS, or registers: one wave on 32 tokens 118 of 128, with uint8 weights
+                          // 130, so 12 of those fit, which step8 and busy8 absorb)
   double step, around, busy, busy_around, step8, busy8;
 };
 // The forms and their times, fitted to 5200 random launches (5 .. 8192 tokens, K 128 .. 16384, 128 .. 32768 channels, uint4
 // and uint8, per-channel scales and groups of 32 .. 128, 20 % with zero points), each in every form, to within 7 .. 11 % in
 // nine of ten.  Many tiles: one wave per tile needs no reduction through LDS and its store overlaps the other tiles of
-// the CU; fewer tiles: more waves share a tile's K.  32-token tiles of 4 waves: four work-groups fit a CU, the best form of short
-// prompts.  Left out since the rest comes within 0.1 % without them: 8 waves on 64 tokens, 2 waves on 32 and 64, and work-groups of
+// the CU; fewer tiles: more waves share a tile's K.  32-token tiles of 4 waves: two work-groups fit a CU (64 KB of LDS each), the best
+// form of short prompts.  Left out since the rest comes within 0.1 % without them: 8 waves on 64 tokens, 2 waves on 32 and 64, and work-groups of
 // two channel tiles.  One rule of rounds of 256 work-groups (8 waves per tile, 4 at 128 tokens) stood here before: over the
 // 3219 launches where every form was timed this one is 1.29 times as fast in the geometric mean (0.9 % behind the best form), 19
 // are slower by more than 4 %.  us, before / now: 8192 x 512 x 14336 210 / 156, 4096 x 1024 x 4096 46.6 / 39, 1000 x 2000 x

@@ -144,10 +144,7 @@ __device__ __forceinline__ float2 WaveStripSum16(const float acc[8]) {
   }
   return make_float2(s2[0], s2[1]);
 }
-// LPR lanes (16 bytes each) cover a row; a wave holds 64 / LPR rows.  Sum over the rows of a wave
-// of the 8 channel sums of every lane; the result of channel (lane % LPR) * 8 + (lane / 8) % 8 is
-// returned in this lane (lanes that differ only in the bits between LPR and 8 hold the same
-// sums).  All 64 lanes must be active.
+
 // v + the value of the lane that differs in one bit of the lane number, as data-parallel moves
 // inside the rows of 16 lanes (no trip through the LDS crossbar): bits 0 and 1 are quad
 // permutations, bit 2 a shift by 4 lanes in either direction, each for the banks it is valid in.
@@ -163,6 +160,10 @@ __device__ __forceinline__ float AddLaneXor4(float v) {
   return v + __uint_as_float(both);
 }
 
+// LPR lanes (16 bytes each) cover a row; a wave holds 64 / LPR rows.  Sum over the rows of a wave
+// of the 8 channel sums of every lane; the result of channel (lane % LPR) * 8 + (lane / 8) % 8 is
+// returned in this lane (lanes that differ only in the bits between LPR and 8 hold the same
+// sums).  All 64 lanes must be active.
 template <int LPR>
 __device__ __forceinline__ float WaveStripSum(const float acc[8], int lane) {
   float s4[4], s2[2];
@@ -310,9 +311,8 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
   const unsigned short out_bias_raw = bias_src[n_out];
   u32x4 w[8];
   u32x2 a[8][M];
-  const bool first = c < c_end;
-  if (first) LoadChunk<M>(p, wcol, rstride, c, w, a, ks_live, act_stride, act_tok0);
-  if (first) {
+  if (c < c_end) {
+    LoadChunk<M>(p, wcol, rstride, c, w, a, ks_live, act_stride, act_tok0);
     while (true) {
       const int cn = c + ROWS;
       const bool more = cn < c_end;
@@ -482,19 +482,6 @@ hipError_t LaunchBatchedM(const StreamParams& p, bool grouped, dim3 grid, hipStr
 }
 
 // ------------------------------------------------------------------------------------------
-// One token over weights packed in output groups of 16 slices (64 channels): the share of a
-// work-group, 64 channels x its range of K, is one contiguous run of 128-byte rows, which HBM
-// delivers at the rate of a plain copy.  Lane = (column of 16 bytes, row): a thread owns 8
-// consecutive K-slices (one 32-channel scale group), its 8 loads are one base address plus
-// immediate offsets, the 8 slices of its activations are 64 contiguous bytes.  Nothing in front of
-// the loads but the address: the kernel's time is the stream's, and every instruction ahead of
-// the first load delays all of it.
-// K reduction: inside a wave by register exchanges that halve the live values per step (the two
-// row halves with v_permlane32_swap, the 16-lane rows with v_permlane16_swap, the 8-lane halves
-// of a row with a DPP rotate), after which lane l holds channel (l % 8) * 8 + l / 8 of the
-// strip; across waves through 4 KB of LDS, fixed order.
-// ------------------------------------------------------------------------------------------
-// ------------------------------------------------------------------------------------------
 // Gated pair: dst = activation(gate(x)) * up(x), the MLP step that follows the gate and up
 // projections in the decoder layers of the LLM sample (samples/llm/gemma3_model_builder.cc:
 // 1054-1090 CreateGeluTanhMulOp, samples/llm/qwen3_model_builder.cc:850-883 CreateSiluMulOp).
@@ -620,6 +607,19 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_gated_stream_kernel(StreamPa
   p.seg[0].dst[((size_t)(n >> 2) * M + m) * 4 + (n & 3)] = __float2half_rn(GatedActivation(activation, gu[0], gu[1]));
 }
 
+// ------------------------------------------------------------------------------------------
+// One token over weights packed in output groups of 16 slices (64 channels): the share of a
+// work-group, 64 channels x its range of K, is one contiguous run of 128-byte rows, which HBM
+// delivers at the rate of a plain copy.  Lane = (column of 16 bytes, row): a thread owns 8
+// consecutive K-slices (one 32-channel scale group), its 8 loads are one base address plus
+// immediate offsets, the 8 slices of its activations are 64 contiguous bytes.  Nothing in front of
+// the loads but the address: the kernel's time is the stream's, and every instruction ahead of
+// the first load delays all of it.
+// K reduction: inside a wave by register exchanges that halve the live values per step (the two
+// row halves with v_permlane32_swap, the 16-lane rows with v_permlane16_swap, the 8-lane halves
+// of a row with a DPP rotate), after which lane l holds channel (l % 8) * 8 + l / 8 of the
+// strip; across waves through 4 KB of LDS, fixed order.
+// ------------------------------------------------------------------------------------------
 // Launch parameters of the strip kernel: what a single-matrix launch reads sits in the first
 // 128 bytes, so that two scalar loads issued at the top of the kernel bring all of it.
 struct StripSegment {
@@ -1680,10 +1680,10 @@ hipError_t LaunchFcW4StreamFused(const FcArgs* args, int count, hipStream_t stre
     p.ksplit = 1;
     const bool wide = (long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 192;
     // One token per row over output groups of 16 slices: the contiguous-strip kernel, from one 64-channel strip for every
-    // second CU on: a strip's K lies in one piece, which counts for more than the idle CUs.  (2 of 8 matrices, 2048 x 4096,
-    // 128 strips: 24.1 -> 17.1 us for the three projections of a layer; of 2041 random launches of 96 .. 260 strips, K 256 ..
-    // 8192, one got 5 % slower by the line's move from 192 to 128.  Below 128 two shapes were timed, 96 strips of 2048 x 768 among
-    // them: 16.0 against 14.3 us, the strip kernel ahead there too; that is no line, and those launches stay on the streaming kernel.)
+    // second CU on: a strip's K lies in one piece, which counts for more than the idle CUs.  (us, strip kernel / half strips of the
+    // streaming kernel in pairs: 2 of 8 matrices 2048 x 4096, 128 strips, 4.9 / 5.1.  104 random launches of 128 .. 300 strips, K
+    // 256 .. 8192: the strip kernel is ahead in each, 0.76 times the time.  229 of 24 .. 127 strips: 0.83 in the geometric mean, but
+    // up to 17 % behind at K of 1088 .. 2048, 96 strips of 2048 x 768 4.6 / 4.5 among them; those stay on the streaming kernel.)
     if ((long)DivUp(p.seg[0].row_u4, 8) * a.rows >= 128 && StripKernelServes(args, count)) {
       if (kernel_name) *kernel_name = "fc_w4_strip_kernel";
       return LaunchStrip(p, args, count, grouped, stream);
