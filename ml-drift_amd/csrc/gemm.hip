@@ -2165,8 +2165,10 @@ hipError_t LaunchDirectGemm(const FcArgs* args, int count, int gate_activation, 
   // Many tokens over one uint4 matrix: both operands shared through LDS, 256 x 256 tiles.  Both
   // kernels run into the same limit on large launches (the chip lowers its clock under dense MFMA
   // work on random data) and finish within a few percent of each other, so the tile counts decide:
-  // the large tiles are taken where they fill one round of the 256 CUs and the 128 x 128 tiles of
-  // the direct kernel would leave its last round half empty (1024 x 4096 x 14336: 131 against 155 us).
+  // the large tiles are taken where they fill one round of the 256 CUs and 128 x 128 tiles would leave a last round half empty.
+  // The line was drawn against work-groups of 4 waves on those (1024 x 4096 x 14336: 131 against 155 us).  Against one wave per
+  // tile, what PlanDirect takes there now, it has no gain left: 72 random launches inside it are 1.07 times the direct
+  // kernel's time in the geometric mean, 0.93 .. 1.17 (1024 x 4096 x 14336 126.9 / 111.0 us).
   {
     const bool tiled_ok = !gated && !packed && count == 1 && a.weight_bits == 4 && a.m % 2 == 0 && p.group_size % 32 == 0;
     const long tiles = (long)DivUp(a.n, 256) * DivUp(a.m, 256);
