@@ -779,35 +779,40 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   wblk_t rw[U][2];
   u32x2 rsc[U], rzp[U], rx[U][NX][2];
   u32x4 rxp[U][NX][2];  // PAIR: {token 2j: 4 halfs, token 2j+1: 4 halfs} per K-slice row
-  auto load_step = [&](int t, bool with_scale, wblk_t (&w)[2], u32x2& sc, u32x2& zpv, u32x2 (&x)[NX][2],
-                       u32x4 (&xp)[NX][2]) {
-    // The scales (and zero points) of a pair of steps (t - 1, t), t odd, which share a group
-    // because a group holds an even number of steps.  They travel with the odd step: by then
-    // both users of the previous pair are done with the registers.  First in the stage, so
-    // that waiting for them holds back as few younger loads as possible.
-    if (with_scale) {
-      sc = __builtin_amdgcn_raw_buffer_load_b64(rsrc_s, vs + (uint32_t)(t >> p.group_shift) * group_bytes, 0, 0);
-      if (ZP) zpv = __builtin_amdgcn_raw_buffer_load_b64(rsrc_z, vs + (uint32_t)(t >> p.group_shift) * group_bytes, 0, 0);
-    }
+  // The scales (and zero points) of a pair of steps (t - 1, t), t odd, which share a group because a group
+  // holds an even number of steps.  They travel with the odd step: by then both users of the previous
+  // pair are done with the registers.
+  auto load_scales = [&](int t, u32x2& sc, u32x2& zpv) {
+    sc = __builtin_amdgcn_raw_buffer_load_b64(rsrc_s, vs + (uint32_t)(t >> p.group_shift) * group_bytes, 0, 0);
+    if (ZP) zpv = __builtin_amdgcn_raw_buffer_load_b64(rsrc_z, vs + (uint32_t)(t >> p.group_shift) * group_bytes, 0, 0);
+  };
+  auto load_weights = [&](int u) {
     if constexpr (WB == 8) {
-      w[0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, vw0, 0, 0);
-      w[1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w1, vw0, 0, 0);
+      rw[u][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, vw0, 0, 0);
+      rw[u][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_w1, vw0, 0, 0);
     } else {
-      w[0] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_w, vw0, 0, 0);
-      w[1] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_w1, vw0, 0, 0);
+      rw[u][0] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_w, vw0, 0, 0);
+      rw[u][1] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_w1, vw0, 0, 0);
     }
     vw0 += step_w;
+  };
+  auto load_act = [&](int u) {
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       if (PAIR) {
-        xp[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, vx[i], 0, 0);
-        xp[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x1, vx[i], 0, 0);
+        rxp[u][i][0] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, vx[i], 0, 0);
+        rxp[u][i][1] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x1, vx[i], 0, 0);
       } else {
-        x[i][0] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_x, vx[i], 0, 0);
-        x[i][1] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_x1, vx[i], 0, 0);
+        rx[u][i][0] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_x, vx[i], 0, 0);
+        rx[u][i][1] = __builtin_amdgcn_raw_buffer_load_b64(rsrc_x1, vx[i], 0, 0);
       }
       vx[i] += step_x;
     }
+  };
+  auto load_step = [&](int t, bool with_scale, int u) {
+    if (with_scale) load_scales(t, rsc[u & ~1], rzp[u & ~1]);
+    load_weights(u);
+    load_act(u);
   };
 
   float16_t acc[4][FM];
@@ -831,7 +836,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    load_step(t_begin + u, u % 2 == 1, rw[u], rsc[u & ~1], rzp[u & ~1], rx[u], rxp[u]);
+    load_step(t_begin + u, u % 2 == 1, u);
     __builtin_amdgcn_sched_barrier(0);
   }
   if constexpr (FM == 1) {
@@ -903,17 +908,22 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
         // refill stage u with step t + U; the fences keep the loads of a stage together and in
         // program order, so that waiting for one stage leaves the younger ones in flight
         __builtin_amdgcn_sched_barrier(0);
-        load_step(t + U, u % 2 == 1, rw[u], rsc[u & ~1], rzp[u & ~1], rx[u], rxp[u]);
+        load_step(t + U, u % 2 == 1, u);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
   } else {
-    // The loop is software-pipelined by one weight operand: while the FM MFMAs of output-channel phase
-    // t4 run, the vector ALU dequantizes the operand of phase t4 + 1 (at t4 = 3: phase 0 of the next
-    // stage), 4 / FM words behind every MFMA.  A wave issues in order, and an MFMA that waits for the
-    // matrix pipe holds back whatever follows it, so a run of MFMAs followed by a run of vector
-    // instructions serialises the two; placed between the MFMAs, the vector instructions issue in the
-    // 32 cycles each MFMA occupies the pipe.  The scheduling groups at the end of a step ask for that order.
+    // The loop is software-pipelined by one weight operand: while the FM MFMAs of output-channel phase t4 run, the vector ALU
+    // dequantizes the operand of phase t4 + 1 (at t4 = 3: phase 0 of the next stage).  What issues behind which MFMA is written
+    // out slot by slot between fences, by what this card does: a wave's MFMA of 32 cycles leaves room for four other instructions,
+    // every further one adds 4 cycles (with two waves on the SIMD: five), and a vector instruction that reads the one before
+    // it takes 8 cycles (12 dequantization instructions per MFMA as chains of three: 94 cycles, four chains side by side
+    // 70).  So the operand's four words go through each step of their dequantization together, and loads, register swaps and
+    // address additions have slots of their own instead of standing behind the last MFMA of a step.  In the order that the
+    // compiler found under a pipeline of scheduling groups (one MFMA, 4 or 8 vector instructions) a step of 128 tokens took about 55
+    // cycles per MFMA, now 39, of 64 tokens 50: 333 x 1656 x 2900 with uint8 weights and zero points 12.04 -> 11.19 us,
+    // 512 x 4096 x 4096 20.0 -> 19.6, 8192 x 4096 x 14336 765 -> 744.  (The two last gain less than the cycles say: under dense MFMA work
+    // on random data the clock gives way, 1.4 GHz in the loop of 128-token tiles and 2.4 around it.)
     struct Stage {
       u32x4 blk, blk8;   // WB == 4: the stage's 32 weights, and the same shifted by 8 bits
       wblk_t w0, w1;     // WB == 8: the two blocks
@@ -926,7 +936,6 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
       st.blk = st.blk8 = u32x4{0u, 0u, 0u, 0u};
       if constexpr (WB == 4) {
         st.blk = u32x4{rw[u][0][0], rw[u][0][1], rw[u][1][0], rw[u][1][1]};
-        st.blk8 = u32x4{st.blk[0] >> 8, st.blk[1] >> 8, st.blk[2] >> 8, st.blk[3] >> 8};
       }
       const u32x2 scr = rsc[u & ~1];
       st.sc01 = AsHalf2(scr[0]);
@@ -938,58 +947,63 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
       }
       return st;
     };
-    // word wd (input channels 2 wd, 2 wd + 1 of the step's 8) of the operand of phase t4
-    auto dequant_word = [&](const Stage& st, int t4, int wd) -> uint32_t {
+    constexpr int kOps = WB == 8 ? 4 : 3;      // vector instructions per word of an operand
+    constexpr int kPerSlot = FM >= 4 ? 4 : 8;  // dequantization instructions behind one MFMA
+    // The operand of one phase on its way: word wd holds input channels 2 wd, 2 wd + 1 of the step's 8.
+    struct Operand {
+      uint32_t part[4];
+      half2_t mzs;
+      u32x4 done;
+    };
+    // Instruction `kind` of word wd of the operand of phase t4: unpack (uint8: two instructions), centre, scale.
+    auto dequant_op = [&](const Stage& st, int t4, int kind, int wd, Operand& o) {
       const half2_t sp = (t4 & 2) ? st.sc23 : st.sc01;
       const half2_t s2 = (t4 & 1) ? __builtin_shufflevector(sp, sp, 1, 1) : __builtin_shufflevector(sp, sp, 0, 0);
-      const half2_t off = WB == 8 ? off_w8 : ((t4 & 1) ? off_hi : off_lo);
-      // zero point: (u - shift) * s - zp * s in one fused step, so that a fractional zero point
-      // costs one extra rounding of zp * s and not a rounding of shift + zp to an integer
-      half2_t mzs = {(_Float16)0.0f, (_Float16)0.0f};
-      if (ZP) {
-        const half2_t zq = (t4 & 2) ? st.zp23 : st.zp01;
-        mzs = -(((t4 & 1) ? __builtin_shufflevector(zq, zq, 1, 1) : __builtin_shufflevector(zq, zq, 0, 0)) * s2);
-      }
-      uint32_t bits;
-      if constexpr (WB == 8) {
-        // bytes t4 of the words of input channels 2*wd, 2*wd + 1 -> the low bytes of two halfs
-        const uint32_t sel = 0x0c000c00u | (uint32_t)t4 | ((uint32_t)(4 + t4) << 16);
-        const wblk_t& wr = (wd >> 1) ? st.w1 : st.w0;
-        bits = __builtin_amdgcn_perm(wr[2 * (wd & 1) + 1], wr[2 * (wd & 1)], sel) | magic_lo;
+      if (kind == 0) {
+        if constexpr (WB == 8) {
+          // bytes t4 of the words of input channels 2*wd, 2*wd + 1 -> the low bytes of two halfs
+          const uint32_t sel = 0x0c000c00u | (uint32_t)t4 | ((uint32_t)(4 + t4) << 16);
+          const wblk_t& wr = (wd >> 1) ? st.w1 : st.w0;
+          o.part[wd] = __builtin_amdgcn_perm(wr[2 * (wd & 1) + 1], wr[2 * (wd & 1)], sel);
+        } else {
+          const uint32_t x = (t4 & 2) ? st.blk8[wd] : st.blk[wd];
+          o.part[wd] = (t4 & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo);
+        }
+      } else if (kind == kOps - 2) {
+        const half2_t off = WB == 8 ? off_w8 : ((t4 & 1) ? off_hi : off_lo);
+        o.part[wd] = AsU32(AsHalf2(o.part[wd]) + off);  // exact: u - shift
+        // zero point: (u - shift) * s - zp * s in one fused step, so that a fractional zero point
+        // costs one extra rounding of zp * s and not a rounding of shift + zp to an integer
+        if (ZP && wd == 0) {
+          const half2_t zq = (t4 & 2) ? st.zp23 : st.zp01;
+          o.mzs = -(((t4 & 1) ? __builtin_shufflevector(zq, zq, 1, 1) : __builtin_shufflevector(zq, zq, 0, 0)) * s2);
+        }
+      } else if (kind == kOps - 1) {
+        o.done[wd] = AsU32(ZP ? __builtin_elementwise_fma(AsHalf2(o.part[wd]), s2, o.mzs) : AsHalf2(o.part[wd]) * s2);
       } else {
-        const uint32_t x = (t4 & 2) ? st.blk8[wd] : st.blk[wd];
-        bits = (t4 & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo);
+        o.part[wd] |= magic_lo;
       }
-      const half2_t centred = AsHalf2(bits) + off;  // exact: u - shift
-      return AsU32(ZP ? __builtin_elementwise_fma(centred, s2, mzs) : centred * s2);
     };
-    // vector instructions per MFMA of a step: 13-14 per phase (3 per word, the scale broadcast, the shifts of a new stage)
-    constexpr int kValuPerMfma = FM >= 4 ? 4 : (FM == 2 ? 8 : 16);
     Stage cur = open_stage(0);
-    u32x4 aop;
+    Operand op = {};
   #pragma unroll
-    for (int wd = 0; wd < 4; ++wd) aop[wd] = dequant_word(cur, 0, wd);
+    for (int i = 0; i < 4 * kOps; ++i) dequant_op(cur, 0, i / 4, i % 4, op);
+    u32x4 aop = op.done;
+    if (PAIR) {
+  #pragma unroll
+      for (int i = 0; i < NX; ++i) SwapRegisters(rxp[0][i][0], rxp[0][i][1]);
+    }
     __builtin_amdgcn_sched_barrier(0);
     for (int tt = 0; tt < per_wave; tt += U) {
   #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int t = t_begin + tt + u;
-        if (PAIR) {
-          // The two 16-byte loads of a token pair hold {token 2j, token 2j+1} of K-slice rows 2q
-          // and 2q+1; exchanging the inner halves makes each of them one token's operand.
-  #pragma unroll
-          for (int i = 0; i < NX; ++i) {
-            SwapRegisters(rxp[u][i][0], rxp[u][i][1]);
-          }
-        }
         Stage nxt = cur;
   #pragma unroll
         for (int t4 = 0; t4 < 4; ++t4) {
           // the operand that follows this one: the next phase of this stage, or phase 0 of the next
           // stage (after the last step: of a stage that was fetched beyond the range and holds zeros)
           if (t4 == 3) nxt = open_stage((u + 1) % U);
-          const int t4n = (t4 + 1) & 3;
-          u32x4 anext;
   #pragma unroll
           for (int fm = 0; fm < FM; ++fm) {
             const u32x4 bop = PAIR ? rxp[u][fm / 2][fm & 1]
@@ -997,23 +1011,33 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
                                            rx[u][PAIR ? 0 : fm][1][1]};
             acc[t4][fm] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, aop),
                                                                  __builtin_bit_cast(half8_t, bop), acc[t4][fm], 0, 0, 0);
-          }
+            __builtin_amdgcn_sched_barrier(0);
   #pragma unroll
-          for (int wd = 0; wd < 4; ++wd) anext[wd] = dequant_word(nxt, t4n, wd);
-          aop = anext;
+            for (int i = fm * kPerSlot; i < (fm + 1) * kPerSlot && i < 4 * kOps; ++i) {
+              dequant_op(nxt, (t4 + 1) & 3, i / 4, i % 4, op);
+              if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            // what else a step has to do, each when its registers are free: behind the last MFMA of a phase
+            if (fm == FM - 1) {
+              if (t4 == 0 && WB == 4) cur.blk8 = u32x4{cur.blk[0] >> 8, cur.blk[1] >> 8, cur.blk[2] >> 8, cur.blk[3] >> 8};
+              if (t4 == (WB == 8 ? 3 : 1)) load_weights(u);
+              if (t4 == 2 && PAIR) {
+                // The two 16-byte loads of a token pair hold {token 2j, token 2j+1} of K-slice rows 2q
+                // and 2q+1; exchanging the inner halves makes each of them one token's operand.
+  #pragma unroll
+                for (int i = 0; i < NX; ++i) SwapRegisters(rxp[(u + 1) % U][i][0], rxp[(u + 1) % U][i][1]);
+              }
+              if (t4 == 3) {
+                if (u % 2 == 1) load_scales(t + U, rsc[u & ~1], rzp[u & ~1]);
+                load_act(u);
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (t4 < 2) nxt = cur;
+          aop = op.done;
         }
         cur = nxt;
-        // the order of the step's instructions: one MFMA, then its share of the vector instructions
-  #pragma unroll
-        for (int i = 0; i < 4 * FM; ++i) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, kValuPerMfma, 0);
-        }
-        // refill stage u with step t + U; the fences keep the loads of a stage together and in
-        // program order, so that waiting for one stage leaves the younger ones in flight
-        __builtin_amdgcn_sched_barrier(0);
-        load_step(t + U, u % 2 == 1, rw[u], rsc[u & ~1], rzp[u & ~1], rx[u], rxp[u]);
-        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
