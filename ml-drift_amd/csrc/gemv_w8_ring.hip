@@ -502,6 +502,172 @@ __global__ __launch_bounds__(THREADS) void fc_w8_ring_i_column_kernel(RingParams
   RingWrite<T, false>(p, wb, ds * 4 + c, ((size_t)ds * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as, row, tok0 + t);
 }
 
+// The same where the window is the whole ring and no runtime bound cuts it.  Then which rows are read does not depend on
+// where the ring starts, only which source slices meet them: row r holds source channels 4 w - sh .. 4 w - sh + 3 with w = r - row0
+// around the ring, whose first part is the slice of row r - 1, around the ring too.  So a thread walks the rows as they lie and
+// requests its weights before the start of the ring is known; the activations follow, and while they and the weights
+// are on their way, scale and bias.  Each of the four shifts has its multiply without selects, and without a zero point the sum
+// of the activations is not needed.  8 tokens x 8192 positions x 256 channels 6.6 -> 6.0 us (profiler figures).  (All activations through LDS,
+// so that nothing but the reads from there waits for the start: 7.2.)
+template <int SH>
+__device__ __forceinline__ void MultiplyShifted(const float (&u)[4][4], const uint32_t* lo, const uint32_t* hi, bool zp, float (&acc)[4],
+                                                float& asum) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = __uint_as_float(i < SH ? lo[4 - SH + i] : hi[i - SH]);
+    if (zp) asum += a;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] = fmaf(a, u[i][c], acc[c]);
+  }
+}
+template <int SH>
+__device__ __forceinline__ void MultiplyShifted(const half2_t (&u)[2][4], const uint32_t* lo, const uint32_t* hi, bool zp, float (&acc)[4],
+                                                float& asum) {
+  uint32_t a01, a23;
+  if (SH == 0) {
+    a01 = hi[0], a23 = hi[1];
+  } else if (SH == 1) {
+    a01 = __builtin_amdgcn_alignbit(hi[0], lo[1], 16), a23 = __builtin_amdgcn_alignbit(hi[1], hi[0], 16);
+  } else if (SH == 2) {
+    a01 = lo[1], a23 = hi[0];
+  } else {
+    a01 = __builtin_amdgcn_alignbit(lo[1], lo[0], 16), a23 = __builtin_amdgcn_alignbit(hi[0], lo[1], 16);
+  }
+  const half2_t one = {(_Float16)1.0f, (_Float16)1.0f};
+  if (zp) asum = __builtin_amdgcn_fdot2(AsHalf2(a23), one, __builtin_amdgcn_fdot2(AsHalf2(a01), one, asum, false), false);
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    acc[c] = __builtin_amdgcn_fdot2(AsHalf2(a23), u[1][c], __builtin_amdgcn_fdot2(AsHalf2(a01), u[0][c], acc[c], false), false);
+}
+// scale, zero point and bias of one output channel, requested ahead of their use
+template <typename T>
+struct RingChannel {
+  float s, z;
+  T bias;
+};
+template <typename T>
+__device__ __forceinline__ RingChannel<T> LoadRingChannel(const RingParams& p, int wb, int n) {
+  RingChannel<T> c = {p.scalar_scale, p.has_zero_point ? p.scalar_zero_point : 0.0f, T()};
+  if (p.scale_kind == kScaleLinear) {
+    c.s = LoadF(static_cast<const T*>(p.scale), (size_t)wb * p.ns * 4 + n);
+    if (p.zero_point) c.z = LoadF(static_cast<const T*>(p.zero_point), (size_t)wb * p.ns * 4 + n);
+  }
+  if (p.bias) c.bias = static_cast<const T*>(p.bias)[n];
+  return c;
+}
+template <typename T>
+__device__ __forceinline__ void RingStoreChannel(const RingParams& p, const RingChannel<T>& c, size_t o, float r) {
+  T* dst = static_cast<T*>(p.dst);
+  if constexpr (std::is_same<T, float>::value) {
+    dst[o] = p.bias ? r + c.bias : r;
+  } else {
+    __half h = __float2half_rn(r);
+    if (p.bias) h = __hadd(h, c.bias);
+    dst[o] = h;
+  }
+}
+
+// (MT as in the column kernel; work-groups are dealt to the XCDs as there)
+template <typename T, int MT, int THREADS, bool ZP>
+__global__ __launch_bounds__(THREADS) void fc_w8_ring_i_turn_kernel(RingParams p) {
+  constexpr int U = 2, WAVES = THREADS / 64, NW = kWordsPerToken<T>;
+  __shared__ float red[WAVES][MT][5];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int kSpreadShift = THREADS == 1024 ? 3 : 5;
+  const int plane = blockIdx.z * ((p.m + MT - 1) / MT) + blockIdx.y;
+  const int j = blockIdx.x >> 3, run = (blockIdx.x - ((plane >> kSpreadShift) & p.xcd_mask) * p.xcd_runs) & 7;
+  const int ds = (j >> 3) * 64 + run * 8 + (j & 7);
+  if (ds >= p.ns) return;  // (the whole work-group)
+  const int row = blockIdx.z, tok_first = blockIdx.y * MT, tok0 = min(tok_first, p.m - MT);
+  int wb = p.batch_ids ? p.batch_ids[row] : 0;
+  wb = min(max(wb, 0), p.weights_batch - 1);
+  const int rows = p.ring_rows;
+  const u32x4* wcol = p.weights + (size_t)wb * rows * p.ns + ds;
+  const size_t act_stride = (size_t)p.src_rows * p.m * 4;
+  const T* act = static_cast<const T*>(p.act) + ((size_t)min(row, p.src_rows - 1) * p.m + tok0) * 4;
+  u32x4 blk[U];
+  auto load_row = [&](int first_row) { return wcol[(size_t)min(first_row + lane, rows - 1) * p.ns]; };
+#pragma unroll
+  for (int u = 0; u < U; ++u) blk[u] = load_row(wave * 64 + u * THREADS);
+  __builtin_amdgcn_sched_barrier(0);
+  const int off = ((p.params[p.ring_index] % p.ring_size) + p.ring_size) % p.ring_size;
+  const int sh = off & 3, row0 = off >> 2;
+  RingChannel<T> channel;
+  if (tid < MT * 4) channel = LoadRingChannel<T>(p, wb, ds * 4 + (tid & 3));
+
+  float acc[MT][4], asum[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    asum[t] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[t][c] = 0.0f;
+  }
+  for (int base = wave * 64; base < rows; base += THREADS * U) {  // (the same for the whole wave: lanes exchange below)
+    uint32_t first[U][MT * NW], hi[U][MT * NW];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int r0 = min(base + u * THREADS, rows - 1);  // (the wave's first row)
+      const int below = r0 - row0 + (r0 > row0 ? -1 : rows - 1);
+      int w = min(r0 + lane, rows - 1) - row0;
+      w = w < 0 ? w + rows : w;
+      LoadTokens<T, MT>(act, (size_t)w * act_stride, hi[u]);
+      LoadTokens<T, MT>(act, (size_t)below * act_stride, first[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (base + u * THREADS + 64 > rows) {  // rows past the ring's last one
+        const bool live = base + u * THREADS + lane < rows;
+#pragma unroll
+        for (int i = 0; i < MT * NW; ++i) hi[u][i] = live ? hi[u][i] : 0u;
+      }
+      typename RingTypes<T>::centred cu;
+      Centre(blk[u], cu);
+      if (base + THREADS * U < rows) blk[u] = load_row(base + THREADS * U + u * THREADS);
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        uint32_t lo[NW];
+        const uint32_t* ht = hi[u] + t * NW;
+        if (sh == 0) {
+          MultiplyShifted<0>(cu, lo, ht, ZP, acc[t], asum[t]);
+        } else {
+          const bool live = base + u * THREADS + lane < rows;
+#pragma unroll
+          for (int i = 0; i < NW; ++i) {
+            lo[i] = __builtin_amdgcn_update_dpp(first[u][t * NW + i], ht[i], 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+            lo[i] = live ? lo[i] : 0u;
+          }
+          if (sh == 1) MultiplyShifted<1>(cu, lo, ht, ZP, acc[t], asum[t]);
+          else if (sh == 2) MultiplyShifted<2>(cu, lo, ht, ZP, acc[t], asum[t]);
+          else MultiplyShifted<3>(cu, lo, ht, ZP, acc[t], asum[t]);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const float v = AddRow16(SwapAdd16(SwapAdd32(acc[t][0], acc[t][2]), SwapAdd32(acc[t][1], acc[t][3])));
+    if ((lane & 15) == 0) red[wave][t][2 * (lane >> 5) + ((lane >> 4) & 1)] = v;
+    if (ZP) {
+      const float s32 = SwapAdd32(asum[t], asum[t]);
+      const float a = AddRow16(SwapAdd16(s32, s32));
+      if (lane == 0) red[wave][t][4] = a;
+    }
+  }
+  __syncthreads();
+  if (tid >= MT * 4) return;
+  const int t = tid >> 2, c = tid & 3, n = ds * 4 + c;
+  if (tok0 + t < tok_first) return;
+  float sum = 0.0f, as = 0.0f;
+#pragma unroll
+  for (int q = 0; q < WAVES; ++q) {
+    sum += red[q][t][c];
+    if (ZP) as += red[q][t][4];
+  }
+  const size_t o = ((size_t)ds * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c;
+  RingStoreChannel<T>(p, channel, o, channel.s * (ZP ? fmaf(-channel.z, as, sum) : sum));
+  if (ZP && RingSumInfinite(as)) RingStore<T>(p, n, o, channel.s * RingSumByProducts<T, false>(row, tok0 + t, n, channel.z));
+}
+
 // ------------------------------------------------------------------------------------------
 // Ring over the output channels of a kOSpatialIOGroupO4I4 buffer (GetRingedOAddresses,
 // fully_connected.cc:411-422, 680-697): query x key cache.  Word (ks, o) of the buffer holds input
@@ -618,31 +784,134 @@ __global__ __launch_bounds__(256) void fc_w8_ring_o_kernel(RingParams p) {
   RingWrite<T, true>(p, wb, slice * 4 + c, ((size_t)slice * p.rows * p.m + (size_t)row * p.m + tok0 + t) * 4 + c, sum, as, row, tok0 + t);
 }
 
-template <typename T, int MT>
-hipError_t LaunchColumnT(const RingParams& p, bool small, hipStream_t stream) {
-  const dim3 grid(DivUp(p.ns, 64) * 64, DivUp(p.m, MT), p.rows);
-  if (small)
-    hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, 256>), grid, dim3(256), 0, stream, p);
+// The same where every channel of the ring is a dst channel: a work-group takes 64 channels as they lie in the ring, so no
+// address of the weights or activations depends on where the ring starts, only the dst channels that the sums are for.
+// 8 tokens x 8192 positions x 256 channels 4.4 -> 4.0 us (profiler figures; a step of 18 layers, keys and values, 198 -> 179 us.  All kernel
+// arguments in one batch of scalar loads at the top, in both kernels: 190).
+template <typename T, int MT, bool ZP>
+__global__ __launch_bounds__(256) void fc_w8_ring_o_turn_kernel(RingParams p) {
+  constexpr int KL = 16, U = 4, NW = kWordsPerToken<T>, CHUNK = 256;
+  __shared__ uint32_t acts[CHUNK][MT * NW];
+  __shared__ float red[4][MT][64], reda[4][MT];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, sl = tid & 15, kl = tid >> 4;
+  const int row = blockIdx.z, tok_first = blockIdx.y * MT, tok0 = min(tok_first, p.m - MT);
+  const size_t act_stride = (size_t)p.src_rows * p.m;
+  const T* act = static_cast<const T*>(p.act) + ((size_t)min(row, p.src_rows - 1) * p.m + tok0) * 4;
+  const int ks_end = RingSrcEndSlices(p);
+  int wb = p.batch_ids ? p.batch_ids[row] : 0;
+  wb = min(max(wb, 0), p.weights_batch - 1);
+  const uint32_t* w32 = reinterpret_cast<const uint32_t*>(p.weights) + (size_t)wb * p.ks * p.ring_size + min((int)blockIdx.x * 16 + sl, p.ns - 1) * 4;
+  float acc[MT][4], asum[MT];
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    asum[t] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[t][c] = 0.0f;
+  }
+  // the sum that this thread finishes: channel c of slice s of the ring for token t
+  const int c = tid & 3, t_out = (tid >> 2) % MT, s = (tid >> 2) / MT;
+  int n = 0;
+  RingChannel<T> channel;
+  for (int chunk = 0; chunk < ks_end || chunk == 0; chunk += CHUNK) {
+    const int count = min(ks_end - chunk, CHUNK);
+    if (chunk > 0) __syncthreads();  // (everybody is done with the chunk before)
+    u32x4 w[U];
+    auto load_weights = [&](int k0) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        w[u] = *reinterpret_cast<const u32x4_word*>(w32 + (size_t)max(chunk + min(k0 + u * KL, count - 1), 0) * p.ring_size);
+    };
+    load_weights(kl);
+    for (int i = tid; i < count; i += 256) {
+      uint32_t v[MT * NW];
+      LoadTokens<T, MT>(act, (size_t)(chunk + i) * act_stride * 4, v);
+#pragma unroll
+      for (int q = 0; q < MT * NW; ++q) acts[i][q] = v[q];
+    }
+    if (chunk == 0) {
+      const int off = ((p.params[p.ring_index] % p.ring_size) + p.ring_size) % p.ring_size;
+      n = (blockIdx.x * 16 + s) * 4 + c - off;
+      n = n < 0 ? n + p.ring_size : n;
+      if (tid < MT * 64 && (int)blockIdx.x * 16 + s < p.ns) channel = LoadRingChannel<T>(p, wb, n);
+    }
+    __syncthreads();
+    for (int k0 = kl; k0 < count; k0 += KL * U) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u * KL;
+        if (k < count) {
+          typename RingTypes<T>::centred cu;
+          CentreO(w[u], cu);
+          uint32_t v[MT * NW];
+#pragma unroll
+          for (int q = 0; q < MT * NW; ++q) v[q] = acts[k][q];
+#pragma unroll
+          for (int t = 0; t < MT; ++t) MultiplyShifted<0>(cu, v + t * NW, v + t * NW, ZP, acc[t], asum[t]);
+        }
+      }
+      if (k0 + KL * U < count) load_weights(k0 + KL * U);
+    }
+  }
+  // lane = slice + 16 x K lane of the wave; two exchanges leave it with channel 2 * (lane / 32) + (lane / 16) % 2
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    red[wave][t][lane] = SwapAdd16(SwapAdd32(acc[t][0], acc[t][2]), SwapAdd32(acc[t][1], acc[t][3]));
+    if (ZP) {
+      const float s32 = SwapAdd32(asum[t], asum[t]);
+      const float a = SwapAdd16(s32, s32);
+      if (lane == 0) reda[wave][t] = a;
+    }
+  }
+  __syncthreads();
+  if (tid >= MT * 64 || (int)blockIdx.x * 16 + s >= p.ns || tok0 + t_out < tok_first) return;
+  float sum = 0.0f, as = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    sum += red[q][t_out][c * 16 + s];
+    if (ZP) as += reda[q][t_out];
+  }
+  const size_t o = ((size_t)(n >> 2) * p.rows * p.m + (size_t)row * p.m + tok0 + t_out) * 4 + (n & 3);
+  RingStoreChannel<T>(p, channel, o, channel.s * (ZP ? fmaf(-channel.z, as, sum) : sum));
+  if (ZP && RingSumInfinite(as)) RingStore<T>(p, n, o, channel.s * RingSumByProducts<T, true>(row, tok0 + t_out, n, channel.z));
+}
+
+// A window that is the whole ring and that no runtime bound cuts.
+bool WholeTurn(const RingParams& p) { return p.src_end_ch_index < 0 && p.k_channels == p.ring_size; }
+
+template <typename T, int MT, int THREADS>
+hipError_t LaunchColumnT(const RingParams& p, hipStream_t stream) {
+  const dim3 grid(DivUp(p.ns, 64) * 64, DivUp(p.m, MT), p.rows), block(THREADS);
+  // (the turn kernel knows no bound of the dst channels)
+  if (WholeTurn(p) && p.dst_end_ch_index < 0 && p.has_zero_point)
+    hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, true>), grid, block, 0, stream, p);
+  else if (WholeTurn(p) && p.dst_end_ch_index < 0)
+    hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, false>), grid, block, 0, stream, p);
   else
-    hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, 1024>), grid, dim3(1024), 0, stream, p);
+    hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, THREADS>), grid, block, 0, stream, p);
   return hipGetLastError();
 }
 template <typename T>
 hipError_t LaunchColumn(const RingParams& p, int slots, bool small, hipStream_t stream) {
-  if (slots == 4) return LaunchColumnT<T, 4>(p, small, stream);
-  if (slots == 2) return LaunchColumnT<T, 2>(p, small, stream);
-  return LaunchColumnT<T, 1>(p, small, stream);
+  if (slots == 4) return small ? LaunchColumnT<T, 4, 256>(p, stream) : LaunchColumnT<T, 4, 1024>(p, stream);
+  if (slots == 2) return small ? LaunchColumnT<T, 2, 256>(p, stream) : LaunchColumnT<T, 2, 1024>(p, stream);
+  return small ? LaunchColumnT<T, 1, 256>(p, stream) : LaunchColumnT<T, 1, 1024>(p, stream);
+}
+template <typename T, int MT>
+hipError_t LaunchRingOT(const RingParams& p, bool turn, hipStream_t stream) {
+  const dim3 grid(DivUp(p.ns, 16), DivUp(p.m, MT), p.rows), block(256);
+  if (turn && p.has_zero_point)
+    hipLaunchKernelGGL((fc_w8_ring_o_turn_kernel<T, MT, true>), grid, block, 0, stream, p);
+  else if (turn)
+    hipLaunchKernelGGL((fc_w8_ring_o_turn_kernel<T, MT, false>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, MT>), grid, block, 0, stream, p);
+  return hipGetLastError();
 }
 template <typename T>
-hipError_t LaunchRingO(const RingParams& p, int slots, hipStream_t stream) {
-  const dim3 grid(DivUp(p.ns, 16), DivUp(p.m, slots), p.rows), block(256);
-  if (slots == 4)
-    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, 4>), grid, block, 0, stream, p);
-  else if (slots == 2)
-    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, 2>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((fc_w8_ring_o_kernel<T, 1>), grid, block, 0, stream, p);
-  return hipGetLastError();
+hipError_t LaunchRingO(const RingParams& p, int slots, bool turn, hipStream_t stream) {
+  if (slots == 4) return LaunchRingOT<T, 4>(p, turn, stream);
+  if (slots == 2) return LaunchRingOT<T, 2>(p, turn, stream);
+  return LaunchRingOT<T, 1>(p, turn, stream);
 }
 
 template <typename T, int LS>
@@ -814,11 +1083,14 @@ hipError_t LaunchFcW8RingO(const FcArgs& a, hipStream_t stream, const char** ker
   if (!FcW8RingOSupported(a)) return hipErrorInvalidValue;
   const RingParams p = MakeRingParams(a);
   if (kernel_name) *kernel_name = "fc_w8_ring_o_kernel";
+  // every channel of the ring is a dst channel (and no runtime bound leaves some out)
+  const bool turn = a.n == a.ring_size && p.dst_end_ch_index < 0;
   // token slots: as ColumnSlots (4 tokens x 8192 positions x 256 channels: 3.6 us with two, 3.9 with four; 8 tokens x 16384 x
-  // 128: 4.2 against 4.1)
-  int slots = (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 4) >= 512 ? 4 : 2;
+  // 128: 4.2 against 4.1; the turn kernel, whose start waits for less, has four ahead from half as many work-groups on: a step of 18
+  // layers of 8 tokens x 8192 x 256, keys and values, 181.4 / 179.0 us)
+  int slots = (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 4) >= (turn ? 256 : 512) ? 4 : 2;
   while (slots > p.m) slots /= 2;
-  return a.act_f16 ? LaunchRingO<__half>(p, slots, stream) : LaunchRingO<float>(p, slots, stream);
+  return a.act_f16 ? LaunchRingO<__half>(p, slots, turn, stream) : LaunchRingO<float>(p, slots, turn, stream);
 }
 
 hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kernel_name) {

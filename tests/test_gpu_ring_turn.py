@@ -1,0 +1,74 @@
+"""GPU parity of the ring kernels where the window is the whole ring (fc_w8_ring_i_turn_kernel, fc_w8_ring_o_turn_kernel): every shift of
+the ring's start against a slice, the last rows of a wave, of a pass of 256 and of 1024 threads and of a second pass, one to several token
+slots with a remainder, matrices of a batch, with and without zero points.  Small whole numbers make every product and sum exact, so
+the results are those of the rolled weights whatever the order of the sums, and those of the unspecialised kernel with an infinite
+activation."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+import mldhip as M
+import workloads as W
+
+SHAPES = [  # axis, ring, other channels, tokens, batch
+    ("i", 4, 8, 1, 1), ("i", 252, 20, 3, 2), ("i", 260, 72, 8, 1), ("i", 2052, 12, 5, 1), ("i", 4104, 260, 6, 1), ("i", 8200, 24, 1, 1),
+    ("i", 16384, 8, 7, 1), ("i", 1024, 1032, 5, 1), ("o", 1024, 256, 1, 1), ("o", 1000, 70, 3, 2), ("o", 8200, 64, 9, 1), ("o", 68, 1030, 6, 1)]
+
+
+@pytest.mark.parametrize("axis,ring,other,tokens,batch", SHAPES)
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("zero_point", [True, False])
+def test_ring_turn(axis, ring, other, tokens, batch, f16, zero_point):
+    import torch
+    td, mt = (torch.float16, M.FLOAT16) if f16 else (torch.float32, M.FLOAT32)
+    rng = np.random.default_rng(ring + other)
+    src_c, dst_c = (ring, other) if axis == "i" else (other, ring)
+    shape = (dst_c, batch, 1, ring) if axis == "i" else (ring, batch, 1, src_c)
+    q = rng.integers(-3, 4, size=shape, dtype=np.int8)
+    q[0, 0, 0, 0], q[-1, -1, 0, -1] = 127, -127
+    desc = M.make_desc(M.UINT8, M.LAYOUT_I4O4 if axis == "i" else M.LAYOUT_O4I4, (shape[0] + 3) // 4)
+    packed = torch.from_numpy(M.rearrange_int8_as_uint8(q, desc)).cuda()
+    # activations of -1, 0 and 1 in 60 channels: sums of at most 60 * 6 + 2 * 131, whole numbers that fp16 holds
+    act = np.zeros((batch * tokens, src_c))
+    for a in act:
+        a[rng.integers(0, src_c, size=60)] = rng.integers(-1, 2, size=60)
+        a[0], a[-1] = 1, 1
+    ns = (dst_c + 3) // 4
+    zp = rng.integers(-3, 4, size=dst_c) if zero_point else np.zeros(dst_c, np.int64)
+    kw = {"ring_%s_offset_index" % axis: 0, "ring_size": ring, ("src" if axis == "i" else "dst") + "_channels": ring}
+    if batch > 1:
+        kw["weights_batch"] = batch
+    op = M.fc_create(M.PRECISION_F32_F16 if f16 else M.PRECISION_F32, mt, mt, shape[0], shape[3], desc, scale_shape=(dst_c, 1),
+                     max_tokens=batch * tokens, has_zero_point_tensor=zero_point, **kw)
+    d_act = torch.from_numpy(W.to_slices(act)).to(td).cuda()
+    params = torch.zeros(1, dtype=torch.int32, device="cuda")
+    srcs = [d_act] + ([torch.arange(batch, dtype=torch.int32, device="cuda")] if batch > 1 else []) + [packed]
+    srcs.append(torch.ones(batch * ns * 4, dtype=td, device="cuda"))
+    if zero_point:
+        srcs.append(torch.from_numpy(np.tile(np.pad(zp, (0, ns * 4 - dst_c)), batch)).to(td).cuda())
+    srcs.append(params)
+
+    def launch(off, generic=0):
+        out = torch.full((ns, batch * tokens, 4), 7.0, dtype=td, device="cuda")
+        op.bind(srcs, [out])
+        op.set_shape(1, batch, tokens)
+        params.fill_(off)
+        print("ring turn", axis, ring, other, "tokens", tokens, "batch", batch, "offset", off, f16, zero_point, flush=True)
+        with M.tuning(force_generic=generic):
+            op.launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert op.kernel_name == ("fc_generic_kernel" if generic else "fc_w8_ring_%s_kernel" % axis)
+        return W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
+
+    for off in (0, 1, 2, 3, ring - 1, ring - 3, ring // 2 + 1, -6):
+        got = launch(off)
+        for b in range(batch):
+            w = q[:, b, 0].astype(np.int64)
+            w = np.roll(w, -off, axis=1 if axis == "i" else 0) - zp[:, None]
+            want = act[b * tokens:(b + 1) * tokens] @ w.T
+            assert np.array_equal(got[b * tokens:(b + 1) * tokens], want), (off, b)
+    d_act[0, 0, 1] = float("inf")
+    d_act[-1, -1, (src_c - 1) % 4] = -float("inf")
+    got, ref = launch(ring // 3), launch(ring // 3, generic=1)
+    assert np.isinf(ref).any() and np.array_equal(got, ref, equal_nan=True)
