@@ -1666,7 +1666,7 @@ __global__ __launch_bounds__(64) void fc_w4_splitk_reduce_kernel(GemmParams p) {
 // lane-constant shift, mask and exponent), which costs L1 bandwidth, not HBM.  A lane holds one
 // token of whole 4-channel slices at the end: one 8-byte store.  Weights are dequantized as in the kernel
 // above (round_fp16((u - 8) * s)): the matrix cores never see the 1024 + u of the unpacking, whose product with a large activation
-// would leave its rounding in channels where the weight is zero.  kSkinnySteps steps of 32 input channels are in flight per wave; the
+// would leave its rounding in channels where the weight is zero.  Up to kSkinnySteps steps of 32 input channels are in flight per wave; the
 // activations' descriptor ends with the wave's share of K, so steps past it add zeros.
 // Bound: first-load latency and the launch for layers of 2048 channels, then the vector ALU's unpacking.
 // Against 32-token tiles of 128 channels (24 work-groups for the q/k/v projections of 2048 channels), in a step
@@ -1684,7 +1684,10 @@ template <int T, int FT, bool ZP, bool MULTI>
 __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(GemmParams p) {
   typedef float float4v_t __attribute__((ext_vector_type(4)));
   constexpr int Q = 4 / T;  // rows per slice; tiles per strip of 16 slices
-  constexpr int U = FT == 1 ? kSkinnySteps : kSkinnySteps / 2;  // (registers)
+  // Steps in flight per wave.  In 64-channel tiles the stream of weights holds back the issue of loads (1 .. 4.7 us for 8 steps of the
+  // gate/up pair of 2048 -> 16384), and with half of them a wave multiplies its first steps meanwhile: 18 layers at 8 tokens 601 -> 592 us,
+  // 30 random stacks at 5 .. 16 tokens 1.03 times as fast (2 steps: 597).  Narrower tiles wait for the first load, not for the stream.
+  constexpr int U = T == 4 || FT == 2 ? kSkinnySteps / 2 : kSkinnySteps;
   __shared__ float4 red[kSkinnyWaves][T * FT][64];
 
   asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.group_shift), "s"(p.b_bytes), "s"(p.act), "s"(p.magic_lo), "s"(p.magic_hi),
