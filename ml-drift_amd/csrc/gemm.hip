@@ -833,6 +833,11 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
   const half2_t off_hi = {(_Float16)-72.0f, (_Float16)-72.0f};
   const half2_t off_w8 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
 
+  // uint8: bytes 2 h, 2 h + 1 (output channels) of the words of two input channels, side by side; one more permute puts the exponent
+  // of 1024 above each byte of channel t.  (1.5 instructions per pair of weights; permute and v_or_b32 took 2: 333 x 1656 x 2900 with zero
+  // points 11.19 -> 10.99 us, 14 random launches of 179 .. 3673 tokens 1.02 times as fast.)
+  auto pair_bytes = [](uint32_t w0, uint32_t w1, int h) { return __builtin_amdgcn_perm(w1, w0, h ? 0x07030602u : 0x05010400u); };
+  auto unpack_bytes = [&](uint32_t pair, int t) { return __builtin_amdgcn_perm(magic_lo, pair, (t & 1) ? 0x07030702u : 0x07010700u); };
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -854,6 +859,13 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
         if constexpr (WB == 4) {
           blk = u32x4{wr[0][0], wr[0][1], wr[1][0], wr[1][1]};
           blk8 = u32x4{blk[0] >> 8, blk[1] >> 8, blk[2] >> 8, blk[3] >> 8};
+        }
+        u32x4 pairs[2];
+        if constexpr (WB == 8) {
+  #pragma unroll
+          for (int h = 0; h < 2; ++h)
+  #pragma unroll
+            for (int wd = 0; wd < 4; ++wd) pairs[h][wd] = pair_bytes(wr[wd >> 1][2 * (wd & 1)], wr[wd >> 1][2 * (wd & 1) + 1], h);
         }
         const half2_t sc01 = AsHalf2(scr[0]), sc23 = AsHalf2(scr[1]);
         half2_t zp01 = {(_Float16)0.0f, (_Float16)0.0f}, zp23 = zp01;
@@ -886,9 +898,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
           for (int wd = 0; wd < 4; ++wd) {
             uint32_t bits;
             if constexpr (WB == 8) {
-              // bytes t4 of the words of input channels 2*wd, 2*wd + 1 -> the low bytes of two halfs
-              const uint32_t sel = 0x0c000c00u | (uint32_t)t4 | ((uint32_t)(4 + t4) << 16);
-              bits = __builtin_amdgcn_perm(wr[wd >> 1][2 * (wd & 1) + 1], wr[wd >> 1][2 * (wd & 1)], sel) | magic_lo;
+              bits = unpack_bytes(pairs[t4 >> 1][wd], t4);
             } else {
               const uint32_t x = (t4 & 2) ? blk8[wd] : blk[wd];
               bits = (t4 & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo);
@@ -925,8 +935,8 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
     // 512 x 4096 x 4096 20.0 -> 19.6, 8192 x 4096 x 14336 765 -> 744.  (The two last gain less than the cycles say: under dense MFMA work
     // on random data the clock gives way, 1.4 GHz in the loop of 128-token tiles and 2.4 around it.)
     struct Stage {
-      u32x4 blk, blk8;   // WB == 4: the stage's 32 weights, and the same shifted by 8 bits
-      wblk_t w0, w1;     // WB == 8: the two blocks
+      u32x4 blk, blk8;  // WB == 4: the stage's 32 weights, and the same shifted by 8 bits; 8: its pairs of bytes, halves 0 and 1
+      wblk_t w0, w1;    // WB == 8: the two blocks
       half2_t sc01, sc23, zp01, zp23;
     };
     auto open_stage = [&](int u) {
@@ -936,6 +946,9 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
       st.blk = st.blk8 = u32x4{0u, 0u, 0u, 0u};
       if constexpr (WB == 4) {
         st.blk = u32x4{rw[u][0][0], rw[u][0][1], rw[u][1][0], rw[u][1][1]};
+      } else {
+  #pragma unroll
+        for (int wd = 0; wd < 4; ++wd) st.blk[wd] = pair_bytes(rw[u][wd >> 1][2 * (wd & 1)], rw[u][wd >> 1][2 * (wd & 1) + 1], 0);
       }
       const u32x2 scr = rsc[u & ~1];
       st.sc01 = AsHalf2(scr[0]);
@@ -947,7 +960,7 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
       }
       return st;
     };
-    constexpr int kOps = WB == 8 ? 4 : 3;      // vector instructions per word of an operand
+    constexpr int kOps = 3;                    // vector instructions per word of an operand: unpack, centre, scale
     constexpr int kPerSlot = FM >= 4 ? 4 : 8;  // dequantization instructions behind one MFMA
     // The operand of one phase on its way: word wd holds input channels 2 wd, 2 wd + 1 of the step's 8.
     struct Operand {
@@ -955,21 +968,14 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
       half2_t mzs;
       u32x4 done;
     };
-    // Instruction `kind` of word wd of the operand of phase t4: unpack (uint8: two instructions), centre, scale.
+    // Instruction `kind` of word wd of the operand of phase t4.
     auto dequant_op = [&](const Stage& st, int t4, int kind, int wd, Operand& o) {
       const half2_t sp = (t4 & 2) ? st.sc23 : st.sc01;
       const half2_t s2 = (t4 & 1) ? __builtin_shufflevector(sp, sp, 1, 1) : __builtin_shufflevector(sp, sp, 0, 0);
       if (kind == 0) {
-        if constexpr (WB == 8) {
-          // bytes t4 of the words of input channels 2*wd, 2*wd + 1 -> the low bytes of two halfs
-          const uint32_t sel = 0x0c000c00u | (uint32_t)t4 | ((uint32_t)(4 + t4) << 16);
-          const wblk_t& wr = (wd >> 1) ? st.w1 : st.w0;
-          o.part[wd] = __builtin_amdgcn_perm(wr[2 * (wd & 1) + 1], wr[2 * (wd & 1)], sel);
-        } else {
-          const uint32_t x = (t4 & 2) ? st.blk8[wd] : st.blk[wd];
-          o.part[wd] = (t4 & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo);
-        }
-      } else if (kind == kOps - 2) {
+        const uint32_t x = (t4 & 2) ? st.blk8[wd] : st.blk[wd];
+        o.part[wd] = WB == 8 ? unpack_bytes(x, t4) : ((t4 & 1) ? ((x & p.mask_hi) | magic_hi) : ((x & p.mask_lo) | magic_lo));
+      } else if (kind == 1) {
         const half2_t off = WB == 8 ? off_w8 : ((t4 & 1) ? off_hi : off_lo);
         o.part[wd] = AsU32(AsHalf2(o.part[wd]) + off);  // exact: u - shift
         // zero point: (u - shift) * s - zp * s in one fused step, so that a fractional zero point
@@ -978,10 +984,8 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
           const half2_t zq = (t4 & 2) ? st.zp23 : st.zp01;
           o.mzs = -(((t4 & 1) ? __builtin_shufflevector(zq, zq, 1, 1) : __builtin_shufflevector(zq, zq, 0, 0)) * s2);
         }
-      } else if (kind == kOps - 1) {
-        o.done[wd] = AsU32(ZP ? __builtin_elementwise_fma(AsHalf2(o.part[wd]), s2, o.mzs) : AsHalf2(o.part[wd]) * s2);
       } else {
-        o.part[wd] |= magic_lo;
+        o.done[wd] = AsU32(ZP ? __builtin_elementwise_fma(AsHalf2(o.part[wd]), s2, o.mzs) : AsHalf2(o.part[wd]) * s2);
       }
     };
     Stage cur = open_stage(0);
@@ -1019,8 +1023,17 @@ __global__ __launch_bounds__(WAVES * 64, FM == 4 ? 1 : 2) void fc_w4_mfma_direct
             }
             // what else a step has to do, each when its registers are free: behind the last MFMA of a phase
             if (fm == FM - 1) {
-              if (t4 == 0 && WB == 4) cur.blk8 = u32x4{cur.blk[0] >> 8, cur.blk[1] >> 8, cur.blk[2] >> 8, cur.blk[3] >> 8};
-              if (t4 == (WB == 8 ? 3 : 1)) load_weights(u);
+              if (t4 == 0) {
+  #pragma unroll
+                for (int wd = 0; wd < 4; ++wd) {
+                  if constexpr (WB == 8)
+                    cur.blk8[wd] = pair_bytes(wd < 2 ? cur.w0[2 * (wd & 1)] : cur.w1[2 * (wd & 1)],
+                                              wd < 2 ? cur.w0[2 * (wd & 1) + 1] : cur.w1[2 * (wd & 1) + 1], 1);
+                  else
+                    cur.blk8[wd] = cur.blk[wd] >> 8;
+                }
+              }
+              if (t4 == 1) load_weights(u);
               if (t4 == 2 && PAIR) {
                 // The two 16-byte loads of a token pair hold {token 2j, token 2j+1} of K-slice rows 2q
                 // and 2q+1; exchanging the inner halves makes each of them one token's operand.
