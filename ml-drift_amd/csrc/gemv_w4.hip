@@ -110,10 +110,30 @@ __device__ __forceinline__ void StoreHalf(__half* dst, size_t i, float r, const 
 // this launch row in it (M and 0 unless the launch has batched weights).
 // wcol: the lane's column of the packed weights (K-slice row 0), rstride: uint4 per K-slice row.
 // ks_live: K-slices that count (p.ks, or fewer under a runtime bound): activations from there on read as zero.
+// whole_rows (one token, alone in its tensor, K-slices in whole chunks): a chunk's activations are 64 contiguous bytes, 16-byte aligned
+// as the tensor is, and nothing is masked: four loads instead of eight, all before the weights.  With the masked form alone, the compiled
+// loop waits for each row of the next chunk before it requests the row behind it, a chain of eight latencies where K takes a
+// second step; beside this form it no longer does, in either.  Batched grouped launches only: their kernels keep three waves a SIMD
+// (130 .. 139 -> 136 .. 143 registers), the others would lose one of four or spill, and a decode step of 18 layers gained nothing
+// (402.7 / 402.4 us).  (us, before / after: three launches a layer, 8 of 128 matrices 2048 x 768 and 768 x 2048, six layers, 87.0 / 83.4;
+// K of 2880, 4 of 128, four layers 88.1 / 62.3; 28 random stacks, K of 512 .. 4032: 1.06 times as fast
+// in the geometric mean.)
 template <int M>
 __device__ __forceinline__ void LoadChunk(const StreamParams& p, const u32x4* wcol, int rstride, int c,
-                                          u32x4 w[8], u32x2 a[8][M], int ks_live, int act_stride = M, int act_tok0 = 0) {
+                                          u32x4 w[8], u32x2 a[8][M], int ks_live, int act_stride = M, int act_tok0 = 0,
+                                          bool whole_rows = false) {
   const int ks0 = c * 8;
+  if (M == 1 && whole_rows) {
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(p.act + (size_t)(ks0 + j) * 4);
+      a[j][0] = u32x2{v[0], v[1]};
+      a[j + 1][0] = u32x2{v[2], v[3]};
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = __builtin_nontemporal_load(wcol + (size_t)(ks0 + j) * rstride);
+    return;
+  }
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int ks = ks0 + j;
@@ -312,7 +332,8 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
   u32x4 w[8];
   u32x2 a[8][M];
   if (c < c_end) {
-    LoadChunk<M>(p, wcol, rstride, c, w, a, ks_live, act_stride, act_tok0);
+    const bool whole_rows = BATCHED && GROUPED && M == 1 && act_stride == 1 && (p.ks & 7) == 0 && ks_live == p.ks;
+    LoadChunk<M>(p, wcol, rstride, c, w, a, ks_live, act_stride, act_tok0, whole_rows);
     while (true) {
       const int cn = c + ROWS;
       const bool more = cn < c_end;
@@ -323,7 +344,7 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
         sv = *reinterpret_cast<const u32x4*>(scale_base + (size_t)g * group_stride + (size_t)2 * pcol * 4);
         if (ZP) zv = *reinterpret_cast<const u32x4*>(zp_base + (size_t)g * group_stride + (size_t)2 * pcol * 4);
       }
-      if (more) LoadChunk<M>(p, wcol, rstride, cn, wn, an, ks_live, act_stride, act_tok0);
+      if (more) LoadChunk<M>(p, wcol, rstride, cn, wn, an, ks_live, act_stride, act_tok0, whole_rows);
       float t[M][8], asum[M];
 #pragma unroll
       for (int m = 0; m < M; ++m) {
