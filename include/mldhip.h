@@ -504,6 +504,9 @@ const char* mldhip_op_kernel_variant(const mldhip_op* op);
 /* How the last launch was cut where that kernel is the "direct" form: tokens of a tile, waves of a work-group, parts of K
  * between work-groups; else zeros.  For tests. */
 int mldhip_op_kernel_tiles(const mldhip_op* op, int* tokens, int* waves, int* k_parts);
+/* 1 where the last launch took the form of its kernel that counts on a whole extent, else 0: under the ring kernels' names a window that
+ * is the whole ring (the turn kernels), under fc_w4_stream_kernel batched matrices that all read one token.  For tests. */
+int mldhip_op_kernel_whole(const mldhip_op* op);
 int mldhip_op_cost(const mldhip_op* op, uint64_t* bytes, uint64_t* flops);
 
 void mldhip_op_destroy(mldhip_op* op);

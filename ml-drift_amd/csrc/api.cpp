@@ -108,6 +108,7 @@ struct mldhip_op {
   const char* last_kernel = "";
   const char* last_variant = "";  // the form of that kernel
   int last_tiles[3] = {0, 0, 0};  // and how its work was cut
+  int last_whole = 0;             // and whether its form counts on a whole extent
   // bytes every object needs at the current shape (kept up to date by create and set_shape, so that
   // a launch checks its bindings without touching the heap)
   std::vector<size_t> need_src, need_dst;
@@ -749,6 +750,8 @@ static int BuildFcArgs(mldhip_op* op, FcArgs* out) {
   a.variant = &op->last_variant;
   std::fill_n(op->last_tiles, 3, 0);
   a.tiles = op->last_tiles;
+  op->last_whole = 0;
+  a.whole = &op->last_whole;
   if (op->idx_params >= 0) {
     a.params = static_cast<const int32_t*>(op->src_ptr[op->idx_params]);
     a.src_end_ch_index = d.src_end_ch_index;
@@ -1002,6 +1005,8 @@ int mldhip_op_kernel_tiles(const mldhip_op* op, int* tokens, int* waves, int* k_
   *k_parts = op->last_tiles[2];
   return MLDHIP_OK;
 }
+
+int mldhip_op_kernel_whole(const mldhip_op* op) { return op ? op->last_whole : 0; }
 
 int mldhip_op_cost(const mldhip_op* op, uint64_t* bytes, uint64_t* flops) {
   if (!op) return Fail(MLDHIP_INVALID_ARGUMENT, "null op");

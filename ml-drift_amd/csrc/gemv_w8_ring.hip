@@ -875,16 +875,15 @@ __global__ __launch_bounds__(256) void fc_w8_ring_o_turn_kernel(RingParams p) {
   if (ZP && RingSumInfinite(as)) RingStore<T>(p, n, o, channel.s * RingSumByProducts<T, true>(row, tok0 + t_out, n, channel.z));
 }
 
-// A window that is the whole ring and that no runtime bound cuts.
-bool WholeTurn(const RingParams& p) { return p.src_end_ch_index < 0 && p.k_channels == p.ring_size; }
+// A window that is the whole ring and that no runtime bound cuts (the turn kernel knows none).
+bool ColumnTurns(const RingParams& p) { return p.src_end_ch_index < 0 && p.dst_end_ch_index < 0 && p.k_channels == p.ring_size; }
 
 template <typename T, int MT, int THREADS>
 hipError_t LaunchColumnT(const RingParams& p, hipStream_t stream) {
   const dim3 grid(DivUp(p.ns, 64) * 64, DivUp(p.m, MT), p.rows), block(THREADS);
-  // (the turn kernel knows no bound of the dst channels)
-  if (WholeTurn(p) && p.dst_end_ch_index < 0 && p.has_zero_point)
+  if (ColumnTurns(p) && p.has_zero_point)
     hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, true>), grid, block, 0, stream, p);
-  else if (WholeTurn(p) && p.dst_end_ch_index < 0)
+  else if (ColumnTurns(p))
     hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, false>), grid, block, 0, stream, p);
   else
     hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, THREADS>), grid, block, 0, stream, p);
@@ -1085,6 +1084,7 @@ hipError_t LaunchFcW8RingO(const FcArgs& a, hipStream_t stream, const char** ker
   if (kernel_name) *kernel_name = "fc_w8_ring_o_kernel";
   // every channel of the ring is a dst channel (and no runtime bound leaves some out)
   const bool turn = a.n == a.ring_size && p.dst_end_ch_index < 0;
+  SetWhole(a.whole, turn);
   // token slots: as ColumnSlots (4 tokens x 8192 positions x 256 channels: 3.6 us with two, 3.9 with four; 8 tokens x 16384 x
   // 128: 4.2 against 4.1; the turn kernel, whose start waits for less, has four ahead from half as many work-groups on: a step of 18
   // layers of 8 tokens x 8192 x 256, keys and values, 181.4 / 179.0 us)
@@ -1103,6 +1103,7 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
     p.xcd_runs = std::min(8, DivUp(p.ns, 8));
     p.xcd_mask = p.xcd_runs == 1 ? 7 : (p.xcd_runs == 2 ? 3 : (p.xcd_runs <= 4 ? 1 : 0));
     SetVariant(a.variant, "column");
+    SetWhole(a.whole, ColumnTurns(p));
     return a.act_f16 ? LaunchColumn<__half>(p, slots, small, stream) : LaunchColumn<float>(p, slots, small, stream);
   }
   SetVariant(a.variant, "split");

@@ -57,6 +57,9 @@ __host__ __device__ inline int DstEndSlice(int end_ch, int ns) {
 inline void SetVariant(const char** variant, const char* name) {
   if (variant) *variant = name;
 }
+inline void SetWhole(int* whole, bool value) {
+  if (whole) *whole = value;
+}
 
 // One FullyConnected launch.  Tensors are slice-major: act [Ks][m][4], dst [Ns][m][4].
 struct FcArgs {
@@ -102,6 +105,7 @@ struct FcArgs {
   int weights_k = 0;  // input channels of the weights buffer (ring_i); 0 = k
   const char** variant = nullptr;  // out: the form of the kernel that was launched (mldhip_op_kernel_variant)
   int* tiles = nullptr;            // out: tokens of a tile, waves, parts of K (mldhip_op_kernel_tiles)
+  int* whole = nullptr;            // out: 1 where the kernel's form counts on a whole extent (mldhip_op_kernel_whole)
 };
 
 // Split-K workspace sizing for the streaming GEMV.

@@ -30,7 +30,7 @@ SYMBOLS = [
     "mldhip_quantization_create", "mldhip_conv_int8_src_type", "mldhip_conv_int8_create",
     "mldhip_op_src_count", "mldhip_op_dst_count", "mldhip_op_src_name", "mldhip_op_dst_name",
     "mldhip_op_set_src", "mldhip_op_set_dst", "mldhip_op_set_shape", "mldhip_op_launch",
-    "mldhip_op_kernel_name", "mldhip_op_kernel_variant", "mldhip_op_kernel_tiles", "mldhip_op_cost", "mldhip_op_destroy", "mldhip_fc_launch_fused",
+    "mldhip_op_kernel_name", "mldhip_op_kernel_variant", "mldhip_op_kernel_tiles", "mldhip_op_kernel_whole", "mldhip_op_cost", "mldhip_op_destroy", "mldhip_fc_launch_fused",
     "mldhip_checkpoint_fc_probe", "mldhip_checkpoint_fc_read", "mldhip_fc_launch_gated",
     "mldhip_scale_to_tensor_batched", "mldhip_fc_batch_ids_create",
     "mldhip_fc_int4_weights_desc_reference", "mldhip_fc_int4_weights_desc_decode", "mldhip_fc_int8_weights_desc_decode", "mldhip_set_tuning", "mldhip_fc_int4_decode_noalloc",
@@ -107,6 +107,7 @@ def lib():
         _lib.mldhip_op_kernel_name.restype = C.c_char_p
         _lib.mldhip_op_kernel_variant.restype = C.c_char_p
         _lib.mldhip_op_kernel_variant.argtypes = [C.c_void_p]
+        _lib.mldhip_op_kernel_whole.argtypes = [C.c_void_p]
         _lib.mldhip_op_kernel_tiles.argtypes = [C.c_void_p] + [C.POINTER(C.c_int)] * 3
         _lib.mldhip_op_src_name.argtypes = [C.c_void_p, C.c_int]
         _lib.mldhip_op_dst_name.argtypes = [C.c_void_p, C.c_int]
@@ -385,6 +386,11 @@ class Op:
         t = [C.c_int() for _ in range(3)]
         check(lib().mldhip_op_kernel_tiles(self.handle, *[C.byref(v) for v in t]))
         return tuple(v.value for v in t)
+
+    @property
+    def kernel_whole(self):
+        """True where the last launch took the form that counts on a whole extent (a whole turn of a ring, one token for all matrices)."""
+        return bool(lib().mldhip_op_kernel_whole(self.handle))
 
     def cost(self):
         b, f = C.c_uint64(), C.c_uint64()

@@ -15,7 +15,7 @@ from test_oracle_fc import (batch_ids_float_weights, batch_ids_int8_exact, make_
 FP16_TOL = 2e-2
 
 
-def run_device(c, td, bias=None, max_tokens=None, group=None):
+def run_device(c, td, bias=None, max_tokens=None, group=None, ops=None):
     import torch
     tt = torch.float16 if td == np.float16 else torch.float32
     mt = M.FLOAT16 if td == np.float16 else M.FLOAT32
@@ -52,6 +52,8 @@ def run_device(c, td, bias=None, max_tokens=None, group=None):
     op.set_shape(1, c["rows"], c["row_tokens"])
     op.launch(torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
+    if ops is not None:  # (for tests that look at the form of the kernel)
+        ops.append(op)
     got = W.from_slices(out.cpu().numpy().astype(np.float32), n).reshape(c["rows"], c["row_tokens"], n)
     return got, op.kernel_name
 

@@ -58,7 +58,7 @@ def test_ring_turn(axis, ring, other, tokens, batch, f16, zero_point):
         with M.tuning(force_generic=generic):
             op.launch(torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        assert op.kernel_name == ("fc_generic_kernel" if generic else "fc_w8_ring_%s_kernel" % axis)
+        assert (op.kernel_name, op.kernel_whole) == (("fc_generic_kernel", False) if generic else ("fc_w8_ring_%s_kernel" % axis, True))
         return W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
 
     for off in (0, 1, 2, 3, ring - 1, ring - 3, ring // 2 + 1, -6):
@@ -72,3 +72,61 @@ def test_ring_turn(axis, ring, other, tokens, batch, f16, zero_point):
     d_act[-1, -1, (src_c - 1) % 4] = -float("inf")
     got, ref = launch(ring // 3), launch(ring // 3, generic=1)
     assert np.isinf(ref).any() and np.array_equal(got, ref, equal_nan=True)
+
+
+# Scales, zero points and biases of their own for every channel and matrix (powers of two and whole numbers: sums, products and results
+# stay exact), the ring's start at all four places against a slice: an index that is off by a channel, a slice or a matrix shows.
+# other channels that fill no slice, batches, several token slots with a remainder; a window one slice shorter than the ring and a bound
+# that cuts nothing stay on the kernels for any window.
+@pytest.mark.parametrize("axis,ring,other,tokens,batch", [("i", 1028, 30, 1, 2), ("i", 2064, 22, 3, 1), ("i", 516, 260, 5, 2), ("o", 1028, 260, 1, 2),
+                                                          ("o", 520, 132, 3, 2), ("o", 1036, 68, 6, 1)])
+@pytest.mark.parametrize("f16", [True, False])
+@pytest.mark.parametrize("zero_point", [True, False])
+@pytest.mark.parametrize("bias", [True, False])
+@pytest.mark.parametrize("form", ["whole", "short", "bound"])
+def test_ring_turn_channel_parameters(axis, ring, other, tokens, batch, f16, zero_point, bias, form):
+    import torch
+    td, mt = (torch.float16, M.FLOAT16) if f16 else (torch.float32, M.FLOAT32)
+    rng = np.random.default_rng(ring + other + tokens)
+    window = ring - 4 if form == "short" else ring
+    src_c, dst_c = (window, other) if axis == "i" else (other, window)
+    w_o, w_i = (other, ring) if axis == "i" else (ring, other)
+    q = rng.integers(-3, 4, size=(w_o, batch, 1, w_i), dtype=np.int8)
+    desc = M.make_desc(M.UINT8, M.LAYOUT_I4O4 if axis == "i" else M.LAYOUT_O4I4, (w_o + 3) // 4)
+    # 12 activations of -1 and 1: |sum| at most 12 * 6 (weights less zero points), times a scale of 1/4 .. 4 plus a bias of at most 15
+    act = np.zeros((batch * tokens, src_c))
+    for a in act:
+        a[rng.choice(src_c, 12, replace=False)] = rng.choice([-1, 1], 12)
+    ns = (dst_c + 3) // 4
+    scale = 2.0 ** rng.integers(-2, 3, size=(batch, dst_c))
+    zp = rng.integers(-3, 4, size=(batch, dst_c)) if zero_point else np.zeros((batch, dst_c), np.int64)
+    b = rng.integers(-15, 16, size=dst_c) if bias else np.zeros(dst_c, np.int64)
+    kw = {"ring_%s_offset_index" % axis: 0, "ring_size": ring, ("src" if axis == "i" else "dst") + "_channels": window}
+    if batch > 1:
+        kw["weights_batch"] = batch
+    if form == "bound":
+        kw["dst_end_ch_index"] = 1
+    op = M.fc_create(M.PRECISION_F32_F16 if f16 else M.PRECISION_F32, mt, mt, w_o, w_i, desc, scale_shape=(dst_c, 1), max_tokens=batch * tokens,
+                     has_zero_point_tensor=zero_point, has_bias=bias, **kw)
+    pad = lambda v: torch.from_numpy(np.pad(v, [(0, 0)] * (v.ndim - 1) + [(0, ns * 4 - dst_c)]).astype(np.float32)).to(td).cuda()
+    ids = np.arange(batch)[::-1].astype(np.int32).copy()
+    srcs = [torch.from_numpy(W.to_slices(act)).to(td).cuda()] + ([torch.from_numpy(ids).cuda()] if batch > 1 else [])
+    srcs += [torch.from_numpy(M.rearrange_int8_as_uint8(q, desc)).cuda(), pad(scale)] + ([pad(zp)] if zero_point else []) + ([pad(b)] if bias else [])
+    params = torch.tensor([0, ring + 64], dtype=torch.int32, device="cuda")
+    out = torch.zeros((ns, batch * tokens, 4), dtype=td, device="cuda")
+    op.bind(srcs + [params], [out])
+    op.set_shape(1, batch, tokens)
+    for off in (0, 1, 2, 3, ring - 2):
+        params[0] = off
+        out.fill_(7.0)
+        print("channel parameters", axis, ring, other, "tokens", tokens, "batch", batch, "offset", off, f16, zero_point, bias, form, flush=True)
+        op.launch(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert (op.kernel_name, op.kernel_whole) == ("fc_w8_ring_%s_kernel" % axis, form == "whole")
+        got = W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
+        for r in range(batch):
+            w = np.roll(q[:, ids[r] if batch > 1 else 0, 0].astype(np.int64), -off, axis=1 if axis == "i" else 0)
+            w = w[:, :window] if axis == "i" else w[:window]
+            m = ids[r] if batch > 1 else 0
+            want = (act[r * tokens:(r + 1) * tokens] @ (w - zp[m][:, None]).T) * scale[m] + b
+            assert np.array_equal(got[r * tokens:(r + 1) * tokens], want), (off, r)
