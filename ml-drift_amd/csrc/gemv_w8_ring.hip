@@ -505,10 +505,14 @@ __global__ __launch_bounds__(THREADS) void fc_w8_ring_i_column_kernel(RingParams
 // The same where the window is the whole ring and no runtime bound cuts it.  Then which rows are read does not depend on
 // where the ring starts, only which source slices meet them: row r holds source channels 4 w - sh .. 4 w - sh + 3 with w = r - row0
 // around the ring, whose first part is the slice of row r - 1, around the ring too.  So a thread walks the rows as they lie and
-// requests its weights before the start of the ring is known; the activations follow, and while they and the weights
-// are on their way, scale and bias.  Each of the four shifts has its multiply without selects, and without a zero point the sum
-// of the activations is not needed.  8 tokens x 8192 positions x 256 channels 6.6 -> 6.0 us (profiler figures).  (All activations through LDS,
-// so that nothing but the reads from there waits for the start: 7.2.)
+// requests its weights before the start of the ring is known, and scale and bias with the activations.  Each of the four shifts has a
+// walk of its own, without selects, and without a zero point the sum of the activations is not needed.  8 tokens x 8192 positions x
+// 256 channels 6.0 us (profiler figures; 6.6 in the column kernel; all activations through LDS, so that nothing but the reads
+// from there waits for the start: 7.2).  One jump for the window and not one for every row and token: those were fetches of instructions
+// that nothing had asked for, and took the kernel behind the column kernel where the activations are summed as well or
+// a thread walks more than two rows (fp16, 367 random launches, geometric means of the speed over the column kernel's with a jump per
+// row / one: no zero points, up to 2044 positions 1.06 / 1.10, up to 8192 1.08 / 1.10, more 1.02 / 1.06; zero points 0.99 / 1.04, 1.00 / 1.02,
+// 0.96 / 1.01; fp32 1.11 .. 1.22 / 1.16 .. 1.27 and 1.10 .. 1.17 / 1.15 .. 1.23).
 template <int SH>
 __device__ __forceinline__ void MultiplyShifted(const float (&u)[4][4], const uint32_t* lo, const uint32_t* hi, bool zp, float (&acc)[4],
                                                 float& asum) {
@@ -605,9 +609,27 @@ __device__ __forceinline__ void RingStoreChannelRaw(const RingParams& p, const R
   if (ZP && RingSumInfinite(asum)) store(s * RingSumByProducts<__half, RING_O>(row, token, n, z));
 }
 
+template <typename F>
+__device__ __forceinline__ void WithShift(int sh, F f) {
+  if (sh == 0) f(std::integral_constant<int, 0>());
+  else if (sh == 1) f(std::integral_constant<int, 1>());
+  else if (sh == 2) f(std::integral_constant<int, 2>());
+  else f(std::integral_constant<int, 3>());
+}
+// Token slots with which the kernel below is there for launches with zero points (ColumnTurns)
+template <typename T, int THREADS>
+constexpr bool TurnWithZeroPoint(int slots) { return std::is_same<T, float>::value || THREADS == 256 || slots <= 2; }
+
+// Token slots with which 1024 threads of the kernel below come in two forms: one work-group per CU (ALONE), two.  Where there is no more than one
+// for every CU of an XCD, two of them are put on one CU all the same where they fit: fp32, 11 tokens x 7172 positions x 16 channels 6.2 us,
+// alone 4.9.  Where there are more, two on a CU hide each other's waits (speed over the column kernel's, geometric means of random
+// launches of 1.25 .. 2 per CU: two fp32 tokens 1.22, alone 1.07; four fp16 tokens 1.27 and 1.15).
+template <typename T, int THREADS>
+constexpr bool TurnAloneOrNot(int slots) { return THREADS == 1024 && sizeof(T) * slots == 8; }
+
 // (MT as in the column kernel; work-groups are dealt to the XCDs as there)
-template <typename T, int MT, int THREADS, bool ZP>
-__global__ __launch_bounds__(THREADS) void fc_w8_ring_i_turn_kernel(RingParams p) {
+template <typename T, int MT, int THREADS, bool ZP, bool ALONE = false>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS / 256, ALONE ? THREADS / 256 : 8))) void fc_w8_ring_i_turn_kernel(RingParams p) {
   constexpr int U = 2, WAVES = THREADS / 64, NW = kWordsPerToken<T>;
   constexpr bool RAW = std::is_same<T, __half>::value;  // (RingChannelRaw)
   __shared__ float red[WAVES][MT][5];
@@ -644,47 +666,50 @@ __global__ __launch_bounds__(THREADS) void fc_w8_ring_i_turn_kernel(RingParams p
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[t][c] = 0.0f;
   }
-  for (int base = wave * 64; base < rows; base += THREADS * U) {  // (the same for the whole wave: lanes exchange below)
-    uint32_t first[U][MT * NW], hi[U][MT * NW];
+  // The window, with SH (0 .. 3) for the ring's start against a slice or, where SH is 4, with sh looked at for every row and token
+  auto walk = [&](auto shift) {
+    constexpr int SH = decltype(shift)::value;
+    for (int base = wave * 64; base < rows; base += THREADS * U) {  // (the same for the whole wave: lanes exchange below)
+      uint32_t first[U][MT * NW], hi[U][MT * NW];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int r0 = min(base + u * THREADS, rows - 1);  // (the wave's first row)
-      const int below = r0 - row0 + (r0 > row0 ? -1 : rows - 1);
-      int w = min(r0 + lane, rows - 1) - row0;
-      w = w < 0 ? w + rows : w;
-      LoadTokens<T, MT>(act, (size_t)w * act_stride, hi[u]);
-      LoadTokens<T, MT>(act, (size_t)below * act_stride, first[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (base + u * THREADS + 64 > rows) {  // rows past the ring's last one
-        const bool live = base + u * THREADS + lane < rows;
-#pragma unroll
-        for (int i = 0; i < MT * NW; ++i) hi[u][i] = live ? hi[u][i] : 0u;
+      for (int u = 0; u < U; ++u) {
+        const int r0 = min(base + u * THREADS, rows - 1);  // (the wave's first row)
+        const int below = r0 - row0 + (r0 > row0 ? -1 : rows - 1);
+        int w = min(r0 + lane, rows - 1) - row0;
+        w = w < 0 ? w + rows : w;
+        LoadTokens<T, MT>(act, (size_t)w * act_stride, hi[u]);
+        LoadTokens<T, MT>(act, (size_t)below * act_stride, first[u]);
       }
-      typename RingTypes<T>::centred cu;
-      Centre(blk[u], cu);
-      if (base + THREADS * U < rows) blk[u] = load_row(base + THREADS * U + u * THREADS);
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        uint32_t lo[NW];
-        const uint32_t* ht = hi[u] + t * NW;
-        if (sh == 0) {
-          MultiplyShifted<0>(cu, lo, ht, ZP, acc[t], asum[t]);
-        } else {
-          const bool live = base + u * THREADS + lane < rows;
+      for (int u = 0; u < U; ++u) {
+        const bool live = base + u * THREADS + lane < rows;  // (rows past the ring's last one count as zero)
+        typename RingTypes<T>::centred cu;
+        Centre(blk[u], cu);
 #pragma unroll
-          for (int i = 0; i < NW; ++i) {
-            lo[i] = __builtin_amdgcn_update_dpp(first[u][t * NW + i], ht[i], 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
-            lo[i] = live ? lo[i] : 0u;
-          }
-          if (sh == 1) MultiplyShifted<1>(cu, lo, ht, ZP, acc[t], asum[t]);
-          else if (sh == 2) MultiplyShifted<2>(cu, lo, ht, ZP, acc[t], asum[t]);
-          else MultiplyShifted<3>(cu, lo, ht, ZP, acc[t], asum[t]);
+        for (int t = 0; t < MT; ++t) {
+          auto multiply = [&](auto row_shift) {
+            constexpr int S = decltype(row_shift)::value;
+            uint32_t lo[NW], hv[NW];
+#pragma unroll
+            for (int i = 0; i < NW; ++i) {
+              if (S > 0) {
+                lo[i] = __builtin_amdgcn_update_dpp(first[u][t * NW + i], hi[u][t * NW + i], 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+                lo[i] = live ? lo[i] : 0u;
+              }
+              hv[i] = live ? hi[u][t * NW + i] : 0u;
+            }
+            MultiplyShifted<S>(cu, lo, hv, ZP, acc[t], asum[t]);
+          };
+          if constexpr (SH < 4) multiply(shift);
+          else WithShift(sh, multiply);
         }
+        if (base + THREADS * U < rows) blk[u] = load_row(base + THREADS * U + u * THREADS);
       }
     }
-  }
+  };
+  // (four fp16 tokens: four walks are 73 registers, one work-group of 1024 threads per CU; with a jump for every row and token 61)
+  if constexpr (std::is_same<T, __half>::value && TurnAloneOrNot<T, THREADS>(MT) && !ALONE) walk(std::integral_constant<int, 4>());
+  else WithShift(sh, walk);
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const float v = AddRow16(SwapAdd16(SwapAdd32(acc[t][0], acc[t][2]), SwapAdd32(acc[t][1], acc[t][3])));
@@ -929,25 +954,31 @@ __global__ __launch_bounds__(256) void fc_w8_ring_o_turn_kernel(RingParams p) {
   }
 }
 
-// A window that is the whole ring and that no runtime bound cuts (the turn kernel knows none).
-bool ColumnTurns(const RingParams& p) { return p.src_end_ch_index < 0 && p.dst_end_ch_index < 0 && p.k_channels == p.ring_size; }
-
+// turn: 0: column kernel; 1: turn kernel; 2: turn kernel, one work-group per CU where there is a form for that
 template <typename T, int MT, int THREADS>
-hipError_t LaunchColumnT(const RingParams& p, hipStream_t stream) {
+hipError_t LaunchColumnT(const RingParams& p, int turn, hipStream_t stream) {
   const dim3 grid(DivUp(p.ns, 64) * 64, DivUp(p.m, MT), p.rows), block(THREADS);
-  if (ColumnTurns(p) && p.has_zero_point)
-    hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, true>), grid, block, 0, stream, p);
-  else if (ColumnTurns(p))
-    hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, false>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, THREADS>), grid, block, 0, stream, p);
+  if (turn > 0 && !p.has_zero_point) {
+    if (TurnAloneOrNot<T, THREADS>(MT) && turn == 2)
+      hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, false, TurnAloneOrNot<T, THREADS>(MT)>), grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, false>), grid, block, 0, stream, p);
+    return hipGetLastError();
+  }
+  if constexpr (TurnWithZeroPoint<T, THREADS>(MT)) {
+    if (turn > 0) {
+      hipLaunchKernelGGL((fc_w8_ring_i_turn_kernel<T, MT, THREADS, true>), grid, block, 0, stream, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((fc_w8_ring_i_column_kernel<T, MT, THREADS>), grid, block, 0, stream, p);
   return hipGetLastError();
 }
 template <typename T>
-hipError_t LaunchColumn(const RingParams& p, int slots, bool small, hipStream_t stream) {
-  if (slots == 4) return small ? LaunchColumnT<T, 4, 256>(p, stream) : LaunchColumnT<T, 4, 1024>(p, stream);
-  if (slots == 2) return small ? LaunchColumnT<T, 2, 256>(p, stream) : LaunchColumnT<T, 2, 1024>(p, stream);
-  return small ? LaunchColumnT<T, 1, 256>(p, stream) : LaunchColumnT<T, 1, 1024>(p, stream);
+hipError_t LaunchColumn(const RingParams& p, int slots, bool small, int turn, hipStream_t stream) {
+  if (slots == 4) return small ? LaunchColumnT<T, 4, 256>(p, turn, stream) : LaunchColumnT<T, 4, 1024>(p, turn, stream);
+  if (slots == 2) return small ? LaunchColumnT<T, 2, 256>(p, turn, stream) : LaunchColumnT<T, 2, 1024>(p, turn, stream);
+  return small ? LaunchColumnT<T, 1, 256>(p, turn, stream) : LaunchColumnT<T, 1, 1024>(p, turn, stream);
 }
 template <typename T, int MT>
 hipError_t LaunchRingOT(const RingParams& p, bool turn, hipStream_t stream) {
@@ -1046,20 +1077,23 @@ RingSplit SplitWindow(const FcArgs& a) {
 // within 17 % in nine of ten.  Their choice is slower than what served these launches without the column kernel by more than 10 %
 // in 49 of them (in 1625 if it takes them all).
 double RingMegabytes(const FcArgs& a) { return 16e-6 * a.rows * DivUp(a.n, 4) * RingWindow(a); }
+// work-groups per CU of the busiest XCD, as the column and the turn kernel deal them
+double ColumnGroupsPerCu(const FcArgs& a, int slots, bool small) {
+  const int ns = DivUp(a.n, 4), runs = std::min(8, DivUp(ns, 8)), copies = runs == 1 ? 8 : (runs == 2 ? 4 : (runs <= 4 ? 2 : 1));
+  const long planes = (long)DivUp(a.m, slots) * a.rows, together = small ? 32 : 8;
+  const long shared = planes <= together ? planes : std::max(together, (planes + copies - 1) / copies);
+  return (ns / 64 * 8 + std::min(8, ns % 64)) * (double)shared / 32.0;
+}
 double ColumnUs(const FcArgs& a) {
   struct Cost {
     double pass, row, act, group;  // per pass of 1024 threads; per 1000 rows: weights, activations; per work-group of 1024 threads
   };
   static const Cost kCost[2][3] = {{{1.5, 1.4, 0.82, 0.18}, {1.8, 1.2, 0.83, 0.46}, {4.3, 1.5, 0.68, 1.1}},   // fp16: 1, 2, 4 slots
                                    {{1.7, 1.2, 0.65, 0.49}, {2.6, 1.2, 0.72, 1.2}, {8.5, 2.0, 0.49, 2.9}}};  // fp32
-  const int ns = DivUp(a.n, 4), window = RingWindow(a), slots = ColumnSlots(a);
+  const int window = RingWindow(a), slots = ColumnSlots(a);
   const bool small = window <= 512;
   const Cost& c = kCost[a.act_f16 ? 0 : 1][slots == 1 ? 0 : (slots == 2 ? 1 : 2)];
-  // work-groups of the busiest XCD, as the kernel deals them
-  const int runs = std::min(8, DivUp(ns, 8)), copies = runs == 1 ? 8 : (runs == 2 ? 4 : (runs <= 4 ? 2 : 1));
-  const long planes = (long)DivUp(a.m, slots) * a.rows, together = small ? 32 : 8;
-  const long shared = planes <= together ? planes : std::max(together, (planes + copies - 1) / copies);
-  const double cus = (ns / 64 * 8 + std::min(8, ns % 64)) * (double)shared / 32.0;  // work-groups per CU
+  const double cus = ColumnGroupsPerCu(a, slots, small);
   const double lines = std::min(1.0, a.src_rows * (double)a.m * (a.act_f16 ? 8 : 16) / 128.0);  // lines that a row's activations touch
   const double chain = small ? 0.0 : std::max(1.0, std::ceil(cus / 2.0)) * DivUp(window, 2048) * c.pass;
   const double work = cus * (window * (c.row + c.act * lines) / 1000.0 + c.group * (small ? 0.31 : 1.0));
@@ -1080,6 +1114,18 @@ double SplitUs(const FcArgs& a) {
 double UnspecialisedUs(const FcArgs& a) {
   const double groups = (double)DivUp(DivUp(a.n, 4), 16) * DivUp(a.m, 4) * a.rows, steps = DivUp(a.k, 64);
   return 5.9 + std::hypot(0.74 * steps, groups / 256 * (0.47 * steps + 1.1)) + 0.24 * RingMegabytes(a);
+}
+// Whether the turn kernel takes a launch from the column kernel: the window is the whole ring and no runtime bound cuts it.  With zero points the
+// activations are summed as in the column kernel, and what is left is the earlier start and the selects.  fp16 (random launches, speed over
+// the column kernel's, geometric mean and least): a thread's two rows cover the ring 1.03, 0.93; more rows 1.01, 0.94; four slots of 1024 threads
+// 1.00, 0.90: there it is ahead only where the ring starts on a whole slice.  fp32 1.05 .. 1.5, but with two slots 1024 threads are 67
+// registers each, 58 in the column kernel: one work-group per CU instead of two; at 1.25 of them per CU still 1.05 .. 1.08, from 1.5 on 0.98, 0.87.
+bool ColumnTurns(const FcArgs& a, int slots, bool small) {
+  if (a.k != a.ring_size || a.src_end_ch_index >= 0 || a.dst_end_ch_index >= 0) return false;
+  if (!a.has_zero_point) return true;
+  if (a.act_f16)
+    return (small ? TurnWithZeroPoint<__half, 256>(slots) : TurnWithZeroPoint<__half, 1024>(slots)) && a.ring_size / 4 <= (small ? 512 : 2048);
+  return slots != 2 || small || ColumnGroupsPerCu(a, slots, small) <= 1.25;
 }
 // (longer windows were not measured in columns, but at 8192 rows x 256 channels and one token: 12.1 us, 8.8 split)
 bool ColumnMeasured(const FcArgs& a) { return RingWindow(a) <= (a.m == 1 ? 4097 : 8193); }
@@ -1157,8 +1203,9 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
     p.xcd_runs = std::min(8, DivUp(p.ns, 8));
     p.xcd_mask = p.xcd_runs == 1 ? 7 : (p.xcd_runs == 2 ? 3 : (p.xcd_runs <= 4 ? 1 : 0));
     SetVariant(a.variant, "column");
-    SetWhole(a.whole, ColumnTurns(p));
-    return a.act_f16 ? LaunchColumn<__half>(p, slots, small, stream) : LaunchColumn<float>(p, slots, small, stream);
+    const int turn = ColumnTurns(a, slots, small) ? (ColumnGroupsPerCu(a, slots, small) <= 1.0 ? 2 : 1) : 0;
+    SetWhole(a.whole, turn > 0);
+    return a.act_f16 ? LaunchColumn<__half>(p, slots, small, turn, stream) : LaunchColumn<float>(p, slots, small, turn, stream);
   }
   SetVariant(a.variant, "split");
   const RingSplit split = SplitWindow(a);

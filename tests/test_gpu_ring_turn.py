@@ -1,6 +1,7 @@
 """GPU parity of the ring kernels where the window is the whole ring (fc_w8_ring_i_turn_kernel, fc_w8_ring_o_turn_kernel): every shift of
 the ring's start against a slice, the last rows of a wave, of a pass of 256 and of 1024 threads and of a second pass, one to several token
-slots with a remainder, matrices of a batch, with and without zero points.  Small whole numbers make every product and sum exact, so
+slots with a remainder, matrices of a batch, with and without zero points, where the sums of the activations leave some launches to the kernel for any window; one
+work-group of 1024 threads per CU and two.  Small whole numbers make every product and sum exact, so
 the results are those of the rolled weights whatever the order of the sums, and those of the unspecialised kernel with an infinite
 activation."""
 import numpy as np
@@ -13,7 +14,24 @@ import workloads as W
 
 SHAPES = [  # axis, ring, other channels, tokens, batch
     ("i", 4, 8, 1, 1), ("i", 252, 20, 3, 2), ("i", 260, 72, 8, 1), ("i", 2052, 12, 5, 1), ("i", 4104, 260, 6, 1), ("i", 8200, 24, 1, 1),
-    ("i", 16384, 8, 7, 1), ("i", 1024, 1032, 5, 1), ("o", 1024, 256, 1, 1), ("o", 1000, 70, 3, 2), ("o", 8200, 64, 9, 1), ("o", 68, 1030, 6, 1)]
+    ("i", 16384, 8, 7, 1), ("i", 1024, 1032, 5, 1), ("i", 4104, 260, 10, 1), ("i", 4096, 516, 6, 1), ("i", 2052, 16, 64, 4), ("i", 2052, 256, 12, 1), ("o", 1024, 256, 1, 1), ("o", 1000, 70, 3, 2), ("o", 8200, 64, 9, 1), ("o", 68, 1030, 6, 1)]
+
+
+def turns(axis, ring, other, tokens, rows, f16, zero_point):
+    """Whether a window that is the whole ring runs on a turn kernel."""
+    if axis == "o" or not zero_point:
+        return True
+    ns, small = (other + 3) // 4, ring // 4 + 1 <= 512  # (256 threads instead of 1024)
+    slots = 4 if ns * rows * ((tokens + 3) // 4) >= 256 else 2
+    while slots > tokens:
+        slots //= 2
+    if f16:  # two rows per thread cover the ring
+        return (small or slots <= 2) and ring // 4 <= (512 if small else 2048)
+    # fp32, two slots, 1024 threads: at most 1.25 work-groups for every CU of the busiest XCD
+    runs = min(8, (ns + 7) // 8)
+    planes, copies = (tokens + 1) // 2 * rows, {1: 8, 2: 4, 3: 2, 4: 2}.get(runs, 1)
+    shared = planes if planes <= 8 else max(8, -(-planes // copies))
+    return slots != 2 or small or (ns // 64 * 8 + min(8, ns % 64)) * shared / 32 <= 1.25
 
 
 @pytest.mark.parametrize("axis,ring,other,tokens,batch", SHAPES)
@@ -58,7 +76,8 @@ def test_ring_turn(axis, ring, other, tokens, batch, f16, zero_point):
         with M.tuning(force_generic=generic):
             op.launch(torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        assert (op.kernel_name, op.kernel_whole) == (("fc_generic_kernel", False) if generic else ("fc_w8_ring_%s_kernel" % axis, True))
+        assert (op.kernel_name, op.kernel_whole) == (
+            ("fc_generic_kernel", False) if generic else ("fc_w8_ring_%s_kernel" % axis, turns(axis, ring, other, tokens, batch, f16, zero_point)))
         return W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
 
     for off in (0, 1, 2, 3, ring - 1, ring - 3, ring // 2 + 1, -6):
@@ -122,7 +141,7 @@ def test_ring_turn_channel_parameters(axis, ring, other, tokens, batch, f16, zer
         print("channel parameters", axis, ring, other, "tokens", tokens, "batch", batch, "offset", off, f16, zero_point, bias, form, flush=True)
         op.launch(torch.cuda.current_stream().cuda_stream)
         torch.cuda.synchronize()
-        assert (op.kernel_name, op.kernel_whole) == ("fc_w8_ring_%s_kernel" % axis, form == "whole")
+        assert (op.kernel_name, op.kernel_whole) == ("fc_w8_ring_%s_kernel" % axis, form == "whole" and turns(axis, ring, other, tokens, batch, f16, zero_point))
         got = W.from_slices(out.cpu().numpy().astype(np.float64), dst_c)
         for r in range(batch):
             w = np.roll(q[:, ids[r] if batch > 1 else 0, 0].astype(np.int64), -off, axis=1 if axis == "i" else 0)
@@ -130,3 +149,13 @@ def test_ring_turn_channel_parameters(axis, ring, other, tokens, batch, f16, zer
             m = ids[r] if batch > 1 else 0
             want = (act[r * tokens:(r + 1) * tokens] @ (w - zp[m][:, None]).T) * scale[m] + b
             assert np.array_equal(got[r * tokens:(r + 1) * tokens], want), (off, r)
+
+
+# Both sides of the lines: rows of a thread's first two, token slots, work-groups per CU
+@pytest.mark.parametrize("ring,channels,tokens,f16,expected", [
+    (2044, 24, 2, True, True), (2048, 24, 2, True, True), (8192, 24, 2, True, True), (8196, 24, 2, True, False), (1024, 1032, 5, True, True),
+    (4096, 1032, 5, True, False), (16384, 24, 1, False, True), (4096, 64, 2, False, True), (4096, 256, 10, False, True),
+    (4096, 256, 12, False, False), (4096, 1032, 5, False, True)])
+def test_ring_turn_lines(ring, channels, tokens, f16, expected):
+    assert turns("i", ring, channels, tokens, 1, f16, True) == expected
+    test_ring_turn("i", ring, channels, tokens, 1, f16, True)
