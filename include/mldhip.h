@@ -501,8 +501,8 @@ const char* mldhip_op_kernel_name(const mldhip_op* op);
  * change): "direct" / "skinny 64x32 k4" (channels x tokens of a work-group, parts of K) / "packed 64x8" (tokens of a tile, waves
  * that share its K) under fc_w4_mfma_gemm_kernel, "column" / "split" under fc_w8_ring_i_kernel; else empty. */
 const char* mldhip_op_kernel_variant(const mldhip_op* op);
-/* How the last launch was cut where that kernel is the "direct" form: tokens of a tile, waves of a work-group, parts of K
- * between work-groups; else zeros.  For tests. */
+/* How the last launch was cut where that kernel is the "direct" form or a ring kernel: tokens of a tile (of a work-group), waves of a
+ * work-group, parts of K (of the window) between work-groups; else zeros.  For tests. */
 int mldhip_op_kernel_tiles(const mldhip_op* op, int* tokens, int* waves, int* k_parts);
 /* 1 where the last launch took the form of its kernel that counts on a whole extent, else 0: under the ring kernels' names a window that
  * is the whole ring (the turn kernels), under fc_w4_stream_kernel batched matrices that all read one token.  For tests. */

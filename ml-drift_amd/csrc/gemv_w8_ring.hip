@@ -1186,10 +1186,13 @@ hipError_t LaunchFcW8RingO(const FcArgs& a, hipStream_t stream, const char** ker
   const bool turn = a.n == a.ring_size && p.dst_end_ch_index < 0;
   SetWhole(a.whole, turn);
   // token slots: as ColumnSlots (4 tokens x 8192 positions x 256 channels: 3.6 us with two, 3.9 with four; 8 tokens x 16384 x
-  // 128: 4.2 against 4.1; the turn kernel, whose start waits for less, has four ahead from half as many work-groups on: a step of 18
-  // layers of 8 tokens x 8192 x 256, keys and values, 181.4 / 179.0 us)
-  int slots = (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 4) >= (turn ? 256 : 512) ? 4 : 2;
+  // 128: 4.2 against 4.1).  The turn kernel, whose start waits for less, has four ahead where two give every CU two work-groups: about half as
+  // many.  (223 random turns of 4 .. 40 tokens with 256 .. 512 work-groups of four slots, speed over the other kernel with four / two slots:
+  // whole fours of tokens or one less 1.11 .. 1.20 / 1.08 .. 1.09; one or two tokens more, where four slots leave two or three empty, below 384
+  // work-groups 1.06 / 1.08 with 0.85 the least, from there on 1.13 / 1.08.)
+  int slots = (turn ? (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 2) : (long)DivUp(p.ns, 16) * p.rows * DivUp(p.m, 4)) >= 512 ? 4 : 2;
   while (slots > p.m) slots /= 2;
+  SetTiles(a.tiles, slots, 4, 1);
   return a.act_f16 ? LaunchRingO<__half>(p, slots, turn, stream) : LaunchRingO<float>(p, slots, turn, stream);
 }
 
@@ -1205,10 +1208,12 @@ hipError_t LaunchFcW8Ring(const FcArgs& a, hipStream_t stream, const char** kern
     SetVariant(a.variant, "column");
     const int turn = ColumnTurns(a, slots, small) ? (ColumnGroupsPerCu(a, slots, small) <= 1.0 ? 2 : 1) : 0;
     SetWhole(a.whole, turn > 0);
+    SetTiles(a.tiles, slots, small ? 4 : 16, 1);
     return a.act_f16 ? LaunchColumn<__half>(p, slots, small, turn, stream) : LaunchColumn<float>(p, slots, small, turn, stream);
   }
   SetVariant(a.variant, "split");
   const RingSplit split = SplitWindow(a);
+  SetTiles(a.tiles, a.m == 1 ? 1 : (a.m == 2 ? 2 : 4), kRingThreads / 64, split.parts);
   const int ls = split.lanes;
   p.parts = split.parts;
   if (a.act_f16) {

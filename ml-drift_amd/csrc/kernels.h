@@ -57,6 +57,12 @@ __host__ __device__ inline int DstEndSlice(int end_ch, int ns) {
 inline void SetVariant(const char** variant, const char* name) {
   if (variant) *variant = name;
 }
+inline void SetTiles(int* tiles, int tokens, int waves, int k_parts) {
+  if (!tiles) return;
+  tiles[0] = tokens;
+  tiles[1] = waves;
+  tiles[2] = k_parts;
+}
 inline void SetWhole(int* whole, bool value) {
   if (whole) *whole = value;
 }

@@ -382,7 +382,7 @@ class Op:
 
     @property
     def kernel_tiles(self):
-        """(tokens of a tile, waves of a work-group, parts of K) of the last launch on the direct GEMM, else zeros."""
+        """(tokens of a tile, waves of a work-group, parts of K) of the last launch on the direct GEMM or a ring kernel, else zeros."""
         t = [C.c_int() for _ in range(3)]
         check(lib().mldhip_op_kernel_tiles(self.handle, *[C.byref(v) for v in t]))
         return tuple(v.value for v in t)

@@ -159,3 +159,29 @@ def test_ring_turn_channel_parameters(axis, ring, other, tokens, batch, f16, zer
 def test_ring_turn_lines(ring, channels, tokens, f16, expected):
     assert turns("i", ring, channels, tokens, 1, f16, True) == expected
     test_ring_turn("i", ring, channels, tokens, 1, f16, True)
+
+
+# Token slots of the keys' kernels: a turn takes four where two give 512 work-groups, a window that is not the whole ring where four do
+@pytest.mark.parametrize("ring,window,tokens,slots", [
+    (8192, 8192, 8, 4), (8188, 8188, 7, 4), (8128, 8128, 8, 2), (10880, 10880, 6, 2), (10944, 10944, 6, 4), (16384, 16384, 4, 4), (16384, 16384, 2, 2),
+    (16320, 16320, 4, 2), (4096, 4096, 1, 1), (16388, 16384, 8, 4), (16324, 16320, 8, 2)])
+def test_ring_o_slots(ring, window, tokens, slots):
+    import torch
+    k, ns, wns = 16, window // 4, ring // 4
+    rng = np.random.default_rng(ring + tokens)
+    q = rng.integers(-3, 4, size=(ring, 1, 1, k), dtype=np.int8)
+    desc = M.make_desc(M.UINT8, M.LAYOUT_O4I4, wns)
+    act = rng.integers(-2, 3, size=(tokens, k)).astype(np.float64)
+    op = M.fc_create(M.PRECISION_F32_F16, M.FLOAT16, M.FLOAT16, ring, k, desc, scale_shape=(window, 1), max_tokens=tokens, ring_o_offset_index=0,
+                     ring_size=ring, dst_channels=window)
+    out = torch.zeros((ns, tokens, 4), dtype=torch.float16, device="cuda")
+    off = ring // 3 + 1
+    op.bind([torch.from_numpy(W.to_slices(act)).half().cuda(), torch.from_numpy(M.rearrange_int8_as_uint8(q, desc)).cuda(),
+             torch.ones(ns * 4, dtype=torch.float16, device="cuda"), torch.tensor([off], dtype=torch.int32, device="cuda")], [out])
+    op.set_shape(1, 1, tokens)
+    print("slots", ring, window, tokens, flush=True)
+    op.launch(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (op.kernel_name, op.kernel_whole, op.kernel_tiles) == ("fc_w8_ring_o_kernel", ring == window, (slots, 4, 1))
+    got = W.from_slices(out.cpu().numpy().astype(np.float64), window)
+    assert np.array_equal(got, act @ np.roll(q[:, 0, 0].astype(np.int64), -off, axis=0)[:window].T)
