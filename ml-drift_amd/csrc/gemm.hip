@@ -1695,7 +1695,7 @@ __global__ __launch_bounds__(64) void fc_w4_splitk_reduce_kernel(GemmParams p) {
 // lane-constant shift, mask and exponent), which costs L1 bandwidth, not HBM.  A lane holds one
 // token of whole 4-channel slices at the end: one 8-byte store.  Weights are dequantized as in the kernel
 // above (round_fp16((u - 8) * s)): the matrix cores never see the 1024 + u of the unpacking, whose product with a large activation
-// would leave its rounding in channels where the weight is zero.  Up to kSkinnySteps steps of 32 input channels are in flight per wave; the
+// would leave its rounding in channels where the weight is zero.  SkinnySteps steps of 32 input channels are in flight per wave; the
 // activations' descriptor ends with the wave's share of K, so steps past it add zeros.
 // Bound: first-load latency and the launch for layers of 2048 channels, then the vector ALU's unpacking.
 // Against 32-token tiles of 128 channels (24 work-groups for the q/k/v projections of 2048 channels), in a step
@@ -1708,15 +1708,17 @@ constexpr int kSkinnySteps = 8;
 constexpr int kSkinnyMaxTokens = 32;        // one token tile
 constexpr int kSkinnyMaxTiledTokens = 384;  // token tiles of 32 along grid.z
 constexpr int kSkinnySplitK = 8192;  // input channels from which K is cut between work-groups
+// Steps in flight per wave.  In 64-channel tiles (T = 4) the stream of weights holds back the issue of loads (1 .. 4.7 us for 8 steps of the
+// gate/up pair of 2048 -> 16384), and with half of them a wave multiplies its first steps meanwhile: 18 layers at 8 tokens 601 -> 592 us,
+// 30 random stacks at 5 .. 16 tokens 1.03 times as fast (2 steps: 597).  Narrower tiles wait for the first load, not for the stream; two token
+// blocks (FT = 2) leave the registers for half.
+constexpr int SkinnySteps(int T, int FT) { return T == 4 || FT == 2 ? kSkinnySteps / 2 : kSkinnySteps; }
 
 template <int T, int FT, bool ZP, bool MULTI>
 __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(GemmParams p) {
   typedef float float4v_t __attribute__((ext_vector_type(4)));
   constexpr int Q = 4 / T;  // rows per slice; tiles per strip of 16 slices
-  // Steps in flight per wave.  In 64-channel tiles the stream of weights holds back the issue of loads (1 .. 4.7 us for 8 steps of the
-  // gate/up pair of 2048 -> 16384), and with half of them a wave multiplies its first steps meanwhile: 18 layers at 8 tokens 601 -> 592 us,
-  // 30 random stacks at 5 .. 16 tokens 1.03 times as fast (2 steps: 597).  Narrower tiles wait for the first load, not for the stream.
-  constexpr int U = T == 4 || FT == 2 ? kSkinnySteps / 2 : kSkinnySteps;
+  constexpr int U = SkinnySteps(T, FT);
   __shared__ float4 red[kSkinnyWaves][T * FT][64];
 
   asm volatile("" : : "s"(p.m), "s"(p.ks), "s"(p.group_shift), "s"(p.b_bytes), "s"(p.act), "s"(p.magic_lo), "s"(p.magic_hi),
@@ -1909,7 +1911,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void fc_w4_mfma_skinny_kernel(Ge
 }
 
 // K split of the kernel for a few tokens.  (16384 -> 2048 channels at 8 tokens: 23 us in 128 tiles of 16 channels
-// without a split, 7.4 + 4.1 us in 32 strips x 8.  2048 channels of K end inside one batch of loads: no split.)
+// without a split, 7.4 + 4.1 us in 32 strips x 8.  2048 channels of K are 8 steps of a wave: no split.)
 int SkinnyKSplit(int k, int n, int token_tiles) {
   if (k < kSkinnySplitK) return 1;
   int s = 1;  // (every wave keeps at least 8 steps)
@@ -1926,8 +1928,10 @@ struct SkinnyPlan {
 // kernel; 16 strips, 32 on each: 4.1 against 6.4).  Us, direct / here: 2048 -> 2048 channels at 64 tokens 8.4 / 5.4, 128
 // 8.4 / 5.7, 256 8.7 / 6.9, 384 9.2 / 10.3 in 384 work-groups; 2048 -> 2560 in three matrices at 128 9.3 / 7.4; 2048 ->
 // 5632 at 64 10.6 / 7.9, 100 10.7 / 11.1 in 352; 5632 -> 2048 at 128 19.2 / 13.4.  Up to 32 tokens, over 280 random launches
-// of more than 256 strips, the direct kernel was 5 to 20 % ahead, except where up to 16 tokens meet a K that fills the one
-// batch of loads (1536..2048 channels), where it was 4 % behind.  More than 384 tokens were not measured.
+// of more than 256 strips, the direct kernel was 5 to 20 % ahead, except where up to 16 tokens meet a K of 6 to 8 steps of a wave
+// (1536..2048 channels), where it was 4 % behind.  That exception was measured with 8 steps in flight in 64-channel tiles, all of such a K, and
+// with the direct kernel's loop of that time; against the loop of today it has no gain left: 65 random launches inside it
+// (1.06 times as fast as then) take 0.91 times their time on the direct kernel in the geometric mean, 0.76..1.18.  More than 384 tokens were not measured.
 // Long K (3471 random launches; direct time / time here, median): up to 32 tokens this kernel is ahead where it is cut at least
 // as often as the direct one (4 and 4 ways 1.20..1.34, 2 and 2 1.23..1.30), else behind (2 against 4 ways 0.91..0.98, whole
 // against 2 ways 0.95 at 17..32 tokens), but for 16 tokens and fewer in whole strips (1.07); two rounds 0.79..0.94 (14336 ->
@@ -1949,13 +1953,14 @@ SkinnyPlan PlanSkinny(int m, int k, int n, int direct_split) {
       if (t == 4 && (m > kSkinnyMaxTokens ? direct_split > 1 : m <= 16 && k <= 512)) return {0, 1};
       return {t, 1};
     }
-  constexpr int kBatch = kSkinnyWaves * kSkinnySteps * 32;  // input channels of one batch of loads
-  return m <= 16 && k <= kBatch && k >= kBatch * 3 / 4 ? SkinnyPlan{4, 1} : SkinnyPlan{0, 1};
+  constexpr int kEightSteps = kSkinnyWaves * 8 * 32;  // input channels of 8 steps of every wave
+  return m <= 16 && k <= kEightSteps && k >= kEightSteps * 3 / 4 ? SkinnyPlan{4, 1} : SkinnyPlan{0, 1};
 }
 
-// The prefetch ends with whole batches of steps in every wave: K-slices up to which offsets are formed.
+// The prefetch ends with whole batches of steps in every wave: K-slices up to which offsets are formed.  (Of the tile with the most
+// steps in flight; 64-channel tiles up to 16 tokens end earlier.)
 bool SkinnyOffsetsFit(const GemmParams& p) {
-  const int unroll = p.m <= 16 ? kSkinnySteps : kSkinnySteps / 2;
+  const int unroll = SkinnySteps(1, p.m <= 16 ? 1 : 2);
   const uint64_t per_slice = (uint64_t)kSkinnyWaves * 8;
   const uint64_t end = ((uint64_t)(p.ksplit - 1) * p.geo_per_wave + (uint64_t)DivUp(p.geo_per_wave, unroll) * unroll) * per_slice;
   const uint64_t past = end > (uint64_t)p.ks ? end - p.ks : 0;

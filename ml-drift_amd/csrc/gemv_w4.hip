@@ -113,7 +113,7 @@ __device__ __forceinline__ void StoreHalf(__half* dst, size_t i, float r, const 
 // whole_rows (one token, alone in its tensor, K-slices in whole chunks): a chunk's activations are 64 contiguous bytes, 16-byte aligned
 // as the tensor is, and nothing is masked: four loads instead of eight, all before the weights.  With the masked form alone, the compiled
 // loop waits for each row of the next chunk before it requests the row behind it, a chain of eight latencies where K takes a
-// second step; beside this form it no longer does, in either.  Batched grouped launches only: their kernels keep three waves a SIMD
+// second step; beside this form it no longer does, in either (what the compiler makes of the two together: no line here asks for it).  Batched grouped launches only: their kernels keep three waves a SIMD
 // (130 .. 139 -> 136 .. 143 registers), the others would lose one of four or spill, and a decode step of 18 layers gained nothing
 // (402.7 / 402.4 us).  (us, before / after: three launches a layer, 8 of 128 matrices 2048 x 768 and 768 x 2048, six layers, 87.0 / 83.4;
 // K of 2880, 4 of 128, four layers 88.1 / 62.3; 28 random stacks, K of 512 .. 4032: 1.06 times as fast
@@ -324,7 +324,8 @@ __global__ __launch_bounds__(WAVES * 64) void fc_w4_stream_kernel(StreamParams p
   // The per-channel scale and the bias of the output this thread writes at the end (output tid % STRIP of the strip, for
   // every token it handles): fetched now, so that their latency does not follow the reduction (behind the weights: 3 % slower
   // over the one-token launches of a mixture of experts).  (Unconditional loads of the raw halfs at a clamped index: a
-  // branch, or a conversion, here would make the kernel wait for them before it issues the weight loads.)
+  // branch, or a conversion, here would make the kernel wait for them before it issues the weight loads.  The compiled whole_rows form of
+  // batched launches waits for the bias in front of its first activations all the same: it is entered by a branch.)
   const int n_out = min(strip * STRIP + tid % STRIP, sg.n_pad - 1);
   const unsigned short* bias_src = reinterpret_cast<const unsigned short*>(sg.bias ? sg.bias : sg.scale);
   const unsigned short out_scale_raw = reinterpret_cast<const unsigned short*>(scale_base)[n_out];

@@ -288,9 +288,9 @@ __global__ __launch_bounds__(256) void fc_w8_ring_finish_kernel(RingParams p) {
 // What bounds it: the dependent launch (1.55 us), then how fast a CU takes pieces that lie in lines of their
 // own: a wave's load of 16-byte blocks a whole row (Ns x 16 bytes) apart touches 64 lines, its load of the
 // activations of two tokens 32.  So the slice below a row's own comes from the neighbouring lane instead
-// of memory and two tokens travel in one load (8 tokens x 8192 positions x 256 channels: 6.4 -> 5.8 us;
-// 74.7 us on the unspecialised kernel that served more than 4 tokens; one token 10.4 us with the window
-// split, 5.0 here).  Neighbouring slices share the lines of the weights, so runs of 8 slices are
+// of memory and two tokens travel in one load (8 tokens x 8192 positions x 256 channels, a ring longer than that: 6.4 -> 5.8 us on
+// one box, 6.6 on the box of the turn kernels' figures below; 74.7 us on the unspecialised kernel that served more than 4 tokens; one
+// token 10.4 us with the window split, 5.0 here).  Neighbouring slices share the lines of the weights, so runs of 8 slices are
 // dealt to one XCD, whose L2 fetches a line once.  A thread owns window rows tid, tid + THREADS, ...; the
 // loads of two rows are in flight per thread, at 1024 threads a cache of 8192 positions at once.
 // ------------------------------------------------------------------------------------------
@@ -751,8 +751,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(THREADS
 // activations, which do not depend on it, go to LDS meanwhile (the 16 lanes of a K-slice read the same
 // 8 or 16 bytes per token), the weights of four K-slices per thread are then in flight at once, and the
 // sums meet by register exchanges inside a wave and through 4 KB of LDS across the waves.  8 tokens x 8192
-// positions x 256 channels, 2.1 MB: 4.0 us (5.3 with the activations from memory and the whole reduction
-// through LDS, 10.1 us on the unspecialised kernel that served it).
+// positions x 256 channels of a longer ring, 2.1 MB: 4.0 us (5.3 with the activations from memory and the whole reduction
+// through LDS, 10.1 us on the unspecialised kernel that served it; 4.5 on the box of the turn kernels' figures below).
 // ------------------------------------------------------------------------------------------
 __device__ __forceinline__ void CentreO(const u32x4& w, float (&u)[4][4]) {
 #pragma unroll
@@ -857,8 +857,8 @@ __global__ __launch_bounds__(256) void fc_w8_ring_o_kernel(RingParams p) {
 
 // The same where every channel of the ring is a dst channel: a work-group takes 64 channels as they lie in the ring, so no
 // address of the weights or activations depends on where the ring starts, only the dst channels that the sums are for.
-// 8 tokens x 8192 positions x 256 channels 4.4 -> 4.0 us (profiler figures; a step of 18 layers, keys and values, 198 -> 179 us.  All kernel
-// arguments in one batch of scalar loads at the top, in both kernels: 190).
+// 8 tokens x 8192 positions x 256 channels 4.5 -> 3.9 us (profiler figures; a step of 18 layers, keys and values, 189 -> 176 us when both kernels
+// were new.  All kernel arguments in one batch of scalar loads at the top, in both: 12 us a step more).
 template <typename T, int MT, bool ZP>
 __global__ __launch_bounds__(256) void fc_w8_ring_o_turn_kernel(RingParams p) {
   constexpr int KL = 16, U = 4, NW = kWordsPerToken<T>, CHUNK = 256;
